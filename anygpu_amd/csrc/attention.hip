@@ -4,8 +4,8 @@
 // three-launch form (q k^T, row softmax, p v) writes and reads 1 GiB of scores twice; this kernel
 // reads q, k, v and writes y.
 //
-// A block of 8 waves owns 128 consecutive queries of one head, 16 per wave (256 and 32 at head
-// dimension 128), so that two waves share a SIMD.  It walks the visible key range in tiles of 64 keys.  Per tile:
+// A block of 8 waves owns 128 consecutive queries of one head, 16 per wave, so that two waves share a SIMD.  It walks the
+// visible key range in tiles of 64 keys.  Per tile:
 //   * K and V rows go global -> LDS directly into two stages; the loads of the next tile are in flight while
 //     this one is being used;
 //   * S^T = K Q^T with v_mfma_f32_16x16x32_f16: the K fragment is the first operand, the Q
@@ -22,9 +22,10 @@
 // slot j <-> key 16 * (2 t + j / 4) + 4 * (lane / 16) + j % 4 of the tile, so no shuffle is needed
 // between the two products.
 //
-// At head dimension 256 a second kernel of the same layout (sdp_attention_fwd_f16_skew_kernel) computes
-// the scores of tile t + 1 beside the softmax of tile t, so that the matrix and the vector instructions of a wave
-// do not depend on each other.
+// This form serves the launches with a mask tensor.  At head dimension 256 without one a second kernel of the same layout
+// (sdp_attention_fwd_f16_skew_kernel) computes the scores of tile t + 1 beside the softmax of tile t, so that the matrix
+// and the vector instructions of a wave do not depend on each other; at 64 and 128 the kernel of attention_f16_q32.hpp has
+// 32 queries per wave.
 //
 // Masks are index rules (causal with the diagonal at n_k - n_q, sliding window); tiles without a
 // visible key are skipped.  A query without any visible key gets zeros.
@@ -930,6 +931,61 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 	}
 }
 
+}  // namespace
+
+}  // namespace anygpu
+
+#include "attention_f16_q32.hpp"
+
+namespace anygpu {
+
+namespace {
+
+template <int D, bool SOFTCAP>
+hipError_t launch_q32(const AttnArgs& args_in, int64_t batch_heads, hipStream_t stream)
+{
+	constexpr int kLdsBytes = 4 * kAttnKeysPerTile * 2 * D;     // two stages of K and V
+	constexpr int kQueriesPerBlock = kQ32QueriesPerBlock;
+	static_assert(kLdsBytes <= 64 * 1024, "the LDS that a launch gets without asking");
+	(void)hipGetLastError();
+	AttnArgs args = args_in;
+	// (masked scores are -inf and meet k_in in a product)
+	if (args.k_in == 0.0f) args.k_in = 1e-30f;
+	const int64_t q_blocks = (args.n_q + kQueriesPerBlock - 1) / kQueriesPerBlock;
+	// The longest blocks in two halves of their key range only under a window, where most blocks are equally long, and where
+	// they make one to two blocks for each CU: up to 1.5 by the plan of the one-block-per-CU kernels (10 / 5 heads x 4096 x 128,
+	// window 1024: 51 -> 47 us); beyond it the rounds are even and a cut gains nothing, so the two-part form that windowed
+	// launches of this size have is left to the latest block of every head (16 / 8 x 4096 x 128, window 1024: 46 us, 58 with all
+	// long ones cut).  Elsewhere two short blocks to a CU even out by themselves, and the partial results' way through
+	// memory costs 8 - 20 % (32 / 8 heads x 3000 x 128 causal 92 -> 100 us).
+	AttnSplitPlan plan{0, 0};
+	const int64_t cus = device_cu_count(), blocks = q_blocks * batch_heads;
+	if (args.window > 0 && blocks > cus && blocks <= 2 * cus)
+	{
+		plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, kQueriesPerBlock,
+		                            kAttnKeysPerTile, D, band::workspace_capacity(stream), blocks * 2 <= cus * 3 ? 0.6 : 0.5);
+		if (blocks * 2 > cus * 3) plan.n_split = std::min<int64_t>(plan.n_split, 1);
+	}
+	// with too few query blocks for the chip, every block in several parts of its key range
+	const int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQueriesPerBlock,
+	                                                                      kAttnKeysPerTile, D, band::workspace_capacity(stream));
+	args.partials = nullptr;
+	if (plan.n_split > 0 || parts_all > 1)
+	{
+		const hipError_t ws_err = band::workspace_acquire(stream, &args.partials);
+		if (ws_err != hipSuccess) return ws_err;
+	}
+	const AttnWalk walk = make_attn_walk(q_blocks, batch_heads, args.q_per_kv, plan.n_split, plan.n_big, parts_all);
+	if (attn_walk_blocks(walk) > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+	sdp_attention_fwd_f16_q32_kernel<D, SOFTCAP><<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * kQ32Waves), kLdsBytes, stream>>>(args, walk);
+	hipError_t err = hipGetLastError();
+	if (err != hipSuccess || walk.n_split == 0) return err;
+	const int64_t items = batch_heads * walk.n_split * kQueriesPerBlock * (D / 4);
+	sdp_attention_merge_halves_kernel<D, half_t><<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream>>>(
+		args.partials, args.y, args.n_q, (int)q_blocks, walk.n_split, kQueriesPerBlock, parts_all > 1 ? (int)parts_all : 2);
+	return hipGetLastError();
+}
+
 // SKEW: the kernel that takes the two halves of a tile's work from different tiles
 template <int D, bool SOFTCAP, int QB, bool SKEW = false, bool MASK = false>
 hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStream_t stream)
@@ -982,26 +1038,17 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 	return hipGetLastError();
 }
 
-// Queries per wave: 16 everywhere (8 waves x 16 queries measured 1.1 - 1.5 x faster than 4 waves x 32: the smaller
-// register footprint lets more waves share a SIMD), except head_dim 128 with enough query blocks to fill the chip,
-// where 8 waves x 32 queries halve the LDS reads per flop and fit the register file (16 x 4096 x 128 causal: 148 us
-// against 172 us).  At head_dim 256 the 32-query form does not fit the registers.
-// The skewed kernel serves head_dim 256 (8 / 4 heads x 8192 x 256 with window 4096, one process: softcap 50
-// 321 -> 276 us, without softcap 277 -> 264 us; 8 heads causal without softcap 381 -> 355 us).  At head_dim 128 and 64 it
-// measured slower than the kernel above (16 x 4096 x 128 causal 128 -> 141 us, 32 x 2048 x 64 causal 45 -> 61 us, before
-// its last tenth), and with 32 queries per wave slower at every head dimension.
+// Head dimensions 64 and 128 take 32 queries per wave and two to three blocks per CU (attention_f16_q32.hpp).  At 256 the accumulators
+// and queries of 32 rows leave that kernel no registers (8 / 4 heads x 8192 x 256, softcap 50, window 4096: 357 us against 300); the
+// skewed kernel serves it (16 queries per wave; the kernel above in one process: softcap 50 321 -> 276 us, without softcap
+// 277 -> 264 us; 8 heads causal without softcap 381 -> 355 us).
 template <int D>
 hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, hipStream_t stream)
 {
-	if constexpr (D == 128)
-	{
-		if (batch_heads * ((args.n_q + 255) / 256) >= 256)
-			return softcap ? launch_variant<D, true, 2>(args, batch_heads, stream) : launch_variant<D, false, 2>(args, batch_heads, stream);
-	}
 	if constexpr (D == 256)
 		return softcap ? launch_variant<D, true, 1, true>(args, batch_heads, stream) : launch_variant<D, false, 1, true>(args, batch_heads, stream);
 	else
-		return softcap ? launch_variant<D, true, 1>(args, batch_heads, stream) : launch_variant<D, false, 1>(args, batch_heads, stream);
+		return softcap ? launch_q32<D, true>(args, batch_heads, stream) : launch_q32<D, false>(args, batch_heads, stream);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -1987,6 +1987,27 @@ def test_sdp_attention_fused_kernel(ops, oracle, case):
     assert rel_l2(got[0], want) <= 2e-3
 
 
+# head dimensions 64 and 128 run 32 queries per wave, four waves and 128 queries per block, tiles of 64 keys: one query and
+# the edges of a wave's and a block's queries, tiles of one key, one short of whole and whole, queries of a wave that see
+# nothing, and the first and last tile of a window that only some waves of a block see
+@pytest.mark.parametrize("n_q,n_k,causal,window", [(1, 65, True, 0), (31, 64, True, 0), (33, 63, False, 0), (127, 129, True, 0), (128, 128, True, 0),
+                                                    (129, 257, True, 70), (160, 100, True, 0), (300, 321, False, 64), (257, 600, True, 1)])
+@pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 0.0, -0.0884), (64, 30.0, 0.0), (128, 50.0, 0.0884)])
+def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, causal, window, d, cap, alpha):
+    heads, kv_heads = 4, 2
+    q = synth.normal(1 + n_q, (1, heads, n_q, d)).astype(np.float16)
+    k = synth.normal(2 + n_k, (1, kv_heads, n_k, d)).astype(np.float16) * np.float16(4.0)        # (scores of tens: the running maximum moves)
+    v = synth.normal(3 + d, (1, kv_heads, n_k, d)).astype(np.float16)
+    got = host(ops.sdp_attention_fwd(dev(q), dev(k), dev(v), alpha, softcap=cap, causal=causal, window=window, decode=False)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=alpha, softcap=cap,
+                                      causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
+    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
+    assert not got[0][blind].any()
+    assert np.isfinite(got).all()
+    # p rounded to fp16 (2^-11 each, weights that sum to 1) and the result's own rounding, values of up to about 4
+    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
+
+
 def _random_attention_cases(count, seed):
     import random
     rnd = random.Random(seed)
