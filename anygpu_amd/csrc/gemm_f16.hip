@@ -467,7 +467,11 @@ hipError_t launch_gemm_f16(const void* A, const void* B, void* C, int64_t M, int
 	const auto done = [&](hipError_t err) { if (finish) finish->handled = true; return err; };
 	if (batch == 1 && b_layout == ANYGPU_B_ROW_MAJOR && !(fin_epi == kEpiBias && fin_bias) && gemm_band_kn_f16_applies(A, B, C, M, N, K, lda, ldb, ldc))
 		return done(launch_gemm_band_kn_f16(A, B, C, M, N, K, lda, ldb, ldc, fin_epi, fin_param, stream));
-	// the same for k-contiguous weights, from three rows on (one and two rows: the skinny kernels): whole 128-byte lines
+	// up to 16 rows against k-contiguous weights: K cut over the waves of a block, one launch
+	if (batch == 1 && gemm_kwave_applies<half_t>(a, b, nullptr, M, N, K, lda, ldb, b_layout, false))
+		return done(launch_gemm_kwave<half_t>(a, b, nullptr, fin_bias, c, M, N, K, lda, ldb, ldc, fin_epi, fin_param, stream));
+	// more rows against k-contiguous weights with the columns of an output head (few rows that the kernel above does not take,
+	// too, from three on; one and two: the skinny kernels): whole 128-byte lines
 	// per weight row and load instruction, an exchange between lane pairs in front of the MFMAs
 	if (batch == 1 && b_layout == ANYGPU_B_COL_MAJOR && M >= 3 && gemm_band_kc_wide_applies<half_t>(a, b, c, M, N, K, lda, ldb, ldc, kWideMaxRowsF16))
 		return done(launch_gemm_band_kc_wide<half_t>(a, b, fin_bias, c, M, N, K, lda, ldb, ldc, fin_epi, fin_param, stream));
@@ -762,6 +766,8 @@ hipError_t launch_gemm_f16_epilogue(const void* A, const void* B, const void* B2
 		const hipError_t err = launch_gemm_f16(A, B, C, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, b_layout, stream, &finish);
 		if (err != hipSuccess || finish.handled) return err;
 	}
+	if (dual && gemm_kwave_applies<half_t>(a, b, b2, M, N, K, lda, ldb, b_layout, true))
+		return launch_gemm_kwave<half_t>(a, b, b2, nullptr, c, M, N, K, lda, ldb, ldc, epilogue, ep_param, stream);
 	if (dual && gemm_band_applies<half_t>(a, b, b2, c, M, N, K, lda, ldb, ldc, b_layout))
 		return launch_gemm_band<half_t>(a, b, b2, nullptr, c, M, N, K, lda, ldb, ldc, epilogue, ep_param, stream);
 	if (!tiles_ok)

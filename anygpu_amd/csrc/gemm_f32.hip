@@ -666,6 +666,9 @@ hipError_t launch_gemm_f32(const float* A, const float* B, const float* bias, fl
 	const int64_t tiles_first_rows = (b_layout == ANYGPU_B_ROW_MAJOR && (double)K * (double)N <= 6.0e6) ? 17 : 33;
 	const bool tiles_first = a_layout == ANYGPU_A_ROW_MAJOR && M >= tiles_first_rows && (b_layout == ANYGPU_B_COL_MAJOR || N <= 65536) &&
 	                         gemm_f32_ring_applies(A, B, M, N, K, lda, ldb, stride_a, stride_b, batch, 0, 64, b_layout);
+	// up to 16 rows against k-contiguous weights: K cut over the waves of a block, one launch
+	if (batch == 1 && a_layout == ANYGPU_A_ROW_MAJOR && gemm_kwave_applies<float>(A, B, nullptr, M, N, K, lda, ldb, b_layout, false))
+		return launch_gemm_kwave<float>(A, B, nullptr, bias, C, M, N, K, lda, ldb, ldc, kEpiBias, 0.0f, stream);
 	// few rows against k-contiguous weights with the columns of an output head: whole lines per row and load instruction
 	if (batch == 1 && a_layout == ANYGPU_A_ROW_MAJOR && b_layout == ANYGPU_B_COL_MAJOR && M >= kWideMinRowsF32 &&
 	    gemm_band_kc_wide_applies<float>(A, B, C, M, N, K, lda, ldb, ldc, kWideMaxRowsF32))
@@ -696,6 +699,8 @@ hipError_t launch_gemm_f32_softcap(const float* A, const float* B, float* C, int
                                    int64_t lda, int64_t ldb, int64_t ldc, int b_layout, float softcap, hipStream_t stream)
 {
 	if (M == 0 || N == 0) return hipSuccess;
+	if (gemm_kwave_applies<float>(A, B, nullptr, M, N, K, lda, ldb, b_layout, false))
+		return launch_gemm_kwave<float>(A, B, nullptr, nullptr, C, M, N, K, lda, ldb, ldc, kEpiSoftcap, softcap, stream);
 	if (b_layout == ANYGPU_B_COL_MAJOR && M >= kWideMinRowsF32 && gemm_band_kc_wide_applies<float>(A, B, C, M, N, K, lda, ldb, ldc, kWideMaxRowsF32))
 		return launch_gemm_band_kc_wide<float>(A, B, nullptr, C, M, N, K, lda, ldb, ldc, kEpiSoftcap, softcap, stream);
 	if (b_layout == ANYGPU_B_COL_MAJOR && M >= kWideMinRowsF32 && gemm_band_kc_wide_split_applies<float>(A, B, C, M, N, K, lda, ldb, ldc, kWideSplitMaxRowsF32, stream))
@@ -792,6 +797,8 @@ hipError_t launch_gemm_f32_gelu_mul(const float* A, const float* B_gate, const f
 			return hipGetLastError();
 		}
 	}
+	if (gemm_kwave_applies<float>(A, B_gate, B_up, M, N, K, lda, ldb, b_layout, true))
+		return launch_gemm_kwave<float>(A, B_gate, B_up, nullptr, C, M, N, K, lda, ldb, ldc, kEpiGeluMul, 0.0f, stream);
 	if (gemm_band_applies<float>(A, B_gate, B_up, C, M, N, K, lda, ldb, ldc, b_layout))
 		return launch_gemm_band<float>(A, B_gate, B_up, nullptr, C, M, N, K, lda, ldb, ldc, kEpiGeluMul, 0.0f, stream);
 	if (b_layout == ANYGPU_B_ROW_MAJOR && gemm_band_ncontig_applies(A, B_gate, B_up, C, M, N, K, lda, ldb, ldc, true))

@@ -199,7 +199,18 @@ hipError_t launch_gemm_band(const T* A, const T* B, const T* B2, const T* bias, 
                             int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                             int epilogue, float ep_param, hipStream_t stream);
 
-// The same for n-contiguous fp32 weights (row-major B) from one row on: there the band kernel is ahead of the
+// Up to 16 rows against k-contiguous weights, K cut over the waves of a block (gemm_kwave.hip): fp32 and fp16, any N, no
+// workspace; `dual`: two weight matrices (kEpiGeluMul).  The launchers ask it before the other few-row kernels.
+template <typename T>
+bool gemm_kwave_applies(const T* A, const T* B, const T* B2, int64_t M, int64_t N, int64_t K,
+                        int64_t lda, int64_t ldb, int b_layout, bool dual);
+
+template <typename T>
+hipError_t launch_gemm_kwave(const T* A, const T* B, const T* B2, const T* bias, T* C,
+                             int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
+                             int epilogue, float ep_param, hipStream_t stream);
+
+// A band of few rows against n-contiguous fp32 weights (row-major B) from one row on: there the band kernel is ahead of the
 // skinny one at every row count (9216 x 2304 weights, 4 rows: 21 us against 50 us).  Any N from 4 on (the last vector of a row is moved back to end at N).
 // `dual`: two weight matrices (kEpiGeluMul), which are limited to 32 rows.
 bool gemm_band_ncontig_applies(const float* A, const float* B, const float* B2, const float* C, int64_t M, int64_t N, int64_t K,

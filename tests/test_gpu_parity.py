@@ -1020,6 +1020,41 @@ def test_mm_row_bands(ops, oracle, dtype, m, k, n):
     assert np.array_equal(got, again)
 
 
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("m,steps,n", [(1, 36, 2304), (2, 16, 300), (3, 17, 1), (8, 36, 9216), (8, 23, 2305), (5, 31, 5003), (4, 16, 7001), (7, 18, 8193),
+                                       (9, 16, 257), (16, 36, 2048), (12, 19, 4099), (16, 17, 6000), (8, 144, 130)])
+def test_mm_few_rows_k_cut_over_waves(ops, oracle, dtype, m, steps, n):
+    # up to 16 rows against k-contiguous weights, K in steps of 128 bytes from 16 of them on (two for each of eight waves), blocks of 1 to
+    # 33 columns that end past N, operands and results inside wider buffers.  Small integers: the sums are exact in both types (below 2048).
+    import torch
+    from anygpu_amd import capi
+    np_dt, t_dt = (np.float16, torch.float16) if dtype == "f16" else (np.float32, torch.float32)
+    pad, k = (8, 64 * steps) if dtype == "f16" else (4, 32 * steps)
+    a, bt, b2t = (synth.integers(s, shape, -2, 2).astype(np_dt) for s, shape in ((m + 1, (m, k)), (n + 2, (n, k)), (n + 3, (n, k))))
+    want = exact_int_product(a, np.ascontiguousarray(bt.T))
+    assert np.max(np.abs(want)) < 2048
+    abuf, bbuf = torch.full((m, k + pad), 9.0, dtype=t_dt, device="cuda"), torch.full((n, k + 2 * pad), 9.0, dtype=t_dt, device="cuda")
+    abuf[:, :k], bbuf[:, :k] = dev(a), dev(bt)
+    cbuf = torch.full((m + 1, n + 3), -7.0, dtype=t_dt, device="cuda")
+    ops.tensor_mm(abuf[:, :k], bbuf[:, :k], out=cbuf[:m, :n], b_layout=capi.B_COL_MAJOR)
+    got = host(cbuf).astype(np.int64)
+    assert np.array_equal(got[:m, :n], want)
+    assert np.all(got[m:, :] == -7) and np.all(got[:, n:] == -7)
+    bias = synth.integers(3, (n,), -9, 9).astype(np_dt)
+    assert np.array_equal(host(ops.tensor_gemm(dev(a), dev(bt), dev(bias), b_layout=capi.B_COL_MAJOR)).astype(np.int64), want + bias.astype(np.int64))
+    # the epilogues on sums of size O(1) (a power of two keeps them exact): half an ulp of the result's type, and 1e-6 of the
+    # arguments for the fp32 tanh (tanh_for_half: 4e-5 of the result)
+    scale = 2.0 ** -6
+    half_ulp = 2.0 ** -11 if dtype == "f16" else 2.0 ** -24
+    s1, s2 = want * scale, exact_int_product(a, np.ascontiguousarray(b2t.T)) * scale
+    got = host(ops.tensor_gemma_linear_softcap(dev((a * scale).astype(np_dt)).reshape(1, m, k), dev(bt), 30.0)).astype(np.float64).reshape(m, n)
+    capped = 30.0 * np.tanh(s1 / 30.0)
+    assert np.all(np.abs(got - capped) <= (half_ulp + (4.4e-5 if dtype == "f16" else 0.0)) * np.abs(capped) + 30.0 * 1e-6)
+    got = host(ops.mlp_gemma2_fused_upproj(dev((a * scale).astype(np_dt)), dev(bt), dev(b2t), b_layout=capi.B_COL_MAJOR)).astype(np.float64)
+    gated = 0.5 * s1 * (1.0 + np.tanh(math.sqrt(2.0 / math.pi) * (s1 + 0.044715 * s1 ** 3))) * s2
+    assert np.all(np.abs(got - gated) <= half_ulp * np.abs(gated) + 1e-6 * np.abs(s1 * s2) + 2.0 ** -24)
+
+
 @pytest.mark.parametrize("m,k,n", [(9, 2304, 9216), (16, 9216, 2304), (17, 512, 1000), (32, 2304, 2052), (12, 72, 68),
                                    (31, 264, 132), (24, 4096, 128), (10, 8, 4), (20, 1000, 132), (13, 16, 3000),
                                    (64, 9216, 2304), (48, 200, 1000), (5, 2304, 4100), (57, 72, 36), (40, 520, 132000),
