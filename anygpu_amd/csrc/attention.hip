@@ -1065,6 +1065,11 @@ hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, h
 // Workspace per (head, split, row): head_dim accumulators + maximum + sum, fp32.
 // ---------------------------------------------------------------------------------------------
 
+// Keys of a tile, and the grain in which they are shared out among the waves: 5001 keys are 157 tiles, five to each of 32 waves of a
+// head; in tiles of 64 they were 79, three (192 keys) to each of 27, and the other waves' SIMDs stood idle (batch 4, 32 / 8 heads
+// x 5001 keys x 128: 21.1 -> 18.9 us with the merge).
+constexpr int kDecodeKeysPerTile = 32;
+
 struct DecodeArgs
 {
 	AttnArgs a;
@@ -1079,11 +1084,10 @@ struct DecodeArgs
 template <int D, bool SOFTCAP>
 __global__ __launch_bounds__(64) void sdp_decode_partial_kernel(const DecodeArgs da)
 {
-	extern __shared__ __align__(16) char lds[];           // the V tile: 64 keys x (2 D + 32) bytes
+	extern __shared__ __align__(16) char lds[];           // the V tile: 32 keys x (2 D + 32) bytes
 	const AttnArgs& a = da.a;
 	constexpr int kPitchV = AttnLds<D>::kPitchV;
 	constexpr int KS = D / 32, DC = D / 16, VPR = D / 8;
-	constexpr int VPT = kAttnKeysPerTile * D / 8 / 64;    // V vectors per lane per tile
 
 	const int lane = threadIdx.x;
 	const int n = lane & 15, g = lane >> 4;
@@ -1118,11 +1122,11 @@ __global__ __launch_bounds__(64) void sdp_decode_partial_kernel(const DecodeArgs
 	const int t0 = da.t_first + split * da.tiles_per_split;
 	int t1 = t0 + da.tiles_per_split - 1;
 	if (t1 > da.t_last) t1 = da.t_last;
-	// The keys are walked in sub-tiles of 32 (one MFMA step of the second product).  The loads of sub-tile u + 1 (K
-	// fragments straight into operand layout, V vectors for the wave's LDS tile) are in flight while sub-tile u is
+	// The keys are walked in tiles of 32 (one MFMA step of the second product).  The loads of tile u + 1 (K
+	// fragments straight into operand layout, V vectors for the wave's LDS tile) are in flight while tile u is
 	// multiplied: a wave that loaded, waited and multiplied in turn left the memory system idle half of the time.
-	constexpr int kSub = 32;
-	constexpr int VPS = kSub * D / 8 / 64;                // V vectors per lane per sub-tile
+	constexpr int kSub = kDecodeKeysPerTile;
+	constexpr int VPS = kSub * D / 8 / 64;                // V vectors per lane per tile
 	half8_t kf[2][2][KS];
 	float4_t vr[2][VPS];
 	auto fetch = [&](half8_t (&kd)[2][KS], float4_t (&vd)[VPS], int key0) {
@@ -1210,8 +1214,8 @@ __global__ __launch_bounds__(64) void sdp_decode_partial_kernel(const DecodeArgs
 		__builtin_amdgcn_s_waitcnt(0xC07F);               // the tile has been read before the next one overwrites it
 		__builtin_amdgcn_wave_barrier();
 	};
-	// sub-tiles u0 .. u1, two per step so that the buffer of a sub-tile is a compile-time constant
-	const int u0 = 2 * t0, u1 = 2 * t1 + 1;
+	// tiles u0 .. u1, two per step so that the buffer of a tile is a compile-time constant
+	const int u0 = t0, u1 = t1;
 	if (u0 <= u1) fetch(kf[0], vr[0], u0 * kSub);
 	for (int u = u0; u <= u1; u += 2)
 	{
@@ -1246,7 +1250,7 @@ __global__ __launch_bounds__(64) void sdp_decode_partial_kernel(const DecodeArgs
 template <int D, bool SOFTCAP>
 hipError_t launch_decode_variant(const DecodeArgs& da, int64_t kv_heads, hipStream_t stream)
 {
-	constexpr int kLdsBytes = kAttnKeysPerTile * AttnLds<D>::kPitchV;
+	constexpr int kLdsBytes = kDecodeKeysPerTile * AttnLds<D>::kPitchV;
 	(void)hipGetLastError();
 	sdp_decode_partial_kernel<D, SOFTCAP><<<dim3(decode_blocks(da.groups, da.splits), (unsigned)kv_heads), dim3(64), kLdsBytes, stream>>>(da);
 	hipError_t e = hipGetLastError();
@@ -1341,7 +1345,7 @@ int64_t sdp_attention_decode_workspace_bytes(int64_t batch_heads, int64_t q_per_
 {
 	if (batch_heads == 0 || n_q == 0) return 0;
 	const int64_t kv_heads = batch_heads / q_per_kv;
-	const DecodePlan p = plan_decode(kv_heads * ((q_per_kv * n_q + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave), n_q, n_k, causal, window, kAttnKeysPerTile);
+	const DecodePlan p = plan_decode(kv_heads * ((q_per_kv * n_q + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave), n_q, n_k, causal, window, kDecodeKeysPerTile);
 	return kv_heads * p.splits * (q_per_kv * n_q) * (head_dim + 2) * (int64_t)sizeof(float);
 }
 
@@ -1351,7 +1355,7 @@ hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const v
 {
 	if (batch_heads == 0 || n_q == 0) return hipSuccess;
 	const int64_t kv_heads = batch_heads / q_per_kv;
-	const DecodePlan p = plan_decode(kv_heads * ((q_per_kv * n_q + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave), n_q, n_k, causal, window, kAttnKeysPerTile);
+	const DecodePlan p = plan_decode(kv_heads * ((q_per_kv * n_q + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave), n_q, n_k, causal, window, kDecodeKeysPerTile);
 	DecodeArgs da;
 	da.a.q = static_cast<const half_t*>(q);
 	da.a.k = static_cast<const half_t*>(k);
