@@ -485,7 +485,7 @@ hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, h
 	args.tile_map = nullptr;
 	args.map_words = 0;
 	std::optional<band::WorkspaceReserve> map_hold;
-	bool mask_two_parts = false;
+	int64_t mask_parts = 0;
 	if constexpr (MASK)
 	{
 		// The visible-tile map of the mask, at the front of the stream's workspace (the partial results of a split key
@@ -502,17 +502,29 @@ hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, h
 		// it does for operand copies (eager launches only), before anything points into it.
 		const int64_t blocks = q_blocks * batch_heads;
 		const int cus = device_cu_count();
-		size_t two_parts_bytes = 0;
-		if (blocks >= cus && blocks < 4 * (int64_t)cus && (args.n_k + KT - 1) / KT >= 32)
-			two_parts_bytes = (size_t)2 * blocks * kQueriesPerBlock * (D + 2) * sizeof(float);
+		// With fewer blocks than CUs but more than half as many, the parts are chosen to fill whole rounds, and the growing
+		// workspace is what lets them: 8 heads x 3001 x 256 are 192 blocks, which the first 64 MB hold in two parts only (384
+		// blocks, one and a half rounds, the first of the causal ones walking 47 of the 36 tiles that a CU averages); four
+		// parts are three whole rounds (us, causal mask 449 -> 422, window of 1024 333 -> 295, no key hidden 899 -> 729; 16 heads x
+		// 1500 x 3000 x 256, likewise 192 blocks: 670 -> 580, 904 -> 722).
+		int64_t want_parts = 0;
+		const int64_t tiles = (args.n_k + KT - 1) / KT;
+		if (blocks >= cus && blocks < 4 * (int64_t)cus && tiles >= 32) want_parts = 2;
+		else if (DIRECT && blocks < cus && 2 * blocks > cus)
+		{
+			const auto filled = [&](int64_t s) { return (double)(blocks * s) / (double)((blocks * s + cus - 1) / cus * cus); };
+			for (int64_t s = 2; s <= 6 && tiles / s >= 16; ++s)
+				if (want_parts == 0 || filled(s) > 1.1 * filled(want_parts)) want_parts = s;
+		}
+		size_t parts_bytes = (size_t)want_parts * blocks * kQueriesPerBlock * (D + 2) * sizeof(float);
 		const size_t map_room = (map_bytes + 255) / 256 * 256 + (1u << 16);
-		if (two_parts_bytes > 0 && band::workspace_copy_capacity(stream) < map_room + two_parts_bytes) two_parts_bytes = 0;
-		if (attention_mask_map_wanted(args.n_q, args.n_k) && (two_parts_bytes > 0 || band::workspace_capacity(stream) >= map_room))
+		if (parts_bytes > 0 && band::workspace_copy_capacity(stream) < map_room + parts_bytes) parts_bytes = 0;
+		if (attention_mask_map_wanted(args.n_q, args.n_k) && (parts_bytes > 0 || band::workspace_capacity(stream) >= map_room))
 		{
 			float* front = nullptr;
-			hipError_t e = band::workspace_acquire(stream, &front, two_parts_bytes > 0 ? map_room + two_parts_bytes : 0);
+			hipError_t e = band::workspace_acquire(stream, &front, parts_bytes > 0 ? map_room + parts_bytes : 0);
 			if (e != hipSuccess) return e;
-			mask_two_parts = two_parts_bytes > 0;
+			if (parts_bytes > 0) mask_parts = want_parts;
 			unsigned long long* map = reinterpret_cast<unsigned long long*>(front);
 			e = launch_attention_mask_tile_map(args.mask, args.mask_stride, args.n_q, args.n_k, kQueriesPerBlock, KT, map, stream);
 			if (e != hipSuccess) return e;
@@ -526,7 +538,7 @@ hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, h
 	// (or, with too few query blocks for the chip, every block in several parts of its key range)
 	int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQueriesPerBlock,
 	                                                                  KT, D, band::workspace_capacity(stream));
-	if (mask_two_parts && plan.n_split == 0 && parts_all == 1) parts_all = 2;
+	if (plan.n_split == 0 && (parts_all == 1 || q_blocks * batch_heads < device_cu_count()) && mask_parts > 0) parts_all = mask_parts;
 	args.partials = nullptr;
 	if (plan.n_split > 0 || parts_all > 1)
 	{

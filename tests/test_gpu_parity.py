@@ -1990,6 +1990,37 @@ def test_sdp_attention_f32_mask_tensor_blocks_in_two_parts_of_their_visible_tile
         assert scaled_rel_err(got[:, h:h + 1], want, 1.0) <= TOL_F32
 
 
+def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops, oracle, monkeypatch):
+    # head dimension 256 with fewer blocks than CUs (16 heads x 10 blocks of 128 queries; 66 key tiles, so up to four parts):
+    # the parts take more than the workspace holds to begin with, which grows; against a caller's workspace that only has
+    # room for the map (whole blocks), and one head against the oracle
+    import torch
+    heads, n_q, n_k, d = 16, 1190, 2090, 256
+    q = synth.normal(81, (1, heads, n_q, d))
+    k = synth.normal(82, (1, heads, n_k, d))
+    v = synth.normal(83, (1, heads, n_k, d))
+    alpha = float(d) ** -0.5
+    rng = np.random.default_rng(84)
+    mask = rng.normal(0.0, 1.0, (n_q, n_k)).astype(np.float32)
+    hide_key_stripes(mask, rng)
+    mask4 = mask.reshape(1, 1, n_q, n_k)
+    dq, dk, dv, dm = dev(q), dev(k), dev(v), dev(mask4)
+    monkeypatch.setenv("ANYGPU_ATTN_MASK_MAP_FROM", "0")
+    got = host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))
+    small = torch.empty(1 << 17, dtype=torch.uint8, device="cuda")
+    ops.set_workspace(small)
+    try:
+        whole = host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))
+    finally:
+        torch.cuda.synchronize()
+        ops.set_workspace(None)
+    assert np.isfinite(got).all()
+    assert scaled_rel_err(got, whole, 1.0) <= 1e-5
+    assert not np.array_equal(got, whole), "the two runs were expected to sum in different orders"
+    want = oracle.sdp_attention_masked_scaled_fwd(q[:, 3:4], k[:, 3:4], v[:, 3:4], mask4, alpha, threads=8)
+    assert scaled_rel_err(got[:, 3:4], want, 1.0) <= TOL_F32
+
+
 ATTN_CASES = [
     # heads, kv_heads, n_q, n_k, d, alpha, softcap, causal, window
     (2, 2, 16, 16, 64, 0.125, 0.0, False, 0),
