@@ -1340,22 +1340,45 @@ bool sdp_attention_decode_f16_supports(int64_t q_per_kv, int64_t n_q, int64_t he
 	return sdp_attention_fwd_f16_supports(head_dim) && q_per_kv >= 1 && n_q >= 1 && q_per_kv * n_q <= kDecodeMaxRows;
 }
 
-int64_t sdp_attention_decode_workspace_bytes(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim,
-                                             int causal, int64_t window)
+namespace {
+
+// Splits in tiles of 32 keys where a wave walks more than one tile of 64 (below that a finer cut only makes more partial results)
+// and `room` bytes of workspace hold the partial results, else in pairs of tiles: 64 keys, the grain whose need is the least
+// that the entry points ask for.
+DecodePlan plan_decode_f16(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim, int causal, int64_t window,
+                           int64_t room)
 {
-	if (batch_heads == 0 || n_q == 0) return 0;
-	const int64_t kv_heads = batch_heads / q_per_kv;
-	const DecodePlan p = plan_decode(kv_heads * ((q_per_kv * n_q + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave), n_q, n_k, causal, window, kDecodeKeysPerTile);
-	return kv_heads * p.splits * (q_per_kv * n_q) * (head_dim + 2) * (int64_t)sizeof(float);
+	const int64_t kv_heads = batch_heads / q_per_kv, rows = q_per_kv * n_q;
+	const int64_t units = kv_heads * ((rows + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave);
+	DecodePlan p = plan_decode(units, n_q, n_k, causal, window, 2 * kDecodeKeysPerTile);
+	if (p.tiles_per_split > 1)
+	{
+		const DecodePlan fine = plan_decode(units, n_q, n_k, causal, window, kDecodeKeysPerTile);
+		if (kv_heads * fine.splits * rows * (head_dim + 2) * (int64_t)sizeof(float) <= room) return fine;
+	}
+	p.t_first *= 2;
+	p.t_last = 2 * p.t_last + 1;
+	p.tiles_per_split *= 2;
+	return p;
 }
 
-hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const void* v, void* y, void* workspace,
+}  // namespace
+
+int64_t sdp_attention_decode_workspace_bytes(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim,
+                                             int causal, int64_t window, bool least)
+{
+	if (batch_heads == 0 || n_q == 0) return 0;
+	const DecodePlan p = plan_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window, least ? 0 : INT64_MAX);
+	return batch_heads / q_per_kv * p.splits * (q_per_kv * n_q) * (head_dim + 2) * (int64_t)sizeof(float);
+}
+
+hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const void* v, void* y, void* workspace, int64_t workspace_bytes,
                                            int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim,
                                            float alpha, float softcap, int causal, int64_t window, hipStream_t stream)
 {
 	if (batch_heads == 0 || n_q == 0) return hipSuccess;
 	const int64_t kv_heads = batch_heads / q_per_kv;
-	const DecodePlan p = plan_decode(kv_heads * ((q_per_kv * n_q + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave), n_q, n_k, causal, window, kDecodeKeysPerTile);
+	const DecodePlan p = plan_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window, workspace_bytes);
 	DecodeArgs da;
 	da.a.q = static_cast<const half_t*>(q);
 	da.a.k = static_cast<const half_t*>(k);

@@ -462,11 +462,11 @@ ANYGPU_EXPORT int anygpu_sdp_attention_decode_f16(const void* q, const void* k, 
 	if (rc != ANYGPU_OK) return rc;
 	if (batch_heads == 0 || n_q == 0) return ANYGPU_OK;
 	if (!anygpu::sdp_attention_decode_f16_supports(q_per_kv, n_q, head_dim)) return ANYGPU_ERR_UNSUPPORTED;
-	const int64_t need = anygpu::sdp_attention_decode_workspace_bytes(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window);
+	const int64_t need = anygpu::sdp_attention_decode_workspace_bytes(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window, true);
 	if (workspace == nullptr) return ANYGPU_ERR_NULL_POINTER;
 	if (workspace_bytes < need) return ANYGPU_ERR_BAD_SHAPE;
 	if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return ANYGPU_ERR_UNSUPPORTED;
-	return (int)anygpu::launch_sdp_attention_decode_f16(q, k, v, y, workspace, batch_heads, q_per_kv, n_q, n_k, head_dim, alpha,
+	return (int)anygpu::launch_sdp_attention_decode_f16(q, k, v, y, workspace, workspace_bytes, batch_heads, q_per_kv, n_q, n_k, head_dim, alpha,
 	                                                    softcap, causal, window, as_stream(stream));
 }
 
@@ -482,9 +482,9 @@ ANYGPU_EXPORT int anygpu_sdp_attention_decode_f16_static(const void* q, const vo
 	if (e != hipSuccess) return (int)e;
 	if (batch_heads == 0 || n_q == 0) return ANYGPU_OK;
 	if (!anygpu::sdp_attention_decode_f16_supports(q_per_kv, n_q, head_dim)) return ANYGPU_ERR_UNSUPPORTED;
-	const int64_t need = anygpu::sdp_attention_decode_workspace_bytes(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window);
+	const int64_t need = anygpu::sdp_attention_decode_workspace_bytes(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window, true);
 	if (need > (int64_t)ANYGPU_DECODE_STATIC_SCRATCH_BYTES) return ANYGPU_ERR_SCRATCH_TOO_SMALL;
-	return (int)anygpu::launch_sdp_attention_decode_f16(q, k, v, y, ws, batch_heads, q_per_kv, n_q, n_k, head_dim, alpha,
+	return (int)anygpu::launch_sdp_attention_decode_f16(q, k, v, y, ws, ANYGPU_DECODE_STATIC_SCRATCH_BYTES, batch_heads, q_per_kv, n_q, n_k, head_dim, alpha,
 	                                                    softcap, causal, window, as_stream(stream));
 }
 

@@ -2330,6 +2330,36 @@ def test_sdp_attention_decode_f32_workspace_and_rejected_arguments(ops):
     assert bool((y == 3.0).all())
 
 
+def test_sdp_attention_decode_takes_the_least_workspace(ops):
+    # 32 key / value heads x 5001 keys: 32 splits of 160 keys by the query, 27 of 192 in the least workspace (fp16), which stays
+    # enough, as does the library's scratch of 8 MB where only that split fits it (8 rows x 256: 7.1 MB against 8.5)
+    import torch
+    from anygpu_amd import capi
+    lib = capi.load()
+    for kv, per, d in ((32, 4, 128), (32, 8, 256)):
+        rng = torch.Generator(device="cuda")
+        rng.manual_seed(7)
+        q = torch.randn((kv * per, 1, d), device="cuda", generator=rng).half()
+        k, v = (torch.randn((kv, 5001, d), device="cuda", generator=rng).half() for _ in range(2))
+        shape = (kv * per, per, 1, 5001, d)
+        need, least = (kv * splits * per * (d + 2) * 4 for splits in (32, 27))
+        assert lib.anygpu_sdp_attention_decode_workspace_bytes(*shape, 1, 0) == need
+        rest = (*shape, d ** -0.5, 0.0, 1, 0, torch.cuda.current_stream().cuda_stream)
+        outs = []
+        for size in (need, least):
+            ws = torch.empty(size, dtype=torch.uint8, device="cuda")
+            outs.append(torch.empty_like(q))
+            assert lib.anygpu_sdp_attention_decode_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[-1].data_ptr(), ws.data_ptr(), size, *rest) == 0
+        ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr())
+        assert lib.anygpu_sdp_attention_decode_f16(*ptrs, outs[-1].data_ptr(), ws.data_ptr(), least - 1, *rest) == capi.ANYGPU_ERR_BAD_SHAPE
+        outs.append(torch.empty_like(q))
+        assert lib.anygpu_sdp_attention_decode_f16_static(*ptrs, outs[-1].data_ptr(), *rest) == 0
+        s = (q.float().view(kv, per, d) @ k.float().transpose(1, 2)) * d ** -0.5
+        want = host((torch.softmax(s, -1) @ v.float()).view(kv * per, 1, d))
+        for out in outs:
+            assert scaled_rel_err(host(out), want, float(np.abs(want).mean())) <= TOL_F16_GEMM
+
+
 def test_sdp_attention_decode_workspace_and_rejected_arguments(ops):
     import torch
     from anygpu_amd import capi
