@@ -579,6 +579,9 @@ hipError_t launch_gemm_f32(const float* A, const float* B, const float* bias, fl
                            int a_layout, int b_layout, hipStream_t stream)
 {
 	if (M == 0 || N == 0 || batch == 0) return hipSuccess;
+	// products of so few tiles that most of the chip would idle
+	if (batch == 1 && a_layout == ANYGPU_A_ROW_MAJOR && gemm_f32_small_applies(A, B, M, N, K, lda, ldb, b_layout))
+		return launch_gemm_f32_small(A, B, bias, C, M, N, K, lda, ldb, ldc, b_layout, stream);
 	// Rows that end a little past a multiple of 64 make a whole further row of tiles, which in fp32 costs matrix-core
 	// time, where the few rows past the multiple would only cost another pass over the weights through the few-row
 	// kernels: where the plans' prices say so, the product is divided into the multiples of 64 and the rest

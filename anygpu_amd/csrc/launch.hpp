@@ -121,6 +121,12 @@ hipError_t launch_gemm_f32(const float* A, const float* B, const float* bias, fl
                            int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t batch,
                            int a_layout, int b_layout, hipStream_t stream);
 
+// The fp32 product (row-major A) in 32 x 32 tiles with K cut over the waves of a block (gemm_f32_small.hip): any sizes, pitches
+// and element alignment.  `applies`: whether it is ahead of the other kernels for these operands.
+bool gemm_f32_small_applies(const float* A, const float* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int b_layout);
+hipError_t launch_gemm_f32_small(const float* A, const float* B, const float* bias, float* C, int64_t M, int64_t N, int64_t K,
+                                 int64_t lda, int64_t ldb, int64_t ldc, int b_layout, hipStream_t stream);
+
 // C = softcap * tanh((A * B) / softcap)
 hipError_t launch_gemm_f32_softcap(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K,
                                    int64_t lda, int64_t ldb, int64_t ldc, int b_layout, float softcap, hipStream_t stream);

@@ -1990,6 +1990,38 @@ def test_sdp_attention_f32_mask_tensor_blocks_in_two_parts_of_their_visible_tile
         assert scaled_rel_err(got[:, h:h + 1], want, 1.0) <= TOL_F32
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 31, 1), (3, 33, 31), (33, 32, 32), (32, 95, 63), (64, 64, 128), (65, 70, 129), (31, 100, 256),
+                                   (40, 33, 385), (128, 128, 768), (97, 130, 1533), (700, 701, 333)])
+@pytest.mark.parametrize("layout", ["kn", "nk"])
+def test_gemm_f32_small_products(ops, oracle, m, n, k, layout):
+    # 32 x 32 tiles with K cut over four waves in steps of 32: edges of tiles, one step, fewer steps than waves, the rest of K in
+    # each wave's turn, padded rows at odd pitches and element alignment.  Integer-valued: every order of summation is
+    # exact.  The buffers behind the operands hold NaN: nothing of them may reach a sum, and what lies between the rows of C stays.
+    import torch
+    from anygpu_amd import capi
+    a = synth.integers(91, (m, k), -8, 8)
+    b = synth.integers(92, (k, n), -8, 8)
+    bias = synth.integers(93, (n,), -8, 8)
+    want = exact_int_product(a, b)
+    b_store = b if layout == "kn" else np.ascontiguousarray(b.T)
+    lay = capi.B_ROW_MAJOR if layout == "kn" else capi.B_COL_MAJOR
+
+    def padded(x, extra, shift):
+        buf = torch.full((x.shape[0] * (x.shape[1] + extra) + shift,), float("nan"), device="cuda")
+        view = buf[shift:].view(x.shape[0], x.shape[1] + extra)[:, :x.shape[1]]
+        view.copy_(dev(x))
+        return view
+
+    for extra, shift in ((0, 0), (3, 1)):
+        out = padded(np.zeros((m, n), np.float32), extra, shift)
+        got = host(ops.tensor_mm(padded(a, extra, shift), padded(b_store, extra, shift), out=out, b_layout=lay))
+        assert np.array_equal(got.astype(np.int64), want)
+        if extra:
+            assert bool(torch.isnan(out._base[shift:].view(m, n + extra)[:, n:]).all())
+    got = host(ops.tensor_gemm(dev(a), dev(b_store), dev(bias), b_layout=lay))
+    assert np.array_equal(got.astype(np.int64), want + bias.astype(np.int64))
+
+
 def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops, oracle, monkeypatch):
     # head dimension 256 with fewer blocks than CUs (16 heads x 10 blocks of 128 queries; 66 key tiles, so up to four parts):
     # the parts take more than the workspace holds to begin with, which grows; against a caller's workspace that only has
