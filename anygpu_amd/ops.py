@@ -13,8 +13,16 @@ import torch
 from . import capi
 
 
+# handle of a device's current stream, and the current device: what torch.cuda.current_stream().cuda_stream comes down to, without
+# the Stream object around it (2.7 us a call, a quarter of what a small call costs the host; 0.15 us this way)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _current_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def _require(cond: bool, msg: str) -> None:
