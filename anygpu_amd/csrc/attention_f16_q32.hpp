@@ -8,7 +8,7 @@
 // softmax, loads and ends run beside the other's products, and causal launches of ordinary prompts have twice as many
 // pieces to pack onto the CUs.  Scores sit 32 to a lane (S^T = K Q^T: a lane holds one query), so row maxima are in-lane
 // but for one exchange of lane halves; sums come out of v_dot2 on the packed halves that the second product uses.
-// Measured, causal (us; before -> now): 32 / 8 heads x 3000 x 128 141 -> 90 (0.82 PFLOP/s), 16 x 4096 x 128 123 -> 95, 64 / 8 x
+// Measured, causal (us; before -> now): 32 / 8 heads x 3000 x 128 126 -> 85 (0.87 PFLOP/s), 16 x 4096 x 128 123 -> 95, 64 / 8 x
 // 1023 x 128 45.7 -> 30.2, 32 / 8 x 8192 x 128 647 -> 541 (1.02 PFLOP/s; a kernel that overlaps the products and the softmax inside
 // a wave ran at the same rate there, as the clock drops under the matrix units' power), 32 x 2048 x 64 43 -> 32.
 #pragma once
