@@ -1020,41 +1020,6 @@ def test_mm_row_bands(ops, oracle, dtype, m, k, n):
     assert np.array_equal(got, again)
 
 
-@pytest.mark.parametrize("dtype", ["f16", "f32"])
-@pytest.mark.parametrize("m,steps,n", [(1, 36, 2304), (2, 16, 300), (3, 17, 1), (8, 36, 9216), (8, 23, 2305), (5, 31, 5003), (4, 16, 7001), (7, 18, 8193),
-                                       (9, 16, 257), (16, 36, 2048), (12, 19, 4099), (16, 17, 6000), (8, 144, 130)])
-def test_mm_few_rows_k_cut_over_waves(ops, oracle, dtype, m, steps, n):
-    # up to 16 rows against k-contiguous weights, K in steps of 128 bytes from 16 of them on (two for each of eight waves), blocks of 1 to
-    # 33 columns that end past N, operands and results inside wider buffers.  Small integers: the sums are exact in both types (below 2048).
-    import torch
-    from anygpu_amd import capi
-    np_dt, t_dt = (np.float16, torch.float16) if dtype == "f16" else (np.float32, torch.float32)
-    pad, k = (8, 64 * steps) if dtype == "f16" else (4, 32 * steps)
-    a, bt, b2t = (synth.integers(s, shape, -2, 2).astype(np_dt) for s, shape in ((m + 1, (m, k)), (n + 2, (n, k)), (n + 3, (n, k))))
-    want = exact_int_product(a, np.ascontiguousarray(bt.T))
-    assert np.max(np.abs(want)) < 2048
-    abuf, bbuf = torch.full((m, k + pad), 9.0, dtype=t_dt, device="cuda"), torch.full((n, k + 2 * pad), 9.0, dtype=t_dt, device="cuda")
-    abuf[:, :k], bbuf[:, :k] = dev(a), dev(bt)
-    cbuf = torch.full((m + 1, n + 3), -7.0, dtype=t_dt, device="cuda")
-    ops.tensor_mm(abuf[:, :k], bbuf[:, :k], out=cbuf[:m, :n], b_layout=capi.B_COL_MAJOR)
-    got = host(cbuf).astype(np.int64)
-    assert np.array_equal(got[:m, :n], want)
-    assert np.all(got[m:, :] == -7) and np.all(got[:, n:] == -7)
-    bias = synth.integers(3, (n,), -9, 9).astype(np_dt)
-    assert np.array_equal(host(ops.tensor_gemm(dev(a), dev(bt), dev(bias), b_layout=capi.B_COL_MAJOR)).astype(np.int64), want + bias.astype(np.int64))
-    # the epilogues on sums of size O(1) (a power of two keeps them exact): half an ulp of the result's type, and 1e-6 of the
-    # arguments for the fp32 tanh (tanh_for_half: 4e-5 of the result)
-    scale = 2.0 ** -6
-    half_ulp = 2.0 ** -11 if dtype == "f16" else 2.0 ** -24
-    s1, s2 = want * scale, exact_int_product(a, np.ascontiguousarray(b2t.T)) * scale
-    got = host(ops.tensor_gemma_linear_softcap(dev((a * scale).astype(np_dt)).reshape(1, m, k), dev(bt), 30.0)).astype(np.float64).reshape(m, n)
-    capped = 30.0 * np.tanh(s1 / 30.0)
-    assert np.all(np.abs(got - capped) <= (half_ulp + (4.4e-5 if dtype == "f16" else 0.0)) * np.abs(capped) + 30.0 * 1e-6)
-    got = host(ops.mlp_gemma2_fused_upproj(dev((a * scale).astype(np_dt)), dev(bt), dev(b2t), b_layout=capi.B_COL_MAJOR)).astype(np.float64)
-    gated = 0.5 * s1 * (1.0 + np.tanh(math.sqrt(2.0 / math.pi) * (s1 + 0.044715 * s1 ** 3))) * s2
-    assert np.all(np.abs(got - gated) <= half_ulp * np.abs(gated) + 1e-6 * np.abs(s1 * s2) + 2.0 ** -24)
-
-
 @pytest.mark.parametrize("m,k,n", [(9, 2304, 9216), (16, 9216, 2304), (17, 512, 1000), (32, 2304, 2052), (12, 72, 68),
                                    (31, 264, 132), (24, 4096, 128), (10, 8, 4), (20, 1000, 132), (13, 16, 3000),
                                    (64, 9216, 2304), (48, 200, 1000), (5, 2304, 4100), (57, 72, 36), (40, 520, 132000),
@@ -1990,69 +1955,6 @@ def test_sdp_attention_f32_mask_tensor_blocks_in_two_parts_of_their_visible_tile
         assert scaled_rel_err(got[:, h:h + 1], want, 1.0) <= TOL_F32
 
 
-@pytest.mark.parametrize("m,n,k", [(17, 31, 1), (3, 33, 31), (33, 32, 32), (32, 95, 63), (64, 64, 128), (65, 70, 129), (31, 100, 256),
-                                   (40, 33, 385), (128, 128, 768), (97, 130, 1533), (700, 701, 333)])
-@pytest.mark.parametrize("layout", ["kn", "nk"])
-def test_gemm_f32_small_products(ops, oracle, m, n, k, layout):
-    # 32 x 32 tiles with K cut over four waves in steps of 32: edges of tiles, one step, fewer steps than waves, the rest of K in
-    # each wave's turn, padded rows at odd pitches and element alignment.  Integer-valued: every order of summation is
-    # exact.  The buffers behind the operands hold NaN: nothing of them may reach a sum, and what lies between the rows of C stays.
-    import torch
-    from anygpu_amd import capi
-    a = synth.integers(91, (m, k), -8, 8)
-    b = synth.integers(92, (k, n), -8, 8)
-    bias = synth.integers(93, (n,), -8, 8)
-    want = exact_int_product(a, b)
-    b_store = b if layout == "kn" else np.ascontiguousarray(b.T)
-    lay = capi.B_ROW_MAJOR if layout == "kn" else capi.B_COL_MAJOR
-
-    def padded(x, extra, shift):
-        buf = torch.full((x.shape[0] * (x.shape[1] + extra) + shift,), float("nan"), device="cuda")
-        view = buf[shift:].view(x.shape[0], x.shape[1] + extra)[:, :x.shape[1]]
-        view.copy_(dev(x))
-        return view
-
-    for extra, shift in ((0, 0), (3, 1)):
-        out = padded(np.zeros((m, n), np.float32), extra, shift)
-        got = host(ops.tensor_mm(padded(a, extra, shift), padded(b_store, extra, shift), out=out, b_layout=lay))
-        assert np.array_equal(got.astype(np.int64), want)
-        if extra:
-            assert bool(torch.isnan(out._base[shift:].view(m, n + extra)[:, n:]).all())
-    got = host(ops.tensor_gemm(dev(a), dev(b_store), dev(bias), b_layout=lay))
-    assert np.array_equal(got.astype(np.int64), want + bias.astype(np.int64))
-
-
-def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops, oracle, monkeypatch):
-    # head dimension 256 with fewer blocks than CUs (16 heads x 10 blocks of 128 queries; 66 key tiles, so up to four parts):
-    # the parts take more than the workspace holds to begin with, which grows; against a caller's workspace that only has
-    # room for the map (whole blocks), and one head against the oracle
-    import torch
-    heads, n_q, n_k, d = 16, 1190, 2090, 256
-    q = synth.normal(81, (1, heads, n_q, d))
-    k = synth.normal(82, (1, heads, n_k, d))
-    v = synth.normal(83, (1, heads, n_k, d))
-    alpha = float(d) ** -0.5
-    rng = np.random.default_rng(84)
-    mask = rng.normal(0.0, 1.0, (n_q, n_k)).astype(np.float32)
-    hide_key_stripes(mask, rng)
-    mask4 = mask.reshape(1, 1, n_q, n_k)
-    dq, dk, dv, dm = dev(q), dev(k), dev(v), dev(mask4)
-    monkeypatch.setenv("ANYGPU_ATTN_MASK_MAP_FROM", "0")
-    got = host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))
-    small = torch.empty(1 << 17, dtype=torch.uint8, device="cuda")
-    ops.set_workspace(small)
-    try:
-        whole = host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))
-    finally:
-        torch.cuda.synchronize()
-        ops.set_workspace(None)
-    assert np.isfinite(got).all()
-    assert scaled_rel_err(got, whole, 1.0) <= 1e-5
-    assert not np.array_equal(got, whole), "the two runs were expected to sum in different orders"
-    want = oracle.sdp_attention_masked_scaled_fwd(q[:, 3:4], k[:, 3:4], v[:, 3:4], mask4, alpha, threads=8)
-    assert scaled_rel_err(got[:, 3:4], want, 1.0) <= TOL_F32
-
-
 ATTN_CASES = [
     # heads, kv_heads, n_q, n_k, d, alpha, softcap, causal, window
     (2, 2, 16, 16, 64, 0.125, 0.0, False, 0),
@@ -2083,27 +1985,6 @@ def test_sdp_attention_fused_kernel(ops, oracle, case):
     # outputs are convex combinations of N(0, 1) values: scale floor 1
     assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2          # p is rounded to fp16 before the second product
     assert rel_l2(got[0], want) <= 2e-3
-
-
-# head dimensions 64 and 128 run 32 queries per wave, four waves and 128 queries per block, tiles of 64 keys: one query and
-# the edges of a wave's and a block's queries, tiles of one key, one short of whole and whole, queries of a wave that see
-# nothing, and the first and last tile of a window that only some waves of a block see
-@pytest.mark.parametrize("n_q,n_k,causal,window", [(1, 65, True, 0), (31, 64, True, 0), (33, 63, False, 0), (127, 129, True, 0), (128, 128, True, 0),
-                                                    (129, 257, True, 70), (160, 100, True, 0), (300, 321, False, 64), (257, 600, True, 1)])
-@pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 0.0, -0.0884), (64, 30.0, 0.0), (128, 50.0, 0.0884)])
-def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, causal, window, d, cap, alpha):
-    heads, kv_heads = 4, 2
-    q = synth.normal(1 + n_q, (1, heads, n_q, d)).astype(np.float16)
-    k = synth.normal(2 + n_k, (1, kv_heads, n_k, d)).astype(np.float16) * np.float16(4.0)        # (scores of tens: the running maximum moves)
-    v = synth.normal(3 + d, (1, kv_heads, n_k, d)).astype(np.float16)
-    got = host(ops.sdp_attention_fwd(dev(q), dev(k), dev(v), alpha, softcap=cap, causal=causal, window=window, decode=False)).astype(np.float32)
-    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=alpha, softcap=cap,
-                                      causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
-    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
-    assert not got[0][blind].any()
-    assert np.isfinite(got).all()
-    # p rounded to fp16 (2^-11 each, weights that sum to 1) and the result's own rounding, values of up to about 4
-    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
 
 def _random_attention_cases(count, seed):
@@ -2360,36 +2241,6 @@ def test_sdp_attention_decode_f32_workspace_and_rejected_arguments(ops):
     assert f(q.data_ptr(), kv.data_ptr(), kv.data_ptr(), y.data_ptr(), ws.data_ptr(), need - 1, *args) == capi.ANYGPU_ERR_BAD_SHAPE
     torch.cuda.synchronize()
     assert bool((y == 3.0).all())
-
-
-def test_sdp_attention_decode_takes_the_least_workspace(ops):
-    # 32 key / value heads x 5001 keys: 32 splits of 160 keys by the query, 27 of 192 in the least workspace (fp16), which stays
-    # enough, as does the library's scratch of 8 MB where only that split fits it (8 rows x 256: 7.1 MB against 8.5)
-    import torch
-    from anygpu_amd import capi
-    lib = capi.load()
-    for kv, per, d in ((32, 4, 128), (32, 8, 256)):
-        rng = torch.Generator(device="cuda")
-        rng.manual_seed(7)
-        q = torch.randn((kv * per, 1, d), device="cuda", generator=rng).half()
-        k, v = (torch.randn((kv, 5001, d), device="cuda", generator=rng).half() for _ in range(2))
-        shape = (kv * per, per, 1, 5001, d)
-        need, least = (kv * splits * per * (d + 2) * 4 for splits in (32, 27))
-        assert lib.anygpu_sdp_attention_decode_workspace_bytes(*shape, 1, 0) == need
-        rest = (*shape, d ** -0.5, 0.0, 1, 0, torch.cuda.current_stream().cuda_stream)
-        outs = []
-        for size in (need, least):
-            ws = torch.empty(size, dtype=torch.uint8, device="cuda")
-            outs.append(torch.empty_like(q))
-            assert lib.anygpu_sdp_attention_decode_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[-1].data_ptr(), ws.data_ptr(), size, *rest) == 0
-        ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr())
-        assert lib.anygpu_sdp_attention_decode_f16(*ptrs, outs[-1].data_ptr(), ws.data_ptr(), least - 1, *rest) == capi.ANYGPU_ERR_BAD_SHAPE
-        outs.append(torch.empty_like(q))
-        assert lib.anygpu_sdp_attention_decode_f16_static(*ptrs, outs[-1].data_ptr(), *rest) == 0
-        s = (q.float().view(kv, per, d) @ k.float().transpose(1, 2)) * d ** -0.5
-        want = host((torch.softmax(s, -1) @ v.float()).view(kv * per, 1, d))
-        for out in outs:
-            assert scaled_rel_err(host(out), want, float(np.abs(want).mean())) <= TOL_F16_GEMM
 
 
 def test_sdp_attention_decode_workspace_and_rejected_arguments(ops):
