@@ -1065,11 +1065,6 @@ hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, h
 // Workspace per (head, split, row): head_dim accumulators + maximum + sum, fp32.
 // ---------------------------------------------------------------------------------------------
 
-// Keys of a tile, and the grain in which they are shared out among the waves: 5001 keys are 157 tiles, five to each of 32 waves of a
-// head; in tiles of 64 they were 79, three (192 keys) to each of 27, and the other waves' SIMDs stood idle (batch 4, 32 / 8 heads
-// x 5001 keys x 128: 21.1 -> 18.9 us with the merge).
-constexpr int kDecodeKeysPerTile = 32;
-
 struct DecodeArgs
 {
 	AttnArgs a;
@@ -1125,7 +1120,7 @@ __global__ __launch_bounds__(64) void sdp_decode_partial_kernel(const DecodeArgs
 	// The keys are walked in tiles of 32 (one MFMA step of the second product).  The loads of tile u + 1 (K
 	// fragments straight into operand layout, V vectors for the wave's LDS tile) are in flight while tile u is
 	// multiplied: a wave that loaded, waited and multiplied in turn left the memory system idle half of the time.
-	constexpr int kSub = kDecodeKeysPerTile;
+	constexpr int kSub = kDecodeF16KeysPerTile;
 	constexpr int VPS = kSub * D / 8 / 64;                // V vectors per lane per tile
 	half8_t kf[2][2][KS];
 	float4_t vr[2][VPS];
@@ -1250,7 +1245,7 @@ __global__ __launch_bounds__(64) void sdp_decode_partial_kernel(const DecodeArgs
 template <int D, bool SOFTCAP>
 hipError_t launch_decode_variant(const DecodeArgs& da, int64_t kv_heads, hipStream_t stream)
 {
-	constexpr int kLdsBytes = kDecodeKeysPerTile * AttnLds<D>::kPitchV;
+	constexpr int kLdsBytes = kDecodeF16KeysPerTile * AttnLds<D>::kPitchV;
 	(void)hipGetLastError();
 	sdp_decode_partial_kernel<D, SOFTCAP><<<dim3(decode_blocks(da.groups, da.splits), (unsigned)kv_heads), dim3(64), kLdsBytes, stream>>>(da);
 	hipError_t e = hipGetLastError();
@@ -1340,36 +1335,12 @@ bool sdp_attention_decode_f16_supports(int64_t q_per_kv, int64_t n_q, int64_t he
 	return sdp_attention_fwd_f16_supports(head_dim) && q_per_kv >= 1 && n_q >= 1 && q_per_kv * n_q <= kDecodeMaxRows;
 }
 
-namespace {
-
-// Splits in tiles of 32 keys where a wave walks more than one tile of 64 (below that a finer cut only makes more partial results)
-// and `room` bytes of workspace hold the partial results, else in pairs of tiles: 64 keys, the grain whose need is the least
-// that the entry points ask for.
-DecodePlan plan_decode_f16(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim, int causal, int64_t window,
-                           int64_t room)
-{
-	const int64_t kv_heads = batch_heads / q_per_kv, rows = q_per_kv * n_q;
-	const int64_t units = kv_heads * ((rows + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave);
-	DecodePlan p = plan_decode(units, n_q, n_k, causal, window, 2 * kDecodeKeysPerTile);
-	if (p.tiles_per_split > 1)
-	{
-		const DecodePlan fine = plan_decode(units, n_q, n_k, causal, window, kDecodeKeysPerTile);
-		if (kv_heads * fine.splits * rows * (head_dim + 2) * (int64_t)sizeof(float) <= room) return fine;
-	}
-	p.t_first *= 2;
-	p.t_last = 2 * p.t_last + 1;
-	p.tiles_per_split *= 2;
-	return p;
-}
-
-}  // namespace
-
 int64_t sdp_attention_decode_workspace_bytes(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim,
                                              int causal, int64_t window, bool least)
 {
 	if (batch_heads == 0 || n_q == 0) return 0;
-	const DecodePlan p = plan_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window, least ? 0 : INT64_MAX);
-	return batch_heads / q_per_kv * p.splits * (q_per_kv * n_q) * (head_dim + 2) * (int64_t)sizeof(float);
+	const DecodePlansF16 plans = plans_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window);
+	return least ? plans.least_bytes() : plans.query_bytes();
 }
 
 hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const void* v, void* y, void* workspace, int64_t workspace_bytes,
@@ -1378,7 +1349,7 @@ hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const v
 {
 	if (batch_heads == 0 || n_q == 0) return hipSuccess;
 	const int64_t kv_heads = batch_heads / q_per_kv;
-	const DecodePlan p = plan_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window, workspace_bytes);
+	const DecodePlan p = plans_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window).within(workspace_bytes);
 	DecodeArgs da;
 	da.a.q = static_cast<const half_t*>(q);
 	da.a.k = static_cast<const half_t*>(k);

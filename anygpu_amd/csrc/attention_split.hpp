@@ -63,6 +63,45 @@ inline DecodePlan plan_decode(int64_t units, int64_t n_q, int64_t n_k, int causa
 	return p;
 }
 
+// Keys of a tile of the fp16 decode form, and the grain in which they are shared out among the waves: 5001 keys are 157 tiles, five
+// to each of 32 waves of a head; in tiles of 64 they were 79, three (192 keys) to each of 27, and the other waves' SIMDs stood idle
+// (batch 4, 32 / 8 heads x 5001 keys x 128: 21.1 -> 18.9 us with the merge).
+constexpr int kDecodeF16KeysPerTile = 32;
+
+// The two ways to cut the key range of a shape into splits, in tiles of 32 keys or in pairs of them (64 keys), and the bytes of
+// workspace that each takes.  Either can be the smaller one: under a window the finer tiles fit both ends of the visible range closer
+// (28 key / value heads, window 4096, 4128 keys: 32 splits, in pairs 33).
+struct DecodePlansF16
+{
+	DecodePlan fine, pairs;
+	int64_t fine_bytes, pairs_bytes;
+	bool take_fine;                                // the cut of a workspace of query_bytes()
+
+	int64_t query_bytes() const { return take_fine ? fine_bytes : pairs_bytes; }
+	// what the entry points ask for: callers that bring the bytes of the pairs are served, with that cut
+	int64_t least_bytes() const { return std::min(query_bytes(), pairs_bytes); }
+	// `room` >= least_bytes()
+	DecodePlan within(int64_t room) const { return take_fine && fine_bytes <= room ? fine : pairs; }
+};
+
+// The finer cut where a wave walks more than 64 keys.
+inline DecodePlansF16 plans_decode_f16(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim, int causal, int64_t window)
+{
+	const int64_t kv_heads = batch_heads / q_per_kv, rows = q_per_kv * n_q;
+	const int64_t units = kv_heads * ((rows + kDecodeRowsPerWave - 1) / kDecodeRowsPerWave);
+	DecodePlansF16 p;
+	p.fine = plan_decode(units, n_q, n_k, causal, window, kDecodeF16KeysPerTile);
+	p.pairs = plan_decode(units, n_q, n_k, causal, window, 2 * kDecodeF16KeysPerTile);
+	p.take_fine = p.pairs.tiles_per_split > 1;
+	p.pairs.t_first *= 2;
+	p.pairs.t_last = 2 * p.pairs.t_last + 1;
+	p.pairs.tiles_per_split *= 2;
+	const int64_t split_bytes = kv_heads * rows * (head_dim + 2) * (int64_t)sizeof(float);
+	p.fine_bytes = p.fine.splits * split_bytes;
+	p.pairs_bytes = p.pairs.splits * split_bytes;
+	return p;
+}
+
 // Which split and which group of 16 rows a block of the partial kernels works on.  The groups of one split read the
 // same keys, so they should run at the same time on the same XCD: consecutive blocks go to the eight XCDs in turn, so
 // block 8 t + x takes split 8 (t / groups) + x of group t % groups.  False: a block past the last split.

@@ -159,3 +159,13 @@ def test_sdp_attention_decode_takes_the_least_workspace(ops):
         want = host((torch.softmax(s, -1) @ v.float()).view(kv * per, 1, d))
         for out in outs:
             assert scaled_rel_err(host(out), want, float(np.abs(want).mean())) <= TOL_F16_GEMM
+
+
+def test_sdp_attention_decode_under_a_window_of_whole_tiles(ops, oracle):
+    # batch 7, 8 / 4 heads, window 4096, 4128 keys: the queried workspace is below that of the cut in tiles of 64
+    q, k, v = (synth.normal(60 + i, (7, h, n, 256)).astype(np.float16) for i, (h, n) in enumerate(((8, 1), (4, 4128), (4, 4128))))
+    got = host(ops.sdp_attention_fwd(dev(q), dev(k), dev(v), 0.0625, softcap=50.0, causal=True, window=4096)).astype(np.float32)
+    for b in (0, 6):
+        want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(np.ascontiguousarray(t[b])) for t in (q, k, v)), alpha=0.0625, softcap=50.0,
+                                          causal=True, window=4096, q_per_kv=2, threads=8)
+        assert scaled_rel_err(got[b], want, 1.0) <= TOL_F16_ROWOPS * 2
