@@ -13,6 +13,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "anygpu_hip.h"
 #include "device_utils.hpp"
 #include "launch.hpp"
 
@@ -25,6 +26,7 @@ constexpr int kDecodeMaxRows = 128;               // eight groups of sixteen
 // all splits) would have eaten that gain, since its time grew with the number of splits.
 constexpr int kDecodeMaxSplits = 256;
 constexpr int kDecodeTargetWaves = 1024;          // one wave per SIMD; two per SIMD measured 5 - 20 % slower
+constexpr int64_t kDecodeStaticBytes = ANYGPU_DECODE_STATIC_SCRATCH_BYTES;
 
 // a workspace row is head_dim + 2 floats long: its 16-byte accesses are aligned to 8 bytes only
 typedef float4_t WsFloat4 __attribute__((aligned(8)));
@@ -84,7 +86,9 @@ struct DecodePlansF16
 	DecodePlan within(int64_t room) const { return take_fine && fine_bytes <= room ? fine : pairs; }
 };
 
-// The finer cut where a wave walks more than 64 keys.
+// The finer cut where a wave walks more than 64 keys, and where the library's fixed scratch of kDecodeStaticBytes holds the partial
+// results of both cuts or of neither: that scratch and a workspace of query_bytes() then always give the same cut, and with
+// it the same bits.
 inline DecodePlansF16 plans_decode_f16(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k, int64_t head_dim, int causal, int64_t window)
 {
 	const int64_t kv_heads = batch_heads / q_per_kv, rows = q_per_kv * n_q;
@@ -92,13 +96,14 @@ inline DecodePlansF16 plans_decode_f16(int64_t batch_heads, int64_t q_per_kv, in
 	DecodePlansF16 p;
 	p.fine = plan_decode(units, n_q, n_k, causal, window, kDecodeF16KeysPerTile);
 	p.pairs = plan_decode(units, n_q, n_k, causal, window, 2 * kDecodeF16KeysPerTile);
-	p.take_fine = p.pairs.tiles_per_split > 1;
+	const bool long_walk = p.pairs.tiles_per_split > 1;
 	p.pairs.t_first *= 2;
 	p.pairs.t_last = 2 * p.pairs.t_last + 1;
 	p.pairs.tiles_per_split *= 2;
 	const int64_t split_bytes = kv_heads * rows * (head_dim + 2) * (int64_t)sizeof(float);
 	p.fine_bytes = p.fine.splits * split_bytes;
 	p.pairs_bytes = p.pairs.splits * split_bytes;
+	p.take_fine = long_walk && (p.fine_bytes <= kDecodeStaticBytes) == (p.pairs_bytes <= kDecodeStaticBytes);
 	return p;
 }
 

@@ -342,7 +342,9 @@ int anygpu_sdp_attention_fwd_masked_f16(const void* q, const void* k, const void
  * unnormalised accumulators, fp32) pass through `workspace` and are merged by a second kernel on the same stream.
  * anygpu_sdp_attention_decode_workspace_bytes returns the bytes needed for a shape (a negative error code for
  * arguments the decode form rejects); workspace must be 16-byte aligned device memory of at least that size and
- * may be reused by the next call on the same stream.  The reference has no decode kernel: its generation step
+ * may be reused by the next call on the same stream.  (The range is cut in tiles of 32 keys; a workspace below that size
+ * which still holds the partial results of a cut in tiles of 64 is accepted and gets that cut, whose sums round
+ * differently.  From that size on the bytes handed in make no difference.)  The reference has no decode kernel: its generation step
  * runs the per-head loop of srcs/transformers/sdp.hpp:258-271 against the cached keys.
  */
 int64_t anygpu_sdp_attention_decode_workspace_bytes(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k,
@@ -359,7 +361,7 @@ int anygpu_sdp_attention_decode_f16(const void* q, const void* k, const void* v,
  * allocation.  It has no counterpart in the reference.  The partial results pass through a fixed array of
  * ANYGPU_DECODE_STATIC_SCRATCH_BYTES of device memory that is part of the library's code object (every GPU the
  * library runs on holds its copy until the process ends); the call allocates and frees nothing.  Same kernels,
- * same split plan and bit-identical results to anygpu_sdp_attention_decode_f16.  A shape for which
+ * same split plan and bit-identical results to anygpu_sdp_attention_decode_f16 with a workspace of the queried size.  A shape for which
  * anygpu_sdp_attention_decode_workspace_bytes exceeds the array is rejected with ANYGPU_ERR_SCRATCH_TOO_SMALL and
  * nothing is launched.  All calls on one GPU share the array: calls on one stream are ordered by the stream, calls
  * that overlap on different streams of one GPU race.  The first call on a device looks up the array's address

@@ -10,6 +10,7 @@ HARNESS = r"""
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
+#define ANYGPU_DECODE_STATIC_SCRATCH_BYTES (8 * 1024 * 1024)
 namespace anygpu {
 %s
 }
@@ -28,6 +29,10 @@ static void check(int64_t kv, int64_t per, int64_t n_q, int64_t n_k, int64_t d, 
 	const auto ok = [&](bool c, const char* what) { expect(c, what, kv, rows, d, n_q, n_k, window); };
 	ok(least <= query, "the entry points ask for more than the size query returns");
 	ok(least <= p.pairs_bytes, "a workspace for the cut in 64 keys is refused");
+	const int64_t static_bytes = ANYGPU_DECODE_STATIC_SCRATCH_BYTES;
+	ok((least <= static_bytes) == (p.pairs_bytes <= static_bytes), "the fixed scratch takes other shapes than those whose cut in 64 keys fits it");
+	if (least <= static_bytes) ok(p.within(static_bytes).splits == p.within(query).splits && p.within(static_bytes).tiles_per_split == p.within(query).tiles_per_split,
+	                              "fixed scratch and queried workspace cut differently");
 	finer_needs_less += p.take_fine && p.fine_bytes < p.pairs_bytes;
 	for (int64_t room : {least, query, (least + query) / 2, query + 1000000})
 	{

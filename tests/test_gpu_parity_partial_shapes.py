@@ -133,30 +133,34 @@ def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, c
 
 def test_sdp_attention_decode_takes_the_least_workspace(ops):
     # 32 key / value heads x 5001 keys: 32 splits of 160 keys by the query, 27 of 192 in the least workspace (fp16), which stays
-    # enough, as does the library's scratch of 8 MB where only that split fits it (8 rows x 256: 7.1 MB against 8.5)
+    # enough.  Where the library's scratch of 8 MB holds the 27 splits only (8 rows x 256: 7.1 MB against 8.5), the query is theirs too,
+    # and with 28 heads and a window of 4096 the finer cut has the fewer splits.  The scratch always gives the bits of a workspace
+    # of the queried size.
     import torch
     from anygpu_amd import capi
     lib = capi.load()
-    for kv, per, d in ((32, 4, 128), (32, 8, 256)):
+    for kv, per, d, n_k, window, query, coarse in ((32, 4, 128, 5001, 0, 32, 27), (32, 8, 256, 5001, 0, 27, 27), (28, 2, 256, 4128, 4096, 32, 33)):
         rng = torch.Generator(device="cuda")
         rng.manual_seed(7)
         q = torch.randn((kv * per, 1, d), device="cuda", generator=rng).half()
-        k, v = (torch.randn((kv, 5001, d), device="cuda", generator=rng).half() for _ in range(2))
-        shape = (kv * per, per, 1, 5001, d)
-        need, least = (kv * splits * per * (d + 2) * 4 for splits in (32, 27))
-        assert lib.anygpu_sdp_attention_decode_workspace_bytes(*shape, 1, 0) == need
-        rest = (*shape, d ** -0.5, 0.0, 1, 0, torch.cuda.current_stream().cuda_stream)
+        k, v = (torch.randn((kv, n_k, d), device="cuda", generator=rng).half() for _ in range(2))
+        shape = (kv * per, per, 1, n_k, d)
+        need, least = (kv * splits * per * (d + 2) * 4 for splits in (query, min(query, coarse)))
+        assert lib.anygpu_sdp_attention_decode_workspace_bytes(*shape, 1, window) == need
+        rest = (*shape, d ** -0.5, 0.0, 1, window, torch.cuda.current_stream().cuda_stream)
+        ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr())
         outs = []
-        for size in (need, least):
+        for size in (need, need + 4096, least):
             ws = torch.empty(size, dtype=torch.uint8, device="cuda")
             outs.append(torch.empty_like(q))
-            assert lib.anygpu_sdp_attention_decode_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), outs[-1].data_ptr(), ws.data_ptr(), size, *rest) == 0
-        ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr())
+            assert lib.anygpu_sdp_attention_decode_f16(*ptrs, outs[-1].data_ptr(), ws.data_ptr(), size, *rest) == 0
         assert lib.anygpu_sdp_attention_decode_f16(*ptrs, outs[-1].data_ptr(), ws.data_ptr(), least - 1, *rest) == capi.ANYGPU_ERR_BAD_SHAPE
         outs.append(torch.empty_like(q))
         assert lib.anygpu_sdp_attention_decode_f16_static(*ptrs, outs[-1].data_ptr(), *rest) == 0
-        s = (q.float().view(kv, per, d) @ k.float().transpose(1, 2)) * d ** -0.5
-        want = host((torch.softmax(s, -1) @ v.float()).view(kv * per, 1, d))
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[3])
+        seen = slice(n_k - window, n_k) if window else slice(0, n_k)
+        s = (q.float().view(kv, per, d) @ k.float()[:, seen].transpose(1, 2).contiguous()) * d ** -0.5
+        want = host((torch.softmax(s, -1) @ v.float()[:, seen]).view(kv * per, 1, d))
         for out in outs:
             assert scaled_rel_err(host(out), want, float(np.abs(want).mean())) <= TOL_F16_GEMM
 
