@@ -7,10 +7,14 @@
 // queries, and two blocks (head dimension 64: three) share a CU without a barrier between them, so that one block's
 // softmax, loads and ends run beside the other's products, and causal launches of ordinary prompts have twice as many
 // pieces to pack onto the CUs.  Scores sit 32 to a lane (S^T = K Q^T: a lane holds one query), so row maxima are in-lane
-// but for one exchange of lane halves; sums come out of v_dot2 on the packed halves that the second product uses.
-// Measured, causal (us; before -> now): 32 / 8 heads x 3000 x 128 126 -> 85 (0.87 PFLOP/s), 16 x 4096 x 128 123 -> 95, 64 / 8 x
-// 1023 x 128 45.7 -> 30.2, 32 / 8 x 8192 x 128 647 -> 541 (1.02 PFLOP/s; a kernel that overlaps the products and the softmax inside
-// a wave ran at the same rate there, as the clock drops under the matrix units' power), 32 x 2048 x 64 43 -> 32.
+// but for one exchange of lane halves.  Sums are those of the fp32 p, and the maximum is exact in every tile, so that the largest p is
+// a power of two, which rounds to a half without an error (a maximum that lags until it is outgrown by 2^8 and sums of the
+// rounded p by v_dot2 measured 5 % faster, but up to a tenth further from 64-bit results: 16 heads x 4096 x 128, q of
+// N(0, 4): 2.36e-4 against 2.17e-4 (2-norm), of which the result's own rounding is 2.1e-4).
+// Measured, causal (us; 16-queries-per-wave kernels -> here): 32 / 8 heads x 3000 x 128 126.6 -> 94.9 (0.78 PFLOP/s), 16 x 4096 x 128 115.9 ->
+// 101.4, 64 / 8 x 1000 x 128 45.1 -> 31.8, 16 x 8192 x 128 367 -> 313 (0.88 PFLOP/s; a kernel that overlaps the products and the softmax
+// inside a wave ran at the same rate there, as the clock drops under the matrix units' power), 32 x 2038 x 64 41.9 -> 36.6; without the causal
+// rule 32 / 8 x 3000 x 128 183 -> 172, but 16 x 8192 x 128 542 -> 570 (the former kernel's rounds are full there).
 #pragma once
 
 #include "attention_walk.hpp"
@@ -23,6 +27,10 @@ namespace {
 
 constexpr int kQ32Waves = 4;
 constexpr int kQ32QueriesPerBlock = 32 * kQ32Waves;
+// p, which the second product takes as halves, is 2^15 for a score at the running maximum: with all of the halves' exponents
+// below it, p is a normal half (11 bits) down to 2^-29 of the maximum instead of 2^-14.  The factor is in the sums and the accumulators
+// alike, also in those that pass through the workspace, and cancels.
+constexpr float kQ32HeadRoom = 15.0f;
 
 // Chunk (16 bytes) of row r that the tile keeps at position c is c ^ swizzle(r): the tile rows are 2 D bytes without padding,
 // filled by direct loads whose lanes land on consecutive 16 bytes.  Both read patterns are free of bank conflicts with it
@@ -224,9 +232,9 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 		for (int i = 1; i < 16; ++i) mt = fmaxf(fmaxf(mt, s[0][i]), s[1][i]);
 		mt = max_over_lane_halves(mt);
 		if constexpr (!SOFTCAP) mt *= k_in;
-		// The maximum is only moved when a query of the wave has outgrown it by 2^8: until then p runs up to 256, which
-		// the halves hold with the same relative precision, and the pass over the accumulators is left out.
-		if (__builtin_amdgcn_ballot_w64(mt > m_run + 8.0f) != 0)
+		// the running maximum settles after some tiles; while no query of the wave raises it, the pass over the accumulators is
+		// left out
+		if (__builtin_amdgcn_ballot_w64(mt > m_run) != 0)
 		{
 			const float m_new = fmaxf(m_run, mt);
 			const float corr = fast_exp2(m_run - (m_new == -INFINITY ? 0.0f : m_new));
@@ -237,21 +245,24 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 #pragma unroll
 				for (int i = 0; i < 16; ++i) o[c][i] *= corr;
 		}
-		const float neg_m = m_run == -INFINITY ? 0.0f : -m_run;
+		const float m_safe = m_run == -INFINITY ? 0.0f : m_run;
+		const float z_add = kQ32HeadRoom - m_safe;
 		half8_t pf[2 * KB];
-		const half2_t ones = {(half_t)1.0f, (half_t)1.0f};
+		float psum[2] = {0.0f, 0.0f};
 #pragma unroll
 		for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
 			for (int i = 0; i < 16; i += 2)
 			{
-				const float z0 = SOFTCAP ? s[kb][i] + neg_m : fmaf(s[kb][i], k_in, neg_m);
-				const float z1 = SOFTCAP ? s[kb][i + 1] + neg_m : fmaf(s[kb][i + 1], k_in, neg_m);
-				const half2_t pp = {(half_t)fast_exp2(z0), (half_t)fast_exp2(z1)};
-				l_run = __builtin_amdgcn_fdot2(pp, ones, l_run, false);
-				pf[2 * kb + i / 8][i % 8] = pp[0];
-				pf[2 * kb + i / 8][i % 8 + 1] = pp[1];
+				const float z0 = SOFTCAP ? s[kb][i] + z_add : fmaf(s[kb][i], k_in, z_add);
+				const float z1 = SOFTCAP ? s[kb][i + 1] + z_add : fmaf(s[kb][i + 1], k_in, z_add);
+				const float p0 = fast_exp2(z0), p1 = fast_exp2(z1);
+				psum[0] += p0;
+				psum[1] += p1;
+				pf[2 * kb + i / 8][i % 8] = (half_t)p0;
+				pf[2 * kb + i / 8][i % 8 + 1] = (half_t)p1;
 			}
+		l_run += psum[0] + psum[1];
 
 		// ---- O^T += V^T P^T ----
 		__builtin_amdgcn_sched_barrier(0);

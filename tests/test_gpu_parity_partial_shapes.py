@@ -131,6 +131,90 @@ def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, c
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
+# many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
+
+def _scores_operands(heads, n_q, k0, d, q0=None):
+    import torch
+    q = torch.zeros((1, heads, n_q, d), dtype=torch.half, device="cuda")
+    q[..., 0] = 1.0 if q0 is None else dev(q0.astype(np.float16))
+    k = torch.zeros((1, 1, len(k0), d), dtype=torch.half, device="cuda")
+    k[0, 0, :, 0] = dev(k0.astype(np.float16))
+    return q, k
+
+
+def _softmax_product(scores, v):
+    w = np.exp(scores - scores.max(axis=-1, keepdims=True))
+    return (w @ v) / w.sum(axis=-1, keepdims=True)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("first", [True, False])
+def test_sdp_attention_32_queries_per_wave_small_weights_keep_their_bits(ops, d, first):
+    # one key with the largest score among keys whose weights are 2^-15 ... 2^-24 of it: as halves below 1 these would be denormal.
+    # The small weights come into the result rounded to 11 bits each (2^-11), as does the result (2^-11)
+    import torch
+    for n, b in ((1000, 17), (4096, 15), (4096, 17), (4096, 20), (4096, 24)):
+        k0 = np.full((n,), -b * math.log(2.0))
+        at = 0 if first else n - 1
+        k0[at] = 0.0
+        q, k = _scores_operands(512, 40, k0, d)
+        v = torch.ones((1, 1, n, d), dtype=torch.half, device="cuda")
+        v[:, :, at] = 0.0
+        small = (n - 1) * math.exp(float(np.float16(k0[n // 2])))
+        got = host(ops.sdp_attention_fwd(q, k, v, 1.0)).astype(np.float64)
+        assert np.abs(got / (small / (1.0 + small)) - 1.0).max() <= 2.0 ** -10 + 1e-5
+    # and into the sum in 32 bits: 65535 of 2^-23.6 each, which halves would round by a quarter
+    n, b = 65536, 23.6
+    k0 = np.full((n,), -b * math.log(2.0))
+    k0[0 if first else n - 1] = 0.0
+    q, k = _scores_operands(512, 40, k0, d)
+    v = torch.zeros((1, 1, n, d), dtype=torch.half, device="cuda")
+    v[:, :, 0 if first else n - 1] = 1.0
+    small = (n - 1) * math.exp(float(np.float16(k0[n // 2])))
+    got = host(ops.sdp_attention_fwd(q, k, v, 1.0)).astype(np.float64)
+    assert np.abs(got * (1.0 + small) - 1.0).max() <= 2.0 ** -11 + 1e-5
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("step", [0.3, 7.9, 8.1, 15.0, -8.1])
+def test_sdp_attention_32_queries_per_wave_moving_maximum(ops, d, step):
+    # the largest score of a tile of 64 keys is 2^step times that of the tile before, for one query of each wave; the other queries see
+    # the steps a hundredth as high.  Whole blocks (512 heads), and 32 heads x 40 queries over 20000 keys in parts, where
+    # the steps come round every seven tiles.  Weights and result rounded to 11 bits, |v| <= 1
+    rng = np.random.default_rng(5)
+    q0 = np.where(np.arange(40) % 32 == 5, 1.0, 0.01)
+    for heads, n in ((512, 7 * 64 - 3), (32, 20000)):
+        k0 = ((np.arange(n) // 64) % 7 * step + rng.uniform(-1.0, 0.0, n)) * math.log(2.0)
+        q, k = _scores_operands(heads, 40, k0, d, q0)
+        v = rng.uniform(-1.0, 1.0, (n, d)).astype(np.float16)
+        got = host(ops.sdp_attention_fwd(q, k, dev(v).reshape(1, 1, n, d), 1.0, decode=False)).astype(np.float64)
+        want = _softmax_product(np.float16(q0).astype(np.float64)[:, None] * np.float16(k0).astype(np.float64)[None, :], v.astype(np.float64))
+        assert np.abs(got[0] - want).max() <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_sdp_attention_32_queries_per_wave_nan_and_infinities(ops, d):
+    # a NaN in a query reaches its row; a NaN in a key, or a score of +inf, the rows that see the key; a score of -inf hides it
+    import torch
+    copies, heads, n = 64, 8, 200
+    q, k, v = (synth.normal(70 + i, (heads, n, d)).astype(np.float16) for i in range(3))
+    q[1, 37, 3] = np.nan
+    k[2, 150, 0] = np.nan
+    k[3, 100, 5] = np.inf
+    q[4, 11, 7] = -np.inf
+    alpha = d ** -0.5
+    got = host(ops.sdp_attention_fwd(*(dev(t).reshape(1, heads, n, d).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, causal=True))
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape), equal_nan=True)
+    s = torch.from_numpy(q).double() @ torch.from_numpy(k).double().transpose(1, 2).contiguous() * alpha
+    s = s.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), -math.inf)
+    want = (torch.softmax(s, -1) @ torch.from_numpy(v).double()).numpy()
+    assert np.array_equal(np.isnan(got[0]), np.isnan(want))
+    assert 0 < np.isnan(want).any(-1).sum() < heads * n // 2
+    seen = ~np.isnan(want)
+    assert scaled_rel_err(got[0].astype(np.float64)[seen], want[seen], 1.0) <= TOL_F16_ROWOPS * 2
+
+
 def test_sdp_attention_decode_takes_the_least_workspace(ops):
     # 32 key / value heads x 5001 keys: 32 splits of 160 keys by the query, 27 of 192 in the least workspace (fp16), which stays
     # enough.  Where the library's scratch of 8 MB holds the 27 splits only (8 rows x 256: 7.1 MB against 8.5), the query is theirs too,
