@@ -246,7 +246,23 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 				for (int i = 0; i < 16; ++i) o[c][i] *= corr;
 		}
 		const float m_safe = m_run == -INFINITY ? 0.0f : m_run;
-		const float z_add = kQ32HeadRoom - m_safe;
+		// p = 2^(z_in s + z_add).  The maximum is a rounded product, which the fma does not see as such: from 2^20 on, before
+		// the rounding can take p out of the halves' range, the difference is taken between rounded products
+		float z_in = SOFTCAP ? 1.0f : k_in, z_add = kQ32HeadRoom - m_safe;
+		if (__builtin_amdgcn_ballot_w64(fabsf(m_safe) > 0x1p20f) != 0)
+		{
+#pragma clang fp contract(off)
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+				for (int i = 0; i < 16; ++i)
+				{
+					const float z = SOFTCAP ? s[kb][i] : s[kb][i] * k_in;
+					s[kb][i] = z - m_safe;
+				}
+			z_in = 1.0f;
+			z_add = kQ32HeadRoom;
+		}
 		half8_t pf[2 * KB];
 		float psum[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -254,8 +270,8 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 #pragma unroll
 			for (int i = 0; i < 16; i += 2)
 			{
-				const float z0 = SOFTCAP ? s[kb][i] + z_add : fmaf(s[kb][i], k_in, z_add);
-				const float z1 = SOFTCAP ? s[kb][i + 1] + z_add : fmaf(s[kb][i + 1], k_in, z_add);
+				const float z0 = SOFTCAP ? s[kb][i] + z_add : fmaf(s[kb][i], z_in, z_add);
+				const float z1 = SOFTCAP ? s[kb][i + 1] + z_add : fmaf(s[kb][i + 1], z_in, z_add);
 				const float p0 = fast_exp2(z0), p1 = fast_exp2(z1);
 				psum[0] += p0;
 				psum[1] += p1;

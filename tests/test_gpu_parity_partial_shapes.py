@@ -194,6 +194,21 @@ def test_sdp_attention_32_queries_per_wave_moving_maximum(ops, d, step):
 
 
 @pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("alpha", [1.0, -1.0])
+def test_sdp_attention_32_queries_per_wave_scores_beyond_the_mantissa(ops, d, alpha):
+    # scores of 10^9 and more, whose rounding as a float is larger than the halves' range of exponents: still the row of the key
+    # with the largest score, bit for bit
+    import torch
+    n, heads = 300, 512
+    order = np.random.default_rng(6).permutation(n)
+    q = torch.full((1, heads, 130, d), 10000.0, dtype=torch.half, device="cuda")
+    k = dev((alpha * (10000.0 - 16.0 * order))[:, None].repeat(d, axis=1).astype(np.float16)).reshape(1, 1, n, d)
+    v = synth.normal(9, (1, 1, n, d)).astype(np.float16)
+    got = host(ops.sdp_attention_fwd(q, k, dev(v), alpha))
+    assert np.array_equal(got, np.broadcast_to(v[0, 0, int(np.argmin(order))], got.shape))
+
+
+@pytest.mark.parametrize("d", [64, 128])
 def test_sdp_attention_32_queries_per_wave_nan_and_infinities(ops, d):
     # a NaN in a query reaches its row; a NaN in a key, or a score of +inf, the rows that see the key; a score of -inf hides it
     import torch
