@@ -110,23 +110,29 @@ def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops,
     assert scaled_rel_err(got[:, 3:4], want, 1.0) <= TOL_F32
 
 
-# head dimensions 64 and 128 run 32 queries per wave, four waves and 128 queries per block, tiles of 64 keys: one query and
+# head dimensions 64 and 128 run 32 queries per wave, four waves and 128 queries per block, tiles of 64 keys, where there are more query
+# blocks than CUs (here: 66 copies of four heads), 16 queries per wave in eight waves where there are fewer: one query and
 # the edges of a wave's and a block's queries, tiles of one key, one short of whole and whole, queries of a wave that see
 # nothing, and the first and last tile of a window that only some waves of a block see
+@pytest.mark.parametrize("copies", [1, 66])
 @pytest.mark.parametrize("n_q,n_k,causal,window", [(1, 65, True, 0), (31, 64, True, 0), (33, 63, False, 0), (127, 129, True, 0), (128, 128, True, 0),
                                                     (129, 257, True, 70), (160, 100, True, 0), (300, 321, False, 64), (257, 600, True, 1)])
 @pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 0.0, -0.0884), (64, 30.0, 0.0), (128, 50.0, 0.0884)])
-def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, causal, window, d, cap, alpha):
+def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, causal, window, d, cap, alpha, copies):
     heads, kv_heads = 4, 2
+    if window and copies > 1:
+        copies *= 2                                              # (under a window from one and a half blocks per CU on)
     q = synth.normal(1 + n_q, (1, heads, n_q, d)).astype(np.float16)
     k = synth.normal(2 + n_k, (1, kv_heads, n_k, d)).astype(np.float16) * np.float16(4.0)        # (scores of tens: the running maximum moves)
     v = synth.normal(3 + d, (1, kv_heads, n_k, d)).astype(np.float16)
-    got = host(ops.sdp_attention_fwd(dev(q), dev(k), dev(v), alpha, softcap=cap, causal=causal, window=window, decode=False)).astype(np.float32)
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, softcap=cap, causal=causal, window=window,
+                                     decode=False)).astype(np.float32)
     want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=alpha, softcap=cap,
                                       causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
     blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
     assert not got[0][blind].any()
     assert np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
     # p rounded to fp16 (2^-11 each, weights that sum to 1) and the result's own rounding, values of up to about 4
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
@@ -195,11 +201,12 @@ def test_sdp_attention_32_queries_per_wave_moving_maximum(ops, d, step):
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("alpha", [1.0, -1.0])
-def test_sdp_attention_32_queries_per_wave_scores_beyond_the_mantissa(ops, d, alpha):
+@pytest.mark.parametrize("heads", [4, 512])
+def test_sdp_attention_scores_beyond_the_mantissa(ops, d, alpha, heads):
     # scores of 10^9 and more, whose rounding as a float is larger than the halves' range of exponents: still the row of the key
-    # with the largest score, bit for bit
+    # with the largest score, bit for bit (16 queries per wave with few heads, 32 with many)
     import torch
-    n, heads = 300, 512
+    n = 300
     order = np.random.default_rng(6).permutation(n)
     q = torch.full((1, heads, 130, d), 10000.0, dtype=torch.half, device="cuda")
     k = dev((alpha * (10000.0 - 16.0 * order))[:, None].repeat(d, axis=1).astype(np.float16)).reshape(1, 1, n, d)
