@@ -941,6 +941,25 @@ namespace anygpu {
 
 namespace {
 
+// Head dimensions 64 and 128, index rules: whether the longest query blocks go out in two halves of their key range (`blocks` of 128
+// queries in all; us, whole / cut).
+//   * Under a window, where most blocks are equally long, while they are one to one and a half for each CU: 9 heads x 4086 x 128, window 1024
+//     55.0 / 43.0, 12 heads 57.1 / 56.6; but 14 heads 46.0 / 62.0, 16 / 8 heads x 4096 52.5 / 61.8.
+//   * One block for each CU: where the blocks run from near nothing to the whole range from 31 tiles on (8 heads x 4086 x 128 78.5 / 61.8, 16 x
+//     2038 45.8 / 46.0; but 32 x 1014 26.7 / 30.0), else from 61 on, where two shorter blocks on a CU overlap enough to pay for the partial
+//     results' way through memory (no causal rule: 4 heads x 8182 x 64 114 / 104, 8 x 4086 x 64 61.6 / 61.0; but 16 x 2038 x 128 51.1 / 58.9).
+//   * More blocks: such a triangle of blocks only, up to one and a quarter for each CU (10 heads x 4086 x 128 81.2 / 69.7; 11 heads 77.7 /
+//     79.2), at head dimension 64 with very long ranges up to two (7 heads x 8182 x 64 122 / 105).
+template <int D>
+bool attention_cut_longest(const AttnArgs& args, int64_t blocks)
+{
+	const int64_t cus = device_cu_count(), tiles = (args.n_k + kAttnKeysPerTile - 1) / kAttnKeysPerTile;
+	if (args.window > 0) return blocks > cus && 2 * blocks <= 3 * cus;
+	const bool triangle = args.causal && 2 * args.diag <= args.n_q;
+	if (blocks <= cus) return tiles > (triangle ? 30 : 60);
+	return triangle && ((tiles > 30 && 4 * blocks <= 5 * cus) || (D == 64 && tiles >= 96 && blocks <= 2 * cus));
+}
+
 // Head dimensions 64 and 128, index rules: whether the kernel with 32 queries per wave takes the launch (`blocks` of 128 queries in all).
 // It does twice the work per wave and tile in half of the waves, which needs two blocks on a CU to pay: with up to one block per CU
 // the 16-queries-per-wave kernel is 7 - 13 % ahead (us, 32 / 16 queries: 8 heads x 64 x 128 5.7 / 5.0, 16 heads x 300 x 64 8.0 / 7.2, 32 heads x 600 x 128 17.5 / 16.5, 16 heads x 1700 x 128 39.6 / 35.5), with
@@ -968,20 +987,10 @@ hipError_t launch_q32(const AttnArgs& args_in, int64_t batch_heads, hipStream_t 
 	// (masked scores are -inf and meet k_in in a product)
 	if (args.k_in == 0.0f) args.k_in = 1e-30f;
 	const int64_t q_blocks = (args.n_q + kQueriesPerBlock - 1) / kQueriesPerBlock;
-	// The longest blocks in two halves of their key range only under a window, where most blocks are equally long, and where
-	// they make one to two blocks for each CU: up to 1.5 by the plan of the one-block-per-CU kernels (10 / 5 heads x 4096 x 128,
-	// window 1024: 51 -> 47 us); beyond it the rounds are even and a cut gains nothing, so the two-part form that windowed
-	// launches of this size have is left to the latest block of every head (16 / 8 x 4096 x 128, window 1024: 46 us, 58 with all
-	// long ones cut).  Elsewhere two short blocks to a CU even out by themselves, and the partial results' way through
-	// memory costs 8 - 20 % (32 / 8 heads x 3000 x 128 causal 92 -> 100 us).
 	AttnSplitPlan plan{0, 0};
-	const int64_t cus = device_cu_count(), blocks = q_blocks * batch_heads;
-	if (args.window > 0 && blocks > cus && blocks <= 2 * cus)
-	{
-		plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, kQueriesPerBlock,
-		                            kAttnKeysPerTile, D, band::workspace_capacity(stream), blocks * 2 <= cus * 3 ? 0.6 : 0.5);
-		if (blocks * 2 > cus * 3) plan.n_split = std::min<int64_t>(plan.n_split, 1);
-	}
+	if (attention_cut_longest<D>(args, q_blocks * batch_heads))
+		plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, kQueriesPerBlock, kAttnKeysPerTile, D,
+		                            band::workspace_capacity(stream));
 	// with too few query blocks for the chip, every block in several parts of its key range
 	const int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQueriesPerBlock,
 	                                                                      kAttnKeysPerTile, D, band::workspace_capacity(stream));
@@ -1032,8 +1041,10 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 	}
 	AttnArgs args = args_in;
 	const int64_t q_blocks = (args.n_q + kQueriesPerBlock - 1) / kQueriesPerBlock;
-	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads,
-	                                                kQueriesPerBlock, kAttnKeysPerTile, D, band::workspace_capacity(stream));
+	AttnSplitPlan plan{0, 0};
+	if (D == 256 || MASK || attention_cut_longest<D>(args, q_blocks * batch_heads))
+		plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads,
+		                            kQueriesPerBlock, kAttnKeysPerTile, D, band::workspace_capacity(stream));
 	// (or, with too few query blocks for the chip, every block in several parts of its key range)
 	const int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQueriesPerBlock,
 	                                                                    kAttnKeysPerTile, D, band::workspace_capacity(stream));

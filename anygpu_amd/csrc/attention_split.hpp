@@ -216,13 +216,13 @@ __global__ __launch_bounds__(256) void sdp_attention_merge_halves_kernel(const f
 }
 
 // How many of a head's latest query blocks to dispatch in two key halves (and how many unsplit ones go out before the
-// halves).  Worth it when whole blocks cannot be packed evenly: at least a block per CU, and the longest block more than
-// `share` of what a CU gets of the whole launch.  Bounded by the workspace of the stream (the K-split workspace of the
+// halves).  Worth it when whole blocks cannot be packed evenly: at least a block per CU, and the longest block a large
+// share of what a CU gets of the whole launch.  Bounded by the workspace of the stream (the K-split workspace of the
 // GEMMs: a caller's, or the library's own for eager launches; none under capture without a caller's: then no split).
 struct AttnSplitPlan { int64_t n_split, n_big; };
 
 inline AttnSplitPlan plan_attention_split(int n_q, int n_k, int causal, int diag, int window, int64_t batch_heads,
-                                          int queries_per_block, int keys_per_tile, int head_dim, size_t capacity, double share = 0.6)
+                                          int queries_per_block, int keys_per_tile, int head_dim, size_t capacity)
 {
 	AttnSplitPlan plan{0, 0};
 	const int64_t q_blocks = (n_q + queries_per_block - 1) / queries_per_block;
@@ -244,8 +244,8 @@ inline AttnSplitPlan plan_attention_split(int n_q, int n_k, int causal, int diag
 		longest = std::max(longest, tiles_of(b));
 	}
 	const double per_cu = (double)total * (double)batch_heads / (double)cus;
-	if (longest < 16 || (double)longest <= share * per_cu) return plan;
-	const int64_t split_min = std::max<int64_t>(16, (int64_t)(share * per_cu));
+	if (longest < 16 || (double)longest <= 0.6 * per_cu) return plan;
+	const int64_t split_min = std::max<int64_t>(16, (int64_t)(0.6 * per_cu));
 	// the latest blocks that are long enough, as far as the workspace holds their partial results
 	const int64_t room = (int64_t)(capacity / ((size_t)batch_heads * 2 * queries_per_block * (head_dim + 2) * sizeof(float)));
 	int64_t n_split = 0;

@@ -237,6 +237,37 @@ def test_sdp_attention_32_queries_per_wave_nan_and_infinities(ops, d):
     assert scaled_rel_err(got[0].astype(np.float64)[seen], want[seen], 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# head dimensions 64 and 128 with 32 queries per wave: the longest blocks in two halves of their key range (causal, 320 blocks; window, 288
+# blocks; long ranges, 448 blocks) and all blocks in parts of a long range (32 blocks x 313 tiles), and 256 blocks with 16 queries per
+# wave in halves: against whole blocks, which a workspace without room gives, and the oracle
+@pytest.mark.parametrize("heads,kv_heads,n_q,n_k,d,causal,window", [(10, 5, 4086, 4086, 128, True, 0), (9, 3, 4086, 4086, 64, True, 1024),
+                                                                     (7, 7, 8182, 8182, 64, True, 0), (16, 2, 200, 20000, 64, True, 0),
+                                                                     (32, 4, 70, 20000, 128, True, 0), (8, 8, 4086, 4086, 64, True, 0)])
+def test_sdp_attention_key_parts_agree_with_whole_blocks(ops, oracle, heads, kv_heads, n_q, n_k, d, causal, window):
+    import torch
+    q = synth.normal(31, (heads, n_q, d)).astype(np.float16)
+    k = synth.normal(32, (kv_heads, n_k, d)).astype(np.float16) * np.float16(2.0)
+    v = synth.normal(33, (kv_heads, n_k, d)).astype(np.float16)
+    alpha = d ** -0.5
+    run = lambda: host(ops.sdp_attention_fwd(dev(q), dev(k), dev(v), alpha, causal=causal, window=window, decode=False)).astype(np.float32)
+    parts = run()
+    tiny = torch.empty((64,), device="cuda")
+    ops.set_workspace(tiny)
+    try:
+        whole = run()
+    finally:
+        torch.cuda.synchronize()
+        ops.set_workspace(None)
+    assert not np.array_equal(parts, whole), "the launch was expected to take parts of the key range"
+    idx = np.array(sorted({0, 31, 63, n_q // 2, n_q - 130, n_q - 70, n_q - 1} & set(range(n_q))), dtype=np.int64)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t) for t in (q, k, v)), alpha=alpha, softcap=0.0, causal=causal, window=window,
+                                      q_per_kv=heads // kv_heads, query_index=idx, threads=8)
+    for got in (parts, whole):
+        assert np.isfinite(got).all()
+        assert scaled_rel_err(got[:, idx, :], want, 1.0) <= TOL_F16_ROWOPS * 2
+    assert scaled_rel_err(parts, whole, 1.0) <= 2e-3
+
+
 def test_sdp_attention_decode_takes_the_least_workspace(ops):
     # 32 key / value heads x 5001 keys: 32 splits of 160 keys by the query, 27 of 192 in the least workspace (fp16), which stays
     # enough.  Where the library's scratch of 8 MB holds the 27 splits only (8 rows x 256: 7.1 MB against 8.5), the query is theirs too,
