@@ -962,18 +962,19 @@ bool attention_cut_longest(const AttnArgs& args, int64_t blocks)
 
 // Head dimensions 64 and 128, index rules: whether the kernel with 32 queries per wave takes the launch (`blocks` of 128 queries in all).
 // It does twice the work per wave and tile in half of the waves, which needs two blocks on a CU to pay: with up to one block per CU
-// the 16-queries-per-wave kernel is 7 - 13 % ahead (us, 32 / 16 queries: 8 heads x 64 x 128 5.7 / 5.0, 16 heads x 300 x 64 8.0 / 7.2, 32 heads x 600 x 128 17.5 / 16.5, 16 heads x 1700 x 128 39.6 / 35.5), with
-// more it falls behind (36 heads x 1014 x 128 28.9 / 31.3, 32 x 1200 x 128 30.5 / 33.5, 32 x 3000 x 128 93 / 107, 16 x 8192 x 64 178 / 197); under a window
-// at head dimension 128 from one and a half blocks on (12 / 4 heads x 4096, window 512 45.8 / 42.9; 13 x 4000, window 1024 43.9 / 57.4).
+// the 16-queries-per-wave kernel is 7 - 13 % ahead (us, 32 / 16 queries: 8 heads x 64 x 128 5.7 / 5.0, 16 heads x 300 x 64 8.0 / 7.2, 32 heads x
+// 600 x 128 17.5 / 16.5, 16 heads x 1700 x 128 39.6 / 35.5), with more it falls behind (36 heads x 1014 x 128 28.9 / 31.3, 32 x 1200 x 128
+// 30.5 / 33.5, 32 x 3000 x 128 93 / 107, 16 x 8192 x 64 178 / 197); under a window at head dimension 128 from one and a half blocks on (12 /
+// 4 heads x 4096, window 512 45.8 / 42.9; 13 x 4000, window 1024 43.9 / 57.4).
 // Launches of up to half a block per CU go out in several parts of their key range per block, which makes the blocks: there 32
-// queries pay from 32 key tiles per CU on, where there is a workspace for the parts (32 / 8 heads x 128 queries x 4000 keys x 128 33.1 / 31.6, 20000 68.0 / 68.4; 64 / 8 x 64 x 20000 80.7 / 98.4,
-// 16 x 1000 x 20000 x 64 116 / 126).
+// queries pay from 32 key tiles per CU on, where the workspace holds the parts' results (32 / 8 heads x 128 queries x 4000 keys x 128
+// 33.1 / 31.6, 20000 68.0 / 68.4; 64 / 8 x 64 x 20000 80.7 / 98.4, 16 x 1000 x 20000 x 64 116 / 126).
 template <int D>
-bool attention_q32_wanted(const AttnArgs& args, int64_t blocks, size_t workspace)
+bool attention_q32_wanted(const AttnArgs& args, int64_t blocks, bool in_parts)
 {
 	const int64_t cus = device_cu_count(), tiles = (args.n_k + kAttnKeysPerTile - 1) / kAttnKeysPerTile;
 	if (args.window > 0) return D == 64 ? blocks > cus : 2 * blocks > 3 * cus;
-	return blocks > cus || (2 * blocks <= cus && blocks * tiles > 32 * cus && workspace > 0);
+	return blocks > cus || (2 * blocks <= cus && blocks * tiles > 32 * cus && in_parts);
 }
 
 template <int D, bool SOFTCAP>
@@ -1077,7 +1078,9 @@ hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, h
 	else
 	{
 		const int64_t blocks = (args.n_q + kQ32QueriesPerBlock - 1) / kQ32QueriesPerBlock * batch_heads;
-		if (attention_q32_wanted<D>(args, blocks, band::workspace_capacity(stream)))
+		const bool in_parts = plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQ32QueriesPerBlock, kAttnKeysPerTile, D,
+		                                           band::workspace_capacity(stream)) > 1;
+		if (attention_q32_wanted<D>(args, blocks, in_parts))
 			return softcap ? launch_q32<D, true>(args, batch_heads, stream) : launch_q32<D, false>(args, batch_heads, stream);
 		return softcap ? launch_variant<D, true, 1>(args, batch_heads, stream) : launch_variant<D, false, 1>(args, batch_heads, stream);
 	}
