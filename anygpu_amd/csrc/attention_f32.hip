@@ -252,25 +252,8 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const
 	};
 	// MASK: the walk visits the tiles that the map has set (all of them without a map); t_next is the tile after t on
 	// that walk, the stages alternate along it
-	// (the word of 64 tiles that the walk is in stays in registers: read anew for every tile it cost a memory latency each)
-	unsigned long long map_word = 0;
-	int map_at = -1;
-	auto next_tile = [&](int t) {
-		if (map_row == nullptr) return t;
-		while (t <= t_last)
-		{
-			if ((t >> 6) != map_at)
-			{
-				map_at = t >> 6;
-				map_word = map_row[map_at];
-			}
-			const unsigned long long bits = map_word >> (t & 63);
-			if (bits != 0) return t + __builtin_ctzll(bits);       // (past t_last: the walk has ended)
-			t = (t | 63) + 1;
-		}
-		return t;
-	};
-	if constexpr (MASK) t_first = next_tile(t_first);
+	AttentionVisibleWalk visible{map_row};
+	if constexpr (MASK) t_first = visible.next(t_first, t_last);
 	if (t_first <= t_last)
 	{
 		if constexpr (MASK) load_mask(mk_next, t_first);
@@ -282,7 +265,7 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const
 	{
 		const float* k_lds = lds_base;
 		const int stage = MASK ? stage_m : (t - t_first) & 1;
-		if constexpr (MASK) t_next = next_tile(t + 1);
+		if constexpr (MASK) t_next = visible.next(t + 1, t_last);
 		else t_next = t + 1;
 		if constexpr (DIRECT)
 		{

@@ -116,6 +116,32 @@ __device__ __forceinline__ int attention_next_visible_tile(const unsigned long l
 	return t_last + 1;
 }
 
+// The same walk with the word of 64 tiles that it is in kept in registers (read anew for every tile it cost the fp32 kernel a memory
+// latency each).  Behind the last set tile the result is any index past t_last.
+struct AttentionVisibleWalk
+{
+	const unsigned long long* map_row;             // nullptr: every tile counts as set
+	unsigned long long word = 0;
+	int at = -1;
+
+	__device__ __forceinline__ int next(int t, int t_last)
+	{
+		if (map_row == nullptr) return t;
+		while (t <= t_last)
+		{
+			if ((t >> 6) != at)
+			{
+				at = t >> 6;
+				word = map_row[at];
+			}
+			const unsigned long long bits = word >> (t & 63);
+			if (bits != 0) return t + __builtin_ctzll(bits);
+			t = (t | 63) + 1;
+		}
+		return t;
+	}
+};
+
 // The share of part `part` of `parts` among the set tiles of [t_first, t_last]: narrows the range to the set tiles number
 // part * per .. (part + 1) * per - 1, per = ceil(set tiles / parts), so that the parts of a query block's key range carry
 // equal numbers of visible tiles wherever the mask hides the others (a sliding window over a long cache leaves most

@@ -1,7 +1,7 @@
 """The scalar helpers with which the attention kernels walk the visible-tile map of a mask tensor
-(anygpu_amd/csrc/attention_tile_map.hpp): the next set tile of a range, and the share of a part among the set tiles.
-Their text is compiled for the host (they use nothing of the device but its qualifiers) and checked against brute
-force over random maps, ranges and part counts.  CPU only."""
+(anygpu_amd/csrc/attention_tile_map.hpp): the next set tile of a range, the walk that keeps the map's word, and the
+share of a part among the set tiles.  Their text is compiled for the host (they use nothing of the device but its
+qualifiers) and checked against brute force over random maps, ranges and part counts.  CPU only."""
 import subprocess
 from pathlib import Path
 
@@ -39,6 +39,18 @@ int main()
 			for (int v : set)
 				if (v >= t) { want = v; break; }
 			if (anygpu_next(map.data(), t, t1) != want) { std::printf("next set tile: mismatch\n"); return 1; }
+		}
+		// the walk that keeps its word, over the set tiles and over every tile (past the last set one: anything past t1)
+		AttentionVisibleWalk walk{map.data()}, steps{map.data()}, all{nullptr};
+		size_t at = 0;
+		for (int t = walk.next(t0, t1); t <= t1; t = walk.next(t + 1, t1), ++at, ++checks)
+			if (at >= set.size() || set[at] != t) { std::printf("walk: mismatch\n"); return 1; }
+		if (at != set.size()) { std::printf("walk: ended early\n"); return 1; }
+		for (int t = t0; t <= t1; ++t, ++checks)
+		{
+			const int got = steps.next(t, t1), want = anygpu_next(map.data(), t, t1);
+			if (want <= t1 ? got != want : got <= t1) { std::printf("step: mismatch\n"); return 1; }
+			if (all.next(t, t1) != t) { std::printf("walk without a map: mismatch\n"); return 1; }
 		}
 		const int parts = 1 + rng() %% 9, total = (int)set.size(), per = (total + parts - 1) / parts;
 		for (int p = 0; p < parts; ++p, ++checks)
