@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
                                        (9, 16, 257), (16, 36, 2048), (12, 19, 4099), (16, 17, 6000), (8, 144, 130)])
 def test_mm_few_rows_k_cut_over_waves(ops, oracle, dtype, m, steps, n):
     # up to 16 rows against k-contiguous weights, K in steps of 128 bytes from 16 of them on (two for each of eight waves), blocks of 1 to
-    # 33 columns that end past N, operands and results inside wider buffers.  Small integers: the sums are exact in both types (below 2048).
+    # 32 columns that end past N, operands and results inside wider buffers.  Small integers: the sums are exact in both types (below 2048).
     import torch
     from anygpu_amd import capi
     np_dt, t_dt = (np.float16, torch.float16) if dtype == "f16" else (np.float32, torch.float32)
@@ -45,6 +45,26 @@ def test_mm_few_rows_k_cut_over_waves(ops, oracle, dtype, m, steps, n):
     got = host(ops.mlp_gemma2_fused_upproj(dev((a * scale).astype(np_dt)), dev(bt), dev(b2t), b_layout=capi.B_COL_MAJOR)).astype(np.float64)
     gated = 0.5 * s1 * (1.0 + np.tanh(math.sqrt(2.0 / math.pi) * (s1 + 0.044715 * s1 ** 3))) * s2
     assert np.all(np.abs(got - gated) <= half_ulp * np.abs(gated) + 1e-6 * np.abs(s1 * s2) + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("m", [3, 8, 16])
+def test_mm_few_rows_k_cut_over_waves_nan_and_infinities(ops, dtype, m):
+    # a NaN or an infinity reaches the row (left operand) or column (weights) that it belongs to and no other, in either half of a step's
+    # chunks and in the shares of different waves; +inf and -inf that meet in a sum give NaN
+    import torch
+    from anygpu_amd import capi
+    t_dt, k, n = (torch.float16, 64 * 19, 300) if dtype == "f16" else (torch.float32, 32 * 19, 300)
+    a, w = (torch.from_numpy(synth.integers(s, shape, -2, 2)).to(t_dt) for s, shape in ((5, (m, k)), (6, (n, k))))
+    a[1, 3] = math.nan
+    a[2, k - 1], w[:, k - 1] = math.inf, 1.0
+    w[7, k // 2 + 9], a[:, k // 2 + 9] = math.nan, 2.0
+    w[9, 17], w[9, k - 40], a[:, 17], a[:, k - 40] = math.inf, -math.inf, 1.0, 1.0
+    w[299, 40], a[:, 40] = -math.inf, 1.0
+    want = a.double() @ w.double().t().contiguous()
+    got = host(ops.tensor_mm(dev(a.numpy()), dev(w.numpy()), b_layout=capi.B_COL_MAJOR)).astype(np.float64)
+    assert np.array_equal(got, want.numpy(), equal_nan=True)
+    assert 0 < np.isnan(got).sum() < got.size // 2
 
 
 @pytest.mark.parametrize("m,n,k", [(17, 31, 1), (3, 33, 31), (33, 32, 32), (32, 95, 63), (64, 64, 128), (65, 70, 129), (31, 100, 256),
@@ -80,11 +100,11 @@ def test_gemm_f32_small_products(ops, oracle, m, n, k, layout):
 
 
 def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops, oracle, monkeypatch):
-    # head dimension 256 with fewer blocks than CUs (16 heads x 10 blocks of 128 queries; 66 key tiles, so up to four parts):
-    # the parts take more than the workspace holds to begin with, which grows; against a caller's workspace that only has
-    # room for the map (whole blocks), and one head against the oracle
+    # head dimension 256 with fewer blocks than CUs (16 heads x 12 blocks of 128 queries; 66 key tiles): four parts, whose results take 101 MB,
+    # more than the workspace holds to begin with, which grows.  Against a caller's workspace of 64 MB, which has room for two parts,
+    # and one that only has room for the map (whole blocks), and one head against the oracle
     import torch
-    heads, n_q, n_k, d = 16, 1190, 2090, 256
+    heads, n_q, n_k, d = 16, 1500, 2090, 256
     q = synth.normal(81, (1, heads, n_q, d))
     k = synth.normal(82, (1, heads, n_k, d))
     v = synth.normal(83, (1, heads, n_k, d))
@@ -95,19 +115,21 @@ def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops,
     mask4 = mask.reshape(1, 1, n_q, n_k)
     dq, dk, dv, dm = dev(q), dev(k), dev(v), dev(mask4)
     monkeypatch.setenv("ANYGPU_ATTN_MASK_MAP_FROM", "0")
-    got = host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))
-    small = torch.empty(1 << 17, dtype=torch.uint8, device="cuda")
-    ops.set_workspace(small)
-    try:
-        whole = host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))
-    finally:
-        torch.cuda.synchronize()
-        ops.set_workspace(None)
-    assert np.isfinite(got).all()
-    assert scaled_rel_err(got, whole, 1.0) <= 1e-5
-    assert not np.array_equal(got, whole), "the two runs were expected to sum in different orders"
+    got = [host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha))]
+    for size in (1 << 26, 1 << 17):
+        workspace = torch.empty(size, dtype=torch.uint8, device="cuda")
+        ops.set_workspace(workspace)
+        try:
+            got.append(host(ops.sdp_attention_masked_scaled_fwd(dq, dk, dv, dm, alpha)))
+        finally:
+            torch.cuda.synchronize()
+            ops.set_workspace(None)
+    assert all(np.isfinite(y).all() for y in got)
+    for i, j in ((0, 1), (0, 2), (1, 2)):
+        assert scaled_rel_err(got[i], got[j], 1.0) <= 1e-5
+        assert not np.array_equal(got[i], got[j]), "the three runs were expected to sum in different orders"
     want = oracle.sdp_attention_masked_scaled_fwd(q[:, 3:4], k[:, 3:4], v[:, 3:4], mask4, alpha, threads=8)
-    assert scaled_rel_err(got[:, 3:4], want, 1.0) <= TOL_F32
+    assert scaled_rel_err(got[0][:, 3:4], want, 1.0) <= TOL_F32
 
 
 # head dimensions 64 and 128 run 32 queries per wave, four waves and 128 queries per block, tiles of 64 keys, where there are more query
