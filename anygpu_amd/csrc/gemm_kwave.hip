@@ -16,9 +16,10 @@
 // 512 of 18), as a CU with one block more than the others is what the launch waits for (2304 columns in 288 blocks of 8: 18 us,
 // in 256 of 9: 11.5), and few, as every block reads the whole left operand.  Two steps in flight per wave, eight waves to a block
 // of up to 16 rows and four to a larger one (depths of 2, 3, 4 and 4, 8, 16 waves were measured).
-// Measured, us before -> now, 8 rows, fp16: 2304 -> 9216 with the GELU of two matrices 29.4 -> 15.2, 9216 -> 2304 13.7 -> 11.5,
-// 2304 -> 2048 8.5 -> 4.5, 4096 -> 4096 11.0 -> 7.9, 3584 -> 18944 33 -> 23.5; fp32: 2304 -> 9216 25.7 -> 18, two matrices 46.8 -> 31.4,
-// 14336 -> 4096 51 -> 42.
+// Measured, us before -> now, 8 rows, weights from memory (700 MB of them walked in turn), fp16: 2304 -> 9216 with the GELU of two matrices
+// 30.7 -> 16.6, 9216 -> 2304 19.8 -> 12.3 (3.5 TB/s), 2304 -> 2048 10.4 -> 4.6, 4096 -> 4096 14.2 -> 8.3, 3584 -> 18944 35.5 -> 25.5 (5.3 TB/s).
+// A matrix that the caches still hold from the product before is read at their rate by either kernel, where the one with a band
+// of A in LDS can be a tenth ahead (9216 x 2304 10.0 / 11.2, 18944 x 3584 22.9 / 25.2; 2304 x 9216 14.2 / 12.9).
 #include "gemm_band.hpp"
 #include "anygpu_hip.h"
 
@@ -206,7 +207,8 @@ hipError_t launch_kwave_rows(const T* A, const T* B, const T* B2, const T* bias,
 
 // Rows of both operands at 16-byte boundaries and whole steps of 128 bytes of K, enough of them for every wave, and the row
 // counts at which it is ahead of what took these products before (us, before / here):
-// one matrix, up to 8 rows: from 2 rows in fp16 (9216 x 2304 weights, 1 row: 7.8 / 8.5, 2 rows: 9.0 / 8.5, 3 rows: 9.7 / 8.9) and
+// one matrix, up to 8 rows: from 2 rows in fp16 (weights from memory, 2 rows: 9216 x 2304 9.8 / 9.8, 2304 x 9216 11.6 / 10.0, 4096 x 4096
+//   8.3 / 7.6, 14336 x 4096 22.8 / 21.2, 3000 x 1024 3.5 / 3.7; out of the caches 9.1 / 9.4, 10.9 / 11.2, 6.8 / 7.8, -, 3.1 / 3.6; 3 rows: 15.3 / 9.6) and
 //   from 3 in fp32 (2 rows: 16.3 / 16.2; 3 rows: 25.3 / 17);
 // one matrix, 9 - 16 rows, where the left operand's way through the L2s grows with the rows: small weight matrices only (fp16,
 //   16 rows: 2048 x 2304 8.5 / 5.6, but 9216 x 2304 9.9 / 12.0; fp32: 2048 x 2048 9.8 / 8.0, 9216 x 2304 26.0 / 26.4);
