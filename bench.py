@@ -68,9 +68,9 @@ MEASURED_TRAFFIC = {
     "attention_gemma2": (530927292, "profiles/sdp_attention_fwd_f16_gemma2_kernel.md"),
     "attention_gemma2_f32": (1308870403, "profiles/sdp_attention_fwd_f32_gemma2_kernel.md"),
     "gated_rmsnorm": (805405955, "profiles/gated_rmsnorm_f16_row_kernel.md"),
-    "attention_decode": (144037358, "profiles/sdp_attention_decode_f16_partial_and_merge_kernels.md"),
-    "lm_head_f32": (2391557676, "profiles/gemma_linear_softcap_head_band_kernels.md"),
-    "lm_head_f16": (1203714309, "profiles/gemma_linear_softcap_head_band_kernels.md"),
+    "attention_decode": (144062464, "profiles/sdp_attention_decode_f16_partial_and_merge_kernels.md"),
+    "lm_head_f32": (2368142029, "profiles/gemma_linear_softcap_head_kwave_kernel.md"),
+    "lm_head_f16": (1184094208, "profiles/gemma_linear_softcap_head_kwave_kernel.md"),
 }
 
 
