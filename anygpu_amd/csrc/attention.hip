@@ -101,16 +101,16 @@ struct AttnLds
 	static constexpr int kBytes = kAttnKeysPerTile * (kPitchK + kPitchV);
 };
 
-// WAVES: waves per block; a block owns 16 * WAVES consecutive queries.
+// QB: 16-query blocks per wave, WAVES: waves per block; a block owns 16 * QB * WAVES consecutive queries.
 // MASK: an additive mask tensor instead of the index rules (the launcher passes none): the four mask values of a lane's four scores
 // of a key block are consecutive in memory; they are requested a tile ahead and added behind scale and softcap; a tile
 // that the mask hides from every query of a wave costs the wave no products (it still issues its share of the next
 // tile's loads); a tile that the visible-tile map of the mask (attention_tile_map.hpp) has not set for the block is
 // neither loaded nor waited for.
-template <int D, bool SOFTCAP, int WAVES, bool MASK = false>
+template <int D, bool SOFTCAP, int QB, int WAVES, bool MASK = false>
 __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const AttnArgs a, const AttnWalk walk)
 {
-	constexpr int kAttnQueriesPerBlock = 16 * WAVES;
+	constexpr int kAttnQueriesPerBlock = 16 * QB * WAVES;
 	extern __shared__ __align__(16) char lds[];
 	using L = AttnLds<D>;
 	// (these follow the stage of the tile in use)
@@ -160,26 +160,42 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 	}
 
 	// this wave's queries as second operands: lane (n, g) holds q[row][32 s + 8 g .. + 7]
-	const int q_row = q0 + 16 * wave + n;
-	half8_t qf[KS];
+	int q_row[QB];
+	half8_t qf[QB][KS];
 #pragma unroll
-	for (int s = 0; s < KS; ++s)
+	for (int b = 0; b < QB; ++b)
 	{
-		half8_t val = {};
-		if (q_row < a.n_q) val = *reinterpret_cast<const half8_t*>(qp + (int64_t)q_row * D + 32 * s + 8 * g);
-		qf[s] = val;
-	}
-	// visible keys of the query this lane serves: lo <= key <= hi
-	int vis_hi = a.causal ? q_row + a.diag : a.n_k - 1;
-	if (vis_hi > a.n_k - 1) vis_hi = a.n_k - 1;
-	const int vis_lo = a.window > 0 ? q_row + a.diag - a.window + 1 : 0;
-
-	float m_run = -INFINITY, l_run = 0.0f;         // l_run: this lane's share of the row sum
-	float4_t o[DC];
+		q_row[b] = q0 + 16 * QB * wave + 16 * b + n;
 #pragma unroll
-	for (int c = 0; c < DC; ++c) o[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+		for (int s = 0; s < KS; ++s)
+		{
+			half8_t val = {};
+			if (q_row[b] < a.n_q) val = *reinterpret_cast<const half8_t*>(qp + (int64_t)q_row[b] * D + 32 * s + 8 * g);
+			qf[b][s] = val;
+		}
+	}
+	// visible keys of each of the two queries this lane serves: lo <= key <= hi
+	int vis_lo[QB], vis_hi[QB];
+#pragma unroll
+	for (int b = 0; b < QB; ++b)
+	{
+		vis_hi[b] = a.causal ? q_row[b] + a.diag : a.n_k - 1;
+		if (vis_hi[b] > a.n_k - 1) vis_hi[b] = a.n_k - 1;
+		vis_lo[b] = a.window > 0 ? q_row[b] + a.diag - a.window + 1 : 0;
+	}
+
+	float m_run[QB], l_run[QB];                    // l_run: this lane's share of the row sum
+	float4_t o[QB][DC];
+#pragma unroll
+	for (int b = 0; b < QB; ++b)
+	{
+		m_run[b] = -INFINITY;
+		l_run[b] = 0.0f;
+#pragma unroll
+		for (int c = 0; c < DC; ++c) o[b][c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+	}
 	// keys visible to every query of this wave need no per-element test: [all_lo, all_hi]
-	const int wq0 = q0 + 16 * wave, wq1 = wq0 + 15;
+	const int wq0 = q0 + 16 * QB * wave, wq1 = wq0 + 16 * QB - 1;
 	const int all_hi = a.causal ? (wq0 + a.diag < a.n_k - 1 ? wq0 + a.diag : a.n_k - 1) : a.n_k - 1;
 	const int all_lo = a.window > 0 ? wq1 + a.diag - a.window + 1 : 0;
 
@@ -231,34 +247,38 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 	// alignment: a whole 128-byte line per query and pair of instructions), and when the tile's turn comes the lane
 	// groups exchange 8-byte pieces by row swaps in the VALU (a 4 x 4 transposition over g).  Keys past the end and
 	// rows past the last query count as hidden.
-	half4_t mk_next[4];
+	half4_t mk_next[MASK ? QB : 1][4];
 	auto load_mask = [&](int t) {
 		typedef half8_t LooseHalf8 __attribute__((aligned(2)));
-		const int key = t * kAttnKeysPerTile + 16 * g;
-		const half_t hidden = (half_t)(-INFINITY);
-		half8_t lo = {hidden, hidden, hidden, hidden, hidden, hidden, hidden, hidden}, hi = lo;
-		if (q_row < a.n_q)
-		{
-			const half_t* src = a.mask + (int64_t)q_row * a.mask_stride + key;
-			if (key + 15 < a.n_k)
-			{
-				lo = *reinterpret_cast<const LooseHalf8*>(src);
-				hi = *reinterpret_cast<const LooseHalf8*>(src + 8);
-			}
-			else
-			{
 #pragma unroll
-				for (int r = 0; r < 8; ++r)
+		for (int b = 0; b < (MASK ? QB : 0); ++b)
+		{
+			const int key = t * kAttnKeysPerTile + 16 * g;
+			const half_t hidden = (half_t)(-INFINITY);
+			half8_t lo = {hidden, hidden, hidden, hidden, hidden, hidden, hidden, hidden}, hi = lo;
+			if (q_row[b] < a.n_q)
+			{
+				const half_t* src = a.mask + (int64_t)q_row[b] * a.mask_stride + key;
+				if (key + 15 < a.n_k)
 				{
-					if (key + r < a.n_k) lo[r] = src[r];
-					if (key + 8 + r < a.n_k) hi[r] = src[8 + r];
+					lo = *reinterpret_cast<const LooseHalf8*>(src);
+					hi = *reinterpret_cast<const LooseHalf8*>(src + 8);
+				}
+				else
+				{
+#pragma unroll
+					for (int r = 0; r < 8; ++r)
+					{
+						if (key + r < a.n_k) lo[r] = src[r];
+						if (key + 8 + r < a.n_k) hi[r] = src[8 + r];
+					}
 				}
 			}
+			mk_next[b][0] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3);
+			mk_next[b][1] = __builtin_shufflevector(lo, lo, 4, 5, 6, 7);
+			mk_next[b][2] = __builtin_shufflevector(hi, hi, 0, 1, 2, 3);
+			mk_next[b][3] = __builtin_shufflevector(hi, hi, 4, 5, 6, 7);
 		}
-		mk_next[0] = __builtin_shufflevector(lo, lo, 0, 1, 2, 3);
-		mk_next[1] = __builtin_shufflevector(lo, lo, 4, 5, 6, 7);
-		mk_next[2] = __builtin_shufflevector(hi, hi, 0, 1, 2, 3);
-		mk_next[3] = __builtin_shufflevector(hi, hi, 4, 5, 6, 7);
 	};
 	// piece j of lane group g <-> piece g of lane group j, for every lane % 16: v_permlane32_swap exchanges the upper half
 	// of its first operand with the lower half of its second, v_permlane16_swap the odd rows of the first with the even
@@ -308,17 +328,21 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 		const bool more = t_next <= t_last;
 		// the mask values of this tile move out of the way of the next tile's, which go out now; they stay halves until
 		// the scores meet them (the float form would not fit the registers at head_dim 256)
-		half4_t mk[4];
+		half4_t mk[MASK ? QB : 1][4];
 		if constexpr (MASK)
 		{
 			bool any_visible = false;
 #pragma unroll
-			for (int kb = 0; kb < 4; ++kb) mk[kb] = mk_next[kb];
-			exchange_mask_pieces(mk);
+			for (int b = 0; b < QB; ++b)
+			{
 #pragma unroll
-			for (int kb = 0; kb < 4; ++kb)
+				for (int kb = 0; kb < 4; ++kb) mk[b][kb] = mk_next[b][kb];
+				exchange_mask_pieces(mk[b]);
 #pragma unroll
-				for (int r = 0; r < 4; ++r) any_visible |= mk[kb][r] > (half_t)(-INFINITY);
+				for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+					for (int r = 0; r < 4; ++r) any_visible |= mk[b][kb][r] > (half_t)(-INFINITY);
+			}
 			if (more) load_mask(t_next);
 			if (__builtin_amdgcn_ballot_w64(any_visible) == 0)
 			{
@@ -331,17 +355,21 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 			}
 		}
 
-		// ---- S^T = K Q^T: s[kb] = scores of the wave's queries against key block kb ----
-		float4_t s[4];
+		// ---- S^T = K Q^T: s[b][kb] = scores of query block b against key block kb ----
+		float4_t s[QB][4];
 #pragma unroll
-		for (int kb = 0; kb < 4; ++kb) s[kb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+		for (int b = 0; b < QB; ++b)
+#pragma unroll
+			for (int kb = 0; kb < 4; ++kb) s[b][kb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
 		for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
 			for (int st = 0; st < KS; ++st)
 			{
 				const half8_t kf = *reinterpret_cast<const half8_t*>(k_lds + (16 * kb + n) * L::kPitchK + (32 * st + 8 * g) * 2);
-				s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[st], s[kb], 0, 0, 0);
+#pragma unroll
+				for (int b = 0; b < QB; ++b)
+					s[b][kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[b][st], s[b][kb], 0, 0, 0);
 				// the next tile's loads, spread behind the key blocks of this product: a wave that issues them in one
 				// burst is held until the CU's vector memory path (64 bytes per clock) has taken them
 				if (st == KS - 1 && more)
@@ -352,63 +380,67 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 			}
 
 		// ---- online softmax; p as the second operand of the next product ----
-		half8_t pf[2];
+		half8_t pf[QB][2];
 		const int tile_key0 = t * kAttnKeysPerTile;
 		const bool interior = tile_key0 >= all_lo && tile_key0 + kAttnKeysPerTile - 1 <= all_hi;   // wave-uniform
-		float z[4][4];
-		float mt = -INFINITY;
-		if (interior && !MASK)
+#pragma unroll
+		for (int b = 0; b < QB; ++b)
 		{
-#pragma unroll
-			for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-				for (int r = 0; r < 4; ++r)
-				{
-					z[kb][r] = logit2<SOFTCAP>(s[kb][r], a.k_in, a.k_cap);
-					mt = fmaxf(mt, z[kb][r]);
-				}
-		}
-		else
-		{
-#pragma unroll
-			for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-				for (int r = 0; r < 4; ++r)
-				{
-					const int key = tile_key0 + 16 * kb + 4 * g + r;
-					const float zz = logit2<SOFTCAP>(s[kb][r], a.k_in, a.k_cap) + (MASK ? (float)mk[kb][r] * kLog2e : 0.0f);
-					z[kb][r] = (MASK || (key >= vis_lo && key <= vis_hi)) ? zz : -INFINITY;
-					mt = fmaxf(mt, z[kb][r]);
-				}
-		}
-		mt = max_over_lane_rows(mt);
-		const float m_new = fmaxf(m_run, mt);
-		const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;   // nothing visible so far: every term is exp2(-inf) = 0
-		float psum = 0.0f;
-		float p[4][4];
-#pragma unroll
-		for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-			for (int r = 0; r < 4; ++r)
+			float z[4][4];
+			float mt = -INFINITY;
+			if (interior && !MASK)
 			{
-				p[kb][r] = fast_exp2(z[kb][r] - m_safe);
-				psum += p[kb][r];
+#pragma unroll
+				for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+					for (int r = 0; r < 4; ++r)
+					{
+						z[kb][r] = logit2<SOFTCAP>(s[b][kb][r], a.k_in, a.k_cap);
+						mt = fmaxf(mt, z[kb][r]);
+					}
 			}
-		// the running maximum settles after a few tiles; when no query of the wave raised it, the
-		// rescale factor is 1 everywhere and the pass over the accumulators is skipped
-		if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0)
-		{
-			const float corr = fast_exp2(m_run - m_safe);
-			l_run *= corr;
+			else
+			{
 #pragma unroll
-			for (int c = 0; c < DC; ++c) o[c] *= corr;
+				for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+					for (int r = 0; r < 4; ++r)
+					{
+						const int key = tile_key0 + 16 * kb + 4 * g + r;
+						const float zz = logit2<SOFTCAP>(s[b][kb][r], a.k_in, a.k_cap) + (MASK ? (float)mk[MASK ? b : 0][kb][r] * kLog2e : 0.0f);
+						z[kb][r] = (MASK || (key >= vis_lo[b] && key <= vis_hi[b])) ? zz : -INFINITY;
+						mt = fmaxf(mt, z[kb][r]);
+					}
+			}
+			mt = max_over_lane_rows(mt);
+			const float m_new = fmaxf(m_run[b], mt);
+			const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;   // nothing visible so far: every term is exp2(-inf) = 0
+			float psum = 0.0f;
+			float p[4][4];
+#pragma unroll
+			for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+				for (int r = 0; r < 4; ++r)
+				{
+					p[kb][r] = fast_exp2(z[kb][r] - m_safe);
+					psum += p[kb][r];
+				}
+			// the running maximum settles after a few tiles; when no query of the wave raised it, the
+			// rescale factor is 1 everywhere and the pass over the accumulators is skipped
+			if (__builtin_amdgcn_ballot_w64(m_new > m_run[b]) != 0)
+			{
+				const float corr = fast_exp2(m_run[b] - m_safe);
+				l_run[b] *= corr;
+#pragma unroll
+				for (int c = 0; c < DC; ++c) o[b][c] *= corr;
+			}
+			l_run[b] += psum;
+			m_run[b] = m_new;
+#pragma unroll
+			for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+				for (int j = 0; j < 8; ++j) pf[b][tt][j] = (half_t)p[2 * tt + j / 4][j % 4];
 		}
-		l_run += psum;
-		m_run = m_new;
-#pragma unroll
-		for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-			for (int j = 0; j < 8; ++j) pf[tt][j] = (half_t)p[2 * tt + j / 4][j % 4];
 
 		// ---- O^T += V^T P^T ----
 #pragma unroll
@@ -420,40 +452,46 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 				const half4_t lo = lds_read_tr_b64(src);
 				const half4_t hi = lds_read_tr_b64(src + 16 * L::kPitchV);
 				const half8_t vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-				o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[tt], o[c], 0, 0, 0);
+#pragma unroll
+				for (int b = 0; b < QB; ++b)
+					o[b][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[b][tt], o[b][c], 0, 0, 0);
 			}
 	}
 
 	// ---- normalise and store: lane (n, g) holds y[row][16 c + 4 g .. + 3] ----
-	float l = l_run;
-	l += __shfl_xor(l, 16);
-	l += __shfl_xor(l, 32);
-	if (parts > 1)
-	{
-		// unnormalised accumulators, running maximum and sum of this half of the keys
-		if (q_row < a.n_q)
-		{
-			float* dst = a.partials + ((((int64_t)bh * walk.n_split + split_slot) * parts + part) * kAttnQueriesPerBlock + (q_row - q0)) * (D + 2);
 #pragma unroll
-			for (int c = 0; c < DC; ++c) *reinterpret_cast<WsFloat4*>(dst + 16 * c + 4 * g) = o[c];
-			if (g == 0)
+	for (int b = 0; b < QB; ++b)
+	{
+		float l = l_run[b];
+		l += __shfl_xor(l, 16);
+		l += __shfl_xor(l, 32);
+		if (parts > 1)
+		{
+			// unnormalised accumulators, running maximum and sum of this half of the keys
+			if (q_row[b] < a.n_q)
 			{
-				dst[D] = m_run;
-				dst[D + 1] = l;
+				float* dst = a.partials + ((((int64_t)bh * walk.n_split + split_slot) * parts + part) * kAttnQueriesPerBlock + (q_row[b] - q0)) * (D + 2);
+#pragma unroll
+				for (int c = 0; c < DC; ++c) *reinterpret_cast<WsFloat4*>(dst + 16 * c + 4 * g) = o[b][c];
+				if (g == 0)
+				{
+					dst[D] = m_run[b];
+					dst[D + 1] = l;
+				}
 			}
+			continue;
 		}
-		return;
-	}
-	const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-	if (q_row < a.n_q)
-	{
-#pragma unroll
-		for (int c = 0; c < DC; ++c)
+		const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+		if (q_row[b] < a.n_q)
 		{
-			half4_t out;
 #pragma unroll
-			for (int r = 0; r < 4; ++r) out[r] = (half_t)(o[c][r] * inv);
-			*reinterpret_cast<half4_t*>(yp + (int64_t)q_row * D + 16 * c + 4 * g) = out;
+			for (int c = 0; c < DC; ++c)
+			{
+				half4_t out;
+#pragma unroll
+				for (int r = 0; r < 4; ++r) out[r] = (half_t)(o[b][c][r] * inv);
+				*reinterpret_cast<half4_t*>(yp + (int64_t)q_row[b] * D + 16 * c + 4 * g) = out;
+			}
 		}
 	}
 }
@@ -464,12 +502,12 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_kernel(const
 //     step B of tile t:  O += V(t)^T P(t)^T        (MFMA + LDS reads)   beside   z(t + 1) = mask(softcap(S(t + 1)))  (VALU)
 // In the kernel above every wave of the block multiplies, then exponentiates, then multiplies (the barriers of a
 // tile keep the eight waves in step), so the matrix cores idle while the VALU works and the other way round.  The
-// LDS holds K of tile t + 1 next to V of tile t (two stages of each, filled global -> LDS directly).  (With
-// two 16-query blocks per wave it measured slower at every head dimension.)
-template <int D, bool SOFTCAP, int WAVES>
+// LDS holds K of tile t + 1 next to V of tile t (two stages of each, filled global -> LDS directly).  QB is 1 in
+// every launch: with two 16-query blocks per wave the kernel measured slower at every head dimension.
+template <int D, bool SOFTCAP, int QB, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(const AttnArgs a, const AttnWalk walk)
 {
-	constexpr int kAttnQueriesPerBlock = 16 * WAVES;
+	constexpr int kAttnQueriesPerBlock = 16 * QB * WAVES;
 	extern __shared__ __align__(16) char lds[];
 	using L = AttnLds<D>;
 	constexpr int KS = D / 32;
@@ -504,27 +542,38 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 	}
 
 	// this wave's queries as second operands: lane (n, g) holds q[row][32 s + 8 g .. + 7]
-	const int q_row = q0 + 16 * wave + n;
-	half8_t qf[KS];
+	int q_row[QB], vis_lo[QB], vis_hi[QB];
+	half8_t qf[QB][KS];
 #pragma unroll
-	for (int s = 0; s < KS; ++s)
+	for (int b = 0; b < QB; ++b)
 	{
-		half8_t val = {};
-		if (q_row < a.n_q) val = *reinterpret_cast<const half8_t*>(qp + (int64_t)q_row * D + 32 * s + 8 * g);
-		qf[s] = val;
+		q_row[b] = q0 + 16 * QB * wave + 16 * b + n;
+#pragma unroll
+		for (int s = 0; s < KS; ++s)
+		{
+			half8_t val = {};
+			if (q_row[b] < a.n_q) val = *reinterpret_cast<const half8_t*>(qp + (int64_t)q_row[b] * D + 32 * s + 8 * g);
+			qf[b][s] = val;
+		}
+		vis_hi[b] = a.causal ? q_row[b] + a.diag : a.n_k - 1;
+		if (vis_hi[b] > a.n_k - 1) vis_hi[b] = a.n_k - 1;
+		vis_lo[b] = a.window > 0 ? q_row[b] + a.diag - a.window + 1 : 0;
 	}
-	int vis_hi = a.causal ? q_row + a.diag : a.n_k - 1;
-	if (vis_hi > a.n_k - 1) vis_hi = a.n_k - 1;
-	const int vis_lo = a.window > 0 ? q_row + a.diag - a.window + 1 : 0;
 	// keys visible to every query of this wave need no per-element test: [all_lo, all_hi]
-	const int wq0 = q0 + 16 * wave, wq1 = wq0 + 15;
+	const int wq0 = q0 + 16 * QB * wave, wq1 = wq0 + 16 * QB - 1;
 	const int all_hi = a.causal ? (wq0 + a.diag < a.n_k - 1 ? wq0 + a.diag : a.n_k - 1) : a.n_k - 1;
 	const int all_lo = a.window > 0 ? wq1 + a.diag - a.window + 1 : 0;
 
-	float m_run = -INFINITY, m_new, l_run = 0.0f;  // l_run: this lane's share of the row sum
-	float4_t o[DC];
+	float m_run[QB], m_new[QB], l_run[QB];         // l_run: this lane's share of the row sum
+	float4_t o[QB][DC];
 #pragma unroll
-	for (int c = 0; c < DC; ++c) o[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+	for (int b = 0; b < QB; ++b)
+	{
+		m_run[b] = -INFINITY;
+		l_run[b] = 0.0f;
+#pragma unroll
+		for (int c = 0; c < DC; ++c) o[b][c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+	}
 
 	// Tiles go global -> LDS without staging registers, K and V in two stages each.  A load instruction fills 1 KB
 	// of consecutive LDS; with padded tile rows a few of its lanes land in the padding and fetch a valid chunk
@@ -574,8 +623,8 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 		__syncthreads();
 		asm volatile("" : "=s"(token));
 	};
-	// z of score e = 4 kb + r against tile t: scale / softcap in the log2 domain, masked keys at -inf
-	auto logit_of_score = [&](auto interior_tag, float sv, int t, int e, int g) {
+	// z of score e = 4 kb + r of query block b against tile t: scale / softcap in the log2 domain, masked keys at -inf
+	auto logit_of_score = [&](auto interior_tag, float sv, int t, int b, int e, int g) {
 		const float zz = logit2<SOFTCAP>(sv, a.k_in, a.k_cap);
 		if constexpr (decltype(interior_tag)::value) return zz;
 		else
@@ -583,7 +632,7 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 			// (a sum, so that the transform is not made conditional on the mask; the bounds pass through an empty
 			// statement, so that the compiler does not keep sixteen pre-combined pairs of them in registers over the
 			// whole kernel)
-			int lo = vis_lo, hi = vis_hi;
+			int lo = vis_lo[b], hi = vis_hi[b];
 			asm volatile("" : "+v"(lo), "+v"(hi));
 			const int key = t * kAttnKeysPerTile + 16 * (e / 4) + 4 * g + e % 4;
 			return zz + ((key >= lo && key <= hi) ? 0.0f : -INFINITY);
@@ -599,13 +648,13 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 		if constexpr (SOFTCAP) return fast_rcp(1.0f + tv);
 		else return tv;
 	};
-	auto logit_finish = [&](auto interior_tag, float rv, int t, int e, int g) {
+	auto logit_finish = [&](auto interior_tag, float rv, int t, int b, int e, int g) {
 		float zz = rv;
 		if constexpr (SOFTCAP) zz = fmaf(rv, -2.0f * a.k_cap, a.k_cap);
 		if constexpr (decltype(interior_tag)::value) return zz;
 		else
 		{
-			int lo = vis_lo, hi = vis_hi;
+			int lo = vis_lo[b], hi = vis_hi[b];
 			asm volatile("" : "+v"(lo), "+v"(hi));
 			const int key = t * kAttnKeysPerTile + 16 * (e / 4) + 4 * g + e % 4;
 			return zz + ((key >= lo && key <= hi) ? 0.0f : -INFINITY);
@@ -616,13 +665,13 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 		return key0 >= all_lo && key0 + kAttnKeysPerTile - 1 <= all_hi;
 	};
 
-	float z[16];
+	float z[QB][16];
 	// running maximum including tile t (m_run: through tile t - 1); known one tile ahead, like z
-	auto row_max = [&]() {
+	auto row_max = [&](int b) {
 		float mt = -INFINITY;
 #pragma unroll
-		for (int e = 0; e < 16; ++e) mt = fmaxf(mt, z[e]);
-		return fmaxf(m_run, max_over_lane_rows(mt));
+		for (int e = 0; e < 16; ++e) mt = fmaxf(mt, z[b][e]);
+		return fmaxf(m_run[b], max_over_lane_rows(mt));
 	};
 	if (t_first <= t_last)
 	{
@@ -641,18 +690,24 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 #pragma unroll
 		for (int kb = 0; kb < 4; ++kb)
 		{
-			float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+			float4_t acc[QB];
+#pragma unroll
+			for (int b = 0; b < QB; ++b) acc[b] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
 			for (int st = 0; st < KS; ++st)
 			{
 				const half8_t kf = *reinterpret_cast<const half8_t*>(lds + (16 * kb + n) * L::kPitchK + (32 * st + 8 * g) * 2);
-				acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[st], acc, 0, 0, 0);
+#pragma unroll
+				for (int b = 0; b < QB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[b][st], acc[b], 0, 0, 0);
 			}
 #pragma unroll
-			for (int r = 0; r < 4; ++r) z[4 * kb + r] = logit_of_score(std::false_type{}, acc[r], t_first, 4 * kb + r, g);
+			for (int b = 0; b < QB; ++b)
+#pragma unroll
+				for (int r = 0; r < 4; ++r) z[b][4 * kb + r] = logit_of_score(std::false_type{}, acc[b][r], t_first, b, 4 * kb + r, g);
 		}
 	}
-	m_new = t_first <= t_last ? row_max() : -INFINITY;
+#pragma unroll
+	for (int b = 0; b < QB; ++b) m_new[b] = t_first <= t_last ? row_max(b) : -INFINITY;
 
 	// One tile.  MORE: tile t + 1 exists (its K is on its way into the other stage); INTERIOR: every key of tile
 	// t + 1 is visible to every query of the wave.  Apart from the rescale at its top the tile is one stretch of
@@ -661,15 +716,20 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 		constexpr bool MORE = decltype(more_tag)::value;
 		// the running maximum settles after a few tiles; when no query of the wave raised it, the rescale factor
 		// is 1 everywhere and the pass over the accumulators is skipped
-		const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;   // nothing visible so far: every term is exp2(-inf) = 0
-		if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0)
-		{
-			const float corr = fast_exp2(m_run - m_safe);
-			l_run *= corr;
+		float m_safe[QB];
 #pragma unroll
-			for (int c = 0; c < DC; ++c) o[c] *= corr;
+		for (int b = 0; b < QB; ++b)
+		{
+			m_safe[b] = (m_new[b] == -INFINITY) ? 0.0f : m_new[b];   // nothing visible so far: every term is exp2(-inf) = 0
+			if (__builtin_amdgcn_ballot_w64(m_new[b] > m_run[b]) != 0)
+			{
+				const float corr = fast_exp2(m_run[b] - m_safe[b]);
+				l_run[b] *= corr;
+#pragma unroll
+				for (int c = 0; c < DC; ++c) o[b][c] *= corr;
+			}
+			m_run[b] = m_new[b];
 		}
-		m_run = m_new;
 		// K(t + 1) and V(t) have landed; K(t) and V(t - 1) are free for the loads issued below
 		tile_barrier();
 		// (the lane's coordinates derived again from a thread number the compiler takes for a new value: a handful of
@@ -683,7 +743,7 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 		const char* v_lds = lds + stage * kStageBytes + kAttnKeysPerTile * L::kPitchK;
 		const int t_k = t + 2 <= t_last ? t + 2 : t_last;       // (past the end: the last tile once more, into the free stage)
 
-		// The tile as steps of one operand out of LDS and the MFMA that uses it (64 at head dimension 256): those of
+		// The tile as steps of one operand out of LDS and the QB MFMAs that use it (64 at head dimension 256): those of
 		// S(t + 1) = K(t + 1) Q^T, the four key blocks in turn so that consecutive MFMAs do not wait for each other's
 		// result, then those of O^T += V(t)^T P(t)^T.  Behind its MFMAs a step issues the LDS reads of the operand
 		// kAhead steps later and does its share of the vector work: in the first half p(t) = exp2(z(t) - m), the 16
@@ -706,33 +766,38 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 			const half4_t hi = lds_read_tr_b64(src + 16 * L::kPitchV);
 			return (half8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 		};
-		float4_t s_next[4];
-		float psum = 0.0f, z_max;
-		half8_t pf[2];
+		float4_t s_next[QB][4];
+		float psum[QB], z_max[QB];
+		half8_t pf[QB][2];
 #pragma unroll
-		for (int kb = 0; kb < 4; ++kb) s_next[kb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-		auto p_of_score = [&](int e) {
-			const float pv = fast_exp2(z[e] - m_safe);
-			psum += pv;
-			pf[e / 8][e % 8] = (half_t)pv;
+		for (int b = 0; b < QB; ++b)
+		{
+			psum[b] = 0.0f;
+#pragma unroll
+			for (int kb = 0; kb < 4; ++kb) s_next[b][kb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+		}
+		auto p_of_score = [&](int b, int e) {
+			const float pv = fast_exp2(z[b][e] - m_safe[b]);
+			psum[b] += pv;
+			pf[b][e / 8][e % 8] = (half_t)pv;
 		};
 		// stage of score e that belongs to step i, if any (see the table at its call)
-		float xa[16], tb[16];
-		auto vector_stage = [&](auto tag, int e, int i) {
+		float xa[QB][16], tb[QB][16];
+		auto vector_stage = [&](auto tag, int b, int e, int i) {
 			constexpr int kStepsB = 2 * DC;
 			const int a0 = e * kStepsA / 16, b0 = kStepsA + e * kStepsB / 16;
-			if (i == a0) xa[e] = fast_exp2(z[e] - m_safe);
+			if (i == a0) xa[b][e] = fast_exp2(z[b][e] - m_safe[b]);
 			if (i == a0 + 1)
 			{
-				psum += xa[e];
-				pf[e / 8][e % 8] = (half_t)xa[e];
+				psum[b] += xa[b][e];
+				pf[b][e / 8][e % 8] = (half_t)xa[b][e];
 			}
-			if (i == b0) tb[e] = logit_begin(s_next[e / 4][e % 4]);
-			if (i == b0 + 1) tb[e] = logit_middle(tb[e]);
+			if (i == b0) tb[b][e] = logit_begin(s_next[b][e / 4][e % 4]);
+			if (i == b0 + 1) tb[b][e] = logit_middle(tb[b][e]);
 			if (i == b0 + 2)
 			{
-				z[e] = logit_finish(tag, tb[e], t + 1, e, g);
-				z_max = e == 0 ? z[0] : fmaxf(z_max, z[e]);
+				z[b][e] = logit_finish(tag, tb[b][e], t + 1, b, e, g);
+				z_max[b] = e == 0 ? z[b][0] : fmaxf(z_max[b], z[b][e]);
 			}
 		};
 #pragma unroll
@@ -740,7 +805,9 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 		if constexpr (!MORE)
 		{
 #pragma unroll
-			for (int e = 0; e < 16; ++e) p_of_score(e);
+			for (int b = 0; b < QB; ++b)
+#pragma unroll
+				for (int e = 0; e < 16; ++e) p_of_score(b, e);
 		}
 		__builtin_amdgcn_sched_barrier(0);
 		// (the step number as a type: every index below is a constant, whatever the optimiser makes of the loop)
@@ -755,8 +822,12 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 				if (((wave >> 2) & 1) == (i == 0 ? 0 : 1)) __builtin_amdgcn_s_setprio(2);
 				else __builtin_amdgcn_s_setprio(0);
 			}
-			if (i < kStepsA) s_next[i % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag[i % kAhead], qf[i / 4], s_next[i % 4], 0, 0, 0);
-			else o[(i - kStepsA) % DC] = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag[i % kAhead], pf[(i - kStepsA) / DC], o[(i - kStepsA) % DC], 0, 0, 0);
+#pragma unroll
+			for (int b = 0; b < QB; ++b)
+			{
+				if (i < kStepsA) s_next[b][i % 4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag[i % kAhead], qf[b][i / 4], s_next[b][i % 4], 0, 0, 0);
+				else o[b][(i - kStepsA) % DC] = __builtin_amdgcn_mfma_f32_16x16x32_f16(frag[i % kAhead], pf[b][(i - kStepsA) / DC], o[b][(i - kStepsA) % DC], 0, 0, 0);
+			}
 			if (i + kAhead < kSteps) frag[i % kAhead] = read_operand(i + kAhead);
 			if constexpr (MORE)
 			{
@@ -778,12 +849,14 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 				// step kStepsA + DC on, so the last scores' second stage may sit in the second half)
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
-					vector_stage(interior_tag, e, i);
+#pragma unroll
+					for (int b = 0; b < QB; ++b) vector_stage(interior_tag, b, e, i);
 				// (p is first used behind the branch that follows the first half: without a use here the compiler moves
 				// the whole half's vector work there)
 				if constexpr (i == kStepsA - 1)
 				{
-					asm volatile("" : "+v"(pf[0]), "+v"(psum));
+#pragma unroll
+					for (int b = 0; b < QB; ++b) asm volatile("" : "+v"(pf[b][0]), "+v"(psum[b]));
 				}
 			}
 			__builtin_amdgcn_sched_barrier(0);
@@ -796,10 +869,15 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 			for (int late = kSteps; late < kSteps + 2; ++late)
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
-					vector_stage(interior_tag, e, late);
+#pragma unroll
+					for (int b = 0; b < QB; ++b) vector_stage(interior_tag, b, e, late);
 		}
-		l_run += psum;
-		if constexpr (MORE) m_new = fmaxf(m_run, max_over_lane_rows(z_max));
+#pragma unroll
+		for (int b = 0; b < QB; ++b)
+		{
+			l_run[b] += psum[b];
+			if constexpr (MORE) m_new[b] = fmaxf(m_run[b], max_over_lane_rows(z_max[b]));
+		}
 	};
 	for (int t = t_first; t < t_last; ++t)
 	{
@@ -815,36 +893,40 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 	int tid_again = threadIdx.x;
 	asm volatile("" : "+v"(tid_again));
 	const int n_out = tid_again & 15, g_out = (tid_again & (kWaveSize - 1)) >> 4;
-	const int row_out = q0 + 16 * wave + n_out;
-	float l = l_run;
-	l += __shfl_xor(l, 16);
-	l += __shfl_xor(l, 32);
-	if (parts > 1)
+#pragma unroll
+	for (int b = 0; b < QB; ++b)
 	{
-		// unnormalised accumulators, running maximum and sum of this half of the keys
+		const int row_out = q0 + 16 * QB * wave + 16 * b + n_out;
+		float l = l_run[b];
+		l += __shfl_xor(l, 16);
+		l += __shfl_xor(l, 32);
+		if (parts > 1)
+		{
+			// unnormalised accumulators, running maximum and sum of this half of the keys
+			if (row_out < a.n_q)
+			{
+				float* dst = a.partials + ((((int64_t)bh * walk.n_split + split_slot) * parts + part) * kAttnQueriesPerBlock + (row_out - q0)) * (D + 2);
+#pragma unroll
+				for (int c = 0; c < DC; ++c) *reinterpret_cast<WsFloat4*>(dst + 16 * c + 4 * g_out) = o[b][c];
+				if (g_out == 0)
+				{
+					dst[D] = m_run[b];
+					dst[D + 1] = l;
+				}
+			}
+			continue;
+		}
+		const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 		if (row_out < a.n_q)
 		{
-			float* dst = a.partials + ((((int64_t)bh * walk.n_split + split_slot) * parts + part) * kAttnQueriesPerBlock + (row_out - q0)) * (D + 2);
 #pragma unroll
-			for (int c = 0; c < DC; ++c) *reinterpret_cast<WsFloat4*>(dst + 16 * c + 4 * g_out) = o[c];
-			if (g_out == 0)
+			for (int c = 0; c < DC; ++c)
 			{
-				dst[D] = m_run;
-				dst[D + 1] = l;
+				half4_t out;
+#pragma unroll
+				for (int r = 0; r < 4; ++r) out[r] = (half_t)(o[b][c][r] * inv);
+				*reinterpret_cast<half4_t*>(yp + (int64_t)row_out * D + 16 * c + 4 * g_out) = out;
 			}
-		}
-		return;
-	}
-	const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-	if (row_out < a.n_q)
-	{
-#pragma unroll
-		for (int c = 0; c < DC; ++c)
-		{
-			half4_t out;
-#pragma unroll
-			for (int r = 0; r < 4; ++r) out[r] = (half_t)(o[c][r] * inv);
-			*reinterpret_cast<half4_t*>(yp + (int64_t)row_out * D + 16 * c + 4 * g_out) = out;
 		}
 	}
 }
@@ -931,17 +1013,17 @@ hipError_t launch_q32(const AttnArgs& args_in, int64_t batch_heads, hipStream_t 
 }
 
 // SKEW: the kernel that takes the two halves of a tile's work from different tiles
-template <int D, bool SOFTCAP, bool SKEW = false, bool MASK = false>
+template <int D, bool SOFTCAP, int QB, bool SKEW = false, bool MASK = false>
 hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStream_t stream)
 {
 	constexpr int WAVES = 8;
 	static_assert(!(SKEW && MASK), "the mask tensor goes through the plain kernel");
 	auto kernel = [] {
-		if constexpr (SKEW) return sdp_attention_fwd_f16_skew_kernel<D, SOFTCAP, WAVES>;
-		else return sdp_attention_fwd_f16_kernel<D, SOFTCAP, WAVES, MASK>;
+		if constexpr (SKEW) return sdp_attention_fwd_f16_skew_kernel<D, SOFTCAP, QB, WAVES>;
+		else return sdp_attention_fwd_f16_kernel<D, SOFTCAP, QB, WAVES, MASK>;
 	}();
 	constexpr int kLdsBytes = 2 * AttnLds<D>::kBytes;           // two stages
-	constexpr int kQueriesPerBlock = 16 * WAVES;
+	constexpr int kQueriesPerBlock = 16 * QB * WAVES;
 	(void)hipGetLastError();
 	if (kLdsBytes > 64 * 1024)
 	{
@@ -992,7 +1074,7 @@ template <int D>
 hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, hipStream_t stream)
 {
 	if constexpr (D == 256)
-		return softcap ? launch_variant<D, true, true>(args, batch_heads, stream) : launch_variant<D, false, true>(args, batch_heads, stream);
+		return softcap ? launch_variant<D, true, 1, true>(args, batch_heads, stream) : launch_variant<D, false, 1, true>(args, batch_heads, stream);
 	else
 	{
 		const int64_t blocks = (args.n_q + kQ32QueriesPerBlock - 1) / kQ32QueriesPerBlock * batch_heads;
@@ -1000,7 +1082,7 @@ hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, h
 		                                           band::workspace_capacity(stream)) > 1;
 		if (attention_q32_wanted<D>(args, blocks, in_parts))
 			return softcap ? launch_q32<D, true>(args, batch_heads, stream) : launch_q32<D, false>(args, batch_heads, stream);
-		return softcap ? launch_variant<D, true>(args, batch_heads, stream) : launch_variant<D, false>(args, batch_heads, stream);
+		return softcap ? launch_variant<D, true, 1>(args, batch_heads, stream) : launch_variant<D, false, 1>(args, batch_heads, stream);
 	}
 }
 
@@ -1266,7 +1348,7 @@ hipError_t launch_sdp_attention_fwd_f16(const void* q, const void* k, const void
 		}
 		// sixteen queries per wave at every head dimension: the mask values of a tile take the registers of a second block
 #define ANYGPU_ATTN_F16_MASK_DIM(DIM) \
-		return capped ? launch_variant<DIM, true, false, true>(args, batch_heads, stream) : launch_variant<DIM, false, false, true>(args, batch_heads, stream)
+		return capped ? launch_variant<DIM, true, 1, false, true>(args, batch_heads, stream) : launch_variant<DIM, false, 1, false, true>(args, batch_heads, stream)
 		switch (head_dim)
 		{
 		case 64: ANYGPU_ATTN_F16_MASK_DIM(64);
