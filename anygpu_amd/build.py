@@ -66,6 +66,8 @@ def build_kernels(verbose: bool = False) -> Path:
     _run([sys.executable, str(CSRC_DIR / "gen_gemm_f16_ring_loop.py"), str(CSRC_DIR / "gemm_f16_ring_loop_4x4.inc"), "4x4"], quiet=not verbose)
     _run([sys.executable, str(CSRC_DIR / "gen_gemm_f16_ring_loop.py"), str(CSRC_DIR / "gemm_f16_ring_loop_8x4kn.inc"), "8x4kn"], quiet=not verbose)
     _run([sys.executable, str(CSRC_DIR / "gen_gemm_f16_ring_loop.py"), str(CSRC_DIR / "gemm_f16_ring_loop_4x4kn.inc"), "4x4kn"], quiet=not verbose)
+    for form in ("kn2", "8x4kn2", "4x4kn2"):
+        _run([sys.executable, str(CSRC_DIR / "gen_gemm_f16_ring_loop.py"), str(CSRC_DIR / f"gemm_f16_ring_loop_{form}.inc"), form], quiet=not verbose)
     _run([sys.executable, str(CSRC_DIR / "gen_gemm_f32_ring_loop.py"), str(CSRC_DIR / "gemm_f32_ring_loop.inc")], quiet=not verbose)
     _run([sys.executable, str(CSRC_DIR / "gen_gemm_f32_ring_loop.py"), str(CSRC_DIR / "gemm_f32_ring_loop_64.inc"), "64"], quiet=not verbose)
     _run([sys.executable, str(CSRC_DIR / "gen_gemm_f32_ring_loop.py"), str(CSRC_DIR / "gemm_f32_ring_loop_kn.inc"), "kn"], quiet=not verbose)

@@ -216,6 +216,7 @@ struct FourWavePrices
 	static constexpr double kSlabHalf[3] = {1.0, 0.575, 0.36};
 	static constexpr double kLaunch[3] = {8.5, 5.5, 3.0};
 	static constexpr double kOperandBytesPerUs = 5.5e6;      // what HBM gives a launch that reads its operands once
+	static constexpr double kDualRoundKN = 2.0;              // what a further round of tiles of two [K, N] products adds to its slabs
 };
 
 struct FourWavePlan
@@ -226,7 +227,7 @@ struct FourWavePlan
 };
 
 // dual: two products side by side in a tile (GELU(gate) * up), which then covers half the output columns
-static FourWavePlan plan_four_wave(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cus, int64_t plane_room, bool dual = false)
+static FourWavePlan plan_four_wave(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t cus, int64_t plane_room, bool dual = false, bool b_kn = false)
 {
 	FourWavePlan best;
 	const int64_t slabs = K / 64;
@@ -250,6 +251,8 @@ static FourWavePlan plan_four_wave(int64_t M, int64_t N, int64_t K, int64_t batc
 			const double stream_us = 2.0 * ((double)M + (double)N) * (double)K * (double)batch / FourWavePrices::kOperandBytesPerUs;
 			if (us < stream_us) us = stream_us;
 			us += FourWavePrices::kLaunch[kind];
+			// (two [K, N] products: 640 x 2304 -> 9216 in three rounds of 128 x 128 tiles 64 us, in one of 256 x 256 57)
+			if (dual && b_kn) us += FourWavePrices::kDualRoundKN * (double)(rounds - 1);
 			if (sp > 1) us += TilePrices::kMergeLaunchUs + 8.0 * (double)sp * (double)M * (double)N / TilePrices::kPlaneBytesPerUs;
 			if (us < best.us)
 			{
@@ -785,11 +788,13 @@ hipError_t launch_gemm_f16_epilogue(const void* A, const void* B, const void* B2
 		return hipGetLastError();
 	}
 	const int64_t cus = device_cu_count();
-	// one product, k-contiguous weights, whole slabs: the four-wave kernels, priced like the unfused product, uncut
-	if (b_layout == ANYGPU_B_COL_MAJOR && gemm_f16_ring_applies(a, b, M, N, K, lda, ldb, 0, 0, 1, b_layout) &&
+	// whole slabs: the four-wave kernels, priced like the unfused product, uncut.  [K, N] weights, us, eight-wave tiles / four-wave:
+	// two matrices 2304 -> 9216 8 rows 26.8 / 19.2, 128 rows 36.4 / 20.7, 1500 rows 118 / 108, 4096 rows 306 / 268 (1.30 PFLOP/s);
+	// bias 2304 -> 9216 256 rows 27 / 17, 4096 -> 4096 640 rows 45 / 28, 4096 rows 112 / 100
+	if (gemm_f16_ring_applies(a, b, M, N, K, lda, ldb, 0, 0, 1, b_layout) &&
 	    (!dual || reinterpret_cast<uintptr_t>(B2) % 16 == 0))
 	{
-		const FourWavePlan four = plan_four_wave(M, N, K, 1, cus, 0, dual);
+		const FourWavePlan four = plan_four_wave(M, N, K, 1, cus, 0, dual, b_layout == ANYGPU_B_ROW_MAJOR);
 		const auto small_blocks = [&](int64_t t) { return ((M + t - 1) / t) * ((N + (dual ? t / 2 : t) - 1) / (dual ? t / 2 : t)); };
 		const double small_us = (double)(K / 64) * slab_us(64, small_blocks(64), cus) + 6.0;
 		if (four.kind >= 0 && four.us < small_us)
@@ -797,15 +802,15 @@ hipError_t launch_gemm_f16_epilogue(const void* A, const void* B, const void* B2
 #define ANYGPU_F16_EPI_FOUR(EPI) \
 			do { \
 				if (four.kind == 0) return launch_gemm_f16_ring<EPI>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, b_layout, bs, ep_param); \
-				if (four.kind == 1) return launch_gemm_f16_ring3<8, 4, EPI>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, bs, ep_param); \
-				return launch_gemm_f16_ring3<4, 4, EPI>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, bs, ep_param); \
+				if (four.kind == 1) return launch_gemm_f16_ring3<8, 4, EPI>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, bs, ep_param, b_layout); \
+				return launch_gemm_f16_ring3<4, 4, EPI>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, bs, ep_param, b_layout); \
 			} while (0)
 			if (epilogue == kEpiSoftcap) ANYGPU_F16_EPI_FOUR(kEpiSoftcap);
 			if (epilogue == kEpiBias) ANYGPU_F16_EPI_FOUR(kEpiBias);
 			// (the second weight matrix travels in the bias argument)
 			if (four.kind == 0) return launch_gemm_f16_ring<kEpiGeluMul>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, b_layout, b2, 0.0f);
-			if (four.kind == 1) return launch_gemm_f16_ring3<8, 4, kEpiGeluMul>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, b2, 0.0f);
-			return launch_gemm_f16_ring3<4, 4, kEpiGeluMul>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, b2, 0.0f);
+			if (four.kind == 1) return launch_gemm_f16_ring3<8, 4, kEpiGeluMul>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, b2, 0.0f, b_layout);
+			return launch_gemm_f16_ring3<4, 4, kEpiGeluMul>(a, b, c, M, N, K, lda, ldb, ldc, 0, 0, 0, 1, stream, nullptr, 0, b2, 0.0f, b_layout);
 #undef ANYGPU_F16_EPI_FOUR
 		}
 	}

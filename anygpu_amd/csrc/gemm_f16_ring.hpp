@@ -35,11 +35,12 @@ struct GemmRingCfg
 // B_KN: B stored [K, N] (row k holds the n), staged as a [64 k][256 n] unit and read through transposing LDS reads; N is a
 // multiple of 8 then, and column chunks past N are read from the last whole chunk of the row.
 // EPI: kEpiNone, kEpiBias (+ bias[n]) or kEpiSoftcap (ep_param * tanh(sum / ep_param)), applied to the fp32 sums; or
-// kEpiGeluMul (k-contiguous weights only): the tile is 128 output columns wide (N and tiles_n count those) and its B unit
+// kEpiGeluMul: the tile is 128 output columns wide (N and tiles_n count those) and its B unit
 // is put together from two matrices: of every wave column's 128 unit rows the first 64 come from B (the gate weights) and
 // the second 64 from `bias`, which then is the second matrix B2 (the up weights, same pitch), both for the same 64 output
 // columns, so that gate and up sums of an output element meet in one lane, A is read once for both products and
-// gelu_tanh(gate) * up goes out.  The wave that loads a quarter of the unit loads it from one matrix.
+// gelu_tanh(gate) * up goes out.  The wave that loads a quarter of the unit loads it from one matrix.  B_KN with kEpiGeluMul: the
+// unit is two [64 k][128 n] halves, one per matrix (gemm_f16_ring_loop_kn2.inc), half a matrix's 32 k rows per wave.
 template <bool RAGGED, bool B_KN, int EPI = kEpiNone>
 __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 	const half_t* __restrict__ A, const half_t* __restrict__ B, half_t* __restrict__ C,
@@ -62,10 +63,10 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 	tile_of_block<4>(blockIdx.x, tiles_m, tiles_n, tile_m, tile_n);
 	const int64_t m0 = (int64_t)tile_m * 256;
 	constexpr bool DUAL = EPI == kEpiGeluMul;
-	static_assert(!DUAL || !B_KN, "two weight matrices: k-contiguous only");
 	const int64_t n0 = (int64_t)tile_n * (DUAL ? 128 : 256);
-	// DUAL: unit rows 64 w .. + 63 of wave w are output columns 64 (w / 2) .. + 63 of the tile, from B (w even) or B2
-	const half_t* const b_of_wave = DUAL && (wave & 1) ? bias : B;
+	// DUAL: unit rows 64 w .. + 63 of wave w are output columns 64 (w / 2) .. + 63 of the tile, from B (w even) or B2; [K, N]: the
+	// first two waves load B, the other two B2
+	const half_t* const b_of_wave = DUAL && (B_KN ? wave >> 1 : wave & 1) ? bias : B;
 	const int b_unit_row = DUAL ? 64 * (wave >> 1) : 64 * wave;       // the wave's first row, as a column of the tile
 
 	// Direct loads.  A unit row is 64 halves = 128 bytes = eight 16-byte chunks; chunk c of row r sits at position
@@ -79,7 +80,10 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 	// (offsets count from the first row of the wave's 64, which keeps them below 2^32 for the row pitches admitted)
 	// A [K, N] unit of B has rows of 256 n = 512 bytes = 32 chunks; one instruction fills 2 k rows: lane -> row lane / 32,
 	// position lane % 32, and the chunk at position p of row k is chunk p ^ kn_row_swizzle(k).  Instruction q of this wave
-	// covers rows 16 wave + 2 q, + 1 of the slab's 64.
+	// covers rows 16 wave + 2 q, + 1 of the slab's 64.  (Two matrices: rows of 128 n = 16 chunks, four k rows to an instruction,
+	// 32 to a wave.)
+	constexpr int kKnRowBytes = DUAL ? 256 : 512, kKnRowsPerLoad = 1024 / kKnRowBytes, kKnChunks = kKnRowBytes / 16;
+	const int kn_first = DUAL ? 32 * (wave & 1) : 16 * wave;   // the wave's first k row
 	int64_t a_first = m0 + 64 * wave, b_first = n0 + b_unit_row;
 	if constexpr (RAGGED)
 	{
@@ -100,8 +104,8 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 		table[64 * q] = (unsigned)(((a_row - a_first) * lda + chunk * 8) * 2);
 		if constexpr (B_KN)
 		{
-			const int k_wave = 2 * q + (lane >> 5);                // the k row, counted from the wave's first
-			int64_t col = (int64_t)(((lane & 31) ^ kn_row_swizzle(16 * wave + k_wave)) << 3);
+			const int k_wave = kKnRowsPerLoad * q + lane / kKnChunks;          // the k row, counted from the wave's first
+			int64_t col = (int64_t)(((lane % kKnChunks) ^ kn_row_swizzle(kn_first + k_wave)) << 3);
 			if constexpr (RAGGED)
 				if (n0 + col + 8 > N) col = N - 8 - n0;
 			table[64 * (8 + q)] = (unsigned)((k_wave * ldb + col) * 2);
@@ -111,7 +115,7 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 	}
 	const unsigned table_addr = lds0 + 4 * Cfg::kUnitBytes + (wave * (16 * 64) + lane) * 4;
 	const uintptr_t a_wave = reinterpret_cast<uintptr_t>(A + a_first * lda);
-	const uintptr_t b_wave = reinterpret_cast<uintptr_t>(B_KN ? B + (int64_t)(16 * wave) * ldb + n0 : b_of_wave + b_first * ldb);
+	const uintptr_t b_wave = reinterpret_cast<uintptr_t>(B_KN ? b_of_wave + (int64_t)kn_first * ldb + n0 : b_of_wave + b_first * ldb);
 	const unsigned wave_share = wave * 8192;               // the wave's 64 rows inside a unit
 	const unsigned lds_wave = lds0 + wave_share;
 	const int slabs = K / 64;
@@ -125,9 +129,10 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 	// columns 4 (r % 4) .. + 3 of the MFMA tile; tile j of the patch lies at chunk pair j ^ (row swizzle / 2), a term the
 	// assembly block adds per tile from `b_swizzle`.
 	const unsigned kn_k = 8 * (lane >> 4) + (frag_row >> 2);
-	const unsigned b_addr = B_KN ? kn_k * 512 + (wn * 16 + ((frag_row & 3) >> 1)) * 16 + 8 * (frag_row & 1) - wave_share
+	// (two matrices: tile j of wave column wn at chunk pair (4 wn + j) ^ (row swizzle / 2) of either half, j < 4)
+	const unsigned b_addr = B_KN ? kn_k * kKnRowBytes + ((DUAL ? 0 : wn * 16) + ((frag_row & 3) >> 1)) * 16 + 8 * (frag_row & 1) - wave_share
 	                             : (wn * 128 + frag_row) * 128 + frag_chunk * 16 - wave_share;
-	[[maybe_unused]] const unsigned b_swizzle = (unsigned)(kn_row_swizzle((int)kn_k) >> 1) << 5;
+	[[maybe_unused]] const unsigned b_swizzle = (unsigned)((kn_row_swizzle((int)kn_k) >> 1) ^ (DUAL ? wn << 2 : 0)) << 5;
 	[[maybe_unused]] const unsigned b_step = (unsigned)(128 * ldb);      // bytes from one [K, N] slab to the next
 
 	// The accumulators leave the block as eight vectors of 32 registers pinned to a[0:255]: row i of the patch's MFMA
@@ -162,7 +167,13 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring_kernel(
 	"v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "v245", "v246", "v247", "v248", "v249", \
 	"v250", "v251", "v252", "v253", "v254", "v255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", \
 	"s69", "s70", "s71", "s72", "s73", "scc", "m0", "memory"
-	if constexpr (B_KN)
+	if constexpr (B_KN && DUAL)
+		asm volatile(
+#include "gemm_f16_ring_loop_kn2.inc"
+			: ANYGPU_RING_OUTPUTS
+			: ANYGPU_RING_INPUTS, [bsx] "v"(b_swizzle), [bstep] "s"(b_step)
+			: ANYGPU_RING_CLOBBERS);
+	else if constexpr (B_KN)
 		asm volatile(
 #include "gemm_f16_ring_loop_kn.inc"
 			: ANYGPU_RING_OUTPUTS
@@ -231,12 +242,8 @@ inline hipError_t launch_gemm_f16_ring(const half_t* A, const half_t* B, half_t*
 	constexpr int kOutN = EPI == kEpiGeluMul ? 128 : 256;             // output columns of a tile
 	const int ragged = (M % 256 != 0 || N % kOutN != 0 || !c_aligned) + 2 * kn;       // which instantiation
 	auto kernel = (ragged & 1) == 0 ? gemm_f16_nt_ring_kernel<false, false, EPI> : gemm_f16_nt_ring_kernel<true, false, EPI>;
-	if constexpr (EPI != kEpiGeluMul)
-	{
-		if (ragged == 2) kernel = gemm_f16_nt_ring_kernel<false, true, EPI>;
-		if (ragged == 3) kernel = gemm_f16_nt_ring_kernel<true, true, EPI>;
-	}
-	else if (kn) return hipErrorInvalidValue;
+	if (ragged == 2) kernel = gemm_f16_nt_ring_kernel<false, true, EPI>;
+	if (ragged == 3) kernel = gemm_f16_nt_ring_kernel<true, true, EPI>;
 	// More than 64 KB of dynamic LDS has to be granted per function and per device, once.
 	static std::atomic<uint64_t> configured_devices[4];
 	(void)hipGetLastError();

@@ -34,7 +34,8 @@ struct GemmRing3Cfg
 // or kEpiGeluMul: the tile is BN / 2 output columns wide and its B unit holds, for every wave column, gate rows (from B) in
 // front of up rows (from `bias`, which then is the second weight matrix), as in gemm_f16_nt_ring_kernel.
 // B_KN: B stored [K, N] (N a multiple of 8): a B unit of 64 k rows x BN n, filled four rows per load, fragments by
-// transposing reads (gemm_f16_ring_loop_8x4kn.inc, _4x4kn.inc); not with kEpiGeluMul.
+// transposing reads (gemm_f16_ring_loop_8x4kn.inc, _4x4kn.inc); with kEpiGeluMul two [64 k][BN / 2 n] halves, one per matrix
+// (_8x4kn2.inc, _4x4kn2.inc).
 template <int TM, int TN, bool RAGGED, bool SPLIT, int EPI = kEpiNone, bool B_KN = false>
 __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	const half_t* __restrict__ A, const half_t* __restrict__ B, half_t* __restrict__ C,
@@ -43,7 +44,6 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	const half_t* __restrict__ bias = nullptr, float ep_param = 0.0f)
 {
 	static_assert(!SPLIT || EPI == kEpiNone, "the planes hold raw sums");
-	static_assert(!B_KN || EPI != kEpiGeluMul, "two weight matrices: k-contiguous only");
 	static_assert(TN == 4, "a [K, N] unit row of 256 bytes: 16 chunks, four k rows per load");
 	using Cfg = GemmRing3Cfg<TM, TN>;
 	extern __shared__ __align__(1024) char lds[];
@@ -67,7 +67,8 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	constexpr bool DUAL = EPI == kEpiGeluMul;
 	const int64_t n0 = (int64_t)tile_n * (DUAL ? Cfg::BN / 2 : Cfg::BN);
 	// DUAL: the unit rows wave w loads are output columns (BN / 4) (w / 2) .. of the tile, from B (w even) or B2
-	const half_t* const b_of_wave = DUAL && (wave & 1) ? bias : B;
+	// ([K, N]: the first two waves load B, the other two B2)
+	const half_t* const b_of_wave = DUAL && (B_KN ? wave >> 1 : wave & 1) ? bias : B;
 	const int b_unit_row = DUAL ? 8 * Cfg::kLoadsB * (wave >> 1) : 8 * Cfg::kLoadsB * wave;
 
 	// Direct loads.  A unit row is 64 halves = eight 16-byte chunks; chunk c of row r sits at position c ^ ((r >> 1) & 7).
@@ -77,6 +78,10 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	const unsigned lds0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
 	const int ld_row = lane >> 3, ld_pos = lane & 7;
 	unsigned* const table = reinterpret_cast<unsigned*>(lds + 3 * Cfg::kStageBytes) + wave * (16 * 64) + lane;
+	// [K, N] units: k rows of 256 bytes, four to an instruction (two matrices: of 128 bytes, eight); the wave's first of them
+	constexpr int kKnRowBytes = DUAL ? 128 : 256, kKnRowsPerLoad = 1024 / kKnRowBytes, kKnChunks = kKnRowBytes / 16;
+	const int kn_first = DUAL ? 32 * (wave & 1) : 16 * wave;
+	const auto kn_swizzle = [](int k) { return DUAL ? kn_half_row_swizzle(k) : kn_row_swizzle(k); };
 	int64_t a_first = m0 + 8 * Cfg::kLoadsA * wave, b_first = n0 + b_unit_row;
 	if constexpr (RAGGED)
 	{
@@ -101,8 +106,8 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 		{
 			// one instruction fills 4 k rows of 256 bytes: lane -> row lane / 16, position lane % 16, and the chunk at
 			// position p of row k is chunk p ^ kn_row_swizzle(k); instruction q covers rows 16 wave + 4 q .. + 3
-			const int k_wave = 4 * q + (lane >> 4);
-			int64_t col = (int64_t)(((lane & 15) ^ kn_row_swizzle(16 * wave + k_wave)) << 3);
+			const int k_wave = kKnRowsPerLoad * q + lane / kKnChunks;
+			int64_t col = (int64_t)(((lane % kKnChunks) ^ kn_swizzle(kn_first + k_wave)) << 3);
 			if constexpr (RAGGED)
 				if (n0 + col + 8 > N) col = N - 8 - n0;
 			table[64 * (8 + q)] = (unsigned)((k_wave * ldb + col) * 2);
@@ -112,7 +117,7 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	}
 	const unsigned table_addr = lds0 + 3 * Cfg::kStageBytes + (wave * (16 * 64) + lane) * 4;
 	const uintptr_t a_wave = reinterpret_cast<uintptr_t>(A + a_first * lda);
-	const uintptr_t b_wave = reinterpret_cast<uintptr_t>(B_KN ? B + (int64_t)(16 * wave) * ldb + n0 : b_of_wave + b_first * ldb);
+	const uintptr_t b_wave = reinterpret_cast<uintptr_t>(B_KN ? b_of_wave + (int64_t)kn_first * ldb + n0 : b_of_wave + b_first * ldb);
 	const unsigned share_a = wave * (Cfg::kLoadsA * 1024);                       // the wave's rows inside a stage
 	const unsigned share_b = Cfg::BM * 128 + wave * (Cfg::kLoadsB * 1024);
 	const int slabs = K / 64;
@@ -126,9 +131,10 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	// columns 4 (r % 4) .. + 3 of the MFMA tile; column tile j of wave column wn lies at chunk pair (4 wn + j) ^ (row
 	// swizzle / 2), which the assembly block adds per tile from `b_swizzle`
 	const unsigned kn_k = 8 * (lane >> 4) + (frag_row >> 2);
-	const unsigned b_addr = B_KN ? Cfg::BM * 128 + kn_k * 256 + ((frag_row & 3) >> 1) * 16 + 8 * (frag_row & 1)
+	// (two matrices: column tile j < 2 of either half at chunk pair (2 wn + j) ^ (row swizzle / 2))
+	const unsigned b_addr = B_KN ? Cfg::BM * 128 + kn_k * kKnRowBytes + ((frag_row & 3) >> 1) * 16 + 8 * (frag_row & 1)
 	                             : Cfg::BM * 128 + (wn * Cfg::kWaveN + frag_row) * 128 + frag_chunk * 16;
-	[[maybe_unused]] const unsigned b_swizzle = (unsigned)((kn_row_swizzle((int)kn_k) >> 1) ^ (wn << 2)) << 5;
+	[[maybe_unused]] const unsigned b_swizzle = (unsigned)((kn_swizzle((int)kn_k) >> 1) ^ (wn << (DUAL ? 1 : 2))) << 5;
 	[[maybe_unused]] const unsigned b_step = (unsigned)(128 * ldb);      // bytes from one [K, N] slab to the next
 
 	// The accumulators leave the block as vectors of 32 registers pinned to a[0 : 4 TM TN): MFMA tile (i, j) in registers
@@ -155,7 +161,19 @@ __global__ __launch_bounds__(256) void gemm_f16_nt_ring3_kernel(
 	"v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "v245", "v246", "v247", "v248", "v249", \
 	"v250", "v251", "v252", "v253", "v254", "v255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", \
 	"s69", "s70", "s71", "s72", "s73", "s74", "scc", "m0", "memory"
-	if constexpr (TM == 8 && B_KN)
+	if constexpr (TM == 8 && B_KN && DUAL)
+		asm volatile(
+#include "gemm_f16_ring_loop_8x4kn2.inc"
+			: "={a[0:31]}"(r0), "={a[32:63]}"(r1), "={a[64:95]}"(r2), "={a[96:127]}"(r3)
+			: ANYGPU_RING3_INPUTS, [bsx] "v"(b_swizzle), [bstep] "s"(b_step)
+			: ANYGPU_RING3_CLOBBERS);
+	else if constexpr (B_KN && DUAL)
+		asm volatile(
+#include "gemm_f16_ring_loop_4x4kn2.inc"
+			: "={a[0:31]}"(r0), "={a[32:63]}"(r1)
+			: ANYGPU_RING3_INPUTS, [bsx] "v"(b_swizzle), [bstep] "s"(b_step)
+			: ANYGPU_RING3_CLOBBERS);
+	else if constexpr (TM == 8 && B_KN)
 		asm volatile(
 #include "gemm_f16_ring_loop_8x4kn.inc"
 			: "={a[0:31]}"(r0), "={a[32:63]}"(r1), "={a[64:95]}"(r2), "={a[96:127]}"(r3)
@@ -228,14 +246,12 @@ inline hipError_t launch_gemm_f16_ring3(const half_t* A, const half_t* B, half_t
 	const bool ragged = M % Cfg::BM != 0 || N % kOutN != 0 || !c_aligned;
 	const int which = planes != nullptr ? 2 : ragged ? 1 : 0;
 	auto kernel = which == 1 ? gemm_f16_nt_ring3_kernel<TM, TN, true, false, EPI> : gemm_f16_nt_ring3_kernel<TM, TN, false, false, EPI>;
+	if (kn) kernel = which == 1 ? gemm_f16_nt_ring3_kernel<TM, TN, true, false, EPI, true> : gemm_f16_nt_ring3_kernel<TM, TN, false, false, EPI, true>;
 	if constexpr (EPI == kEpiNone)
 	{
-		if (which == 2) kernel = gemm_f16_nt_ring3_kernel<TM, TN, true, true, kEpiNone>;
-		if (kn)
-			kernel = which == 2 ? gemm_f16_nt_ring3_kernel<TM, TN, true, true, kEpiNone, true>
-			       : which == 1 ? gemm_f16_nt_ring3_kernel<TM, TN, true, false, kEpiNone, true> : gemm_f16_nt_ring3_kernel<TM, TN, false, false, kEpiNone, true>;
+		if (which == 2) kernel = kn ? gemm_f16_nt_ring3_kernel<TM, TN, true, true, kEpiNone, true> : gemm_f16_nt_ring3_kernel<TM, TN, true, true, kEpiNone>;
 	}
-	else if (which == 2 || kn) return hipErrorInvalidValue;
+	else if (which == 2) return hipErrorInvalidValue;
 	// More than 64 KB of dynamic LDS has to be granted per function and per device, once.
 	static std::atomic<uint64_t> configured_devices[6];
 	(void)hipGetLastError();

@@ -143,6 +143,13 @@ __device__ __forceinline__ int kn_row_swizzle(int k)
 	return 2 * ((k & 3) | (((k >> 3) & 1) << 2));
 }
 
+// The same for rows of 128 bytes: two rows to a sweep of the banks, so the row's parity picks one half of them and s(k) = ((k >> 1) & 1) |
+// ((k >> 3) & 1) << 1 one of the four 32-byte slots in it.
+__device__ __forceinline__ int kn_half_row_swizzle(int k)
+{
+	return 2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1));
+}
+
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
 // ds_read_b64_tr_b16: within each group of 16 lanes, lane i receives element (i % 4) of the

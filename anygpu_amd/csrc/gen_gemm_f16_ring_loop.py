@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Writes gemm_f16_ring_loop.inc and gemm_f16_ring_loop_kn.inc: the main loop of the 256 x 256 fp16 GEMM tile kernel of gemm_f16_ring.hpp (four waves, a
+"""Writes gemm_f16_ring_loop.inc, gemm_f16_ring_loop_kn.inc and gemm_f16_ring_loop_kn2.inc: the main loop of the 256 x 256 fp16 GEMM tile kernel of gemm_f16_ring.hpp (four waves, a
 128 x 128 patch per wave) as the text of one inline-assembly block, every instruction in issue order.
 
 Why assembly: with one wave per SIMD nothing hides a stall, and the 256 accumulator registers of a lane fill the AGPR file
@@ -22,6 +22,11 @@ row), filled two rows per load, and a fragment is put together by two transposin
 each).  The swizzle permutes the eight column tiles of the patch differently in every lane, so each tile has an address
 register of its own: v[80:87] inside a unit, v[88:95] in the unit being read; a slab of B is 64 rows further on in
 memory, s73 holds the upper half of that product.
+
+Two matrices stored [K, N] (the "kn2" forms, GELU(gate) * up): a B unit is two halves of 64 k rows, one per matrix, with
+half of the tile's unit columns each (rows half as long), so that every load instruction reads one matrix.  Of a wave's
+column tiles the first half comes from the first matrix, the second half from the second at the same columns: the same
+address registers, the second half unit in the offset of the read.
 
 LDS holds five operand units of 32 KB: a unit is the 256 rows x 64 k (128-byte rows, 16-byte chunks swizzled by the row) of
 A or of B for one 64-deep slab.  Operand slab n of the sequence A(0), B(0), A(1), B(1), ... lives in unit n mod 5.  While
@@ -50,7 +55,7 @@ v112 / v113 and v114 / v115 the fragment addresses of the first and of the secon
 addresses inside a stage with bit 6 flipped.  Operands: vtab, aaddr, baddr (inside a stage), abaselo .. bbasehi, slabs as
 above, lds0 (SGPR: LDS address of stage 0), ldsa / ldsb (SGPR: offset of the wave's share of the A / B unit in a stage).
 
-Usage: gen_gemm_f16_ring_loop.py OUTPUT [kn | 8x4 | 4x4 | 8x4kn | 4x4kn]
+Usage: gen_gemm_f16_ring_loop.py OUTPUT [kn | kn2 | 8x4 | 4x4 | 8x4kn | 4x4kn | 8x4kn2 | 4x4kn2]
 """
 import sys
 
@@ -79,8 +84,17 @@ def afrag(buf, i):
     return f"v[{r}:{r + 3}]"
 
 
-def generate(kn):
-    """the block's instructions as (text, comment) pairs; kn: B stored [K, N]"""
+def kn_reads(buf, cols, row, dual, second_half):
+    """the transposing fragment reads of `cols` column tiles out of a [k][n] unit with rows of `row` bytes: the second
+    32-deep half of the slab lies 32 rows further on, the upper four k of a lane's eight 4 rows, the second matrix 64 rows"""
+    own = cols // 2 if dual else cols            # column tiles with an address register of their own
+    off = 32 * row if second_half else 0
+    return [f"ds_read_b64_tr_b16 {bfrag(buf, q // 2, q % 2)}, v{V_BCUR + q // 2 % own} offset:{off + 4 * row * (q % 2) + 64 * row * (q // 2 // own)}"
+            for q in range(2 * cols)]
+
+
+def generate(kn, dual=False):
+    """the block's instructions as (text, comment) pairs; kn: B stored [K, N]; dual: two such matrices"""
     lines = []
     # address arithmetic starts behind this MFMA (the reads of the step have been issued by then)
     extra_from = 47 if kn else 33
@@ -117,18 +131,16 @@ def generate(kn):
 
     def reads(buf, va, vb, second_half):
         """the fragment reads of a step.  k-contiguous operand: MFMA tile i of the patch lies 16 rows = 2048 bytes further
-        on.  B stored [K, N]: per column tile its own address, the second 32-deep half of the slab 32 rows = 16 KB
-        further on, the upper four k of a lane's eight 4 rows = 2 KB further on."""
+        on.  B stored [K, N]: per column tile its own address (rows of 512 bytes, 256 with two matrices)."""
         if kn:
-            off = 16384 if second_half else 0
-            out = [f"ds_read_b64_tr_b16 {bfrag(buf, q // 2, q % 2)}, v{V_BCUR + q // 2} offset:{off + 2048 * (q % 2)}" for q in range(16)]
+            out = kn_reads(buf, 8, 256 if dual else 512, dual, second_half)
         else:
             out = [f"ds_read_b128 {bfrag(buf, q)}, {vb} offset:{q * 2048}" for q in range(8)]
         out += [f"ds_read_b128 {afrag(buf, q)}, {va} offset:{q * 2048}" for q in range(8)]
         return out
 
     def b_unit_addresses(unit_reg):
-        return [f"v_add_u32 v{V_BCUR + j}, {unit_reg}, v{V_BUNIT + j}" for j in range(8)]
+        return [f"v_add_u32 v{V_BCUR + j}, {unit_reg}, v{V_BUNIT + j}" for j in range(4 if dual else 8)]
 
     # ---- prologue: A(0), B(0), A(1), B(1) into units 0 .. 3, fragments of the first step
     emit(f"s_mov_b32 {S_T}, 0", "prologue")
@@ -140,7 +152,7 @@ def generate(kn):
     emit("s_waitcnt lgkmcnt(0)")
     emit(f"v_xor_b32 {V_A1}, 64, %[aaddr]")
     if kn:
-        for j in range(8):
+        for j in range(4 if dual else 8):
             emit(f"v_xor_b32 v{V_BUNIT + j}, {32 * j}, %[bsx]")
             emit(f"v_add_u32 v{V_BUNIT + j}, %[baddr], v{V_BUNIT + j}")
     else:
@@ -223,10 +235,10 @@ def generate(kn):
     return lines
 
 
-def generate_three_stages(tm, tn, kn=False):
+def generate_three_stages(tm, tn, kn=False, dual=False):
     """the block for a patch of tm x tn MFMA tiles per wave (tile 32 tm x 32 tn), three LDS stages; kn: B stored [K, N]
     (a B unit of 64 k rows x 32 tn n, fragments by transposing reads through one address register per column tile, as in
-    the kn form of the 256 x 256 tile; s64 and s74 hold the halves of the slab's byte offset)"""
+    the kn form of the 256 x 256 tile; s64 and s74 hold the halves of the slab's byte offset); dual: two such matrices"""
     lines = []
     bm, bn = 32 * tm, 32 * tn
     stage = (bm + bn) * 128
@@ -269,19 +281,19 @@ def generate_three_stages(tm, tn, kn=False):
                         f"global_load_lds_dwordx4 v{v}, {A_CUR if operand == 'a' else B_CUR}"))
         return out
 
-    row_kn = 64 * tn                            # bytes of a [k][n] unit row
+    row_kn = 32 * tn if dual else 64 * tn       # bytes of a [k][n] unit row
+    own = tn // 2 if dual else tn               # column tiles with an address register of their own
 
     def reads(buf, va, vb, second_half=False):
         if kn:
-            off = 32 * row_kn if second_half else 0
-            out = [f"ds_read_b64_tr_b16 {bfrag(buf, q // 2, q % 2)}, v{V_BCUR + q // 2} offset:{off + 4 * row_kn * (q % 2)}" for q in range(2 * tn)]
+            out = kn_reads(buf, tn, row_kn, dual, second_half)
         else:
             out = [f"ds_read_b128 {bfrag(buf, q)}, {vb} offset:{q * 2048}" for q in range(tn)]
         out += [f"ds_read_b128 {afrag(buf, q)}, {va} offset:{q * 2048}" for q in range(tm)]
         return out
 
     def b_stage_addresses(stage_reg):
-        return [f"v_add_u32 v{V_BCUR + j}, {stage_reg}, v{V_BUNIT + j}" for j in range(tn)]
+        return [f"v_add_u32 v{V_BCUR + j}, {stage_reg}, v{V_BUNIT + j}" for j in range(own)]
 
     # ---- prologue: slabs 0 and 1 and the first half of the loads of slab 2, fragments of the first step
     emit(f"s_mov_b32 {S_T}, 0", "prologue")
@@ -295,7 +307,7 @@ def generate_three_stages(tm, tn, kn=False):
     emit("s_waitcnt lgkmcnt(0)")
     emit(f"v_xor_b32 {V_A64}, 64, %[aaddr]")
     if kn:
-        for j in range(tn):
+        for j in range(own):
             emit(f"v_xor_b32 v{V_BUNIT + j}, {32 * j}, %[bsx]")
             emit(f"v_add_u32 v{V_BUNIT + j}, %[baddr], v{V_BUNIT + j}")
     else:
@@ -398,9 +410,10 @@ if __name__ == "__main__":
     form = sys.argv[2] if len(sys.argv) > 2 else ""
     with open(sys.argv[1], "w") as f:
         f.write("// Written by gen_gemm_f16_ring_loop.py (the register plan and the schedule are explained there): do not edit.\n")
-        kn = form.endswith("kn")
-        patch = form[:-2] if kn else form
-        for s, c in (generate_three_stages(*(int(x) for x in patch.split("x")), kn) if "x" in patch else generate(kn)):
+        dual = form.endswith("kn2")
+        kn = dual or form.endswith("kn")
+        patch = form.split("kn")[0]
+        for s, c in (generate_three_stages(*(int(x) for x in patch.split("x")), kn, dual) if patch else generate(kn, dual)):
             if c:
                 f.write(f"// {c}\n")
             f.write(f'"{s}\\n\\t"\n')

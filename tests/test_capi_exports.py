@@ -93,7 +93,9 @@ def test_generated_gemm_loop_is_current(tmp_path):
         assert out.read_text() == (csrc / name).read_text()
     for name, form in (("gemm_f16_ring_loop.inc", []), ("gemm_f16_ring_loop_kn.inc", ["kn"]),
                        ("gemm_f16_ring_loop_8x4.inc", ["8x4"]), ("gemm_f16_ring_loop_4x4.inc", ["4x4"]),
-                       ("gemm_f16_ring_loop_8x4kn.inc", ["8x4kn"]), ("gemm_f16_ring_loop_4x4kn.inc", ["4x4kn"])):
+                       ("gemm_f16_ring_loop_8x4kn.inc", ["8x4kn"]), ("gemm_f16_ring_loop_4x4kn.inc", ["4x4kn"]),
+                       ("gemm_f16_ring_loop_kn2.inc", ["kn2"]), ("gemm_f16_ring_loop_8x4kn2.inc", ["8x4kn2"]),
+                       ("gemm_f16_ring_loop_4x4kn2.inc", ["4x4kn2"])):
         out = tmp_path / name
         subprocess.run([sys.executable, str(csrc / "gen_gemm_f16_ring_loop.py"), str(out), *form], check=True)
         assert out.read_text() == (csrc / name).read_text()

@@ -332,3 +332,20 @@ def test_sdp_attention_decode_under_a_window_of_whole_tiles(ops, oracle):
         want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(np.ascontiguousarray(t[b])) for t in (q, k, v)), alpha=0.0625, softcap=50.0,
                                           causal=True, window=4096, q_per_kv=2, threads=8)
         assert scaled_rel_err(got[b], want, 1.0) <= TOL_F16_ROWOPS * 2
+
+
+@pytest.mark.parametrize("m,n,k", [(130, 72, 64), (200, 1000, 128), (300, 2056, 192), (256, 2048, 320), (2000, 4072, 320), (2048, 4096, 320),
+                                   (4090, 4072, 320), (4096, 4096, 320)])
+def test_upproj_and_bias_f16_row_major_weights_in_whole_slabs(ops, m, n, k):
+    # [K, N] weights, K in whole slabs of 64: one and two matrices in 128 x 128, 256 x 128 and 256 x 256 tiles, whole and ending past M and N.
+    # Small integers times a power of two: the sums are exact; bounds as in test_mm_few_rows_k_cut_over_waves
+    a, w1, w2 = (synth.integers(s, shape, -2, 2).astype(np.float16) for s, shape in ((m, (m, k)), (n + 2, (k, n)), (n + 3, (k, n))))
+    bias = synth.integers(3, (n,), -9, 9).astype(np.float16)
+    s1 = exact_int_product(a, w1)
+    assert np.array_equal(host(ops.tensor_gemm(dev(a), dev(w1), dev(bias))).astype(np.int64), s1 + bias.astype(np.int64))
+    scale = 2.0 ** -6
+    s1, s2 = s1 * scale, exact_int_product(a, w2) * scale
+    got = host(ops.mlp_gemma2_fused_upproj(dev((a * scale).astype(np.float16)), dev(w1), dev(w2))).astype(np.float64)
+    gated = 0.5 * s1 * (1.0 + np.tanh(math.sqrt(2.0 / math.pi) * (s1 + 0.044715 * s1 ** 3))) * s2
+    # (the half epilogue's tanh: 4.4e-5 of the gate's factor)
+    assert np.all(np.abs(got - gated) <= 2.0 ** -11 * np.abs(gated) + 5e-5 * np.abs(s1 * s2) + 2.0 ** -24)
