@@ -2,12 +2,11 @@
 // sliding-window masks) fused in.  HBM-bound: every visible input element is read once and
 // every output element written once, with 16-byte accesses.
 //
-// Fast kernel: one wave owns one row and keeps it in registers (VPL 16-byte vectors per
-// lane), runs an online max/sum over the vectors as they arrive, combines the 64 lane
-// states with DPP reductions, then normalises from registers.  Vectors that lie wholly
-// outside the visible key interval [lo, hi] of the row are never loaded; their outputs are
-// stored as zeros.
-// Short rows (up to 64 vectors) share a wave four at a time; rows longer than a block's registers hold are walked
+// Without a mask tensor (softmax_rows_kernel): a row of lanes, a wave or a block owns one row and keeps its visible part in
+// registers; rows of any width and pitch.  Vectors that lie wholly outside the visible key interval [lo, hi] of the row are never
+// loaded; their outputs are stored as zeros.
+// With one, or where x and y are not aligned alike (softmax_rows_wave_kernel): the same with an online max/sum over the vectors as they
+// arrive.  Rows longer than a block's registers hold are walked
 // twice by a block of 1024 threads with 16-byte accesses, at any width, stride or alignment.
 // An additive mask tensor [q_len, cols] shared by the heads of a batch is read with ordinary (cached) loads, and the
 // blocks are dealt so that the heads of a mask row run side by side on one XCD (block_rows).
@@ -278,16 +277,18 @@ __global__ __launch_bounds__(256) void softmax_rows_wave_kernel(const SoftmaxArg
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp16 fast kernel.  One wave per row, the VISIBLE part of the row in registers: lane l owns the
-// 16-byte vectors 64 (c_lo + t) + l (t < VPL), where c_lo is the 64-vector chunk of the row that
-// holds the first visible key, so a sliding window of W keys needs (W / 8 + 63) / 64 + 1 vectors per
-// lane however long the row is.  Vectors without a visible key are never loaded; they are stored as zeros.
+// Rows without a mask tensor.  GROUP threads share a row (16: a row of lanes, 64: a wave, 256 and 512: the block) and keep its VISIBLE part in
+// registers as fp32 logits: the vectors kGroup (c_lo + t) + lane (t < VPL), where c_lo is the chunk of GROUP vectors that holds the
+// first visible key, so a sliding window of W keys needs W / (EPV GROUP) + 2 vectors per lane however long the row is.  Vectors
+// without a visible key are never loaded; they are stored as zeros.  Three passes over the registers: logit and maximum, exp2 and sum,
+// scale and store, so that an element costs the logit's transcendentals and one more, and is rounded once.
 //
-// One pass over the registers runs the online max/sum recurrence per vector and leaves
-// e = exp2(z - m_t) (m_t = running maximum after vector t) in the registers as halves, in place
-// of the input; the sum is accumulated in fp32 from the unrounded values.  After the DPP
-// reductions a second pass over the registers multiplies by exp2(m_t - M) / S in fp32 and rounds
-// to the fp16 output.  The logit transform (scale, softcap) therefore runs once per element.
+// Rows of any width and pitch: the vectors lie at 16-byte boundaries of memory (a wave's chunks at whole lines) and not at the row's own start; the
+// elements in front of the row in its first vector and behind it in its last are another row's: loaded where they are inside the
+// tensor, never stored.  x and y have to be aligned alike (rows_alike).  A row of odd width walked from its own start splits every access over
+// two lines and its ends into eight element accesses.  us before / here (softcap 50, causal, fp16): 16 heads x 4615 x 4615
+// under a window of 4096 354 / 182, 32 x 1629 x 1629 85 / 51, 8 x 1038 x 16310 181 / 93; float32 without softcap 32 x 1629 x 1629 118 / 87; rows
+// that were aligned all along, whose halves were rounded twice before: 8 x 8192 x 8192 window 4096 277 / 244 (6.1 TB/s of needed bytes).
 // ---------------------------------------------------------------------------------------------
 template <bool SOFTCAP>
 __device__ __forceinline__ float logit2_fast(float x, float k_in, float k_cap)
@@ -303,57 +304,89 @@ __device__ __forceinline__ float logit2_fast(float x, float k_in, float k_cap)
 	return x * k_in;
 }
 
-template <int VPL, bool SOFTCAP>
-__global__ __launch_bounds__(256) void softmax_rows_f16_window_kernel(const SoftmaxArgs a)
+template <typename T, int VPL, int GROUP, bool SOFTCAP>
+__global__ __launch_bounds__(GROUP > 256 ? GROUP : 256) void softmax_rows_kernel(const SoftmaxArgs a)
 {
-	constexpr int EPV = 8;
-	const int lane = threadIdx.x & (kWaveSize - 1);
-	const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-	if (row >= a.rows) return;  // uniform over the wave
+	static_assert(GROUP == 16 || GROUP == 64 || GROUP == 256 || GROUP == 512, "a row of lanes, a wave or the block per row");
+	constexpr int kThreads = GROUP > 256 ? GROUP : 256, kWaves = GROUP > 64 ? GROUP / 64 : 1;
+	constexpr int EPV = 16 / (int)sizeof(T);
+	// what the vectors count from: a 16-byte boundary, or the line, so that the accesses of a wave are whole lines
+	constexpr int kStart = GROUP == 16 ? EPV : 128 / (int)sizeof(T);
+	using Vec = typename Vec16<T>::type;
+	__shared__ float red_m[kWaves], red_s[kWaves];
+	const int lane = threadIdx.x & (GROUP - 1);
+	const int64_t row = (int64_t)blockIdx.x * (kThreads / GROUP) + threadIdx.x / GROUP;
+	if (row >= a.rows) return;  // uniform over the group
 	const RowSpan span = row_span(a, row);
-	const half8_t* __restrict__ xr = reinterpret_cast<const half8_t*>(static_cast<const half_t*>(a.x) + row * a.xs);
-	half8_t* __restrict__ yr = reinterpret_cast<half8_t*>(static_cast<half_t*>(a.y) + row * a.ys);
-	const int nvec = (int)(a.cols / EPV);
-	const int lo = (int)span.lo, hi = (int)span.hi;
-	const half8_t zeros = {};
-
+	const T* const xr = static_cast<const T*>(a.x) + row * a.xs;
+	T* const yr = static_cast<T*>(a.y) + row * a.ys;
+	const int shift = (int)(reinterpret_cast<uintptr_t>(yr) / sizeof(T) % kStart);
+	const Vec* __restrict__ xv = reinterpret_cast<const Vec*>(xr - shift);
+	Vec* __restrict__ yv = reinterpret_cast<Vec*>(yr - shift);
+	// element numbers from there: the row is [shift, end), its visible part [lo, hi]
+	const int end = shift + (int)a.cols;
+	const int lo = (int)span.lo + shift, hi = (int)span.hi + shift;
+	const int v_first = shift / EPV, v_end = (end - 1) / EPV;
+	const Vec zeros = {};
+	auto put = [&](int v, const Vec& val) {
+		const int from = shift - v * EPV, to = end - v * EPV;         // elements [from, to) of the vector are the row's
+		if (from <= 0 && to >= EPV) __builtin_nontemporal_store(val, yv + v);
+		else
+		{
+#pragma unroll
+			for (int e = 0; e < EPV; ++e)
+				if (e >= from && e < to) reinterpret_cast<T*>(yv + v)[e] = val[e];
+		}
+	};
 	if (hi < lo)
 	{
-		for (int v = lane; v < nvec; v += kWaveSize) __builtin_nontemporal_store(zeros, yr + v);
+		for (int v = v_first + lane; v <= v_end; v += GROUP) put(v, zeros);
 		return;
 	}
 	const int v_lo = lo / EPV, v_hi = hi / EPV;
-	// Every load and store of the wave covers one whole 1 KB chunk of the row (64 vectors from a multiple of 64), whatever
-	// the visible interval: lanes outside it load nothing and store zeros.  A run of stores that starts inside a chunk
-	// leaves the memory partial lines at both ends of every instruction, and a launch whose runs start at an odd vector
-	// writes a fifth slower for it (8 heads x 8192 x 8192, window 4096: 295 -> 272 us).
-	const int c_lo = v_lo / kWaveSize, c_hi = v_hi / kWaveSize;
+	// Every load and store of the group covers whole chunks, whatever the visible interval: lanes outside it load nothing and store
+	// zeros.  A run of stores that starts inside a chunk leaves the memory partial lines at both ends of every instruction, and a launch
+	// whose runs start at an odd vector writes a fifth slower for it (8 heads x 8192 x 8192, window 4096: 295 -> 272 us).
+	const int c_lo = v_lo / GROUP, c_hi = v_hi / GROUP;
 
-	half8_t reg[VPL];
+	Vec raw[VPL];
 #pragma unroll
 	for (int t = 0; t < VPL; ++t)
 	{
-		const int v = (c_lo + t) * kWaveSize + lane;
-		half8_t val = {};
-		if (v >= v_lo && v <= v_hi) val = __builtin_nontemporal_load(xr + v);
-		reg[t] = val;
+		const int v = (c_lo + t) * GROUP + lane;
+		Vec val = {};
+		if (v >= v_lo && v <= v_hi)
+		{
+			// (the first vector of the first row and the last of the last may reach past the tensor)
+			const int from = row == 0 ? shift - v * EPV : 0, to = row == a.rows - 1 ? end - v * EPV : EPV;
+			if (from <= 0 && to >= EPV) val = __builtin_nontemporal_load(xv + v);
+			else
+			{
+#pragma unroll
+				for (int e = 0; e < EPV; ++e)
+					if (e >= from && e < to) val[e] = reinterpret_cast<const T*>(xv + v)[e];
+			}
+		}
+		raw[t] = val;
 	}
 
 	const float k_in = SOFTCAP ? 2.0f * kLog2e * a.alpha * a.inv_cap : a.alpha_log2e;
 	const float k_cap = a.cap_log2e;
-
-	OnlineState st;
-	float m_at[VPL];
+	float z[VPL][EPV];
+	float m = -INFINITY;
+	__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
 	for (int t = 0; t < VPL; ++t)
 	{
-		const int v = (c_lo + t) * kWaveSize + lane;
-		m_at[t] = -INFINITY;
+		const int v = (c_lo + t) * GROUP + lane;
 		if (v >= v_lo && v <= v_hi)
 		{
-			float z[EPV];
 #pragma unroll
-			for (int e = 0; e < EPV; ++e) z[e] = logit2_fast<SOFTCAP>((float)reg[t][e], k_in, k_cap);
+			for (int e = 0; e < EPV; ++e)
+			{
+				if constexpr (sizeof(T) == 2) z[t][e] = logit2_fast<SOFTCAP>((float)raw[t][e], k_in, k_cap);
+				else z[t][e] = SOFTCAP ? k_cap * tanh_f32(raw[t][e] * a.alpha * a.inv_cap) : raw[t][e] * a.alpha_log2e;
+			}
 			if (v == v_lo || v == v_hi)
 			{
 				// only the two end vectors can hold keys outside [lo, hi]
@@ -361,66 +394,100 @@ __global__ __launch_bounds__(256) void softmax_rows_f16_window_kernel(const Soft
 				for (int e = 0; e < EPV; ++e)
 				{
 					const int j = v * EPV + e;
-					if (j < lo || j > hi) z[e] = -INFINITY;
+					if (j < lo || j > hi) z[t][e] = -INFINITY;
 				}
 			}
-			float vmax = z[0];
 #pragma unroll
-			for (int e = 1; e < EPV; ++e) vmax = fmaxf(vmax, z[e]);
-			const float mn = fmaxf(st.m, vmax);
-			const float shift = (mn == -INFINITY) ? 0.0f : mn;
-			float acc = st.s * fast_exp2(st.m - shift);
-			half8_t ev;
-#pragma unroll
-			for (int e = 0; e < EPV; ++e)
-			{
-				const float p = fast_exp2(z[e] - shift);
-				acc += p;
-				ev[e] = (half_t)p;
-			}
-			reg[t] = ev;
-			m_at[t] = mn;
-			st.s = acc;
-			st.m = mn;
+			for (int e = 0; e < EPV; ++e) m = fmaxf(m, z[t][e]);
 		}
 	}
-
-	const float M = wave_allreduce(st.m, MaxOp());
-	const float S = wave_allreduce(st.s * exp2_shift(st.m, M), SumOp());
-	const float inv = S > 0.0f ? 1.0f / S : 0.0f;
-
-	// the whole row goes out in address order, chunk by chunk: zeros, the chunks with visible keys, zeros
-	for (int c = 0; c < c_lo; ++c)
-		__builtin_nontemporal_store(zeros, yr + c * kWaveSize + lane);
+	float M = GROUP == 16 ? row_allreduce(m, MaxOp()) : wave_allreduce(m, MaxOp());
+	if constexpr (kWaves > 1)
+	{
+		if ((threadIdx.x & 63) == 0) red_m[threadIdx.x >> 6] = M;
+		__syncthreads();
+#pragma unroll
+		for (int w = 0; w < kWaves; ++w) M = fmaxf(M, red_m[w]);
+	}
+	const float m_safe = M == -INFINITY ? 0.0f : M;
+	float sum[2] = {0.0f, 0.0f};
 #pragma unroll
 	for (int t = 0; t < VPL; ++t)
 	{
-		const int v = (c_lo + t) * kWaveSize + lane;
-		if (c_lo + t <= c_hi && v < nvec)
+		const int v = (c_lo + t) * GROUP + lane;
+		if (v >= v_lo && v <= v_hi)
 		{
-			half8_t out = zeros;
-			if (v >= v_lo && v <= v_hi)
-			{
-				const float scale = exp2_shift(m_at[t], M) * inv;
 #pragma unroll
-				for (int e = 0; e < EPV; ++e) out[e] = (half_t)((float)reg[t][e] * scale);
+			for (int e = 0; e < EPV; ++e)
+			{
+				z[t][e] = fast_exp2(z[t][e] - m_safe);
+				sum[e % 2] += z[t][e];
 			}
-			__builtin_nontemporal_store(out, yr + v);
 		}
 	}
-	for (int v = (c_hi + 1) * kWaveSize + lane; v < nvec; v += kWaveSize) __builtin_nontemporal_store(zeros, yr + v);
+	float S = GROUP == 16 ? row_allreduce(sum[0] + sum[1], SumOp()) : wave_allreduce(sum[0] + sum[1], SumOp());
+	if constexpr (kWaves > 1)
+	{
+		if ((threadIdx.x & 63) == 0) red_s[threadIdx.x >> 6] = S;
+		__syncthreads();
+		S = 0.0f;
+#pragma unroll
+		for (int w = 0; w < kWaves; ++w) S += red_s[w];
+	}
+	const float inv = S > 0.0f ? 1.0f / S : 0.0f;
+
+	// the whole row goes out in address order, chunk by chunk: zeros, the chunks with visible keys, zeros
+	for (int v = lane; v < c_lo * GROUP; v += GROUP)
+		if (v >= v_first) put(v, zeros);
+#pragma unroll
+	for (int t = 0; t < VPL; ++t)
+	{
+		const int v = (c_lo + t) * GROUP + lane;
+		if (c_lo + t <= c_hi && v >= v_first && v <= v_end)
+		{
+			Vec out = zeros;
+			if (v >= v_lo && v <= v_hi)
+			{
+#pragma unroll
+				for (int e = 0; e < EPV; ++e) out[e] = (T)(z[t][e] * inv);
+			}
+			put(v, out);
+		}
+	}
+	for (int v = (c_hi + 1) * GROUP + lane; v <= v_end; v += GROUP) put(v, zeros);
 }
 
-template <int VPL>
-static hipError_t launch_f16_window(const SoftmaxArgs& a, hipStream_t stream)
+// Whether the vectors of x and y can be counted from the same 16-byte boundaries in every row.
+static bool rows_alike(const SoftmaxArgs& a, int elem_bytes)
 {
-	const unsigned blocks = (unsigned)((a.rows + 3) / 4);
+	return (reinterpret_cast<uintptr_t>(a.x) - reinterpret_cast<uintptr_t>(a.y)) % 16 == 0 && (a.xs - a.ys) * elem_bytes % 16 == 0 &&
+	       reinterpret_cast<uintptr_t>(a.y) % elem_bytes == 0;
+}
+
+template <typename T, int VPL, int GROUP>
+static hipError_t launch_rows(const SoftmaxArgs& a, hipStream_t stream)
+{
+	constexpr int kThreads = GROUP > 256 ? GROUP : 256;
+	const unsigned blocks = (unsigned)((a.rows + kThreads / GROUP - 1) / (kThreads / GROUP));
 	discard_stale_error();
-	if (a.inv_cap != 0.0f)
-		softmax_rows_f16_window_kernel<VPL, true><<<dim3(blocks), dim3(256), 0, stream>>>(a);
-	else
-		softmax_rows_f16_window_kernel<VPL, false><<<dim3(blocks), dim3(256), 0, stream>>>(a);
+	if (a.inv_cap != 0.0f) softmax_rows_kernel<T, VPL, GROUP, true><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
+	else softmax_rows_kernel<T, VPL, GROUP, false><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
 	return hipGetLastError();
+}
+
+// Vectors per lane that hold the visible part of any row: its keys, the elements that the first vector starts early, and, under a
+// window, the rest of the chunk that the interval starts in (without one every interval starts in the row's first chunk).
+template <typename T>
+static int64_t rows_vectors(const SoftmaxArgs& a, int group)
+{
+	constexpr int EPV = 16 / (int)sizeof(T);
+	const int64_t start = group == 16 ? EPV : 128 / (int)sizeof(T);
+	const bool whole = a.ys % start == 0 && reinterpret_cast<uintptr_t>(a.y) % (start * sizeof(T)) == 0;      // no row starts early
+	const int64_t row_vecs = (a.cols + (whole ? 0 : start - 1) + EPV - 1) / EPV;
+	if (a.window == 0) return (row_vecs + group - 1) / group;
+	const int64_t span = a.causal ? std::min<int64_t>(a.cols, a.window) : a.cols;
+	const int64_t vecs = (span + EPV - 1) / EPV + 1 + group - 1;
+	return std::min<int64_t>((row_vecs + group - 1) / group, (vecs + group - 1) / group);
 }
 
 // Rows longer than a block's registers hold (more than 32768 elements: the logits of an output head): a block of 1024
@@ -575,8 +642,9 @@ static hipError_t launch_wave(const SoftmaxArgs& a, hipStream_t stream)
 {
 	const unsigned blocks = blocks_for_rows(a, 256 / GROUP);
 	discard_stale_error();
-	if (a.mask != nullptr) softmax_rows_wave_kernel<T, VPL, LOOSE, GROUP, true><<<dim3(blocks), dim3(256), 0, stream>>>(a);
-	else softmax_rows_wave_kernel<T, VPL, LOOSE, GROUP, false><<<dim3(blocks), dim3(256), 0, stream>>>(a);
+	// (without a mask tensor only rows of x and y that are not aligned alike get here)
+	if (!LOOSE || a.mask != nullptr) softmax_rows_wave_kernel<T, VPL, LOOSE, GROUP, true><<<dim3(blocks), dim3(256), 0, stream>>>(a);
+	else softmax_rows_wave_kernel<T, VPL, true, GROUP, false><<<dim3(blocks), dim3(256), 0, stream>>>(a);
 	return hipGetLastError();
 }
 
@@ -612,6 +680,35 @@ hipError_t launch_softmax_rows(const void* x, void* y, int64_t rows, int64_t col
 	                    (reinterpret_cast<uintptr_t>(x) % 16 == 0) && (reinterpret_cast<uintptr_t>(y) % 16 == 0) &&
 	                    (mask == nullptr || (mask_stride % EPV == 0 && reinterpret_cast<uintptr_t>(mask) % 16 == 0));
 	const int64_t nvec = cols / EPV;
+	if (mask == nullptr && rows_alike(a, (int)sizeof(T)) && !((cols + EPV - 1) / EPV > 2048 && rows < 256))
+	{
+		// short rows (up to 64 vectors: 512 halves, 256 floats): sixteen lanes per row, four rows per wave
+		if ((cols + EPV - 1) / EPV <= 64 && rows >= 64)
+		{
+			const int64_t per_lane = rows_vectors<T>(a, 16);
+			if (per_lane <= 1) return launch_rows<T, 1, 16>(a, stream);
+			if (per_lane <= 2) return launch_rows<T, 2, 16>(a, stream);
+			if (per_lane <= 4) return launch_rows<T, 4, 16>(a, stream);
+			if (per_lane <= 5) return launch_rows<T, 5, 16>(a, stream);
+		}
+		// A wave per row while that takes up to 6 vectors per lane, else the block: the logits of 9 vectors leave a SIMD three waves (us, wave /
+		// block: 8 heads x 8192 x 8192 window 4096 264 / 244, 1 x 7796 x 7796 39 / 34, 8 x 4096 x 4096 floats 141 / 128; up to 6 the block's two
+		// barriers cost more: 32 x 3001 x 3001 143 / 177); blocks of 512 threads from 8 vectors per thread of 256 on (4 x 4096 x 28000 halves,
+		// softcap: 373 us with 1024 threads, 300)
+		const int64_t per_lane = rows_vectors<T>(a, 64), per_thread = rows_vectors<T>(a, 256);
+		if (per_lane <= 1) return launch_rows<T, 1, 64>(a, stream);
+		if (per_lane <= 2) return launch_rows<T, 2, 64>(a, stream);
+		if (per_lane <= 3) return launch_rows<T, 3, 64>(a, stream);
+		if (per_lane <= 4) return launch_rows<T, 4, 64>(a, stream);
+		if (per_lane <= 6) return launch_rows<T, 6, 64>(a, stream);
+		if (per_thread <= 2) return launch_rows<T, 2, 256>(a, stream);
+		if (per_thread <= 3) return launch_rows<T, 3, 256>(a, stream);
+		if (per_thread <= 4) return launch_rows<T, 4, 256>(a, stream);
+		if (per_thread <= 6) return launch_rows<T, 6, 256>(a, stream);
+		if (per_thread <= 8) return launch_rows<T, 8, 256>(a, stream);
+		if (rows_vectors<T>(a, 512) <= 6) return launch_rows<T, 6, 512>(a, stream);
+		if (rows_vectors<T>(a, 512) <= 8) return launch_rows<T, 8, 512>(a, stream);
+	}
 	// short rows (up to 64 vectors: 512 halves, 256 floats): sixteen lanes per row, four rows per wave
 	if (vec_ok && nvec <= 64 && rows >= 64)
 	{
@@ -626,30 +723,8 @@ hipError_t launch_softmax_rows(const void* x, void* y, int64_t rows, int64_t col
 		if (loose <= 32) return launch_wave<T, 2, true, 16>(a, stream);
 		return launch_wave<T, 4, true, 16>(a, stream);
 	}
-	if constexpr (sizeof(T) == 2)
-	{
-		// vectors a row can touch: its visible keys (the window when causal + window, else the
-		// whole row) plus one for an interval that starts inside a vector
-		const int64_t span = (causal && window > 0) ? std::min<int64_t>(cols, window) : cols;
-		int64_t span_vecs = std::min<int64_t>(nvec, (span + EPV - 1) / EPV + 1);
-		// (the kernel counts in whole chunks of 64 vectors from the chunk the interval starts in; without a window every
-		// interval starts at the start of the row)
-		if (window > 0) span_vecs = std::min<int64_t>((nvec + kWaveSize - 1) / kWaveSize * kWaveSize, span_vecs + kWaveSize - 1);
-		if (vec_ok && mask == nullptr)
-		{
-			if (span_vecs <= kWaveSize * 1) return launch_f16_window<1>(a, stream);
-			if (span_vecs <= kWaveSize * 2) return launch_f16_window<2>(a, stream);
-			if (span_vecs <= kWaveSize * 4) return launch_f16_window<4>(a, stream);
-			if (span_vecs <= kWaveSize * 6) return launch_f16_window<6>(a, stream);
-			if (span_vecs <= kWaveSize * 9) return launch_f16_window<9>(a, stream);
-			if (span_vecs <= kWaveSize * 12) return launch_f16_window<12>(a, stream);
-			if (span_vecs <= kWaveSize * 16) return launch_f16_window<16>(a, stream);
-		}
-	}
-	// A wave holds up to 16 vectors per lane of its row (32 of float32 fit the registers, but leave a SIMD with too few
-	// waves: 16384 x 8192 float32 353 us that way, 185 us with the block per row); the block per row up to 16 as well
-	// (32768 halves, 16384 floats); longer rows, and long rows too few to give every CU a block, are walked twice by
-	// 1024 threads (8192 x 32768 float32: 751 us in registers, 426 us walked twice; 128 x 32768 halves: 18 -> 10 us).
+	// A wave holds up to 16 vectors per lane of its row, the block per row as well (32768 halves, 16384 floats); longer rows, and long
+	// rows too few to give every CU a block, are walked twice by 1024 threads (8192 x 32768 float32: 751 us in registers, 426 us walked twice; 128 x 32768 halves: 18 -> 10 us).
 	constexpr int kMaxVpl = 16;
 	const bool walk_twice = nvec > (int64_t)256 * kMaxVpl || (nvec > 2048 && rows < 256);
 	if (vec_ok && walk_twice)

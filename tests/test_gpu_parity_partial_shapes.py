@@ -349,3 +349,29 @@ def test_upproj_and_bias_f16_row_major_weights_in_whole_slabs(ops, m, n, k):
     gated = 0.5 * s1 * (1.0 + np.tanh(math.sqrt(2.0 / math.pi) * (s1 + 0.044715 * s1 ** 3))) * s2
     # (the half epilogue's tanh: 4.4e-5 of the gate's factor)
     assert np.all(np.abs(got - gated) <= 2.0 ** -11 * np.abs(gated) + 5e-5 * np.abs(s1 * s2) + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("rows,cols,pad,off,window", [(64, 1, 0, 0, 0), (70, 7, 0, 3, 0), (65, 8, 1, 5, 0), (64, 63, 2, 1, 0), (80, 505, 0, 7, 100), (64, 512, 3, 2, 0),
+                                                      (3, 65, 0, 1, 0), (5, 449, 5, 63, 0), (9, 1473, 0, 0, 1000), (7, 1537, 1, 33, 0), (5, 3009, 0, 9, 2049),
+                                                      (6, 3073, 3, 62, 0), (9, 4097, 0, 1, 4096), (4, 8129, 0, 31, 0), (3, 16321, 7, 2, 0), (300, 16385, 0, 0, 4096),
+                                                      (260, 32705, 1, 3, 0)])
+def test_softmax_rows_of_any_width_and_start(ops, oracle, dtype, rows, cols, pad, off, window):
+    # rows that start at any element and share their first and last 16 bytes with other rows: what lies between the rows (NaN here) reaches
+    # no result, and nothing is stored there; x and y start at different places of the same 16 bytes, lines apart
+    import torch
+    np_dt, t_dt = (np.float16, torch.float16) if dtype == "f16" else (np.float32, torch.float32)
+    epv, pitch = 16 // np.dtype(np_dt).itemsize, cols + pad
+    x = synth.normal(cols + rows, (rows, cols), std=8.0).astype(np_dt)
+    xbuf, ybuf = torch.full((off + rows * pitch + 64,), math.nan, dtype=t_dt, device="cuda"), torch.full((off + 3 * epv + rows * pitch + 64,), -7.0, dtype=t_dt, device="cuda")
+    xv, yv = torch.as_strided(xbuf, (rows, cols), (pitch, 1), off), torch.as_strided(ybuf, (rows, cols), (pitch, 1), off + 3 * epv)
+    xv.copy_(dev(x))
+    kw = dict(alpha=0.5, softcap=20.0 if off % 2 else 0.0, causal=window > 0, window=window, q_len=rows, diag=cols - rows)
+    ops.tensor_softmax(xv, out=yv, **kw)
+    got = host(yv).astype(np.float64)
+    want = oracle.attention_softmax(oracle.cvt_f16_to_f32(x) if dtype == "f16" else x, **kw).reshape(rows, cols).astype(np.float64)
+    tol = TOL_F16_ROWOPS if dtype == "f16" else TOL_F32
+    assert np.max(np.abs(got - want) / (want + want.max(axis=1, keepdims=True))) <= tol
+    assert np.all(got[want == 0] == 0)
+    yv.fill_(-7.0)
+    assert bool((ybuf == -7.0).all())
