@@ -4,6 +4,7 @@ CPU oracle used by the tests (gcc, through oracle/Makefile).
 
 Everything is built in-tree so that the shared objects travel with the source tree:
     anygpu_amd/lib/libanygpu_hip.so     kernels + C ABI (include/anygpu_hip.h)
+    anygpu_amd/lib/_torch_calls.so      the native callers behind ops.py (extension module)
     anygpu_amd/lib/anygpu_host_tests    reference-style C++ test harness over Tensor<dtype, device>
     oracle/liboracle.so                 CPU oracle (test infrastructure)
 """
@@ -107,6 +108,23 @@ def build_host_harness(verbose: bool = False) -> Path | None:
     return out
 
 
+def build_torch_calls(verbose: bool = False) -> Path:
+    """Compile the extension module that ops.py calls through (host C++ against torch's headers)."""
+    import sysconfig
+
+    import torch
+    torch_dir = Path(torch.__file__).resolve().parent
+    out = LIB_DIR / "_torch_calls.so"
+    clangxx = ROCM_DIR / "lib" / "llvm" / "bin" / "clang++"
+    _run([str(clangxx), "-std=c++20", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          f"-I{INCLUDE_DIR}", f"-isystem{torch_dir / 'include'}", f"-isystem{torch_dir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+          f"-isystem{ROCM_DIR / 'include'}", f"-isystem{sysconfig.get_paths()['include']}", "-Wall",
+          str(CSRC_DIR / "torch_calls.cpp"), "-o", str(out), f"-L{LIB_DIR}", "-lanygpu_hip", f"-L{torch_dir / 'lib'}", "-lc10", "-lc10_hip",
+          "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"], quiet=not verbose)
+    return out
+
+
 def build_oracle(verbose: bool = False) -> Path:
     """Build the CPU oracle (tests only)."""
     _run(["make", "-C", str(ORACLE_DIR), "-B"], quiet=not verbose)
@@ -114,7 +132,7 @@ def build_oracle(verbose: bool = False) -> Path:
 
 
 def build_all(verbose: bool = False) -> dict[str, str]:
-    built = {"kernels": str(build_kernels(verbose))}
+    built = {"kernels": str(build_kernels(verbose)), "torch_calls": str(build_torch_calls(verbose))}
     harness = build_host_harness(verbose)
     if harness is not None:
         built["host_harness"] = str(harness)

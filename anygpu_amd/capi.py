@@ -10,6 +10,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libanygpu_hip.so"
+TORCH_CALLS_PATH = LIB_PATH.with_name("_torch_calls.so")
 
 ANYGPU_OK = 0
 ANYGPU_ERR_NULL_POINTER = -1
@@ -141,3 +142,16 @@ def error_string(code: int) -> str:
 def check(fn: str, code: int) -> None:
     if code != ANYGPU_OK:
         raise AnyGpuError(fn, code, error_string(code))
+
+
+def load_torch_calls():
+    """The extension module behind ops.py (csrc/torch_calls.cpp).  Raises if it is not built."""
+    load()
+    if not TORCH_CALLS_PATH.exists():
+        raise RuntimeError(f"{TORCH_CALLS_PATH} is not built; run `python anygpu_amd/build.py` first.")
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("_torch_calls", TORCH_CALLS_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.set_check(check)
+    return module

@@ -12,6 +12,17 @@ import torch
 
 from . import capi
 
+_native = None
+
+
+def _calls():
+    """The native callers (csrc/torch_calls.cpp).  Each returns None for anything but plain dense device tensors that fit: the Python below
+    it then checks in full, and raises or makes the call itself."""
+    global _native
+    if _native is None:
+        _native = capi.load_torch_calls()
+    return _native
+
 
 # handle of a device's current stream, and the current device: what torch.cuda.current_stream().cuda_stream comes down to, without
 # the Stream object around it (2.7 us a call, a quarter of what a small call costs the host; 0.15 us this way)
@@ -59,6 +70,9 @@ def tensor_mm(lhs: torch.Tensor, rhs: torch.Tensor, out: torch.Tensor | None = N
     stride(1) == 1); with A_COL_MAJOR (float32 only) lhs is the [K, M] storage of A.
     With b_layout == B_ROW_MAJOR rhs is [K, N]; with B_COL_MAJOR rhs is the [N, K] storage of B.
     float16 (fp32 accumulate) and float32 are supported."""
+    got = (_native or _calls()).mm(lhs, rhs, out, b_layout, a_layout)
+    if got is not None:
+        return got if out is None else out
     _check_device(lhs, rhs)
     _require(lhs.dim() == 2 and rhs.dim() == 2, "matrix multiplication requires compatible matrices")
     _require(lhs.dtype == rhs.dtype, "operands must share a dtype")
@@ -94,6 +108,9 @@ def tensor_mm(lhs: torch.Tensor, rhs: torch.Tensor, out: torch.Tensor | None = N
 def tensor_gemm(xt: torch.Tensor, wt: torch.Tensor, bt: torch.Tensor,
                 b_layout: int = capi.B_ROW_MAJOR) -> torch.Tensor:
     """xt @ wt + bt (bias per output column), float32 or float16 (fp32 sums, bias added before the rounding)."""
+    got = (_native or _calls()).gemm(xt, wt, bt, b_layout)
+    if got is not None:
+        return got
     _check_device(xt, wt, bt)
     _require(xt.dim() == 2 and wt.dim() == 2, "matrix multiplication requires compatible matrices")
     _require(xt.dtype in (torch.float32, torch.float16) and wt.dtype == xt.dtype and bt.dtype == xt.dtype,
@@ -122,6 +139,9 @@ def tensor_gemma_linear_softcap(xt: torch.Tensor, wt: torch.Tensor, final_softca
 
     Same contract as tensor_gemma_linear_softcap of the reference (srcs/models/gemma2/gemma_linsoftcap.hpp:12-41).
     """
+    got = (_native or _calls()).linear_softcap(xt, wt, final_softcapping)
+    if got is not None:
+        return got
     _check_device(xt, wt)
     _require(xt.dim() == 3, "xt should be 3 dim")
     _require(wt.dim() == 2 and xt.shape[2] == wt.shape[1], "hidden size should match for xt and wt")
@@ -149,6 +169,9 @@ def mlp_gemma2_fused_upproj(xt: torch.Tensor, wt_gp: torch.Tensor, wt_up: torch.
 
     Same contract as cu_mlp_gemma2_fused_upproj_f32_v1 / _v2 (srcs/kernels/cuda/mlp_gemma2_fused_upproj.cuh:6-16).
     """
+    got = (_native or _calls()).upproj(xt, wt_gp, wt_up, b_layout)
+    if got is not None:
+        return got
     _check_device(xt, wt_gp, wt_up)
     _require(wt_gp.dim() == 2 and tuple(wt_gp.shape) == tuple(wt_up.shape), "gate and up weights must agree")
     k, n = wt_gp.shape if b_layout == capi.B_ROW_MAJOR else (wt_gp.shape[1], wt_gp.shape[0])
@@ -167,6 +190,9 @@ def mlp_gemma2_fused_upproj(xt: torch.Tensor, wt_gp: torch.Tensor, wt_up: torch.
 def tensor_softmax(x: torch.Tensor, out: torch.Tensor | None = None, *, alpha: float = 1.0, softcap: float = 0.0,
                    causal: bool = False, window: int = 0, q_len: int = 0, diag: int = 0) -> torch.Tensor:
     """Row softmax of a 2-D tensor with the fused prologue (scale -> softcap -> masks)."""
+    got = (_native or _calls()).softmax(x, out, alpha, softcap, causal, window, q_len, diag)
+    if got is not None:
+        return got if out is None else out
     _check_device(x)
     _require(x.dim() == 2, "softmax expects 2 dimensional tensors")
     _require(x.stride(1) == 1 or x.shape[1] <= 1, "rows must be contiguous")
@@ -192,6 +218,9 @@ def tensor_softmax(x: torch.Tensor, out: torch.Tensor | None = None, *, alpha: f
 def tensor_causal_conv1d(xt: torch.Tensor, wt: torch.Tensor, bt: torch.Tensor,
                          out: torch.Tensor | None = None) -> torch.Tensor:
     """silu(depthwise causal conv1d(xt, wt) + bt); xt [batch, dims, seq_len], wt [dims, width], bt [dims]."""
+    got = (_native or _calls()).conv1d(xt, wt, bt, out)
+    if got is not None:
+        return got
     _check_device(xt, wt, bt)
     _require(xt.dim() == 3, "xt needs to be 3 dimensional")
     _require(xt.shape[1] == wt.shape[0], "xt and wt need to have the same dims")
@@ -217,6 +246,9 @@ def tensor_causal_conv1d(xt: torch.Tensor, wt: torch.Tensor, bt: torch.Tensor,
 def tensor_causal_conv1d_update(xt: torch.Tensor, state: torch.Tensor, wt: torch.Tensor, bt: torch.Tensor) -> torch.Tensor:
     """One decode step of tensor_causal_conv1d: xt [batch, dims] is the new sample of every row, state
     [batch, dims, width - 1] holds the samples in front of it (oldest first) and is updated in place."""
+    got = (_native or _calls()).conv1d_update(xt, state, wt, bt)
+    if got is not None:
+        return got
     _check_device(xt, state, wt, bt)
     _require(xt.dim() == 2 and state.dim() == 3, "xt needs to be 2 and state 3 dimensional")
     _require(xt.shape[1] == wt.shape[0], "xt and wt need to have the same dims")
@@ -242,6 +274,9 @@ def tensor_causal_conv1d_update(xt: torch.Tensor, state: torch.Tensor, wt: torch
 def tensor_rms_norm(xt: torch.Tensor, wt: torch.Tensor, eps: float, zero_centered: bool = False,
                     gate: torch.Tensor | None = None) -> torch.Tensor:
     """rms_norm(xt * silu(gate)) * (wt + zero_centered) over the last axis; gate None: plain RMS norm."""
+    got = (_native or _calls()).rms_norm(xt, wt, eps, zero_centered, gate)
+    if got is not None:
+        return got
     _check_device(xt, wt) if gate is None else _check_device(xt, wt, gate)
     _require(wt.dim() == 1 and xt.dim() >= 1 and xt.shape[-1] == wt.shape[0], "wt shape is incorrect")
     _require(gate is None or tuple(gate.shape) == tuple(xt.shape), "tensors are not elementwise compatible")
@@ -322,6 +357,9 @@ def sdp_attention_masked_scaled_fwd(qw: torch.Tensor, kw: torch.Tensor, vw: torc
                                     alpha: float) -> torch.Tensor:
     """softmax(alpha q k^T + mask) v over [..., n, d] tensors (reference: srcs/transformers/sdp.hpp:207-274):
     one batched GEMM for q k^T (k in its own storage), one fused softmax, one batched GEMM for p v."""
+    got = (_native or _calls()).attention_masked(qw, kw, vw, mask, alpha)
+    if got is not None:
+        return got
     _require(qw.dim() == kw.dim() == vw.dim() == mask.dim() and qw.dim() >= 2, "dimension missmatch")
     n_q, d = qw.shape[-2:]
     n_k, d_v = kw.shape[-2], vw.shape[-1]
@@ -350,6 +388,9 @@ def sdp_attention_fwd(qw: torch.Tensor, kw: torch.Tensor, vw: torch.Tensor, alph
     """softmax(mask(softcap(alpha q k^T))) v in one kernel; q [..., heads, n_q, d], k and v [..., kv_heads, n_k, d]
     with heads a multiple of kv_heads, float16 or float32; masks are index rules with the causal diagonal at
     n_k - n_q.  decode: True / False forces the split-key decode form or the fused form, None picks by shape."""
+    got = (_native or _calls()).attention(qw, kw, vw, alpha, softcap, causal, window, decode)
+    if got is not None:
+        return got
     _check_device(qw, kw, vw)
     _require(qw.dim() == kw.dim() == vw.dim() and qw.dim() >= 3, "dimension missmatch")
     _require(qw.dtype == kw.dtype == vw.dtype and qw.dtype in (torch.float16, torch.float32), "Unsupported data types")
