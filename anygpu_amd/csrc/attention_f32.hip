@@ -20,12 +20,23 @@
 // At 32 cycles per MFMA the matrix pipe is the bound by a wide margin (the softmax arithmetic of a tile is
 // about 2 % of its MFMA time); the K and V tiles of the next step are in flight meanwhile.
 //
+// Most launches take a second form (attend_f32_split, attend_f32_split16; the rule: attention_split_wanted).  The fp32 instruction has a
+// sixteenth of the bf16 one's rate, and a float is the sum of three bf16 exactly, so a product of floats is six bf16 products whose missing
+// terms lie below 2^-23 of it: 6 / 16 of the matrix time, summed in fp32 as before, in fewer roundings.  Error against float64 (2-norm), fp32
+// instruction / bf16 parts, q, k, v of N(0, 1): 16 heads x 1000 x 128 3.8e-7 / 2.8e-7, 16 / 4 x 1000 x 64 5.0e-7 / 3.5e-7, 8 / 4 x 1500 x 256 under softcap
+// and window 2.10e-6 / 2.08e-6, 8 x 1000 x 256 with q of four times the scale 1.46e-6 / 1.17e-6, a bias mask 8 x 2100 x 256 7.3e-7 / 6.6e-7.
+// K and V are cut into their parts on their way into LDS (three planes each, once per block), p in its registers.  Bound: the bf16 matrix rate (and
+// the power that goes with it).  us, before / now: 8 / 4 heads x 8192 x 256, softcap, window 4096 1801 / 1051 (196 TFLOP/s, so 1.18 PFLOP/s of bf16
+// products), 16 x 2000 x 128 324 / 185, 32 / 8 x 3000 x 128 causal 701 / 419, 32 x 2000 x 64 causal 180 / 122, 8 x 1000 x 256 79.6 / 59.1; with a mask tensor
+// 8 x 3001 x 256 causal 412 / 264, dense bias 738 / 420, 64 x 1393 x 128 causal 564 / 240.
+//
 // Masks are index rules (causal with the diagonal at n_k - n_q, sliding window); tiles without a visible key
 // are skipped.  A query without any visible key gets zeros.
 #include "device_utils.hpp"
 #include "attention_walk.hpp"
 #include "attention_split.hpp"
 #include "attention_tile_map.hpp"
+#include "attention_balance.hpp"
 #include "gemm_band.hpp"
 #include "launch.hpp"
 
@@ -95,16 +106,29 @@ __device__ __forceinline__ void wait_vmem_all()
 // of a key block are consecutive in memory; they are requested in front of the tile's first product and added behind
 // scale and softcap.  A tile that the mask hides from every query of a wave costs the wave no products; a tile that the
 // visible-tile map of the mask (attention_tile_map.hpp) has not set for the block is neither loaded nor waited for.
+// x summed over the four groups of 16 lanes, in all of them (max_over_lane_rows has the manner)
+__device__ __forceinline__ float sum_over_lane_rows(float x)
+{
+	float a = x, b = x;
+	asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+	const float sum = a + b;
+	a = sum;
+	b = sum;
+	asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+	return a + b;
+}
+
+// One query block over the tiles [t_first, t_last] (MASK: the set ones of map_row, if there is a map).  partial: NULL, or where the block's
+// [query][D accumulators, maximum, sum] go instead of y.
 template <int D, bool SOFTCAP, int WAVES, int KT, bool DIRECT, bool MASK>
-__global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const AttnArgsF32 a, const AttnWalk walk)
+__device__ __forceinline__ void attend_f32(const AttnArgsF32& a, float* const lds_base, int bh, int q_block, int t_first, int t_last,
+                                           const unsigned long long* __restrict__ map_row, float* partial)
 {
 	constexpr int kKeysPerTile = KT;
 	static_assert(!DIRECT || D == 256, "one load instruction per tile row");
 	constexpr int kQueriesPerBlock = 16 * WAVES;
 	constexpr int THREADS = 64 * WAVES;
-	extern __shared__ __align__(16) char lds_raw[];
 	using L = AttnLdsF32<D, KT>;
-	float* const lds_base = reinterpret_cast<float*>(lds_raw);
 	typedef __attribute__((address_space(3))) void lds_void;
 	typedef const __attribute__((address_space(1))) void global_void;
 	constexpr int KS = D / 16;                      // 16-element groups of the head dimension (q k^T: 4 MFMAs each)
@@ -114,45 +138,18 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const
 	constexpr int VPT = kKeysPerTile * VPR / THREADS;   // vectors per thread per tile and matrix
 	static_assert(kKeysPerTile * VPR % THREADS == 0, "the tile divides over the threads");
 
-	const int tid = threadIdx.x;
+	int tid = threadIdx.x;
+	asm volatile("" : "+v"(tid));                   // (a caller's loop keeps nothing of a lane's addresses in registers)
+	__builtin_assume(tid >= 0 && tid < 512);
 	const int lane = tid & (kWaveSize - 1);
 	const int wave = tid >> 6;
 	const int n = lane & 15;                        // query inside the wave's block (second MFMA operand index)
 	const int g = lane >> 4;                        // lane group: summation slot g of an MFMA
-	int bh, q_block, part, parts, split_slot;
-	if (!attn_walk_locate_part(walk, blockIdx.x, bh, q_block, part, parts, split_slot)) return;       // the whole block
 	const int q0 = q_block * kQueriesPerBlock;
 	const float* qp = a.q + (int64_t)bh * a.n_q * D;
 	const float* kp = a.k + (int64_t)(bh / a.q_per_kv) * a.n_k * D;
 	const float* vp = a.v + (int64_t)(bh / a.q_per_kv) * a.n_k * D;
 	float* yp = a.y + (int64_t)bh * a.n_q * D;
-
-	// visible key range of the whole block: from the first key of its first query to the last of its last
-	const int q_last = (q0 + kQueriesPerBlock - 1 < a.n_q ? q0 + kQueriesPerBlock - 1 : a.n_q - 1);
-	int key_hi = a.n_k - 1;
-	if (a.causal && q_last + a.diag < key_hi) key_hi = q_last + a.diag;
-	int key_lo = 0;
-	if (a.window > 0 && q0 + a.diag - a.window + 1 > 0) key_lo = q0 + a.diag - a.window + 1;
-	int t_first = key_lo / kKeysPerTile;
-	int t_last = key_hi >= 0 ? key_hi / kKeysPerTile : -1;
-	// MASK: the visible-tile map of the mask, where the launcher has made one: the words of this query block
-	const unsigned long long* map_row = nullptr;
-	if constexpr (MASK)
-	{
-		if (a.tile_map != nullptr) map_row = a.tile_map + (int64_t)q_block * a.map_words;
-	}
-	if (parts > 1)
-	{
-		// one part of the block's key tiles; the other parts are other blocks', a merge kernel combines them.  With a
-		// map the parts divide the VISIBLE tiles among them, else the range
-		if (MASK && map_row != nullptr) attention_visible_share(map_row, part, parts, t_first, t_last);
-		else
-		{
-			const int per = (t_last - t_first + parts) / parts;
-			t_first += part * per;
-			if (t_first + per - 1 < t_last) t_last = t_first + per - 1;
-		}
-	}
 
 	// this lane's query as second operand: q[row][16 s + 4 g .. + 3]
 	const int q_row = q0 + 16 * wave + n;
@@ -416,15 +413,13 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const
 	}
 
 	// ---- normalise and store: register r of accumulator (c, e) is y[row][64 c + 4 (4 g + r) + e] ----
-	float l = l_run;
-	l += __shfl_xor(l, 16);
-	l += __shfl_xor(l, 32);
-	if (parts > 1)
+	const float l = sum_over_lane_rows(l_run);
+	if (partial != nullptr)
 	{
-		// unnormalised accumulators, running maximum and sum of this half of the keys
+		// unnormalised accumulators, running maximum and sum of this part of the keys
 		if (q_row < a.n_q)
 		{
-			float* dst = a.partials + ((((int64_t)bh * walk.n_split + split_slot) * parts + part) * kQueriesPerBlock + (q_row - q0)) * (D + 2);
+			float* dst = partial + (int64_t)(q_row - q0) * (D + 2);
 #pragma unroll
 			for (int c = 0; c < DC; ++c)
 #pragma unroll
@@ -452,93 +447,791 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const
 	}
 }
 
-template <int D, bool SOFTCAP, bool MASK>
-hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, hipStream_t stream)
+// Which head and query block this block works on, the key tiles of it, and where a partial result goes (NULL: y).  False: a padding block.
+template <int D, int QUERIES, int KT, bool MASK>
+__device__ __forceinline__ bool attention_block_f32(const AttnArgsF32& a, const AttnWalk& walk, int& bh, int& q_block, int& t_first, int& t_last,
+                                                    const unsigned long long*& map_row, float*& partial)
 {
-	// head dimension 256: 8 waves (two per SIMD) on tiles of 32 keys in two stages, 130 KB, one block per CU.  Two
-	// alternatives with two blocks of 4 waves per CU, for a better balance of long and short blocks under the causal
-	// rule, measured 5 - 12 % slower: tiles of 16 keys, and one K and one V buffer refilled in turn.
-	constexpr bool DIRECT = (D == 256);
-	constexpr int WAVES = DIRECT ? 8 : 4;
-	constexpr int KT = DIRECT ? 32 : 64;
-	auto kernel = sdp_attention_fwd_f32_kernel<D, SOFTCAP, WAVES, KT, DIRECT, MASK>;
-	constexpr int kLdsBytes = AttnLdsF32<D, KT>::kStageFloats * 4 * (DIRECT ? 2 : 1);
-	constexpr int kQueriesPerBlock = 16 * WAVES;
-	(void)hipGetLastError();
-	if (kLdsBytes > 64 * 1024)
-	{
-		// more than 64 KB of dynamic LDS has to be granted per function and per device, once
-		static std::atomic<uint64_t> configured_devices{0};
-		int device = 0;
-		hipError_t e = hipGetDevice(&device);
-		if (e != hipSuccess) return e;
-		const uint64_t bit = 1ull << (device & 63);
-		if ((configured_devices.load(std::memory_order_relaxed) & bit) == 0)
-		{
-			e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-			if (e != hipSuccess) return e;
-			configured_devices.fetch_or(bit, std::memory_order_relaxed);
-		}
-	}
-	AttnArgsF32 args = args_in;
-	const int64_t q_blocks = (args.n_q + kQueriesPerBlock - 1) / kQueriesPerBlock;
-	args.tile_map = nullptr;
-	args.map_words = 0;
-	std::optional<band::WorkspaceReserve> map_hold;
-	int64_t mask_parts = 0;
+	int part, parts, split_slot;
+	if (!attn_walk_locate_part(walk, blockIdx.x, bh, q_block, part, parts, split_slot)) return false;
+	const int q0 = q_block * QUERIES;
+	// visible key range of the whole block: from the first key of its first query to the last of its last
+	const int q_last = (q0 + QUERIES - 1 < a.n_q ? q0 + QUERIES - 1 : a.n_q - 1);
+	int key_hi = a.n_k - 1;
+	if (a.causal && q_last + a.diag < key_hi) key_hi = q_last + a.diag;
+	int key_lo = 0;
+	if (a.window > 0 && q0 + a.diag - a.window + 1 > 0) key_lo = q0 + a.diag - a.window + 1;
+	t_first = key_lo / KT;
+	t_last = key_hi >= 0 ? key_hi / KT : -1;
+	// MASK: the visible-tile map of the mask, where the launcher has made one: the words of this query block
+	map_row = nullptr;
 	if constexpr (MASK)
 	{
-		// The visible-tile map of the mask, at the front of the stream's workspace (the partial results of a split key
-		// range go behind it): worth its pass over the mask for large masks and long key ranges
-		// (attention_mask_map_wanted), and left out where the stream has no workspace to offer (a capture without a
-		// caller's workspace).  For whole query blocks the results are the same bit for bit: the map only saves the loads
-		// and barriers of tiles that every wave of a block would skip.
-		const int64_t words = attention_tile_map_words(args.n_k, KT);
-		const size_t map_bytes = (size_t)(q_blocks * words) * sizeof(unsigned long long);
-		// With as many blocks as one to four rounds of the chip the rounds do not even out where the mask leaves the
-		// blocks unequal shares of their key range (a sliding window: the late query blocks carry the full window, the
-		// early ones little): every block then goes out in two parts, each with half of its VISIBLE tiles.  Their
-		// partial results may take more than the library's own workspace holds to begin with; it grows for them as
-		// it does for operand copies (eager launches only), before anything points into it.
-		const int64_t blocks = q_blocks * batch_heads;
-		const int cus = device_cu_count();
-		// With fewer blocks than CUs but more than half as many, the parts are chosen to fill whole rounds, and the growing
-		// workspace is what lets them: 8 heads x 3001 x 256 are 192 blocks, which the first 64 MB hold in two parts only (384
-		// blocks, one and a half rounds, the first of the causal ones walking 47 of the 36 tiles that a CU averages); four
-		// parts are three whole rounds (us, causal mask 449 -> 422, window of 1024 333 -> 295, no key hidden 899 -> 729; 16 heads x
-		// 1500 x 3000 x 256, likewise 192 blocks: 670 -> 580, 904 -> 722).
-		int64_t want_parts = 0;
-		const int64_t tiles = (args.n_k + KT - 1) / KT;
-		if (blocks >= cus && blocks < 4 * (int64_t)cus && tiles >= 32) want_parts = 2;
-		else if (DIRECT && blocks < cus && 2 * blocks > cus)
+		if (a.tile_map != nullptr) map_row = a.tile_map + (int64_t)q_block * a.map_words;
+	}
+	partial = nullptr;
+	if (parts > 1)
+	{
+		// one part of the block's key tiles; the other parts are other blocks', a merge kernel combines them.  With a
+		// map the parts divide the VISIBLE tiles among them, else the range
+		if (MASK && map_row != nullptr) attention_visible_share(map_row, part, parts, t_first, t_last);
+		else
 		{
-			const auto filled = [&](int64_t s) { return (double)(blocks * s) / (double)((blocks * s + cus - 1) / cus * cus); };
-			for (int64_t s = 2; s <= 6 && tiles / s >= 16; ++s)
-				if (want_parts == 0 || filled(s) > 1.1 * filled(want_parts)) want_parts = s;
+			const int per = (t_last - t_first + parts) / parts;
+			t_first += part * per;
+			if (t_first + per - 1 < t_last) t_last = t_first + per - 1;
 		}
-		size_t parts_bytes = (size_t)want_parts * blocks * kQueriesPerBlock * (D + 2) * sizeof(float);
-		const size_t map_room = (map_bytes + 255) / 256 * 256 + (1u << 16);
-		if (parts_bytes > 0 && band::workspace_copy_capacity(stream) < map_room + parts_bytes) parts_bytes = 0;
-		if (attention_mask_map_wanted(args.n_q, args.n_k) && (parts_bytes > 0 || band::workspace_capacity(stream) >= map_room))
+		partial = a.partials + (((int64_t)bh * walk.n_split + split_slot) * parts + part) * ((int64_t)QUERIES * (D + 2));
+	}
+	return true;
+}
+
+// The launch of the form above: every block finds its query block and the tiles of it.
+template <int D, bool SOFTCAP, int WAVES, int KT, bool DIRECT, bool MASK>
+__global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f32_kernel(const AttnArgsF32 a, const AttnWalk walk)
+{
+	extern __shared__ __align__(16) char lds_raw[];
+	int bh, q_block, t_first, t_last;
+	const unsigned long long* map_row;
+	float* partial;
+	if (!attention_block_f32<D, 16 * WAVES, KT, MASK>(a, walk, bh, q_block, t_first, t_last, map_row, partial)) return;
+	attend_f32<D, SOFTCAP, WAVES, KT, DIRECT, MASK>(a, reinterpret_cast<float*>(lds_raw), bh, q_block, t_first, t_last, map_row, partial);
+}
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
+typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
+typedef short short4_t __attribute__((ext_vector_type(4)));
+
+// A float as the sum of three bf16 (8 bits each, cut off, which together are all of its 24 bits): the first is the upper half of the
+// float's bits, the others are those of what is left.  (What is left below 2^-133, the smallest bf16, is lost: of floats below 2^-110.)
+__device__ __forceinline__ void split_bits(float x, unsigned& b1, unsigned& b2, unsigned& b3)
+{
+	b1 = __builtin_bit_cast(unsigned, x);
+	const float r1 = x - __builtin_bit_cast(float, b1 & 0xFFFF0000u);
+	b2 = __builtin_bit_cast(unsigned, r1);
+	const float r2 = r1 - __builtin_bit_cast(float, b2 & 0xFFFF0000u);
+	b3 = __builtin_bit_cast(unsigned, r2);
+}
+// the upper halves of two words, the first below
+__device__ __forceinline__ unsigned upper_halves(unsigned lo, unsigned hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
+
+constexpr int kSplitQueries = 128, kSplitKeys = 32;
+constexpr int64_t kSplitMaskStride = 1 << 22;   // mask rows at most this far apart: byte offsets in a query block fit 32 bits
+// The form with 16 queries per wave, eight waves (the other: 32, four): where 32 leave no registers.
+constexpr bool split_narrow(int head_dim, bool mask) { return head_dim == 256 || (head_dim == 128 && mask); }
+constexpr int split_threads(int head_dim, bool mask) { return split_narrow(head_dim, mask) ? 512 : 256; }
+
+template <int D, bool NARROW>
+struct AttnLdsSplit
+{
+	// bytes of a row of a plane: both read patterns without bank conflicts (the lane groups that read V together are four keys apart
+	// in the narrow form, else sixteen columns)
+	static constexpr int kPitchK = 2 * D + 32, kPitchV = NARROW ? 2 * D + 32 : 2 * D + 64;
+	static constexpr int kPlaneK = kSplitKeys * kPitchK, kPlaneV = kSplitKeys * kPitchV;
+	static constexpr int kBytes = 3 * (kPlaneK + kPlaneV);
+};
+
+// Whether any thread of the block says so.  (Smaller than __syncthreads_or, whose lane numbers the compiler kept in registers through the
+// key loop.)  The LDS may be in use before, and is free again behind the caller's next barrier.
+template <int WAVES>
+__device__ __forceinline__ bool any_of_block(bool said, char* const lds, int wave)
+{
+	int* const flags = reinterpret_cast<int*>(lds);
+	const int of_wave = __builtin_amdgcn_ballot_w64(said) != 0;
+	__syncthreads();
+	flags[wave] = of_wave;
+	__syncthreads();
+	int any = 0;
+#pragma unroll
+	for (int i = 0; i < WAVES; ++i) any |= flags[i];
+	return __builtin_amdgcn_readfirstlane(any) != 0;
+}
+
+// A query block of 128 with every product of floats as six products of bf16 parts on v_mfma_f32_32x32x16_bf16, accumulated in fp32:
+// x y = x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1; the terms left out are below 2^-23 of x y.
+// False, with nothing stored, where a result is not finite (the parts of an infinity are no numbers): the caller takes the form above.
+template <int D, bool SOFTCAP, bool MASK>
+__device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* const lds, int bh, int q_block, int t_first, int t_last,
+                                                 const unsigned long long* __restrict__ map_row, float* partial)
+{
+	constexpr int KT = kSplitKeys, THREADS = 256;
+	using L = AttnLdsSplit<D, false>;
+	constexpr int KS = D / 16;                      // MFMA steps along the head dimension
+	constexpr int DC = D / 32;                      // 32-wide column blocks of the output
+	constexpr int VPR = D / 4;                      // float4 per row
+	constexpr int VPT = KT * VPR / THREADS;         // float4 per thread and tile
+
+	int tid = threadIdx.x;
+	asm volatile("" : "+v"(tid));                   // (a caller's loop keeps nothing of a lane's addresses in registers)
+	__builtin_assume(tid >= 0 && tid < 512);
+	const int lane = tid & (kWaveSize - 1);
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int n = lane & 31;                        // query of the wave (second MFMA operand index)
+	const int h = lane >> 5;                        // lane half: k slots 8 h .. 8 h + 7 of an MFMA
+	const int q0 = q_block * kSplitQueries;
+	const float* qp = a.q + (int64_t)bh * a.n_q * D;
+	const float* kp = a.k + (int64_t)(bh / a.q_per_kv) * a.n_k * D;
+	const float* vp = a.v + (int64_t)(bh / a.q_per_kv) * a.n_k * D;
+	float* yp = a.y + (int64_t)bh * a.n_q * D;
+
+	// this lane's query as second operands: q[row][16 s + 8 h .. + 7] in three parts
+	const int wq0 = q0 + 32 * wave;
+	const int q_row = wq0 + n;
+	bf16x8_t qf[3][KS];
+#pragma unroll
+	for (int s = 0; s < KS; ++s)
+	{
+		float4_t x[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+		if (q_row < a.n_q)
 		{
-			float* front = nullptr;
-			hipError_t e = band::workspace_acquire(stream, &front, parts_bytes > 0 ? map_room + parts_bytes : 0);
-			if (e != hipSuccess) return e;
-			if (parts_bytes > 0) mask_parts = want_parts;
-			unsigned long long* map = reinterpret_cast<unsigned long long*>(front);
-			e = launch_attention_mask_tile_map(args.mask, args.mask_stride, args.n_q, args.n_k, kQueriesPerBlock, KT, map, stream);
-			if (e != hipSuccess) return e;
-			args.tile_map = map;
-			args.map_words = (int)words;
-			map_hold.emplace(map_bytes);
+			x[0] = *reinterpret_cast<const float4_t*>(qp + (int64_t)q_row * D + 16 * s + 8 * h);
+			x[1] = *reinterpret_cast<const float4_t*>(qp + (int64_t)q_row * D + 16 * s + 8 * h + 4);
+		}
+		uint4_t w[3];
+#pragma unroll
+		for (int e = 0; e < 8; e += 2)
+		{
+			unsigned lo[3], hi[3];
+			split_bits(x[e / 4][e % 4], lo[0], lo[1], lo[2]);
+			split_bits(x[e / 4][e % 4 + 1], hi[0], hi[1], hi[2]);
+#pragma unroll
+			for (int p = 0; p < 3; ++p) w[p][e / 2] = upper_halves(lo[p], hi[p]);
+		}
+#pragma unroll
+		for (int p = 0; p < 3; ++p) qf[p][s] = __builtin_bit_cast(bf16x8_t, w[p]);
+	}
+	// keys visible to every query of this wave need no per-element test: [all_lo, all_hi]
+	const int all_hi = a.causal ? (wq0 + a.diag < a.n_k - 1 ? wq0 + a.diag : a.n_k - 1) : a.n_k - 1;
+	const int all_lo = a.window > 0 ? wq0 + 31 + a.diag - a.window + 1 : 0;
+
+	float m_run = -INFINITY, l_run = 0.0f;          // l_run: this lane's share of the row sum
+	float16_t o[DC];
+#pragma unroll
+	for (int c = 0; c < DC; ++c)
+#pragma unroll
+		for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
+
+	// A tile goes through registers, where its floats are cut into their parts, into the planes: VPT pieces per thread.  Rows past the last
+	// key repeat it (their scores are masked, their p is 0).
+	float4_t staged[VPT];
+	auto fetch = [&](const float* src, int t) {
+		const char* base = reinterpret_cast<const char*>(src) + (int64_t)t * (KT * D * 4);
+		const int last = a.n_k - 1 - t * KT;        // KT - 1 and more: a whole tile
+#pragma unroll
+		for (int i = 0; i < VPT; ++i)
+		{
+			const int idx = tid + THREADS * i;
+			const int over = idx / VPR > last ? idx / VPR - last : 0;
+			staged[i] = *reinterpret_cast<const float4_t*>(base + (unsigned)(idx * 16 - over * (D * 4)));
+		}
+	};
+	auto put = [&](bool of_v, int i) {
+		const int idx = tid + THREADS * i;
+		const int pitch = of_v ? L::kPitchV : L::kPitchK, plane = of_v ? L::kPlaneV : L::kPlaneK;
+		char* const dst = lds + (of_v ? 3 * L::kPlaneK : 0) + (idx / VPR) * pitch + (idx % VPR) * 8;
+		unsigned b[4][3];
+#pragma unroll
+		for (int e = 0; e < 4; ++e) split_bits(staged[i][e], b[e][0], b[e][1], b[e][2]);
+#pragma unroll
+		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{upper_halves(b[0][p], b[1][p]), upper_halves(b[2][p], b[3][p])};
+	};
+
+	// MASK: the mask values of this lane's scores, keys 8 j + 4 h .. + 3 of the tile: four consecutive floats at any alignment, as they come.
+	// Keys past the end read nothing and count as hidden.
+	float4_t mk[MASK ? 4 : 1];
+	const char* const mask_block = MASK ? reinterpret_cast<const char*>(a.mask + q0 * a.mask_stride) : nullptr;
+	const unsigned mask_at = MASK ? (unsigned)((q_row < a.n_q ? q_row : a.n_q - 1) - q0) * (unsigned)(a.mask_stride * 4) + 16u * h : 0u;   // (32 bits: kSplitMaskStride)
+	auto load_mask = [&](int t) {
+		typedef float4_t LooseF4 __attribute__((aligned(4)));
+		const float* const at = reinterpret_cast<const float*>(mask_block + (int64_t)t * (KT * 4) + mask_at);
+		if ((t + 1) * KT <= a.n_k)
+		{
+#pragma unroll
+			for (int j = 0; j < (MASK ? 4 : 0); ++j) mk[j] = *reinterpret_cast<const LooseF4*>(at + 8 * j);
+			return;
+		}
+#pragma unroll
+		for (int j = 0; j < (MASK ? 4 : 0); ++j)
+#pragma unroll
+			for (int r = 0; r < 4; ++r)
+			{
+				const int key = t * KT + 8 * j + 4 * h + r;
+				mk[j][r] = key < a.n_k ? at[8 * j + r] : -INFINITY;
+			}
+	};
+	AttentionVisibleWalk visible{map_row};
+	if constexpr (MASK) t_first = visible.next(t_first, t_last);
+	if (t_first <= t_last)
+	{
+		fetch(kp, t_first);
+		if constexpr (MASK) load_mask(t_first);
+		__syncthreads();                            // (the query block before has been read by everybody)
+#pragma unroll
+		for (int i = 0; i < VPT; ++i) put(false, i);
+		fetch(vp, t_first);
+	}
+	// Each product is a sequence of steps: a fragment (of V: of two column blocks), the third, second and first part in turn, and its one, two
+	// or three products; a step's fragments are read some steps ahead, and the tile that the other product needs next is cut into the
+	// planes behind the steps of the second half, its loads having had the first.  Neighbouring MFMAs use different accumulators.
+	constexpr int kStepsQ = 3 * KS, kAheadQ = 4, kStepsV = 3 * DC, kAheadV = 2;
+	static_assert(DC % 2 == 0, "column blocks in pairs");
+	bf16x8_t frag[4];
+	auto read_k = [&](int f) {
+		const int st = f / 3, p = 2 - f % 3;
+		frag[f % kAheadQ] = *reinterpret_cast<const bf16x8_t*>(lds + p * L::kPlaneK + n * L::kPitchK + (16 * st + 8 * h) * 2);
+	};
+	// slot (h, j) of 16-key step u is key 16 u + 8 (j / 4) + 4 h + j % 4
+	auto read_v = [&](int f) {
+		const int pair = f / 3, p = 2 - f % 3, u = pair / (DC / 2), c = 2 * (pair % (DC / 2));
+		typedef __attribute__((address_space(3))) short4_t* LdsShort4;
+#pragma unroll
+		for (int i = 0; i < 2; ++i)
+		{
+			const char* src = lds + 3 * L::kPlaneK + p * L::kPlaneV + (16 * u + 4 * h + ((lane & 15) >> 2)) * L::kPitchV +
+			                  (32 * (c + i) + 16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+			const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsShort4)(src));
+			const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsShort4)(src + 8 * L::kPitchV));
+			frag[2 * (f % kAheadV) + i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+		}
+	};
+	// piece of the staged tile that goes behind step f of `steps`, or -1
+	auto piece_at = [](int f, int steps) {
+		const int half = steps / 2, every = half / VPT;
+		return f >= half && (f - half) % every == 0 && (f - half) / every < VPT ? (f - half) / every : -1;
+	};
+	static_assert(kStepsQ / 2 >= VPT && kStepsV / 2 >= VPT, "steps for the pieces");
+	int t_next = 0;
+	for (int t = t_first; t <= t_last; t = t_next)
+	{
+		if constexpr (MASK) t_next = visible.next(t + 1, t_last);
+		else t_next = t + 1;
+		__syncthreads();                            // K(t) is complete, V of the tile before has been read by everybody
+		// ---- S^T = K Q^T ----
+		float16_t s;
+#pragma unroll
+		for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+		for (int f = 0; f < kAheadQ; ++f) read_k(f);
+		__builtin_amdgcn_sched_barrier(0);
+		__builtin_amdgcn_s_setprio(1);              // (the SIMD's other block has its softmax in between: 1 - 4 %)
+#pragma unroll
+		for (int f = 0; f < kStepsQ; ++f)
+		{
+#pragma unroll
+			for (int x = f % 3; x >= 0; --x) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[f % kAheadQ], qf[x][f / 3], s, 0, 0, 0);
+			if (f + kAheadQ < kStepsQ) read_k(f + kAheadQ);
+			if (piece_at(f, kStepsQ) >= 0) put(true, piece_at(f, kStepsQ));
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		__builtin_amdgcn_s_setprio(0);
+		// ---- online softmax: score i of this lane is key 8 (i / 4) + 4 h + i % 4 ----
+		const int tile_key0 = t * KT;
+		const bool interior = tile_key0 >= all_lo && tile_key0 + KT - 1 <= all_hi;   // wave-uniform
+#pragma unroll
+		for (int i = 0; i < 16; ++i)
+		{
+			s[i] = logit2<SOFTCAP>(s[i], a.k_in, a.k_cap);
+			if constexpr (MASK) s[i] += mk[MASK ? i / 4 : 0][i % 4] * kLog2e;
+		}
+		if (!MASK && !interior)                     // (a mask's values past the last key hide them)
+		{
+			int row = n;
+			asm volatile("" : "+v"(row));           // (found anew at each such tile: two registers)
+			row += wq0;
+			const int vis_hi = a.causal && row + a.diag < a.n_k - 1 ? row + a.diag : a.n_k - 1;
+			const int vis_lo = a.window > 0 ? row + a.diag - a.window + 1 : 0;
+#pragma unroll
+			for (int i = 0; i < 16; ++i)
+			{
+				const int key = tile_key0 + 8 * (i / 4) + 4 * h + i % 4;
+				s[i] = (key >= vis_lo && key <= vis_hi) ? s[i] : -INFINITY;
+			}
+		}
+		float mt = s[0];
+#pragma unroll
+		for (int i = 1; i < 16; ++i) mt = fmaxf(mt, s[i]);
+		mt = fmaxf(mt, __shfl_xor(mt, 32));
+		const float m_new = fmaxf(m_run, mt);
+		const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;   // nothing visible so far: every term is exp2(-inf) = 0
+		// the running maximum settles after a few tiles; when no query of the wave raised it, the
+		// rescale factor is 1 everywhere and the pass over the accumulators is skipped
+		if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0)
+		{
+			const float corr = fast_exp2(m_run - m_safe);
+			l_run *= corr;
+#pragma unroll
+			for (int c = 0; c < DC; ++c)
+#pragma unroll
+				for (int i = 0; i < 16; ++i) o[c][i] *= corr;
+		}
+		m_run = m_new;
+		float psum[2] = {0.0f, 0.0f};
+		bf16x8_t pf[3][2];
+#pragma unroll
+		for (int u = 0; u < 2; ++u)
+		{
+			uint4_t w[3];
+#pragma unroll
+			for (int j = 0; j < 8; j += 2)
+			{
+				const float p0 = fast_exp2(s[8 * u + j] - m_safe), p1 = fast_exp2(s[8 * u + j + 1] - m_safe);
+				psum[0] += p0;
+				psum[1] += p1;
+				unsigned lo[3], hi[3];
+				split_bits(p0, lo[0], lo[1], lo[2]);
+				split_bits(p1, hi[0], hi[1], hi[2]);
+#pragma unroll
+				for (int p = 0; p < 3; ++p) w[p][j / 2] = upper_halves(lo[p], hi[p]);
+			}
+#pragma unroll
+			for (int p = 0; p < 3; ++p) pf[p][u] = __builtin_bit_cast(bf16x8_t, w[p]);
+		}
+		l_run += psum[0] + psum[1];
+		// (behind the last tile: that tile once more, of no consequence)
+		const int t_load = t_next <= t_last ? t_next : t;
+		if constexpr (MASK) load_mask(t_load);
+		fetch(kp, t_load);
+		__syncthreads();                            // V(t) is complete, K(t) has been read by everybody
+		// ---- O^T += V^T P^T ----
+#pragma unroll
+		for (int f = 0; f < kAheadV; ++f) read_v(f);
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int f = 0; f < kStepsV; ++f)
+		{
+			const int pair = f / 3, u = pair / (DC / 2), c = 2 * (pair % (DC / 2));
+#pragma unroll
+			for (int x = f % 3; x >= 0; --x)
+#pragma unroll
+				for (int i = 0; i < 2; ++i) o[c + i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[2 * (f % kAheadV) + i], pf[x][u], o[c + i], 0, 0, 0);
+			if (f + kAheadV < kStepsV) read_v(f + kAheadV);
+			if (piece_at(f, kStepsV) >= 0) put(false, piece_at(f, kStepsV));
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		fetch(vp, t_load);
+	}
+
+	// ---- normalise and store: lane (n, h) holds y[row][32 c + 8 (i / 4) + 4 h + i % 4] ----
+	const float l = l_run + __shfl_xor(l_run, 32);
+	float all = l;                                  // not finite where anything that entered it is not
+#pragma unroll
+	for (int c = 0; c < DC; ++c)
+#pragma unroll
+		for (int i = 0; i < 16; ++i) all = fmaf(o[c][i], 0.0f, all);
+	if (any_of_block<THREADS / kWaveSize>(!(fabsf(all) < INFINITY), lds, wave)) return false;
+	if (q_row >= a.n_q) return true;
+	if (partial != nullptr)
+	{
+		// unnormalised accumulators, running maximum and sum of this part of the keys
+		float* dst = partial + (int64_t)(q_row - q0) * (D + 2);
+#pragma unroll
+		for (int c = 0; c < DC; ++c)
+#pragma unroll
+			for (int r = 0; r < 4; ++r)
+				*reinterpret_cast<WsFloat4*>(dst + 32 * c + 8 * r + 4 * h) = float4_t{o[c][4 * r], o[c][4 * r + 1], o[c][4 * r + 2], o[c][4 * r + 3]};
+		if (h == 0)
+		{
+			dst[D] = m_run;
+			dst[D + 1] = l;
+		}
+		return true;
+	}
+	const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+	for (int c = 0; c < DC; ++c)
+#pragma unroll
+		for (int r = 0; r < 4; ++r)
+			*reinterpret_cast<float4_t*>(yp + (int64_t)q_row * D + 32 * c + 8 * r + 4 * h) =
+				float4_t{o[c][4 * r] * inv, o[c][4 * r + 1] * inv, o[c][4 * r + 2] * inv, o[c][4 * r + 3] * inv};
+	return true;
+}
+
+// The same for head dimension 256, where a wave of 32 queries has no registers left: eight waves of 16 queries, v_mfma_f32_16x16x32_bf16.
+template <int D, bool SOFTCAP, bool MASK>
+__device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* const lds, int bh, int q_block, int t_first, int t_last,
+                                                 const unsigned long long* __restrict__ map_row, float* partial)
+{
+	constexpr int KT = kSplitKeys, THREADS = 512;
+	using L = AttnLdsSplit<D, true>;
+	constexpr int KS = D / 32;                      // MFMA steps along the head dimension
+	constexpr int DC = D / 16;                      // 16-wide column blocks of the output
+	constexpr int KB = KT / 16;                     // 16-key blocks per tile
+	constexpr int VPR = D / 4;                      // float4 per row
+	constexpr int VPT = KT * VPR / THREADS;         // float4 per thread and tile
+
+	int tid = threadIdx.x;
+	asm volatile("" : "+v"(tid));                   // (a caller's loop keeps nothing of a lane's addresses in registers)
+	__builtin_assume(tid >= 0 && tid < 512);
+	const int lane = tid & (kWaveSize - 1);
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int n = lane & 15;                        // query of the wave (second MFMA operand index)
+	const int g = lane >> 4;                        // lane group: k slots 8 g .. 8 g + 7 of an MFMA
+	const int q0 = q_block * kSplitQueries;
+	const float* qp = a.q + (int64_t)bh * a.n_q * D;
+	const float* kp = a.k + (int64_t)(bh / a.q_per_kv) * a.n_k * D;
+	const float* vp = a.v + (int64_t)(bh / a.q_per_kv) * a.n_k * D;
+	float* yp = a.y + (int64_t)bh * a.n_q * D;
+
+	// this lane's query as second operands: q[row][32 s + 8 g .. + 7] in three parts
+	const int wq0 = q0 + 16 * wave;
+	const int q_row = wq0 + n;
+	bf16x8_t qf[3][KS];
+#pragma unroll
+	for (int s = 0; s < KS; ++s)
+	{
+		float4_t x[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+		if (q_row < a.n_q)
+		{
+			x[0] = *reinterpret_cast<const float4_t*>(qp + (int64_t)q_row * D + 32 * s + 8 * g);
+			x[1] = *reinterpret_cast<const float4_t*>(qp + (int64_t)q_row * D + 32 * s + 8 * g + 4);
+		}
+		uint4_t w[3];
+#pragma unroll
+		for (int e = 0; e < 8; e += 2)
+		{
+			unsigned lo[3], hi[3];
+			split_bits(x[e / 4][e % 4], lo[0], lo[1], lo[2]);
+			split_bits(x[e / 4][e % 4 + 1], hi[0], hi[1], hi[2]);
+#pragma unroll
+			for (int p = 0; p < 3; ++p) w[p][e / 2] = upper_halves(lo[p], hi[p]);
+		}
+#pragma unroll
+		for (int p = 0; p < 3; ++p) qf[p][s] = __builtin_bit_cast(bf16x8_t, w[p]);
+	}
+	// keys visible to every query of this wave need no per-element test: [all_lo, all_hi]
+	const int all_hi = a.causal ? (wq0 + a.diag < a.n_k - 1 ? wq0 + a.diag : a.n_k - 1) : a.n_k - 1;
+	const int all_lo = a.window > 0 ? wq0 + 15 + a.diag - a.window + 1 : 0;
+
+	float m_run = -INFINITY, l_run = 0.0f;          // l_run: this lane's share of the row sum
+	float4_t o[DC];
+#pragma unroll
+	for (int c = 0; c < DC; ++c) o[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+	// A tile goes through registers, where its floats are cut into their parts, into the planes: VPT pieces per thread.  Rows past the last
+	// key repeat it (their scores are masked, their p is 0).
+	float4_t staged[VPT];
+	auto fetch = [&](const float* src, int t) {
+		const char* base = reinterpret_cast<const char*>(src) + (int64_t)t * (KT * D * 4);
+		const int last = a.n_k - 1 - t * KT;        // KT - 1 and more: a whole tile
+#pragma unroll
+		for (int i = 0; i < VPT; ++i)
+		{
+			const int idx = tid + THREADS * i;
+			const int over = idx / VPR > last ? idx / VPR - last : 0;
+			staged[i] = *reinterpret_cast<const float4_t*>(base + (unsigned)(idx * 16 - over * (D * 4)));
+		}
+	};
+	auto put = [&](bool of_v, int i) {
+		const int idx = tid + THREADS * i;
+		const int pitch = of_v ? L::kPitchV : L::kPitchK, plane = of_v ? L::kPlaneV : L::kPlaneK;
+		char* const dst = lds + (of_v ? 3 * L::kPlaneK : 0) + (idx / VPR) * pitch + (idx % VPR) * 8;
+		unsigned b[4][3];
+#pragma unroll
+		for (int e = 0; e < 4; ++e) split_bits(staged[i][e], b[e][0], b[e][1], b[e][2]);
+#pragma unroll
+		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{upper_halves(b[0][p], b[1][p]), upper_halves(b[2][p], b[3][p])};
+	};
+
+	// MASK: the mask values of this lane's scores, keys 16 j + 4 g .. + 3 of the tile: four consecutive floats at any alignment, as they come.
+	// Keys past the end read nothing and count as hidden.
+	float4_t mk[MASK ? KB : 1];
+	const char* const mask_block = MASK ? reinterpret_cast<const char*>(a.mask + q0 * a.mask_stride) : nullptr;
+	const unsigned mask_at = MASK ? (unsigned)((q_row < a.n_q ? q_row : a.n_q - 1) - q0) * (unsigned)(a.mask_stride * 4) + 16u * g : 0u;   // (32 bits: kSplitMaskStride)
+	auto load_mask = [&](int t) {
+		typedef float4_t LooseF4 __attribute__((aligned(4)));
+		const float* const at = reinterpret_cast<const float*>(mask_block + (int64_t)t * (KT * 4) + mask_at);
+		if ((t + 1) * KT <= a.n_k)
+		{
+#pragma unroll
+			for (int j = 0; j < (MASK ? KB : 0); ++j) mk[j] = *reinterpret_cast<const LooseF4*>(at + 16 * j);
+			return;
+		}
+#pragma unroll
+		for (int j = 0; j < (MASK ? KB : 0); ++j)
+#pragma unroll
+			for (int r = 0; r < 4; ++r)
+			{
+				const int key = t * KT + 16 * j + 4 * g + r;
+				mk[j][r] = key < a.n_k ? at[16 * j + r] : -INFINITY;
+			}
+	};
+	AttentionVisibleWalk visible{map_row};
+	if constexpr (MASK) t_first = visible.next(t_first, t_last);
+	if (t_first <= t_last)
+	{
+		fetch(kp, t_first);
+		__syncthreads();                            // (the query block before has been read by everybody)
+#pragma unroll
+		for (int i = 0; i < VPT; ++i) put(false, i);
+		fetch(vp, t_first);
+	}
+	// Each product is a sequence of steps: a fragment (of V: of two column blocks), the third, second and first part in turn, and its one, two
+	// or three products; a step's fragments are read some steps ahead, and the tile that the other product needs next is cut into the
+	// planes behind the steps of the second half, its loads having had the first.  Neighbouring MFMAs use different accumulators.
+	constexpr int kStepsQ = 3 * KS * KB, kAheadQ = 4, kStepsV = 3 * DC / 2, kAheadV = 2;
+	static_assert(DC % 2 == 0 && KB == 2, "column blocks in pairs; one 32-key step");
+	bf16x8_t frag[4];
+	auto read_k = [&](int f) {
+		const int u = f / 3, p = 2 - f % 3, st = u / KB, kb = u % KB;
+		frag[f % kAheadQ] = *reinterpret_cast<const bf16x8_t*>(lds + p * L::kPlaneK + (16 * kb + n) * L::kPitchK + (32 * st + 8 * g) * 2);
+	};
+	// slot (g, j) of the 32-key step is key 16 (j / 4) + 4 g + j % 4
+	auto read_v = [&](int f) {
+		const int c = 2 * (f / 3), p = 2 - f % 3;
+		typedef __attribute__((address_space(3))) short4_t* LdsShort4;
+#pragma unroll
+		for (int i = 0; i < 2; ++i)
+		{
+			const char* src = lds + 3 * L::kPlaneK + p * L::kPlaneV + (4 * g + (n >> 2)) * L::kPitchV + (16 * (c + i) + 4 * (n & 3)) * 2;
+			const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsShort4)(src));
+			const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsShort4)(src + 16 * L::kPitchV));
+			frag[2 * (f % kAheadV) + i] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+		}
+	};
+	// piece of the staged tile that goes behind step f of `steps`, or -1
+	auto piece_at = [](int f, int steps) {
+		const int half = steps / 2, every = half / VPT;
+		return f >= half && (f - half) % every == 0 && (f - half) / every < VPT ? (f - half) / every : -1;
+	};
+	static_assert(kStepsQ / 2 >= VPT && kStepsV / 2 >= VPT, "steps for the pieces");
+	int t_next = 0;
+	for (int t = t_first; t <= t_last; t = t_next)
+	{
+		if constexpr (MASK) t_next = visible.next(t + 1, t_last);
+		else t_next = t + 1;
+		__syncthreads();                            // K(t) is complete, V of the tile before has been read by everybody
+		if constexpr (MASK) load_mask(t);
+		// ---- S^T = K Q^T ----
+		float4_t s[KB];
+#pragma unroll
+		for (int kb = 0; kb < KB; ++kb) s[kb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+		for (int f = 0; f < kAheadQ; ++f) read_k(f);
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int f = 0; f < kStepsQ; ++f)
+		{
+			const int u = f / 3, st = u / KB, kb = u % KB;
+#pragma unroll
+			for (int x = f % 3; x >= 0; --x) s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag[f % kAheadQ], qf[x][st], s[kb], 0, 0, 0);
+			if (f + kAheadQ < kStepsQ) read_k(f + kAheadQ);
+			if (piece_at(f, kStepsQ) >= 0) put(true, piece_at(f, kStepsQ));
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		// ---- online softmax: score (kb, r) of this lane is key 16 kb + 4 g + r ----
+		const int tile_key0 = t * KT;
+		const bool interior = tile_key0 >= all_lo && tile_key0 + KT - 1 <= all_hi;   // wave-uniform
+		float z[4 * KB];
+#pragma unroll
+		for (int i = 0; i < 4 * KB; ++i)
+		{
+			z[i] = logit2<SOFTCAP>(s[i / 4][i % 4], a.k_in, a.k_cap);
+			if constexpr (MASK) z[i] += mk[MASK ? i / 4 : 0][i % 4] * kLog2e;
+		}
+		if (!MASK && !interior)                     // (a mask's values past the last key hide them)
+		{
+			int row = n;
+			asm volatile("" : "+v"(row));           // (found anew at each such tile: two registers)
+			row += wq0;
+			const int vis_hi = a.causal && row + a.diag < a.n_k - 1 ? row + a.diag : a.n_k - 1;
+			const int vis_lo = a.window > 0 ? row + a.diag - a.window + 1 : 0;
+#pragma unroll
+			for (int i = 0; i < 4 * KB; ++i)
+			{
+				const int key = tile_key0 + 16 * (i / 4) + 4 * g + i % 4;
+				z[i] = (key >= vis_lo && key <= vis_hi) ? z[i] : -INFINITY;
+			}
+		}
+		float mt = z[0];
+#pragma unroll
+		for (int i = 1; i < 4 * KB; ++i) mt = fmaxf(mt, z[i]);
+		mt = max_over_lane_rows(mt);
+		const float m_new = fmaxf(m_run, mt);
+		const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;   // nothing visible so far: every term is exp2(-inf) = 0
+		// the running maximum settles after a few tiles; when no query of the wave raised it, the
+		// rescale factor is 1 everywhere and the pass over the accumulators is skipped
+		if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0)
+		{
+			const float corr = fast_exp2(m_run - m_safe);
+			l_run *= corr;
+#pragma unroll
+			for (int c = 0; c < DC; ++c) o[c] *= corr;
+		}
+		m_run = m_new;
+		float psum[2] = {0.0f, 0.0f};
+		bf16x8_t pf[3];
+		uint4_t w[3];
+#pragma unroll
+		for (int j = 0; j < 8; j += 2)
+		{
+			const float p0 = fast_exp2(z[j] - m_safe), p1 = fast_exp2(z[j + 1] - m_safe);
+			psum[0] += p0;
+			psum[1] += p1;
+			unsigned lo[3], hi[3];
+			split_bits(p0, lo[0], lo[1], lo[2]);
+			split_bits(p1, hi[0], hi[1], hi[2]);
+#pragma unroll
+			for (int p = 0; p < 3; ++p) w[p][j / 2] = upper_halves(lo[p], hi[p]);
+		}
+#pragma unroll
+		for (int p = 0; p < 3; ++p) pf[p] = __builtin_bit_cast(bf16x8_t, w[p]);
+		l_run += psum[0] + psum[1];
+		// (behind the last tile: that tile once more, of no consequence)
+		const int t_load = t_next <= t_last ? t_next : t;
+		fetch(kp, t_load);
+		__syncthreads();                            // V(t) is complete, K(t) has been read by everybody
+		// ---- O^T += V^T P^T ----
+#pragma unroll
+		for (int f = 0; f < kAheadV; ++f) read_v(f);
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int f = 0; f < kStepsV; ++f)
+		{
+			const int c = 2 * (f / 3);
+#pragma unroll
+			for (int x = f % 3; x >= 0; --x)
+#pragma unroll
+				for (int i = 0; i < 2; ++i) o[c + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag[2 * (f % kAheadV) + i], pf[x], o[c + i], 0, 0, 0);
+			if (f + kAheadV < kStepsV) read_v(f + kAheadV);
+			if (piece_at(f, kStepsV) >= 0) put(false, piece_at(f, kStepsV));
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		fetch(vp, t_load);
+	}
+
+	// ---- normalise and store: lane (n, g) holds y[row][16 c + 4 g .. + 3] ----
+	const float l = sum_over_lane_rows(l_run);
+	float all = l;                                  // not finite where anything that entered it is not
+#pragma unroll
+	for (int c = 0; c < DC; ++c)
+#pragma unroll
+		for (int r = 0; r < 4; ++r) all = fmaf(o[c][r], 0.0f, all);
+	if (any_of_block<THREADS / kWaveSize>(!(fabsf(all) < INFINITY), lds, wave)) return false;
+	if (q_row >= a.n_q) return true;
+	if (partial != nullptr)
+	{
+		// unnormalised accumulators, running maximum and sum of this part of the keys
+		float* dst = partial + (int64_t)(q_row - q0) * (D + 2);
+#pragma unroll
+		for (int c = 0; c < DC; ++c) *reinterpret_cast<WsFloat4*>(dst + 16 * c + 4 * g) = o[c];
+		if (g == 0)
+		{
+			dst[D] = m_run;
+			dst[D + 1] = l;
+		}
+		return true;
+	}
+	const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+	for (int c = 0; c < DC; ++c) *reinterpret_cast<float4_t*>(yp + (int64_t)q_row * D + 16 * c + 4 * g) = o[c] * inv;
+	return true;
+}
+
+// The launch of that form: every block finds its query block and the tiles of it, or (BALANCED: MASK with a map) its range of the launch's
+// set tiles (attention_balance.hpp), and walks it query block after query block.  One range per resident block: with two for each CU 16 heads x 2500 x 128 215 us, with one 199.
+template <int D, bool SOFTCAP, bool MASK, bool BALANCED>
+__global__ __launch_bounds__(split_threads(D, MASK), 2) void sdp_attention_fwd_f32_split_kernel(const AttnArgsF32 a, const AttnWalk walk, const AttnBalance balance)
+{
+	static_assert(!BALANCED || MASK, "ranges of a mask's set tiles");
+	extern __shared__ __align__(16) char lds_raw[];
+	const auto attend = [&](int bh, int q_block, int t_first, int t_last, const unsigned long long* map_row, float* partial) {
+		if constexpr (split_narrow(D, MASK))
+		{
+			if (attend_f32_split16<D, SOFTCAP, MASK>(a, lds_raw, bh, q_block, t_first, t_last, map_row, partial)) return;
+		}
+		else if (attend_f32_split<D, SOFTCAP, MASK>(a, lds_raw, bh, q_block, t_first, t_last, map_row, partial)) return;
+		// (16 queries to a wave: with four waves the block's queries in two halves)
+		constexpr int kWaves = split_threads(D, MASK) / 64, kHalves = kSplitQueries / (16 * kWaves);
+		for (int i = 0; i < kHalves; ++i)
+		{
+			__syncthreads();
+			attend_f32<D, SOFTCAP, kWaves, kSplitKeys, D == 256, MASK>(a, reinterpret_cast<float*>(lds_raw), bh, kHalves * q_block + i, t_first, t_last, map_row,
+			                                                           partial ? partial + i * (16 * kWaves) * (D + 2) : nullptr);
+		}
+	};
+	if constexpr (!BALANCED)
+	{
+		int bh, q_block, t_first, t_last;
+		const unsigned long long* map_row;
+		float* partial;
+		if (!attention_block_f32<D, kSplitQueries, kSplitKeys, MASK>(a, walk, bh, q_block, t_first, t_last, map_row, partial)) return;
+		attend(bh, q_block, t_first, t_last, map_row, partial);
+	}
+	else
+	{
+		constexpr int64_t kPartialFloats = (int64_t)kSplitQueries * (D + 2);
+		// (a run of ranges to each XCD: neighbours share a head's keys)
+		const int64_t range = balance.ranges % 8 == 0 ? (int64_t)(blockIdx.x % 8) * (balance.ranges / 8) + blockIdx.x / 8 : blockIdx.x;
+		const BalanceScan scan(a.tile_map, balance);
+		int64_t at = range * scan.per;
+		const int64_t range_end = min(at + scan.per, (int64_t)scan.per_head * balance.heads);
+		if (at >= range_end) return;
+		int bh = (int)(at / scan.per_head), q_block, first;
+		const int x = (int)(at - (int64_t)bh * scan.per_head);
+		scan.locate(a.tile_map, balance, x, q_block, first);
+		q_block = __builtin_amdgcn_readfirstlane(q_block);
+		int in_block = __builtin_amdgcn_readfirstlane(x - first);              // tiles of the query block in front of the range
+		float* slot = a.partials + 2 * range * kPartialFloats;       // of the query block that the range starts inside; the next one's
+		for (;;)
+		{
+			const unsigned long long* const map_row = a.tile_map + (int64_t)q_block * a.map_words;
+			// (the same in every lane, which the compiler does not see by itself)
+			const int count = __builtin_amdgcn_readfirstlane(balance_tiles(a.tile_map, balance, q_block));
+			const int taken = __builtin_amdgcn_readfirstlane((int)min((int64_t)(count - in_block), range_end - at));
+			const int t_first = __builtin_amdgcn_readfirstlane(balance_nth_tile(map_row, balance.words, in_block));
+			int t_last = __builtin_amdgcn_readfirstlane(balance_nth_tile(map_row, balance.words, in_block + taken - 1));
+			if (t_first > (a.n_k - 1) / kSplitKeys) t_last = t_first - 1;       // (no set tile at all: zeros)
+			attend(bh, q_block, t_first, t_last, map_row, taken == count ? nullptr : slot);
+			at += taken;
+			if (at >= range_end) return;
+			in_block = 0;
+			slot = a.partials + (2 * range + 1) * kPartialFloats;
+			if (++q_block == balance.q_blocks)
+			{
+				q_block = 0;
+				++bh;
+			}
 		}
 	}
-	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads,
-	                                                kQueriesPerBlock, KT, D, band::workspace_capacity(stream));
+}
+
+// More than 64 KB of dynamic LDS has to be granted per function and per device, once.
+template <typename Kernel>
+hipError_t grant_lds(Kernel kernel, int bytes, std::atomic<uint64_t>& configured_devices)
+{
+	if (bytes <= 64 * 1024) return hipSuccess;
+	int device = 0;
+	hipError_t e = hipGetDevice(&device);
+	if (e != hipSuccess) return e;
+	const uint64_t bit = 1ull << (device & 63);
+	if ((configured_devices.load(std::memory_order_relaxed) & bit) == 0)
+	{
+		e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+		if (e != hipSuccess) return e;
+		configured_devices.fetch_or(bit, std::memory_order_relaxed);
+	}
+	return hipSuccess;
+}
+
+template <int D, bool MASK>
+constexpr int split_lds_bytes()
+{
+	constexpr int kPlainBytes = AttnLdsF32<D, kSplitKeys>::kStageFloats * 4 * (D == 256 ? 2 : 1);     // (the form that takes over from it)
+	constexpr int kPlanes = AttnLdsSplit<D, split_narrow(D, MASK)>::kBytes;
+	return kPlanes > kPlainBytes ? kPlanes : kPlainBytes;
+}
+
+// One launch over query blocks of QUERIES and tiles of KEYS, with the merge of whatever goes out in parts of its key range.
+template <int D, int QUERIES, int KEYS, typename Launch>
+hipError_t launch_blocks_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t stream, Launch launch)
+{
+	const int64_t q_blocks = (args.n_q + QUERIES - 1) / QUERIES;
+	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, QUERIES, KEYS, D,
+	                                                band::workspace_capacity(stream));
 	// (or, with too few query blocks for the chip, every block in several parts of its key range)
-	int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQueriesPerBlock,
-	                                                                  KT, D, band::workspace_capacity(stream));
-	if (plan.n_split == 0 && (parts_all == 1 || q_blocks * batch_heads < device_cu_count()) && mask_parts > 0) parts_all = mask_parts;
+	const int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, QUERIES, KEYS, D,
+	                                                                        band::workspace_capacity(stream));
 	args.partials = nullptr;
 	if (plan.n_split > 0 || parts_all > 1)
 	{
@@ -547,13 +1240,118 @@ hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, h
 	}
 	const AttnWalk walk = make_attn_walk(q_blocks, batch_heads, args.q_per_kv, plan.n_split, plan.n_big, parts_all);
 	if (attn_walk_blocks(walk) > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-	kernel<<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * WAVES), kLdsBytes, stream>>>(args, walk);
-	const hipError_t err = hipGetLastError();
+	const hipError_t err = launch(walk);
 	if (err != hipSuccess || walk.n_split == 0) return err;
-	const int64_t items = batch_heads * walk.n_split * kQueriesPerBlock * (D / 4);
+	const int64_t items = batch_heads * walk.n_split * QUERIES * (D / 4);
 	sdp_attention_merge_halves_kernel<D, float><<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream>>>(
-		args.partials, args.y, args.n_q, (int)q_blocks, walk.n_split, kQueriesPerBlock, parts_all > 1 ? (int)parts_all : 2);
+		args.partials, args.y, args.n_q, (int)q_blocks, walk.n_split, QUERIES, parts_all > 1 ? (int)parts_all : 2);
 	return hipGetLastError();
+}
+
+template <int D, bool SOFTCAP, bool MASK>
+hipError_t launch_split_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t stream)
+{
+	return launch_blocks_f32<D, kSplitQueries, kSplitKeys>(args, batch_heads, stream, [&](const AttnWalk& walk) {
+		auto kernel = sdp_attention_fwd_f32_split_kernel<D, SOFTCAP, MASK, false>;
+		static std::atomic<uint64_t> configured_devices{0};
+		const hipError_t err = grant_lds(kernel, split_lds_bytes<D, MASK>(), configured_devices);
+		if (err != hipSuccess) return err;
+		kernel<<<dim3((unsigned)attn_walk_blocks(walk)), dim3(split_threads(D, MASK)), split_lds_bytes<D, MASK>(), stream>>>(args, walk, AttnBalance{});
+		return hipGetLastError();
+	});
+}
+
+template <int D, bool SOFTCAP, bool MASK>
+hipError_t launch_plain_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t stream)
+{
+	// head dimension 256: 8 waves (two per SIMD) on tiles of 32 keys in two stages, 130 KB, one block per CU.  Two
+	// alternatives with two blocks of 4 waves per CU, for a better balance of long and short blocks under the causal
+	// rule, measured 5 - 12 % slower: tiles of 16 keys, and one K and one V buffer refilled in turn.
+	constexpr bool DIRECT = (D == 256);
+	constexpr int WAVES = DIRECT ? 8 : 4;
+	constexpr int KT = DIRECT ? 32 : 64;
+	constexpr int kLdsBytes = AttnLdsF32<D, KT>::kStageFloats * 4 * (DIRECT ? 2 : 1);
+	return launch_blocks_f32<D, 16 * WAVES, KT>(args, batch_heads, stream, [&](const AttnWalk& walk) {
+		auto kernel = sdp_attention_fwd_f32_kernel<D, SOFTCAP, WAVES, KT, DIRECT, MASK>;
+		static std::atomic<uint64_t> configured_devices{0};
+		const hipError_t err = grant_lds(kernel, kLdsBytes, configured_devices);
+		if (err != hipSuccess) return err;
+		kernel<<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * WAVES), kLdsBytes, stream>>>(args, walk);
+		return hipGetLastError();
+	});
+}
+
+// Whether the launch takes the bf16 parts (us, fp32 matrix instruction / bf16 parts).
+//   * Index rules: at head dimension 256 always (8 heads x 64 x 64 21.2 / 15.9, 8 / 4 x 8192, window 4096 1801 / 1051); at 64 and 128, where the
+//     other form has blocks of 64 queries, from some ten tiles on (32 heads x 1000 x 128 111 / 75, 400 38 / 32, 16 x 2000 x 128 324 / 185; but
+//     32 x 150 x 128 18.1 / 19.3, 64 x 250 x 64 15.2 / 19.9), at 64 for more than a block of queries (8 x 64 x 4000 28.8 / 34.1, 32 x 100 x 1000 21.1 / 22.6).
+//   * A mask tensor: with its visible-tile map, as there is no test of a tile by each wave.  The pass that makes the map and a range's start cost
+//     20 - 30 us: head dimension 256 from 150 K mask values on (8 heads x 250 x 600 58.3 / 56.7, 400 58.5 / 54.7, 2000 301 / 139); 128 from 6 M values
+//     over all heads (8 x 100 x 8000 86.7 / 69.0, 8 x 1000 60.4 / 45.2; but 8 x 797 39.0 / 42.6, 32 x 250 x 600 39.5 / 43.7); 64 from 11 M in masks of
+//     600 K (8 x 830 x 1800 51.6 / 48.1, 32 x 797 55.6 / 50.3; but 8 x 1000 33.1 / 37.8, 32 x 400 26.6 / 37.3).
+template <int D, bool MASK>
+bool attention_split_wanted(const AttnArgsF32& args, int64_t batch_heads)
+{
+	if constexpr (MASK)
+	{
+		const int64_t values = (int64_t)args.n_q * args.n_k;
+		if (args.mask_stride > kSplitMaskStride) return false;
+		if (D == 64) return values >= 600 * 1000 && batch_heads * values >= 11 * 1000 * 1000;
+		return values >= 150 * 1000 && (D == 256 || batch_heads * values >= 6 * 1000 * 1000);
+	}
+	else return D == 256 || (args.n_k >= 350 && (D == 128 || args.n_q > 128));
+}
+
+template <int D, bool SOFTCAP, bool MASK>
+hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, hipStream_t stream)
+{
+	(void)hipGetLastError();
+	AttnArgsF32 args = args_in;
+	args.tile_map = nullptr;
+	args.map_words = 0;
+	const bool split = attention_split_wanted<D, MASK>(args, batch_heads);
+	if constexpr (!MASK) return split ? launch_split_f32<D, SOFTCAP, false>(args, batch_heads, stream) : launch_plain_f32<D, SOFTCAP, false>(args, batch_heads, stream);
+	else
+	{
+		// The visible-tile map of the mask, at the front of the stream's workspace (partial results go behind it), for large masks and long key
+		// ranges (attention_mask_map_wanted), and left out where the stream has no workspace to offer (a capture without a
+		// caller's workspace).
+		const int queries = split || D == 256 ? kSplitQueries : 64, keys = split || D == 256 ? kSplitKeys : 64;
+		const int64_t q_blocks = (args.n_q + queries - 1) / queries, words = attention_tile_map_words(args.n_k, keys);
+		const size_t map_bytes = ((size_t)(q_blocks * words) * sizeof(unsigned long long) + 255) / 256 * 256;
+		if (!attention_mask_map_wanted(args.n_q, args.n_k, split) || band::workspace_capacity(stream) < map_bytes + (1u << 16))
+			return launch_plain_f32<D, SOFTCAP, true>(args, batch_heads, stream);
+		// Up to four rounds of query blocks: the launch's set tiles in equal shares, whose partial results may need more than the library's own
+		// workspace holds to begin with (it grows for them as it does for operand copies, eager launches only).
+		const int64_t ranges = (split_narrow(D, true) ? 1 : 2) * (int64_t)device_cu_count();
+		const size_t shares_bytes = map_bytes + (size_t)(2 * ranges) * kSplitQueries * (D + 2) * sizeof(float);
+		const bool balanced = split && q_blocks * batch_heads < 4 * ranges && band::workspace_copy_capacity(stream) >= shares_bytes;
+		float* front = nullptr;
+		hipError_t e = band::workspace_acquire(stream, &front, balanced ? shares_bytes : 0);
+		if (e != hipSuccess) return e;
+		unsigned long long* map = reinterpret_cast<unsigned long long*>(front);
+		e = launch_attention_mask_tile_map(args.mask, args.mask_stride, args.n_q, args.n_k, queries, keys, map, stream);
+		if (e != hipSuccess) return e;
+		args.tile_map = map;
+		args.map_words = (int)words;
+		if (!balanced)
+		{
+			const band::WorkspaceReserve map_hold(map_bytes);
+			return split ? launch_split_f32<D, SOFTCAP, true>(args, batch_heads, stream) : launch_plain_f32<D, SOFTCAP, true>(args, batch_heads, stream);
+		}
+		args.partials = reinterpret_cast<float*>(reinterpret_cast<char*>(front) + map_bytes);
+		const AttnBalance balance{(int)ranges, (int)batch_heads, (int)q_blocks, (int)words, 4};
+		auto kernel = sdp_attention_fwd_f32_split_kernel<D, SOFTCAP, true, true>;
+		static std::atomic<uint64_t> configured_devices{0};
+		e = grant_lds(kernel, split_lds_bytes<D, MASK>(), configured_devices);
+		if (e != hipSuccess) return e;
+		kernel<<<dim3((unsigned)ranges), dim3(split_threads(D, MASK)), split_lds_bytes<D, MASK>(), stream>>>(args, AttnWalk{}, balance);
+		e = hipGetLastError();
+		if (e != hipSuccess) return e;
+		sdp_attention_merge_ranges_kernel<D, float><<<dim3(kSplitQueries * (D / 4) / 256, (unsigned)q_blocks, (unsigned)batch_heads), dim3(256), 0, stream>>>(
+			args.partials, args.y, args.n_q, kSplitQueries, map, balance);
+		return hipGetLastError();
+	}
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -72,11 +72,12 @@ __global__ __launch_bounds__(1024) void attention_mask_tile_map_kernel(const T* 
 // on whatever the queries (a sliding window over a long cache hides most of them from a few queries as well).  The
 // environment variable ANYGPU_ATTN_MASK_MAP_FROM, read at every launch, replaces the rule by "from that many mask values
 // on" (0: always, a huge value: never).
-inline bool attention_mask_map_wanted(int64_t n_q, int64_t n_k)
+// `needed`: the launch's kernel works on the map.
+inline bool attention_mask_map_wanted(int64_t n_q, int64_t n_k, bool needed = false)
 {
 	const char* text = std::getenv("ANYGPU_ATTN_MASK_MAP_FROM");
 	if (text != nullptr && *text != 0) return n_q * n_k >= std::atoll(text);
-	return n_q * n_k >= (4ll << 20) || n_k >= 16384;
+	return needed || n_q * n_k >= (4ll << 20) || n_k >= 16384;
 }
 
 // 64-bit words of the map per query block
