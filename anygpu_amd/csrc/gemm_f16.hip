@@ -6,8 +6,8 @@
 // (the reference layout, transposed on the way out of LDS); the smaller two also cut along K.
 // Eight-wave and 64 x 64 tile kernels (gemm_f16_tile.hpp): everything the above do not take (a K tail, few rows).
 // Operands the 16-byte chunk loads cannot fetch are copied aligned into the stream's workspace first (gemm_repack.hip);
-// where that is not possible or not worth it, the edge kernel: 64 x 64 tiles, guarded scalar loads and stores, either
-// B layout, any shape, stride and alignment.
+// small products of such operands go as they lie through gemm_f16_small.hip; where neither is possible or worth it, the edge kernel:
+// 128 x 128 tiles, guarded scalar loads and stores, either B layout, any shape, stride and alignment.
 #include <algorithm>
 
 #include "device_utils.hpp"
@@ -403,6 +403,12 @@ hipError_t launch_gemm_f16(const void* A, const void* B, void* C, int64_t M, int
 	// 166 us against 198 us; small weights 9 us against 13 us), and whatever the tile kernels cannot take goes to the
 	// band kernels (5 .. 64 rows) or the skinny ones.
 	const bool tiles_first = tiles_ok && (b_layout == ANYGPU_B_ROW_MAJOR || M >= 3);
+	// small products of such operands (the rule and both sides: gemm_f16_small_applies)
+	if (!tiles_ok && batch == 1 && gemm_f16_small_applies(M, N, K, b_layout, finish != nullptr))
+	{
+		if (finish) finish->handled = true;
+		return launch_gemm_f16_small(A, B, fin_bias, C, M, N, K, lda, ldb, ldc, b_layout, fin_epi, fin_param, stream);
+	}
 	// Operands the tile kernels cannot fetch (an odd start or row pitch, K no multiple of 8, [K, N] weights with such an
 	// N) are copied into the stream's workspace as aligned k-contiguous rows, zeros up to the next multiple of 64 behind
 	// K, and the product runs on the copies: 4096 x 4100 . [4096, 4100] weights 270 -> 117 us (vendor 105 - 110).  From

@@ -121,6 +121,11 @@ hipError_t launch_gemm_f32(const float* A, const float* B, const float* bias, fl
                            int64_t stride_a, int64_t stride_b, int64_t stride_c, int64_t batch,
                            int a_layout, int b_layout, hipStream_t stream);
 
+// The fp16 product with operands straight from memory at element alignment (gemm_f16_small.hip), for small ragged ones; epilogue: kEpiBias
+// (bias may be NULL) or kEpiSoftcap
+bool gemm_f16_small_applies(int64_t M, int64_t N, int64_t K, int b_layout, bool with_epilogue);
+hipError_t launch_gemm_f16_small(const void* A, const void* B, const void* bias, void* C, int64_t M, int64_t N, int64_t K,
+                                 int64_t lda, int64_t ldb, int64_t ldc, int b_layout, int epilogue, float ep_param, hipStream_t stream);
 // The fp32 product (row-major A) in 32 x 32 tiles with K cut over the waves of a block (gemm_f32_small.hip): any sizes, pitches
 // and element alignment.  `applies`: whether it is ahead of the other kernels for these operands.
 bool gemm_f32_small_applies(const float* A, const float* B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int b_layout);

@@ -375,3 +375,43 @@ def test_softmax_rows_of_any_width_and_start(ops, oracle, dtype, rows, cols, pad
     assert np.all(got[want == 0] == 0)
     yv.fill_(-7.0)
     assert bool((ybuf == -7.0).all())
+
+
+@pytest.mark.parametrize("layout", ["kn", "nk"])
+@pytest.mark.parametrize("m,n,k,shift", [(3, 1, 1, 0), (1, 333, 211, 1), (5, 33, 31, 0), (32, 32, 32, 1), (33, 31, 33, 0), (64, 65, 127, 1), (31, 97, 129, 3),
+                                         (100, 40, 160, 1), (70, 130, 161, 2), (45, 300, 543, 0), (200, 129, 1000, 1), (17, 50, 1502, 2), (2, 1001, 700, 0)])
+def test_mm_f16_small_products_as_they_lie(ops, m, n, k, layout, shift):
+    # 32 x 32 tiles and steps of 32 of K from before to behind their ends, none to a dozen steps per wave; operands `shift` halves into wider buffers of
+    # NaN, so that rows start at odd halves and at words that are no multiple of 16 bytes, the result likewise.  Small integers: exact.
+    import torch
+    from anygpu_amd import capi
+    lay = capi.B_ROW_MAJOR if layout == "kn" else capi.B_COL_MAJOR
+    a, b = (synth.integers(s + m, shape, -2, 2).astype(np.float16) for s, shape in ((1, (m, k)), (2, (k, n))))
+    want = exact_int_product(a, b)
+    assert np.max(np.abs(want)) < 2000
+    w = b if layout == "kn" else np.ascontiguousarray(b.T)
+
+    def inside(x):
+        buf = torch.full((x.shape[0], x.shape[1] + 5), math.nan, dtype=torch.float16, device="cuda")
+        view = buf[:, shift:shift + x.shape[1]]
+        view.copy_(dev(x))
+        return view
+    av, wv = inside(a), inside(w)
+    out = torch.full((m + 1, n + 4), -7.0, dtype=torch.float16, device="cuda")
+    ops.tensor_mm(av, wv, out=out[:m, shift:shift + n], b_layout=lay)
+    got = host(out).astype(np.int64)
+    assert np.array_equal(got[:m, shift:shift + n], want)
+    assert np.all(got[m:] == -7) and np.all(got[:, :shift] == -7) and np.all(got[:, shift + n:] == -7)
+    bias = synth.integers(3, (n,), -9, 9).astype(np.float16)
+    assert np.array_equal(host(ops.tensor_gemm(dev(a), dev(w), dev(bias), b_layout=lay)).astype(np.int64), want + bias.astype(np.int64))
+    if layout == "nk":
+        # half an ulp of the result, 4.4e-5 of it for the fp16 tanh
+        scale = 2.0 ** -6
+        got = host(ops.tensor_gemma_linear_softcap(dev((a * scale).astype(np.float16)).reshape(1, m, k), dev(w), 30.0)).astype(np.float64).reshape(m, n)
+        capped = 30.0 * np.tanh(want * scale / 30.0)
+        assert np.all(np.abs(got - capped) <= (2.0 ** -11 + 4.4e-5) * np.abs(capped) + 30.0 * 1e-6)
+    # a NaN or an infinity reaches its row or column and no other
+    av[0, k - 1], wv[(k // 2, n - 1) if layout == "kn" else (n - 1, k // 2)] = math.nan, math.inf
+    got = host(ops.tensor_mm(av, wv, b_layout=lay)).astype(np.float64)
+    assert np.all(np.isnan(got[0])) and not np.isfinite(got[1:, n - 1]).any()
+    assert np.array_equal(got[1:, :n - 1], want[1:, :n - 1])
