@@ -291,9 +291,9 @@ int anygpu_sdp_attention_fwd_f16(const void* q, const void* k, const void* v, vo
                                  float alpha, float softcap, int causal, int64_t window, void* stream);
 
 /*
- * anygpu_sdp_attention_fwd_f16 in float32: operands, scores, sums and output are fp32 and both products run on the
- * fp32 matrix instruction, so results agree with the unfused float32 path to fp32 rounding.  Same arguments and
- * rules.  Replaces cu_flash_sdpa_fwd_d256_v1 (srcs/kernels/cuda/flash_sdpa_fwd.cuh:6-15: one head, head_dim 256,
+ * anygpu_sdp_attention_fwd_f16 in float32: operands, scores, sums and output are fp32.  A product of floats is six products
+ * of their bf16 parts, summed in fp32 (what is left out lies below 2^-23 of it), small launches and results that are not finite
+ * run on the fp32 matrix instruction; results agree with the unfused float32 path to fp32 rounding.  Same arguments and rules.  Replaces cu_flash_sdpa_fwd_d256_v1 (srcs/kernels/cuda/flash_sdpa_fwd.cuh:6-15: one head, head_dim 256,
  * no mask; here any number of heads, head_dim 64 / 128 / 256, the index-rule masks) and, for masks that are
  * index rules, the per-head loop of sdp_attention_masked_scaled_fwd (srcs/transformers/sdp.hpp:258-271).
  */
@@ -313,10 +313,12 @@ int anygpu_sdp_attention_fwd_f32(const float* q, const float* k, const float* v,
  * under a capture without a caller's workspace there is none, every tile is loaded and the hidden ones cost no products.
  * The results are the same bit for bit either way, except where few query blocks go out in parts of their key range:
  * with the note the parts divide the visible tiles among them (a sliding window over a long cache leaves most equal
- * parts of the range empty), without it the range, and the sums are taken in another order.  With as many query blocks as
- * one to four rounds of the device's compute units the float32 form sends every block out in two such parts; for their
- * partial results an eager launch without a caller's workspace lets the library's own grow (as operand copies do, up to
- * 1 GiB; 192 MiB for 8 heads x 8192 queries x 256).  Callers whose mask is an index rule are still better served by
+ * parts of the range empty), without it the range, and the sums are taken in another order.  The float32 form's products of bf16
+ * parts need the note: masks for which they pay (150 K values and more at head dimension 256) get one whatever their size, unless
+ * the environment variable is set, and a launch without one runs on the fp32 matrix instruction (the same to rounding).  With
+ * fewer query blocks than four rounds of the device the note's set tiles are cut into one equal range per resident block; for their
+ * partial results (68 MB at head dimension 256) an eager launch without a caller's workspace lets the library's own grow
+ * (as operand copies do, up to 1 GiB).  Callers whose mask is an index rule are still better served by
  * anygpu_sdp_attention_fwd_f32.  Same key splits through the stream's workspace as that entry point.
  */
 int anygpu_sdp_attention_fwd_masked_f32(const float* q, const float* k, const float* v, const float* mask, float* y,
