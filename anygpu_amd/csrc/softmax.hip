@@ -5,8 +5,8 @@
 // Without a mask tensor (softmax_rows_kernel): a row of lanes, a wave or a block owns one row and keeps its visible part in
 // registers; rows of any width and pitch.  Vectors that lie wholly outside the visible key interval [lo, hi] of the row are never
 // loaded; their outputs are stored as zeros.
-// With one, or where x and y are not aligned alike (softmax_rows_wave_kernel): the same with an online max/sum over the vectors as they
-// arrive.  Rows longer than a block's registers hold are walked
+// With one, where x and y are not aligned alike, or where a row's vectors just fill a block (softmax_rows_wave_kernel): the same with an
+// online max/sum over the vectors as they arrive.  Rows longer than a block's registers hold are walked
 // twice by a block of 1024 threads with 16-byte accesses, at any width, stride or alignment.
 // An additive mask tensor [q_len, cols] shared by the heads of a batch is read with ordinary (cached) loads, and the
 // blocks are dealt so that the heads of a mask row run side by side on one XCD (block_rows).
@@ -642,9 +642,10 @@ static hipError_t launch_wave(const SoftmaxArgs& a, hipStream_t stream)
 {
 	const unsigned blocks = blocks_for_rows(a, 256 / GROUP);
 	discard_stale_error();
-	// (without a mask tensor only rows of x and y that are not aligned alike get here)
-	if (!LOOSE || a.mask != nullptr) softmax_rows_wave_kernel<T, VPL, LOOSE, GROUP, true><<<dim3(blocks), dim3(256), 0, stream>>>(a);
-	else softmax_rows_wave_kernel<T, VPL, true, GROUP, false><<<dim3(blocks), dim3(256), 0, stream>>>(a);
+	// Without a mask tensor: rows at element alignment, and aligned ones whose vectors just fill a block's registers (launch_softmax_rows).
+	if (a.mask != nullptr) softmax_rows_wave_kernel<T, VPL, LOOSE, GROUP, true><<<dim3(blocks), dim3(256), 0, stream>>>(a);
+	else if constexpr (LOOSE || (GROUP == 256 && VPL == 16)) softmax_rows_wave_kernel<T, VPL, LOOSE, GROUP, false><<<dim3(blocks), dim3(256), 0, stream>>>(a);
+	else return hipErrorInvalidValue;
 	return hipGetLastError();
 }
 
@@ -708,6 +709,7 @@ hipError_t launch_softmax_rows(const void* x, void* y, int64_t rows, int64_t col
 		if (per_thread <= 8) return launch_rows<T, 8, 256>(a, stream);
 		if (rows_vectors<T>(a, 512) <= 6) return launch_rows<T, 6, 512>(a, stream);
 		if (rows_vectors<T>(a, 512) <= 8) return launch_rows<T, 8, 512>(a, stream);
+		// (rows of 4089 to 4096 vectors that start inside a line have a ninth vector per thread: the forms below)
 	}
 	// short rows (up to 64 vectors: 512 halves, 256 floats): sixteen lanes per row, four rows per wave
 	if (vec_ok && nvec <= 64 && rows >= 64)

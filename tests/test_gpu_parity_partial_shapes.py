@@ -377,6 +377,27 @@ def test_softmax_rows_of_any_width_and_start(ops, oracle, dtype, rows, cols, pad
     assert bool((ybuf == -7.0).all())
 
 
+@pytest.mark.parametrize("dtype,rows,cols,off", [("f16", 256, 32712, 0), ("f16", 300, 32760, 0), ("f32", 256, 16356, 0), ("f32", 300, 16380, 0), ("f16", 256, 32768, 8), ("f32", 256, 16384, 4)])
+@pytest.mark.parametrize("window", [0, 16000])
+def test_softmax_aligned_rows_that_just_fill_a_block(ops, oracle, dtype, rows, cols, off, window):
+    # 4089 to 4096 vectors of 16 bytes in rows that start inside a line: more than the block of 512 threads counts, as many as 256 hold
+    import torch
+    np_dt, t_dt = (np.float16, torch.float16) if dtype == "f16" else (np.float32, torch.float32)
+    x = synth.normal(cols + rows, (rows, cols), std=8.0).astype(np_dt)
+    xbuf, ybuf = (torch.full((off + rows * cols + 64,), -7.0, dtype=t_dt, device="cuda") for _ in range(2))
+    xv, yv = (torch.as_strided(buf, (rows, cols), (cols, 1), off) for buf in (xbuf, ybuf))
+    xv.copy_(dev(x))
+    kw = dict(alpha=0.5, softcap=20.0, causal=window > 0, window=window, q_len=rows, diag=cols - rows)
+    ops.tensor_softmax(xv, out=yv, **kw)
+    got = host(yv).astype(np.float64)
+    want = oracle.attention_softmax(oracle.cvt_f16_to_f32(x) if dtype == "f16" else x, **kw).reshape(rows, cols).astype(np.float64)
+    tol = TOL_F16_ROWOPS if dtype == "f16" else TOL_F32
+    assert np.max(np.abs(got - want) / (want + want.max(axis=1, keepdims=True))) <= tol
+    assert np.all(got[want == 0] == 0)
+    yv.fill_(-7.0)
+    assert bool((ybuf == -7.0).all())
+
+
 @pytest.mark.parametrize("layout", ["kn", "nk"])
 @pytest.mark.parametrize("m,n,k,shift", [(3, 1, 1, 0), (1, 333, 211, 1), (5, 33, 31, 0), (32, 32, 32, 1), (33, 31, 33, 0), (64, 65, 127, 1), (31, 97, 129, 3),
                                          (100, 40, 160, 1), (70, 130, 161, 2), (45, 300, 543, 0), (200, 129, 1000, 1), (17, 50, 1502, 2), (2, 1001, 700, 0)])
