@@ -14,6 +14,7 @@
 #include "launch.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace anygpu {
 
@@ -304,7 +305,21 @@ __device__ __forceinline__ float logit2_fast(float x, float k_in, float k_cap)
 	return x * k_in;
 }
 
-template <typename T, int VPL, int GROUP, bool SOFTCAP>
+// The softcap of softmax_rows_kernel.  The short form is off by 1.5e-7 of the cap in the logit, so by 1e-5 of a probability at a cap of 64, a
+// fiftieth of a half's rounding; beyond (halves) and for floats a form whose error vanishes with the logit.  2-norm error of halves, N(0, 16) scores,
+// short / full form: cap 50 1.98e-4 / 1.98e-4, 1000 1.88e-4 / 1.86e-4, 1e5 2.6e-3 / 1.9e-4.
+// tanh below a sixteenth, to 4e-9 of it
+constexpr float kTanhNearZero = 0.0625f;
+__device__ __forceinline__ float tanh_near_zero(float x)
+{
+	const float x2 = x * x;
+	return x * (1.0f + x2 * (-1.0f / 3.0f + x2 * (2.0f / 15.0f)));
+}
+
+enum : int { kCapNone, kCapShort, kCapFull };
+constexpr float kCapShortMost = 64.0f;
+
+template <typename T, int VPL, int GROUP, int CAP>
 __global__ __launch_bounds__(GROUP > 256 ? GROUP : 256) void softmax_rows_kernel(const SoftmaxArgs a)
 {
 	static_assert(GROUP == 16 || GROUP == 64 || GROUP == 256 || GROUP == 512, "a row of lanes, a wave or the block per row");
@@ -370,7 +385,7 @@ __global__ __launch_bounds__(GROUP > 256 ? GROUP : 256) void softmax_rows_kernel
 		raw[t] = val;
 	}
 
-	const float k_in = SOFTCAP ? 2.0f * kLog2e * a.alpha * a.inv_cap : a.alpha_log2e;
+	const float k_in = CAP == kCapShort ? 2.0f * kLog2e * a.alpha * a.inv_cap : a.alpha_log2e;
 	const float k_cap = a.cap_log2e;
 	float z[VPL][EPV];
 	float m = -INFINITY;
@@ -384,8 +399,24 @@ __global__ __launch_bounds__(GROUP > 256 ? GROUP : 256) void softmax_rows_kernel
 #pragma unroll
 			for (int e = 0; e < EPV; ++e)
 			{
-				if constexpr (sizeof(T) == 2) z[t][e] = logit2_fast<SOFTCAP>((float)raw[t][e], k_in, k_cap);
-				else z[t][e] = SOFTCAP ? k_cap * tanh_f32(raw[t][e] * a.alpha * a.inv_cap) : raw[t][e] * a.alpha_log2e;
+				if constexpr (CAP == kCapFull && sizeof(T) == 4) z[t][e] = k_cap * tanh_f32(raw[t][e] * a.alpha * a.inv_cap);
+				else if constexpr (CAP == kCapFull) z[t][e] = tanh_near_zero((float)raw[t][e] * a.alpha * a.inv_cap) * k_cap;
+				else z[t][e] = logit2_fast<CAP == kCapShort>((float)raw[t][e], k_in, k_cap);
+			}
+			if constexpr (CAP == kCapFull && sizeof(T) == 2)
+			{
+				// (a cap far beyond the scores leaves whole vectors near zero: 8 x 8192 x 8192 at a cap of 1000 394 us with both forms
+				// everywhere, 332 this way, as in the short form; at a cap of 100 366)
+				float far = 0.0f;
+#pragma unroll
+				for (int e = 0; e < EPV; ++e) far = fmaxf(far, fabsf((float)raw[t][e] * a.alpha * a.inv_cap));
+				if (__builtin_amdgcn_ballot_w64(!(far < kTanhNearZero)) != 0)
+#pragma unroll
+					for (int e = 0; e < EPV; ++e)
+					{
+						const float u = (float)raw[t][e] * a.alpha * a.inv_cap;
+						z[t][e] = fabsf(u) < kTanhNearZero ? z[t][e] : logit2_fast<true>((float)raw[t][e], 2.0f * kLog2e * a.alpha * a.inv_cap, k_cap);
+					}
 			}
 			if (v == v_lo || v == v_hi)
 			{
@@ -470,8 +501,9 @@ static hipError_t launch_rows(const SoftmaxArgs& a, hipStream_t stream)
 	constexpr int kThreads = GROUP > 256 ? GROUP : 256;
 	const unsigned blocks = (unsigned)((a.rows + kThreads / GROUP - 1) / (kThreads / GROUP));
 	discard_stale_error();
-	if (a.inv_cap != 0.0f) softmax_rows_kernel<T, VPL, GROUP, true><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
-	else softmax_rows_kernel<T, VPL, GROUP, false><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
+	if (a.inv_cap == 0.0f) softmax_rows_kernel<T, VPL, GROUP, kCapNone><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
+	else if (sizeof(T) == 2 && std::fabs(a.cap_log2e) <= kCapShortMost * kLog2e) softmax_rows_kernel<T, VPL, GROUP, kCapShort><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
+	else softmax_rows_kernel<T, VPL, GROUP, kCapFull><<<dim3(blocks), dim3(kThreads), 0, stream>>>(a);
 	return hipGetLastError();
 }
 

@@ -398,6 +398,19 @@ def test_softmax_aligned_rows_that_just_fill_a_block(ops, oracle, dtype, rows, c
     assert bool((ybuf == -7.0).all())
 
 
+@pytest.mark.parametrize("softcap", [50.0, 64.0, 65.0, 1e5, -1e5])
+@pytest.mark.parametrize("cols", [500, 1001, 12000])
+def test_softmax_f16_softcap_of_any_size(ops, softcap, cols):
+    # the logit keeps its precision however far the cap lies beyond the scores.  One rounding to half (2^-11, 2^-25 below the smallest normal half), the logit to
+    # 1.5e-7 of a cap of up to 64 or of a score of up to 32, some roundings of the fp32 sum and of exp2 (1e-6 each)
+    x = synth.normal(cols, (64, cols), std=4.0).astype(np.float16)
+    got = host(ops.tensor_softmax(dev(x), softcap=softcap)).astype(np.float64)
+    z = softcap * np.tanh(x.astype(np.float64) / softcap)
+    want = np.exp(z - z.max(axis=1, keepdims=True))
+    want /= want.sum(axis=1, keepdims=True)
+    assert np.all(np.abs(got - want) <= (2.0 ** -11 + 1.5e-5) * want + 2.0 ** -25)
+
+
 @pytest.mark.parametrize("layout", ["kn", "nk"])
 @pytest.mark.parametrize("m,n,k,shift", [(3, 1, 1, 0), (1, 333, 211, 1), (5, 33, 31, 0), (32, 32, 32, 1), (33, 31, 33, 0), (64, 65, 127, 1), (31, 97, 129, 3),
                                          (100, 40, 160, 1), (70, 130, 161, 2), (45, 300, 543, 0), (200, 129, 1000, 1), (17, 50, 1502, 2), (2, 1001, 700, 0)])

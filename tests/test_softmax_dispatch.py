@@ -28,6 +28,8 @@ using std::max;
 inline int64_t min(int64_t a, int64_t b) { return a < b ? a : b; }
 inline int64_t max(int64_t a, int64_t b) { return a > b ? a : b; }
 %(args)s
+enum : int { kCapNone, kCapShort, kCapFull };
+constexpr float kCapShortMost = 64.0f;
 static long picked[4] = {};
 [[noreturn]] static void fail(const char* what, const SoftmaxArgs& a, int bytes, int vpl, int group)
 {
