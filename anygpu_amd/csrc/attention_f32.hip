@@ -22,9 +22,10 @@
 //
 // Most launches take a second form (attend_f32_split, attend_f32_split16; the rule: attention_split_wanted).  The fp32 instruction has a
 // sixteenth of the bf16 one's rate, and a float is the sum of three bf16 exactly, so a product of floats is six bf16 products whose missing
-// terms lie below 2^-23 of it: 6 / 16 of the matrix time, summed in fp32 as before, in fewer roundings.  Error against float64 (2-norm), fp32
-// instruction / bf16 parts, q, k, v of N(0, 1): 16 heads x 1000 x 128 3.8e-7 / 2.8e-7, 16 / 4 x 1000 x 64 5.0e-7 / 3.5e-7, 8 / 4 x 1500 x 256 under softcap
-// and window 2.10e-6 / 2.08e-6, 8 x 1000 x 256 with q of four times the scale 1.46e-6 / 1.17e-6, a bias mask 8 x 2100 x 256 7.3e-7 / 6.6e-7.
+// terms lie below 2^-24 of it, of either sign: 6 / 16 of the matrix time, summed in fp32 as before, in fewer roundings.  Error against float64 (2-norm),
+// fp32 instruction / bf16 parts: q, k, v of N(0, 1) 24 heads x 800 x 64 5.9e-7 / 3.4e-7, 10 x 800 x 128 6.4e-7 / 3.6e-7, 3 x 800 x 256
+// 5.9e-7 / 4.6e-7; all mantissas 0x00FFFF 6.2e-7 / 3.6e-7, 6.8e-7 / 4.6e-7, 5.1e-7 / 5.2e-7; all mantissas 0x007FC0, which lose the most, 5.6e-7 / 3.2e-7,
+// 5.7e-7 / 4.1e-7, 3.3e-7 / 6.4e-7.
 // K and V are cut into their parts on their way into LDS (three planes each, once per block), p in its registers.  Bound: the bf16 matrix rate (and
 // the power that goes with it).  us, before / now: 8 / 4 heads x 8192 x 256, softcap, window 4096 1801 / 1051 (196 TFLOP/s, so 1.18 PFLOP/s of bf16
 // products), 16 x 2000 x 128 324 / 185, 32 / 8 x 3000 x 128 causal 701 / 419, 32 x 2000 x 64 causal 180 / 122, 8 x 1000 x 256 79.6 / 59.1; with a mask tensor
@@ -503,18 +504,24 @@ typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
 typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
-// A float as the sum of three bf16 (8 bits each, cut off, which together are all of its 24 bits): the first is the upper half of the
-// float's bits, the others are those of what is left.  (What is left below 2^-133, the smallest bf16, is lost: of floats below 2^-110.)
-__device__ __forceinline__ void split_bits(float x, unsigned& b1, unsigned& b2, unsigned& b3)
+// Two floats as sums of three bf16 each: the float rounded to nearest, what is left rounded likewise, and the rest, at most 2^-9, 2^-18 of the
+// power of two below the float (8 bits each with their own signs, which together are all of its 24 bits).  Word p of w: part p of both, the
+// first below.  Cut-off parts, twice as large and all of the float's sign, left 4.7e-7 of a product out of the six below, always
+// towards zero; these 5.9e-8 (2^-24) at most and 5.3e-9 (root mean square over all mantissas) of either sign.  (What is left below 2^-133, the smallest
+// bf16, is lost: of floats below 2^-110.)
+__device__ __forceinline__ void split_pair(float lo, float hi, unsigned (&w)[3])
 {
-	b1 = __builtin_bit_cast(unsigned, x);
-	const float r1 = x - __builtin_bit_cast(float, b1 & 0xFFFF0000u);
-	b2 = __builtin_bit_cast(unsigned, r1);
-	const float r2 = r1 - __builtin_bit_cast(float, b2 & 0xFFFF0000u);
-	b3 = __builtin_bit_cast(unsigned, r2);
+	typedef float float2_t __attribute__((ext_vector_type(2)));
+	typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+	for (int p = 0; p < 3; ++p)
+	{
+		w[p] = __builtin_bit_cast(unsigned, __builtin_convertvector(float2_t{lo, hi}, bf16x2_t));
+		if (p == 2) break;
+		lo -= __builtin_bit_cast(float, w[p] << 16);
+		hi -= __builtin_bit_cast(float, w[p] & 0xFFFF0000u);
+	}
 }
-// the upper halves of two words, the first below
-__device__ __forceinline__ unsigned upper_halves(unsigned lo, unsigned hi) { return __builtin_amdgcn_perm(hi, lo, 0x07060302u); }
 
 constexpr int kSplitQueries = 128, kSplitKeys = 32;
 constexpr int64_t kSplitMaskStride = 1 << 22;   // mask rows at most this far apart: byte offsets in a query block fit 32 bits
@@ -549,8 +556,9 @@ __device__ __forceinline__ bool any_of_block(bool said, char* const lds, int wav
 }
 
 // A query block of 128 with every product of floats as six products of bf16 parts on v_mfma_f32_32x32x16_bf16, accumulated in fp32:
-// x y = x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1; the terms left out are below 2^-23 of x y.
-// False, with nothing stored, where a result is not finite (the parts of an infinity are no numbers): the caller takes the form above.
+// x y = x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1; the terms left out are below 2^-24 of x y.
+// False, with nothing stored, where a result is not finite (the parts of an infinity, and of the floats that round to one, are no numbers): the
+// caller takes the form above.
 template <int D, bool SOFTCAP, bool MASK>
 __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* const lds, int bh, int q_block, int t_first, int t_last,
                                                  const unsigned long long* __restrict__ map_row, float* partial)
@@ -592,11 +600,10 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 #pragma unroll
 		for (int e = 0; e < 8; e += 2)
 		{
-			unsigned lo[3], hi[3];
-			split_bits(x[e / 4][e % 4], lo[0], lo[1], lo[2]);
-			split_bits(x[e / 4][e % 4 + 1], hi[0], hi[1], hi[2]);
+			unsigned parts[3];
+			split_pair(x[e / 4][e % 4], x[e / 4][e % 4 + 1], parts);
 #pragma unroll
-			for (int p = 0; p < 3; ++p) w[p][e / 2] = upper_halves(lo[p], hi[p]);
+			for (int p = 0; p < 3; ++p) w[p][e / 2] = parts[p];
 		}
 #pragma unroll
 		for (int p = 0; p < 3; ++p) qf[p][s] = __builtin_bit_cast(bf16x8_t, w[p]);
@@ -630,11 +637,11 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 		const int idx = tid + THREADS * i;
 		const int pitch = of_v ? L::kPitchV : L::kPitchK, plane = of_v ? L::kPlaneV : L::kPlaneK;
 		char* const dst = lds + (of_v ? 3 * L::kPlaneK : 0) + (idx / VPR) * pitch + (idx % VPR) * 8;
-		unsigned b[4][3];
+		unsigned parts[2][3];
+		split_pair(staged[i][0], staged[i][1], parts[0]);
+		split_pair(staged[i][2], staged[i][3], parts[1]);
 #pragma unroll
-		for (int e = 0; e < 4; ++e) split_bits(staged[i][e], b[e][0], b[e][1], b[e][2]);
-#pragma unroll
-		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{upper_halves(b[0][p], b[1][p]), upper_halves(b[2][p], b[3][p])};
+		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{parts[0][p], parts[1][p]};
 	};
 
 	// MASK: the mask values of this lane's scores, keys 8 j + 4 h .. + 3 of the tile: four consecutive floats at any alignment, as they come.
@@ -778,11 +785,10 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 				const float p0 = fast_exp2(s[8 * u + j] - m_safe), p1 = fast_exp2(s[8 * u + j + 1] - m_safe);
 				psum[0] += p0;
 				psum[1] += p1;
-				unsigned lo[3], hi[3];
-				split_bits(p0, lo[0], lo[1], lo[2]);
-				split_bits(p1, hi[0], hi[1], hi[2]);
+				unsigned parts[3];
+				split_pair(p0, p1, parts);
 #pragma unroll
-				for (int p = 0; p < 3; ++p) w[p][j / 2] = upper_halves(lo[p], hi[p]);
+				for (int p = 0; p < 3; ++p) w[p][j / 2] = parts[p];
 			}
 #pragma unroll
 			for (int p = 0; p < 3; ++p) pf[p][u] = __builtin_bit_cast(bf16x8_t, w[p]);
@@ -890,11 +896,10 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 #pragma unroll
 		for (int e = 0; e < 8; e += 2)
 		{
-			unsigned lo[3], hi[3];
-			split_bits(x[e / 4][e % 4], lo[0], lo[1], lo[2]);
-			split_bits(x[e / 4][e % 4 + 1], hi[0], hi[1], hi[2]);
+			unsigned parts[3];
+			split_pair(x[e / 4][e % 4], x[e / 4][e % 4 + 1], parts);
 #pragma unroll
-			for (int p = 0; p < 3; ++p) w[p][e / 2] = upper_halves(lo[p], hi[p]);
+			for (int p = 0; p < 3; ++p) w[p][e / 2] = parts[p];
 		}
 #pragma unroll
 		for (int p = 0; p < 3; ++p) qf[p][s] = __builtin_bit_cast(bf16x8_t, w[p]);
@@ -926,11 +931,11 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 		const int idx = tid + THREADS * i;
 		const int pitch = of_v ? L::kPitchV : L::kPitchK, plane = of_v ? L::kPlaneV : L::kPlaneK;
 		char* const dst = lds + (of_v ? 3 * L::kPlaneK : 0) + (idx / VPR) * pitch + (idx % VPR) * 8;
-		unsigned b[4][3];
+		unsigned parts[2][3];
+		split_pair(staged[i][0], staged[i][1], parts[0]);
+		split_pair(staged[i][2], staged[i][3], parts[1]);
 #pragma unroll
-		for (int e = 0; e < 4; ++e) split_bits(staged[i][e], b[e][0], b[e][1], b[e][2]);
-#pragma unroll
-		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{upper_halves(b[0][p], b[1][p]), upper_halves(b[2][p], b[3][p])};
+		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{parts[0][p], parts[1][p]};
 	};
 
 	// MASK: the mask values of this lane's scores, keys 16 j + 4 g .. + 3 of the tile: four consecutive floats at any alignment, as they come.
@@ -1068,11 +1073,10 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 			const float p0 = fast_exp2(z[j] - m_safe), p1 = fast_exp2(z[j + 1] - m_safe);
 			psum[0] += p0;
 			psum[1] += p1;
-			unsigned lo[3], hi[3];
-			split_bits(p0, lo[0], lo[1], lo[2]);
-			split_bits(p1, hi[0], hi[1], hi[2]);
+			unsigned parts[3];
+			split_pair(p0, p1, parts);
 #pragma unroll
-			for (int p = 0; p < 3; ++p) w[p][j / 2] = upper_halves(lo[p], hi[p]);
+			for (int p = 0; p < 3; ++p) w[p][j / 2] = parts[p];
 		}
 #pragma unroll
 		for (int p = 0; p < 3; ++p) pf[p] = __builtin_bit_cast(bf16x8_t, w[p]);

@@ -292,7 +292,7 @@ int anygpu_sdp_attention_fwd_f16(const void* q, const void* k, const void* v, vo
 
 /*
  * anygpu_sdp_attention_fwd_f16 in float32: operands, scores, sums and output are fp32.  A product of floats is six products
- * of their bf16 parts, summed in fp32 (what is left out lies below 2^-23 of it), small launches and results that are not finite
+ * of their bf16 parts, summed in fp32 (what is left out lies below 2^-24 of it, of either sign), small launches and results that are not finite
  * run on the fp32 matrix instruction; results agree with the unfused float32 path to fp32 rounding.  Same arguments and rules.  Replaces cu_flash_sdpa_fwd_d256_v1 (srcs/kernels/cuda/flash_sdpa_fwd.cuh:6-15: one head, head_dim 256,
  * no mask; here any number of heads, head_dim 64 / 128 / 256, the index-rule masks) and, for masks that are
  * index rules, the per-head loop of sdp_attention_masked_scaled_fwd (srcs/transformers/sdp.hpp:258-271).

@@ -11,7 +11,7 @@ from test_gpu_parity import dev, host
 
 pytestmark = pytest.mark.gpu
 
-# A product of two floats as six products of their parts is off by 3 x 2^-24 at most, fp32 sums of some thousand of them by 1e-6 of the terms' norm; the
+# A product of two floats as six products of their parts is off by 2^-24 at most, fp32 sums of some thousand of them by 1e-6 of the terms' norm; the
 # softcap's tanh from exp2 and a reciprocal by 2e-6 of the cap.
 TOL = 1e-5
 
@@ -54,6 +54,28 @@ def test_attention_f32_in_bf16_parts(ops, d, heads, kv, n_q, n_k, softcap, causa
     want = attend64(q[0], k[0], v[0], alpha, softcap, hidden_keys(n_q, n_k, causal, window))
     assert scaled_rel_err(got, want, 1.0) <= TOL
     assert not got[want.any(axis=-1) == 0].any()
+
+
+@pytest.mark.parametrize("d,heads", [(64, 24), (128, 10), (256, 3)])
+def test_attention_f32_in_bf16_parts_of_like_mantissas(ops, monkeypatch, d, heads):
+    # products that all leave out what they can with one sign: no further from float64 than on the fp32 instruction, to a seventh
+    n = 800
+    rng = np.random.default_rng(d)
+
+    def alike():
+        exponent_and_sign = rng.integers(126, 129, (heads, n, d)) << 23 | rng.integers(0, 2, (heads, n, d)) << 31
+        return (exponent_and_sign | 0x00FFFF).astype(np.uint32).view(np.float32)
+    q, k, v = alike(), alike(), alike()
+    args = [dev(t[None]) for t in (q, k, v)]
+    mask = np.zeros((1, 1, n, n), dtype=np.float32)
+    want = attend64(q, k, v, d ** -0.5)
+
+    def err(y):
+        return np.linalg.norm(host(y)[0] - want) / np.linalg.norm(want)
+    rules, masked = err(ops.sdp_attention_fwd(*args, d ** -0.5, decode=False)), err(ops.sdp_attention_masked_scaled_fwd(*args, dev(mask), d ** -0.5))
+    monkeypatch.setenv("ANYGPU_ATTN_MASK_MAP_FROM", str(1 << 60))
+    plain = err(ops.sdp_attention_masked_scaled_fwd(*args, dev(mask), d ** -0.5))
+    assert max(rules, masked) <= 1.15 * plain
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
