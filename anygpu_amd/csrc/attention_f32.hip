@@ -507,11 +507,10 @@ typedef short short4_t __attribute__((ext_vector_type(4)));
 // Two floats as sums of three bf16 each: the float rounded to nearest, what is left rounded likewise, and the rest, at most 2^-9, 2^-18 of the
 // power of two below the float (8 bits each with their own signs, which together are all of its 24 bits).  Word p of w: part p of both, the
 // first below.  Cut-off parts, twice as large and all of the float's sign, left 4.7e-7 of a product out of the six below, always
-// towards zero; these 5.9e-8 (2^-24) at most and 5.3e-9 (root mean square over all mantissas) of either sign.  (What is left below 2^-133, the smallest
-// bf16, is lost: of floats below 2^-110.)
-__device__ __forceinline__ void split_pair(float lo, float hi, unsigned (&w)[3])
+// towards zero; these 5.9e-8 (2^-24) at most and 5.3e-9 (root mean square over all mantissas) of either sign.
+// Returned: what stands in the last part.  What lies below 2^-133 of it, the smallest bf16, is lost, of floats below 2^-110 (RestBits).
+__device__ __forceinline__ float2_t split_pair(float lo, float hi, unsigned (&w)[3])
 {
-	typedef float float2_t __attribute__((ext_vector_type(2)));
 	typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 #pragma unroll
 	for (int p = 0; p < 3; ++p)
@@ -521,7 +520,17 @@ __device__ __forceinline__ void split_pair(float lo, float hi, unsigned (&w)[3])
 		lo -= __builtin_bit_cast(float, w[p] << 16);
 		hi -= __builtin_bit_cast(float, w[p] & 0xFFFF0000u);
 	}
+	return float2_t{lo, hi};
 }
+
+// Whether parts have lost bits: the lower half of a last part's float is zero unless it has bits below the smallest bf16.
+struct RestBits
+{
+	unsigned bits = 0;
+	// (as an expression of its own it kept the last parts of a whole tile in registers)
+	__device__ __forceinline__ void take(float2_t rest) { asm("v_or3_b32 %0, %1, %2, %0" : "+v"(bits) : "v"(rest[0]), "v"(rest[1])); }
+	__device__ __forceinline__ bool lost() const { return (bits & 0xFFFFu) != 0; }
+};
 
 constexpr int kSplitQueries = 128, kSplitKeys = 32;
 constexpr int64_t kSplitMaskStride = 1 << 22;   // mask rows at most this far apart: byte offsets in a query block fit 32 bits
@@ -557,8 +566,8 @@ __device__ __forceinline__ bool any_of_block(bool said, char* const lds, int wav
 
 // A query block of 128 with every product of floats as six products of bf16 parts on v_mfma_f32_32x32x16_bf16, accumulated in fp32:
 // x y = x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1; the terms left out are below 2^-24 of x y.
-// False, with nothing stored, where a result is not finite (the parts of an infinity, and of the floats that round to one, are no numbers): the
-// caller takes the form above.
+// False, with nothing stored, where a result is not finite (the parts of an infinity, and of the floats that round to one, are no numbers) or
+// the parts of an operand have lost bits: the caller takes the form above.
 template <int D, bool SOFTCAP, bool MASK>
 __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* const lds, int bh, int q_block, int t_first, int t_last,
                                                  const unsigned long long* __restrict__ map_row, float* partial)
@@ -587,6 +596,7 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 	const int wq0 = q0 + 32 * wave;
 	const int q_row = wq0 + n;
 	bf16x8_t qf[3][KS];
+	RestBits rest;                                  // of q, k and v (weights below 2^-110 of the row's largest may lose bits)
 #pragma unroll
 	for (int s = 0; s < KS; ++s)
 	{
@@ -601,7 +611,7 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 		for (int e = 0; e < 8; e += 2)
 		{
 			unsigned parts[3];
-			split_pair(x[e / 4][e % 4], x[e / 4][e % 4 + 1], parts);
+			rest.take(split_pair(x[e / 4][e % 4], x[e / 4][e % 4 + 1], parts));
 #pragma unroll
 			for (int p = 0; p < 3; ++p) w[p][e / 2] = parts[p];
 		}
@@ -638,8 +648,8 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 		const int pitch = of_v ? L::kPitchV : L::kPitchK, plane = of_v ? L::kPlaneV : L::kPlaneK;
 		char* const dst = lds + (of_v ? 3 * L::kPlaneK : 0) + (idx / VPR) * pitch + (idx % VPR) * 8;
 		unsigned parts[2][3];
-		split_pair(staged[i][0], staged[i][1], parts[0]);
-		split_pair(staged[i][2], staged[i][3], parts[1]);
+		rest.take(split_pair(staged[i][0], staged[i][1], parts[0]));
+		rest.take(split_pair(staged[i][2], staged[i][3], parts[1]));
 #pragma unroll
 		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{parts[0][p], parts[1][p]};
 	};
@@ -825,7 +835,7 @@ __device__ __forceinline__ bool attend_f32_split(const AttnArgsF32& a, char* con
 	for (int c = 0; c < DC; ++c)
 #pragma unroll
 		for (int i = 0; i < 16; ++i) all = fmaf(o[c][i], 0.0f, all);
-	if (any_of_block<THREADS / kWaveSize>(!(fabsf(all) < INFINITY), lds, wave)) return false;
+	if (any_of_block<THREADS / kWaveSize>(rest.lost() || !(fabsf(all) < INFINITY), lds, wave)) return false;
 	if (q_row >= a.n_q) return true;
 	if (partial != nullptr)
 	{
@@ -883,6 +893,7 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 	const int wq0 = q0 + 16 * wave;
 	const int q_row = wq0 + n;
 	bf16x8_t qf[3][KS];
+	RestBits rest;                                  // of q, k and v (weights below 2^-110 of the row's largest may lose bits)
 #pragma unroll
 	for (int s = 0; s < KS; ++s)
 	{
@@ -897,7 +908,7 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 		for (int e = 0; e < 8; e += 2)
 		{
 			unsigned parts[3];
-			split_pair(x[e / 4][e % 4], x[e / 4][e % 4 + 1], parts);
+			rest.take(split_pair(x[e / 4][e % 4], x[e / 4][e % 4 + 1], parts));
 #pragma unroll
 			for (int p = 0; p < 3; ++p) w[p][e / 2] = parts[p];
 		}
@@ -932,8 +943,8 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 		const int pitch = of_v ? L::kPitchV : L::kPitchK, plane = of_v ? L::kPlaneV : L::kPlaneK;
 		char* const dst = lds + (of_v ? 3 * L::kPlaneK : 0) + (idx / VPR) * pitch + (idx % VPR) * 8;
 		unsigned parts[2][3];
-		split_pair(staged[i][0], staged[i][1], parts[0]);
-		split_pair(staged[i][2], staged[i][3], parts[1]);
+		rest.take(split_pair(staged[i][0], staged[i][1], parts[0]));
+		rest.take(split_pair(staged[i][2], staged[i][3], parts[1]));
 #pragma unroll
 		for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2_t*>(dst + p * plane) = uint2_t{parts[0][p], parts[1][p]};
 	};
@@ -1111,7 +1122,7 @@ __device__ __forceinline__ bool attend_f32_split16(const AttnArgsF32& a, char* c
 	for (int c = 0; c < DC; ++c)
 #pragma unroll
 		for (int r = 0; r < 4; ++r) all = fmaf(o[c][r], 0.0f, all);
-	if (any_of_block<THREADS / kWaveSize>(!(fabsf(all) < INFINITY), lds, wave)) return false;
+	if (any_of_block<THREADS / kWaveSize>(rest.lost() || !(fabsf(all) < INFINITY), lds, wave)) return false;
 	if (q_row >= a.n_q) return true;
 	if (partial != nullptr)
 	{

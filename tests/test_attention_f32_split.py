@@ -15,6 +15,7 @@ HARNESS = r"""
 #include <random>
 #define __device__
 #define __forceinline__ inline
+typedef float float2_t __attribute__((ext_vector_type(2)));
 %s
 static std::mt19937_64 rng(1);
 static float from_bits(uint32_t b) { return __builtin_bit_cast(float, b); }
@@ -72,7 +73,7 @@ int main()
 
 def test_bf16_parts_of_floats(tmp_path):
     text = (REPO / "anygpu_amd" / "csrc" / "attention_f32.hip").read_text()
-    begin = text.index("__device__ __forceinline__ void split_pair(")
+    begin = text.index("__device__ __forceinline__ float2_t split_pair(")
     src, exe = tmp_path / "parts_check.cpp", tmp_path / "parts_check"
     src.write_text(HARNESS % text[begin:text.index("\n}\n", begin) + 3])
     subprocess.run([str(build.ROCM_DIR / "lib" / "llvm" / "bin" / "clang++"), "-O2", "-std=c++20", "-o", str(exe), str(src)], check=True)

@@ -78,6 +78,36 @@ def test_attention_f32_in_bf16_parts_of_like_mantissas(ops, monkeypatch, d, head
     assert max(rules, masked) <= 1.15 * plain
 
 
+@pytest.mark.parametrize("d,heads", [(64, 24), (128, 10), (256, 3)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_f32_in_bf16_parts_of_small_operands(ops, d, heads, masked):
+    # floats below 2^-110 have parts below the smallest bf16: blocks that hold one keep the precision of float32 all the same (fp32 sums: 1e-6), and
+    # the other heads keep their bits.  Normal floats all of them: magnitudes from one to two times a power of two.
+    n = 800
+    q, k, v = (synth.normal(s, (heads, n, d)) for s in (1, 2, 3))
+    k, v = (np.sign(t) * (1 + np.abs(t) % 1) for t in (k, v))
+    mask = np.zeros((1, 1, n, n), dtype=np.float32)
+
+    def run(*qkv):
+        args = [dev(t.astype(np.float32)[None]) for t in qkv]
+        return host(ops.sdp_attention_masked_scaled_fwd(*args, dev(mask), d ** -0.5) if masked else ops.sdp_attention_fwd(*args, d ** -0.5, decode=False))[0]
+
+    def small(t, exponent):
+        t = t.copy()
+        t[0] = np.ldexp(t[0], exponent)
+        return t.astype(np.float32)
+    base, want = run(q, k, v), attend64(q[:1].astype(np.float32), k[:1].astype(np.float32), v[:1].astype(np.float32), d ** -0.5)
+    for exponent in (-110, -112, -118, -125):
+        for at, got in ((exponent, run(q, k, small(v, exponent))), (0, run(small(q, -exponent), small(k, exponent), v)), (0, run(small(q, exponent), small(k, -exponent), v))):
+            assert np.array_equal(got[1:], base[1:])
+            got = np.ldexp(got[0].astype(np.float64), -at)
+            if at == 0 or exponent > -118:
+                assert np.linalg.norm(got - want) <= 2e-6 * np.linalg.norm(want), exponent
+            else:
+                # (results here are floats below the smallest normal one: half a step of 2^-149 each)
+                assert np.all(np.abs(got - want) <= 1e-5 * np.abs(want).max() + 2.0 ** (-150 - at)), exponent
+
+
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("masked", [False, True])
 def test_attention_f32_in_bf16_parts_of_values_without_parts(ops, d, masked):
