@@ -448,15 +448,11 @@ __device__ __forceinline__ void attend_f32(const AttnArgsF32& a, float* const ld
 	}
 }
 
-// Which head and query block this block works on, the key tiles of it, and where a partial result goes (NULL: y).  False: a padding block.
-template <int D, int QUERIES, int KT, bool MASK>
-__device__ __forceinline__ bool attention_block_f32(const AttnArgsF32& a, const AttnWalk& walk, int& bh, int& q_block, int& t_first, int& t_last,
-                                                    const unsigned long long*& map_row, float*& partial)
+// The key tiles that some query of a block of QUERIES sees under the index rules: from the first key of its first query to the last of its last.
+template <int QUERIES, int KT>
+__device__ __forceinline__ void visible_tiles_f32(const AttnArgsF32& a, int q_block, int& t_first, int& t_last)
 {
-	int part, parts, split_slot;
-	if (!attn_walk_locate_part(walk, blockIdx.x, bh, q_block, part, parts, split_slot)) return false;
 	const int q0 = q_block * QUERIES;
-	// visible key range of the whole block: from the first key of its first query to the last of its last
 	const int q_last = (q0 + QUERIES - 1 < a.n_q ? q0 + QUERIES - 1 : a.n_q - 1);
 	int key_hi = a.n_k - 1;
 	if (a.causal && q_last + a.diag < key_hi) key_hi = q_last + a.diag;
@@ -464,6 +460,16 @@ __device__ __forceinline__ bool attention_block_f32(const AttnArgsF32& a, const 
 	if (a.window > 0 && q0 + a.diag - a.window + 1 > 0) key_lo = q0 + a.diag - a.window + 1;
 	t_first = key_lo / KT;
 	t_last = key_hi >= 0 ? key_hi / KT : -1;
+}
+
+// Which head and query block this block works on, the key tiles of it, and where a partial result goes (NULL: y).  False: a padding block.
+template <int D, int QUERIES, int KT, bool MASK>
+__device__ __forceinline__ bool attention_block_f32(const AttnArgsF32& a, const AttnWalk& walk, int& bh, int& q_block, int& t_first, int& t_last,
+                                                    const unsigned long long*& map_row, float*& partial)
+{
+	int part, parts, split_slot;
+	if (!attn_walk_locate_part(walk, blockIdx.x, bh, q_block, part, parts, split_slot)) return false;
+	visible_tiles_f32<QUERIES, KT>(a, q_block, t_first, t_last);
 	// MASK: the visible-tile map of the mask, where the launcher has made one: the words of this query block
 	map_row = nullptr;
 	if constexpr (MASK)
@@ -1161,7 +1167,16 @@ __global__ __launch_bounds__(split_threads(D, MASK), 2) void sdp_attention_fwd_f
 		for (int i = 0; i < kHalves; ++i)
 		{
 			__syncthreads();
-			attend_f32<D, SOFTCAP, kWaves, kSplitKeys, D == 256, MASK>(a, reinterpret_cast<float*>(lds_raw), bh, kHalves * q_block + i, t_first, t_last, map_row,
+			// (a value that is not finite reaches every query of a block whose tiles hold its key: those of each half, as where blocks have 64 queries)
+			int first = t_first, last = t_last;
+			if constexpr (kHalves > 1 && !MASK)
+			{
+				int of_half_first, of_half_last;
+				visible_tiles_f32<16 * kWaves, kSplitKeys>(a, kHalves * q_block + i, of_half_first, of_half_last);
+				first = max(first, of_half_first);
+				last = min(last, of_half_last);
+			}
+			attend_f32<D, SOFTCAP, kWaves, kSplitKeys, D == 256, MASK>(a, reinterpret_cast<float*>(lds_raw), bh, kHalves * q_block + i, first, last, map_row,
 			                                                           partial ? partial + i * (16 * kWaves) * (D + 2) : nullptr);
 		}
 	};

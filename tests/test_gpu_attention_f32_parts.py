@@ -145,6 +145,24 @@ def test_attention_f32_in_bf16_parts_of_values_without_parts(ops, d, masked):
     assert scaled_rel_err(got * 2.0 ** -100, base, 1.0) <= TOL
 
 
+@pytest.mark.parametrize("d,block", [(64, 64), (128, 64), (256, 128)])
+@pytest.mark.parametrize("heads,window", [(2, 0), (2, 200), (50, 0)])
+def test_attention_f32_value_that_is_not_finite_reaches_its_query_block(ops, d, block, heads, window):
+    # the queries that see its key, and of those that the rules hide it from at most the rest of a block of 64 (head dimension 256: 128): the blocks of the fp32 instruction
+    n, key = 800, 485
+    q, k, v = (synth.normal(s, (1, heads, n, d)) for s in (1, 2, 3))
+    v[0, 0, key, 5], v[0, 1, key] = math.nan, math.inf
+    got = host(ops.sdp_attention_fwd(dev(q), dev(k), dev(v), d ** -0.5, causal=True, window=window, decode=False))[0]
+    # (a block walks whole tiles: its last query that sees a key of the tile of 32 that holds this one, its first likewise)
+    tile = key // 32 * 32
+    first, last = tile // block * block, n if window == 0 else min(n, (tile + 31 + window - 1) // block * block + block)
+    for h, cols in ((0, [5]), (1, range(d))):
+        assert not np.isfinite(got[h][key:key + window or n, cols]).any()
+        assert np.isfinite(got[h][:first]).all() and np.isfinite(got[h][last:]).all()
+        assert np.isfinite(np.delete(got[h], cols, axis=1)).all()
+    assert np.isfinite(got[2:]).all()
+
+
 @pytest.mark.parametrize("heads,n_q,n_k,d,kind", [
     (1, 800, 801, 256, "causal"), (2, 1000, 600, 256, "bias"), (3, 780, 1300, 256, "blind blocks"), (1, 130, 5003, 256, "window"), (7, 775, 775, 256, "nothing"),
     (25, 900, 773, 128, "blind blocks"), (1, 300, 520, 256, "bias"), (9, 830, 1001, 128, "window"), (26, 790, 790, 64, "window"), (24, 1000, 700, 64, "bias"), (300, 800, 800, 256, "window"), (40, 770, 800, 128, "causal")])
