@@ -32,6 +32,9 @@ const at::Tensor* plain(PyObject* obj)
 	return &t;
 }
 
+// A result tensor that the caller brings: the operands' type and device.
+bool fits(const at::Tensor& out, const at::Tensor& like) { return out.scalar_type() == like.scalar_type() && out.device() == like.device(); }
+
 bool half_or_float(const at::Tensor& t) { return t.scalar_type() == at::kHalf || t.scalar_type() == at::kFloat; }
 
 bool as_int(PyObject* obj, int64_t* out)
@@ -114,7 +117,7 @@ PyObject* mm(PyObject*, PyObject* const* args, Py_ssize_t n_args)
 	else
 	{
 		const at::Tensor* given = plain(args[2]);
-		DECLINE_UNLESS(given && given->dim() == 2 && given->size(0) == m && given->size(1) == n && given->stride(1) == 1);
+		DECLINE_UNLESS(given && fits(*given, *a) && given->dim() == 2 && given->size(0) == m && given->size(1) == n && given->stride(1) == 1);
 		out = *given;
 	}
 	const int64_t lda = a->size(0) > 1 ? a->stride(0) : at_least_one(a->size(1));
@@ -215,7 +218,7 @@ PyObject* softmax(PyObject*, PyObject* const* args, Py_ssize_t n_args)
 	else
 	{
 		const at::Tensor* given = plain(args[1]);
-		DECLINE_UNLESS(given && given->dim() == 2 && given->size(0) == rows && given->size(1) == cols);
+		DECLINE_UNLESS(given && fits(*given, *x) && given->dim() == 2 && given->size(0) == rows && given->size(1) == cols && (given->stride(1) == 1 || cols <= 1));
 		out = *given;
 	}
 	const int64_t xs = rows > 1 ? x->stride(0) : at_least_one(cols), ys = rows > 1 ? out.stride(0) : at_least_one(cols);

@@ -46,6 +46,12 @@ def _check_device(*tensors: torch.Tensor) -> None:
         _require(t.is_cuda, "anygpu ops take device tensors only (no CPU fallback)")
 
 
+def _check_out(out: torch.Tensor, like: torch.Tensor) -> None:
+    """A result tensor that the caller brings: the kernels write it as elements of the operands' type in their memory."""
+    _check_device(out)
+    _require(out.dtype == like.dtype and out.device == like.device, "the result needs the operands' dtype and device")
+
+
 def set_workspace(workspace: torch.Tensor | None, stream: torch.cuda.Stream | None = None) -> None:
     """Hand the GEMM entry points a caller-owned K-split workspace for `stream` (default: the current stream), or take
     it back with None.  The tensor must stay alive while launches or graphs that used it can still run."""
@@ -86,6 +92,7 @@ def tensor_mm(lhs: torch.Tensor, rhs: torch.Tensor, out: torch.Tensor | None = N
         n = rhs.shape[0]
     if out is None:
         out = torch.empty((m, n), dtype=lhs.dtype, device=lhs.device)
+    _check_out(out, lhs)
     _require(tuple(out.shape) == (m, n) and out.stride(1) == 1, "result mtx shape is wrong")
     lib = capi.load()
     lda = lhs.stride(0) if lhs.shape[0] > 1 else max(lhs.shape[1], 1)
@@ -199,7 +206,9 @@ def tensor_softmax(x: torch.Tensor, out: torch.Tensor | None = None, *, alpha: f
     rows, cols = x.shape
     if out is None:
         out = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
+    _check_out(out, x)
     _require(tuple(out.shape) == (rows, cols), "result shape is wrong")
+    _require(out.stride(1) == 1 or cols <= 1, "rows must be contiguous")
     xs = x.stride(0) if rows > 1 else max(cols, 1)
     ys = out.stride(0) if rows > 1 else max(cols, 1)
     lib = capi.load()
@@ -230,6 +239,8 @@ def tensor_causal_conv1d(xt: torch.Tensor, wt: torch.Tensor, bt: torch.Tensor,
     _require(xt.is_contiguous() and wt.is_contiguous() and bt.is_contiguous(), "dense operands expected")
     if out is None:
         out = torch.empty_like(xt)
+    _check_out(out, xt)
+    _require(tuple(out.shape) == tuple(xt.shape) and out.is_contiguous(), "result shape is wrong")
     b, d, s = xt.shape
     lib = capi.load()
     if xt.dtype == torch.float16:

@@ -97,3 +97,24 @@ def test_native_calls_decline_what_they_do_not_check(ops):
     # the C ABI's own refusal comes back as the package's error
     with pytest.raises(capi.AnyGpuError):
         native.softmax(a, None, 1.0, 0.0, False, -1, 0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,other", [("float32", "float16"), ("float16", "float32"), ("float32", "int32")])
+def test_results_of_another_type_or_layout_are_refused(ops, dtype, other):
+    # elements of the operands' type would run past the end of a narrower result, rows of a transposed one over each other
+    import torch
+    from anygpu_amd import capi
+    native = capi.load_torch_calls()
+    dtype, other = getattr(torch, dtype), getattr(torch, other)
+    a, b, x = torch.zeros(4, 8, dtype=dtype, device="cuda"), torch.zeros(8, 6, dtype=dtype, device="cuda"), torch.zeros(2, 3, 8, dtype=dtype, device="cuda")
+    mm_out, rows_out, conv_out = (torch.full(shape, 7, dtype=other, device="cuda") for shape in ((4, 6), (4, 8), (2, 3, 8)))
+    w, bias = torch.zeros(3, 4, dtype=dtype, device="cuda"), torch.zeros(3, dtype=dtype, device="cuda")
+    turned, turned_conv = torch.full((8, 4), 7, dtype=dtype, device="cuda").T, torch.full((2, 8, 3), 7, dtype=dtype, device="cuda").transpose(1, 2)
+    assert native.mm(a, b, mm_out, 0, 0) is None and native.softmax(a, rows_out, 1.0, 0.0, False, 0, 0, 0) is None
+    assert native.softmax(a, turned, 1.0, 0.0, False, 0, 0, 0) is None
+    for call in (lambda: ops.tensor_mm(a, b, out=mm_out), lambda: ops.tensor_softmax(a, out=rows_out), lambda: ops.tensor_softmax(a, out=turned), lambda: ops.tensor_mm(a, b, out=mm_out.cpu()),
+                 lambda: ops.tensor_softmax(a, out=rows_out.cpu()), lambda: ops.tensor_causal_conv1d(x, w, bias, out=conv_out), lambda: ops.tensor_causal_conv1d(x, w, bias, out=turned_conv)):
+        with pytest.raises(ValueError):
+            call()
+    assert all(bool((t == 7).all()) for t in (mm_out, rows_out, conv_out, turned, turned_conv))
