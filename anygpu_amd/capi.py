@@ -145,10 +145,10 @@ def check(fn: str, code: int) -> None:
 
 
 def load_torch_calls():
-    """The extension module behind ops.py (csrc/torch_calls.cpp).  Raises if it is not built."""
+    """The extension module behind ops.py (csrc/torch_calls.cpp).  Raises ImportError if it is not built, or built against another torch."""
     load()
     if not TORCH_CALLS_PATH.exists():
-        raise RuntimeError(f"{TORCH_CALLS_PATH} is not built; run `python anygpu_amd/build.py` first.")
+        raise ImportError(f"{TORCH_CALLS_PATH} is not built; run `python anygpu_amd/build.py` first.")
     import importlib.util
     spec = importlib.util.spec_from_file_location("_torch_calls", TORCH_CALLS_PATH)
     module = importlib.util.module_from_spec(spec)

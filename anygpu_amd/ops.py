@@ -8,6 +8,8 @@ additional keyword arguments the C ABI carries.
 """
 from __future__ import annotations
 
+import warnings
+
 import torch
 
 from . import capi
@@ -15,12 +17,25 @@ from . import capi
 _native = None
 
 
+class _NoNativeCalls:
+    """Stands in where the extension module cannot be loaded: every call is left to the Python below it."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _calls():
     """The native callers (csrc/torch_calls.cpp).  Each returns None for anything but plain dense device tensors that fit: the Python below
-    it then checks in full, and raises or makes the call itself."""
+    it then checks in full, and raises or makes the call itself.  Without the module, or with one built against another torch, the
+    same kernels are called through ctypes, 2 - 3 us later."""
     global _native
     if _native is None:
-        _native = capi.load_torch_calls()
+        capi.load()
+        try:
+            _native = capi.load_torch_calls()
+        except ImportError as err:
+            warnings.warn(f"anygpu ops call the kernels through ctypes: {err}", RuntimeWarning, stacklevel=3)
+            _native = _NoNativeCalls()
     return _native
 
 

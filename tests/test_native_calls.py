@@ -118,3 +118,23 @@ def test_results_of_another_type_or_layout_are_refused(ops, dtype, other):
         with pytest.raises(ValueError):
             call()
     assert all(bool((t == 7).all()) for t in (mm_out, rows_out, conv_out, turned, turned_conv))
+
+
+@pytest.mark.parametrize("content", [None, b"not a library"])
+def test_without_the_extension_module_the_python_path_calls_the_library(monkeypatch, tmp_path, content):
+    import torch
+    from anygpu_amd import capi, ops
+    path = tmp_path / "_torch_calls.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(capi, "TORCH_CALLS_PATH", path)
+    monkeypatch.setattr(ops, "_native", None)
+    a = torch.zeros(2, 2)
+    with pytest.warns(RuntimeWarning, match="ctypes"), pytest.raises(ValueError, match="device tensors only"):
+        ops.tensor_mm(a, a)
+    with pytest.raises(ValueError, match="device tensors only"):         # (the warning comes once)
+        ops.tensor_softmax(a)
+    monkeypatch.setattr(capi, "load", lambda: (_ for _ in ()).throw(RuntimeError("no library")))
+    monkeypatch.setattr(ops, "_native", None)
+    with pytest.raises(RuntimeError, match="no library"):                # there is no way around the library itself
+        ops.tensor_mm(a, a)
