@@ -4,12 +4,13 @@ CPU oracle used by the tests (gcc, through oracle/Makefile).
 
 Everything is built in-tree so that the shared objects travel with the source tree:
     anygpu_amd/lib/libanygpu_hip.so     kernels + C ABI (include/anygpu_hip.h)
-    anygpu_amd/lib/_torch_calls.so      the native callers behind ops.py (extension module)
+    anygpu_amd/lib/_torch_calls.so      the native callers behind ops.py (extension module; where torch is installed)
     anygpu_amd/lib/anygpu_host_tests    reference-style C++ test harness over Tensor<dtype, device>
     oracle/liboracle.so                 CPU oracle (test infrastructure)
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -132,11 +133,14 @@ def build_oracle(verbose: bool = False) -> Path:
 
 
 def build_all(verbose: bool = False) -> dict[str, str]:
-    built = {"kernels": str(build_kernels(verbose)), "torch_calls": str(build_torch_calls(verbose))}
+    built = {"kernels": str(build_kernels(verbose))}
     harness = build_host_harness(verbose)
     if harness is not None:
         built["host_harness"] = str(harness)
     built["oracle"] = str(build_oracle(verbose))
+    # (last, and only where torch is: the C ABI and the host layer do not need it)
+    if importlib.util.find_spec("torch") is not None:
+        built["torch_calls"] = str(build_torch_calls(verbose))
     return built
 
 

@@ -138,3 +138,15 @@ def test_without_the_extension_module_the_python_path_calls_the_library(monkeypa
     monkeypatch.setattr(ops, "_native", None)
     with pytest.raises(RuntimeError, match="no library"):                # there is no way around the library itself
         ops.tensor_mm(a, a)
+
+
+def test_everything_but_the_extension_module_is_built_without_torch(monkeypatch):
+    import importlib.util
+
+    from anygpu_amd import build
+    for name in ("build_kernels", "build_host_harness", "build_oracle", "build_torch_calls"):
+        monkeypatch.setattr(build, name, lambda verbose, name=name: name)
+    assert list(build.build_all().values()) == ["build_kernels", "build_host_harness", "build_oracle", "build_torch_calls"]
+    find = importlib.util.find_spec
+    monkeypatch.setattr(importlib.util, "find_spec", lambda name, *rest: None if name == "torch" else find(name, *rest))
+    assert list(build.build_all().values()) == ["build_kernels", "build_host_harness", "build_oracle"]
