@@ -308,6 +308,14 @@ __device__ __forceinline__ float logit2_fast(float x, float k_in, float k_cap)
 // The softcap of softmax_rows_kernel.  The short form is off by 1.5e-7 of the cap in the logit, so by 1e-5 of a probability at a cap of 64, a
 // fiftieth of a half's rounding; beyond (halves) and for floats a form whose error vanishes with the logit.  2-norm error of halves, N(0, 16) scores,
 // short / full form: cap 50 1.98e-4 / 1.98e-4, 1000 1.88e-4 / 1.86e-4, 1e5 2.6e-3 / 1.9e-4.
+// Elements of the tensor in front of a row and behind it, as far as they can share a vector with it.  (Rows shorter than a vector, or on top of
+// each other in memory, have several rows in the tensor's first and last 16 bytes.)
+struct RowNeighbours { int before, behind; };
+__device__ __forceinline__ RowNeighbours row_neighbours(const SoftmaxArgs& a, int64_t row)
+{
+	return {(int)min(row * a.xs, (int64_t)8), (int)min((a.rows - 1 - row) * a.xs, (int64_t)8)};
+}
+
 // tanh below a sixteenth, to 4e-9 of it
 constexpr float kTanhNearZero = 0.0625f;
 __device__ __forceinline__ float tanh_near_zero(float x)
@@ -342,6 +350,7 @@ __global__ __launch_bounds__(GROUP > 256 ? GROUP : 256) void softmax_rows_kernel
 	const int end = shift + (int)a.cols;
 	const int lo = (int)span.lo + shift, hi = (int)span.hi + shift;
 	const int v_first = shift / EPV, v_end = (end - 1) / EPV;
+	const RowNeighbours near = row_neighbours(a, row);
 	const Vec zeros = {};
 	auto put = [&](int v, const Vec& val) {
 		const int from = shift - v * EPV, to = end - v * EPV;         // elements [from, to) of the vector are the row's
@@ -372,8 +381,7 @@ __global__ __launch_bounds__(GROUP > 256 ? GROUP : 256) void softmax_rows_kernel
 		Vec val = {};
 		if (v >= v_lo && v <= v_hi)
 		{
-			// (the first vector of the first row and the last of the last may reach past the tensor)
-			const int from = row == 0 ? shift - v * EPV : 0, to = row == a.rows - 1 ? end - v * EPV : EPV;
+			const int from = shift - v * EPV - near.before, to = end - v * EPV + near.behind;        // elements [from, to) of the vector are the tensor's
 			if (from <= 0 && to >= EPV) val = __builtin_nontemporal_load(xv + v);
 			else
 			{

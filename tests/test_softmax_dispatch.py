@@ -51,6 +51,15 @@ void softmax_rows_kernel(const SoftmaxArgs& a)
 		const int shift = (int)(y / sizeof(T) %% kStart);
 		const RowSpan span = row_span(a, row);
 		if (span.hi < span.lo) continue;
+		// a vector that holds elements of the row: those of its elements that are loaded are the tensor's, and all of the row's are among them
+		const RowNeighbours near = row_neighbours(a, row);
+		const int end = shift + (int)a.cols;
+		for (int v : {((int)span.lo + shift) / EPV, ((int)span.hi + shift) / EPV})
+		{
+			const int from = std::max(0, shift - v * EPV - near.before), to = std::min(EPV, end - v * EPV + near.behind);
+			const int64_t at = row * a.xs - shift + (int64_t)v * EPV, tensor = (a.rows - 1) * a.xs + a.cols;
+			if (at + from < 0 || at + to > tensor || from > std::max(0, shift - v * EPV) || to < std::min(EPV, end - v * EPV)) fail("outside", a, sizeof(T), VPL, GROUP);
+		}
 		const int c_lo = ((int)span.lo + shift) / EPV / GROUP, c_hi = ((int)span.hi + shift) / EPV / GROUP;
 		if (c_hi - c_lo + 1 > VPL) fail("capacity", a, sizeof(T), VPL, GROUP);
 	}
@@ -112,6 +121,7 @@ def test_softmax_kernels_are_picked_by_the_mask_and_hold_their_rows(tmp_path):
     text = (REPO / "anygpu_amd" / "csrc" / "softmax.hip").read_text()
     args = [_between(text, start, "\n}") + end for start, end in (("struct SoftmaxArgs", ";"), ("__device__ __forceinline__ int64_t query_of_row", ""),
                                                                   ("static inline unsigned blocks_for_rows", ""))]
+    args += [_between(text, "struct RowNeighbours", ";") + " };", _between(text, "__device__ __forceinline__ RowNeighbours row_neighbours", "\n}")]
     args += [_between(text, "struct RowSpan", ";") + " };", _between(text, "__device__ __forceinline__ RowSpan row_span", "\n}")]
     rule = [_between(text, start, "\n}") for start in ("static bool rows_alike", "template <typename T, int VPL, int GROUP>\nstatic hipError_t launch_rows",
                                                        "template <typename T>\nstatic int64_t rows_vectors", "template <typename T, int VPL, bool LOOSE = false, int GROUP = 64>",
