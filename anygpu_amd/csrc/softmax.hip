@@ -775,14 +775,14 @@ hipError_t launch_softmax_rows(const void* x, void* y, int64_t rows, int64_t col
 		softmax_rows_long_kernel<T><<<dim3(blocks_for_rows(a, 1)), dim3(1024), 0, stream>>>(a);
 		return hipGetLastError();
 	}
-	// (with a mask tensor, whose vectors sit in registers beside the row's, a wave takes up to 8 vectors per lane)
-	if (vec_ok && nvec <= (int64_t)kWaveSize * (mask ? 8 : kMaxVpl))
+	// (with a mask tensor, whose vectors sit in registers beside the row's, a wave takes up to 8 vectors per lane; aligned rows without one
+	// come here only where they just fill the block)
+	if (vec_ok && nvec <= (int64_t)kWaveSize * 8)
 	{
 		if (nvec <= kWaveSize * 1) return launch_wave<T, 1>(a, stream);
 		if (nvec <= kWaveSize * 2) return launch_wave<T, 2>(a, stream);
 		if (nvec <= kWaveSize * 4) return launch_wave<T, 4>(a, stream);
-		if (nvec <= kWaveSize * 8) return launch_wave<T, 8>(a, stream);
-		return launch_wave<T, 16>(a, stream);
+		return launch_wave<T, 8>(a, stream);
 	}
 	if (vec_ok && nvec <= (int64_t)256 * kMaxVpl) return launch_long_rows<T, false>(a, nvec, stream);
 	// rows at element alignment, any width: the same wave kernel with element-aligned vector accesses
