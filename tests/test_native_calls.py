@@ -120,6 +120,19 @@ def test_results_of_another_type_or_layout_are_refused(ops, dtype, other):
     assert all(bool((t == 7).all()) for t in (mm_out, rows_out, conv_out, turned, turned_conv))
 
 
+@pytest.mark.gpu
+def test_a_dense_convolution_result_of_another_shape_takes_the_samples_in_order(ops):
+    import torch
+    x, w, bias = (torch.arange(n, dtype=torch.float32, device="cuda").reshape(shape) / n for n, shape in ((2 * 9 * 64, (2, 9, 64)), (9 * 4, (9, 4)), (9, (9,))))
+    want = ops.tensor_causal_conv1d(x, w, bias)
+    flat, larger = torch.full((18 * 64,), 7.0, device="cuda"), torch.full((20, 64), 7.0, device="cuda")
+    assert ops.tensor_causal_conv1d(x, w, bias, out=flat) is flat and ops.tensor_causal_conv1d(x, w, bias, out=larger) is larger
+    assert torch.equal(flat.view(2, 9, 64), want) and torch.equal(larger[:18].view(2, 9, 64), want) and bool((larger[18:] == 7).all())
+    with pytest.raises(ValueError):
+        ops.tensor_causal_conv1d(x, w, bias, out=flat[:-1])
+    assert torch.equal(flat.view(2, 9, 64), want)
+
+
 @pytest.mark.parametrize("content", [None, b"not a library"])
 def test_without_the_extension_module_the_python_path_calls_the_library(monkeypatch, tmp_path, content):
     import torch
