@@ -452,10 +452,11 @@ def bench_softmax(torch, ops, synth, steps, warmup, cpu_seconds, *, name, heads,
     out = {
         "name": name, "workload": workload,
         **timing_fields(t), "value": dense / sec / 1e9, "unit": "GB/s", "dtype": "f16",
-        "roofline": {"bound": "hbm", "achieved": dense / sec / 1e9, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                     "frac": dense / sec / 1e9 / PEAK_HBM_GBS, **traffic_fields(key),
-                     "algorithmic_bytes": dense, "mask_aware_bytes": mask_aware,
-                     "mask_aware_gbs": mask_aware / sec / 1e9, "physical_gbs": MEASURED_TRAFFIC[key][0] / sec / 1e9},
+        # (hidden scores are not read: the roofline counts what is)
+        "roofline": {"bound": "hbm", "achieved": mask_aware / sec / 1e9, "peak": PEAK_HBM_GBS, "unit": "GB/s",
+                     "frac": mask_aware / sec / 1e9 / PEAK_HBM_GBS, **traffic_fields(key),
+                     "algorithmic_bytes": mask_aware, "dense_bytes": dense, "dense_gbs": dense / sec / 1e9,
+                     "physical_gbs": MEASURED_TRAFFIC[key][0] / sec / 1e9},
     }
     if cpu_seconds > 0:
         import oracle
