@@ -27,9 +27,9 @@
 // 5.9e-7 / 4.6e-7; all mantissas 0x00FFFF 6.2e-7 / 3.6e-7, 6.8e-7 / 4.6e-7, 5.1e-7 / 5.2e-7; all mantissas 0x007FC0, which lose the most, 5.6e-7 / 3.2e-7,
 // 5.7e-7 / 4.1e-7, 3.3e-7 / 6.4e-7.
 // K and V are cut into their parts on their way into LDS (three planes each, once per block), p in its registers.  Bound: the bf16 matrix rate (and
-// the power that goes with it).  us, before / now: 8 / 4 heads x 8192 x 256, softcap, window 4096 1801 / 1051 (196 TFLOP/s, so 1.18 PFLOP/s of bf16
-// products), 16 x 2000 x 128 324 / 185, 32 / 8 x 3000 x 128 causal 701 / 419, 32 x 2000 x 64 causal 180 / 122, 8 x 1000 x 256 79.6 / 59.1; with a mask tensor
-// 8 x 3001 x 256 causal 412 / 264, dense bias 738 / 420, 64 x 1393 x 128 causal 564 / 240.
+// the power that goes with it).  us, fp32 instruction / bf16 parts: 8 / 4 heads x 8192 x 256, softcap, window 4096 1711 / 1039 (198 TFLOP/s, so 1.19 PFLOP/s of bf16
+// products), 16 x 2000 x 128 297 / 181, 32 / 8 x 3000 x 128 causal 654 / 430, 32 x 2000 x 64 causal 175 / 124, 8 x 1000 x 256 causal 82.8 / 59.2; with a mask
+// tensor 8 x 3001 x 256 causal 394 / 265, dense bias 679 / 424, 64 x 1393 x 128 causal 556 / 232.
 //
 // Masks are index rules (causal with the diagonal at n_k - n_q, sliding window); tiles without a visible key
 // are skipped.  A query without any visible key gets zeros.
@@ -1312,13 +1312,13 @@ hipError_t launch_plain_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t 
 }
 
 // Whether the launch takes the bf16 parts (us, fp32 matrix instruction / bf16 parts).
-//   * Index rules: at head dimension 256 always (8 heads x 64 x 64 21.2 / 15.9, 8 / 4 x 8192, window 4096 1801 / 1051); at 64 and 128, where the
-//     other form has blocks of 64 queries, from some ten tiles on (32 heads x 1000 x 128 111 / 75, 400 38 / 32, 16 x 2000 x 128 324 / 185; but
+//   * Index rules: at head dimension 256 always (8 heads x 64 x 64 21.7 / 15.6, 8 / 4 x 8192, window 4096 1711 / 1039); at 64 and 128, where the
+//     other form has blocks of 64 queries, from some ten tiles on (32 heads x 1000 x 128 153 / 109, 400 41.6 / 38.3, 64 heads x 400 x 64 causal 28.7 / 25.9; but
 //     32 x 150 x 128 18.1 / 19.3, 64 x 250 x 64 15.2 / 19.9), at 64 for more than a block of queries (8 x 64 x 4000 28.8 / 34.1, 32 x 100 x 1000 21.1 / 22.6).
 //   * A mask tensor: with its visible-tile map, as there is no test of a tile by each wave.  The pass that makes the map and a range's start cost
-//     20 - 30 us: head dimension 256 from 150 K mask values on (8 heads x 250 x 600 58.3 / 56.7, 400 58.5 / 54.7, 2000 301 / 139); 128 from 6 M values
-//     over all heads (8 x 100 x 8000 86.7 / 69.0, 8 x 1000 60.4 / 45.2; but 8 x 797 39.0 / 42.6, 32 x 250 x 600 39.5 / 43.7); 64 from 11 M in masks of
-//     600 K (8 x 830 x 1800 51.6 / 48.1, 32 x 797 55.6 / 50.3; but 8 x 1000 33.1 / 37.8, 32 x 400 26.6 / 37.3).
+//     20 - 30 us: head dimension 256 from 150 K mask values on (causal 8 heads x 250 x 600 58.8 / 57.2, 400 58.4 / 54.8, 2000 231 / 139); 128 from 6 M values
+//     over all heads (8 x 100 x 8000 87.5 / 69.1, 8 x 1000 60.8 / 44.9; but 8 x 797 39.0 / 42.6, 32 x 250 x 600 39.5 / 43.7); 64 from 11 M in masks of
+//     600 K (8 x 830 x 1800 51.3 / 48.3, 32 x 797 55.7 / 51.1; but 8 x 1000 33.1 / 37.8, 32 x 400 26.6 / 37.3).
 template <int D, bool MASK>
 bool attention_split_wanted(const AttnArgsF32& args, int64_t batch_heads)
 {

@@ -288,8 +288,9 @@ __global__ __launch_bounds__(256) void softmax_rows_wave_kernel(const SoftmaxArg
 // elements in front of the row in its first vector and behind it in its last are another row's: loaded where they are inside the
 // tensor, never stored.  x and y have to be aligned alike (rows_alike).  A row of odd width walked from its own start splits every access over
 // two lines and its ends into eight element accesses.  us before / here (softcap 50, causal, fp16): 16 heads x 4615 x 4615
-// under a window of 4096 354 / 182, 32 x 1629 x 1629 85 / 51, 8 x 1038 x 16310 181 / 93; float32 without softcap 32 x 1629 x 1629 118 / 87; rows
-// that were aligned all along, whose halves were rounded twice before: 8 x 8192 x 8192 window 4096 277 / 244 (6.1 TB/s of needed bytes).
+// under a window of 4096 341 / 195, 32 x 1629 x 1629 82 / 52, 8 x 1038 x 16310 173 / 90; float32 without softcap 32 x 1629 x 1629 116 / 91; rows
+// that were aligned all along, whose halves were rounded twice before (2-norm error 2.30e-4 / 2.01e-4): 8 x 8192 x 8192 window 4096 272 / 244
+// (6.1 TB/s of needed bytes).
 // ---------------------------------------------------------------------------------------------
 template <bool SOFTCAP>
 __device__ __forceinline__ float logit2_fast(float x, float k_in, float k_cap)
@@ -305,9 +306,6 @@ __device__ __forceinline__ float logit2_fast(float x, float k_in, float k_cap)
 	return x * k_in;
 }
 
-// The softcap of softmax_rows_kernel.  The short form is off by 1.5e-7 of the cap in the logit, so by 1e-5 of a probability at a cap of 64, a
-// fiftieth of a half's rounding; beyond (halves) and for floats a form whose error vanishes with the logit.  2-norm error of halves, N(0, 16) scores,
-// short / full form: cap 50 1.98e-4 / 1.98e-4, 1000 1.88e-4 / 1.86e-4, 1e5 2.6e-3 / 1.9e-4.
 // Elements of the tensor in front of a row and behind it, as far as they can share a vector with it.  (Rows shorter than a vector, or on top of
 // each other in memory, have several rows in the tensor's first and last 16 bytes.)
 struct RowNeighbours { int before, behind; };
@@ -324,6 +322,9 @@ __device__ __forceinline__ float tanh_near_zero(float x)
 	return x * (1.0f + x2 * (-1.0f / 3.0f + x2 * (2.0f / 15.0f)));
 }
 
+// The softcap of softmax_rows_kernel.  The short form is off by 1.5e-7 of the cap in the logit, so by 1e-5 of a probability at a cap of 64, a
+// fiftieth of a half's rounding; beyond (halves) and for floats a form whose error vanishes with the logit.  2-norm error of halves, N(0, 16) scores,
+// short / full form: cap 50 1.98e-4 / 1.98e-4, 1000 1.88e-4 / 1.86e-4, 1e5 2.6e-3 / 1.9e-4.
 enum : int { kCapNone, kCapShort, kCapFull };
 constexpr float kCapShortMost = 64.0f;
 

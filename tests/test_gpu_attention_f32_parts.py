@@ -140,7 +140,7 @@ def test_attention_f32_in_bf16_parts_of_values_without_parts(ops, d, masked):
     assert np.array_equal(got[2:], base[2:])
     assert np.all(np.isnan(got[0, 500:])) and np.isfinite(got[0, :384]).all()
     assert np.isfinite(got[1, 790]).all()                                # the key's score is -inf there: no weight
-    # scores of order one from tiny queries and large keys; a large result (parts below 2^-133 are lost: queries of 2^-110 have all of theirs)
+    # scores of order one from tiny queries and large keys; a large result (floats from 2^-110 on have all of their parts)
     got = run((q * np.float32(2.0 ** -105)), (k * np.float32(2.0 ** 105)), (v * np.float32(2.0 ** 100)))
     assert scaled_rel_err(got * 2.0 ** -100, base, 1.0) <= TOL
 
