@@ -64,10 +64,10 @@ MEASURED_TRAFFIC = {
     "gemm_f16": (235046242, "profiles/gemm_f16_4096_ring_kernel.md"),
     "gemm_f32": (117654803, "profiles/gemm_f32_2048_kernel.md"),
     "conv1d": (277197415, "profiles/causal_conv1d_silu_zamba2_tile_kernel.md"),
-    "softmax_causal": (407016345, "profiles/softmax_causal_32x2048x2048_window_kernel.md"),
-    "softmax_gemma2": (1482778727, "profiles/softmax_gemma2_8x8192x8192_window_kernel.md"),
+    "softmax_causal": (407008806, "profiles/softmax_causal_32x2048x2048_window_kernel.md"),
+    "softmax_gemma2": (1482728761, "profiles/softmax_gemma2_8x8192x8192_window_kernel.md"),
     "attention_gemma2": (530927292, "profiles/sdp_attention_fwd_f16_gemma2_kernel.md"),
-    "attention_gemma2_f32": (1331299024, "profiles/sdp_attention_fwd_f32_gemma2_kernel.md"),
+    "attention_gemma2_f32": (1331564678, "profiles/sdp_attention_fwd_f32_gemma2_kernel.md"),
     "gated_rmsnorm": (805405955, "profiles/gated_rmsnorm_f16_row_kernel.md"),
     "attention_decode": (144062464, "profiles/sdp_attention_decode_f16_partial_and_merge_kernels.md"),
     "lm_head_f32": (2368142029, "profiles/gemma_linear_softcap_head_kwave_kernel.md"),
