@@ -1311,10 +1311,34 @@ hipError_t launch_plain_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t 
 	});
 }
 
+// Head dimensions 64 and 128, index rules: whether the blocks of 128 queries have enough tiles of 32 keys each (`longest`), which a short window
+// does not leave them, nor a long key range that goes out in many parts (in tiles of 32 keys twice as many as in the other form's of 64).
+// us, fp32 matrix instruction / bf16 parts, causal:
+//   * Whole blocks under a window: 24 heads x 700 x 64, window 500 (20 tiles) 30.3 / 38.4, 16 / 8 x 1500, window 1000 (36 tiles) 64.3 / 44.6; with a block
+//     for every CU from 5 tiles on (32 x 4000 x 64, window 30 50.8 / 38.8).
+//   * In parts: 16 / 8 x 700 x 64, window 100 (8 tiles in 5 parts) 12.6 / 23.0, window 500 (20 in 5) 28.3 / 25.0, 4 x 300 x 3000 x 64 (94 in 23) 27.1 / 30.8, 2 x
+//     300 x 6000 x 64 (188 in 47) 34.7 / 46.0, x 128 48.4 / 55.6, 16 / 8 x 700 x 128, window 100 21.1 / 30.2, window 300 (14 in 5) 35.5 / 32.2.
+template <int D>
+bool attention_split_fills(const AttnArgsF32& args, int64_t batch_heads)
+{
+	constexpr size_t kRoom = band::kBandPartialBytes;      // the library's own workspace, whatever the stream has: the form does not depend on it
+	const int64_t q_blocks = (args.n_q + kSplitQueries - 1) / kSplitQueries;
+	int64_t longest = 0;
+	for (int64_t b = q_blocks - 1, step = q_blocks / 64 + 1; b >= 0; b = args.window > 0 ? b - step : -1)
+		longest = std::max(longest, attention_block_tiles(b, args.n_q, args.n_k, args.causal, args.diag, args.window, kSplitQueries, kSplitKeys));
+	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, kSplitQueries, kSplitKeys, D, kRoom);
+	const int64_t parts = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kSplitQueries, kSplitKeys, D, kRoom);
+	if (parts == 1) return args.window == 0 || longest >= 21 || (longest >= 5 && q_blocks * batch_heads >= device_cu_count());
+	if (longest < 11) return false;
+	if (D == 64) return longest >= 8 * parts || (parts <= 32 && 5 * longest >= 21 * parts);
+	return longest > 4 * parts || (parts <= 16 && 2 * longest >= 5 * parts);
+}
+
 // Whether the launch takes the bf16 parts (us, fp32 matrix instruction / bf16 parts).
-//   * Index rules: at head dimension 256 always (8 heads x 64 x 64 21.7 / 15.6, 8 / 4 x 8192, window 4096 1711 / 1039); at 64 and 128, where the
-//     other form has blocks of 64 queries, from some ten tiles on (32 heads x 1000 x 128 153 / 109, 400 41.6 / 38.3, 64 heads x 400 x 64 causal 28.7 / 25.9; but
-//     32 x 150 x 128 18.1 / 19.3, 64 x 250 x 64 15.2 / 19.9), at 64 for more than a block of queries (8 x 64 x 4000 28.8 / 34.1, 32 x 100 x 1000 21.1 / 22.6).
+//   * Index rules: at head dimension 256 always (8 heads x 64 x 64 21.7 / 15.6, 8 / 4 x 8192, window 4096 1711 / 1039; 4 x 700, window 1 30.0 / 25.1);
+//     at 64 and 128, where the other form has blocks of 64 queries, from some ten tiles on (attention_split_fills; 32 heads x 1000 x 128 153 /
+//     109, 400 41.6 / 38.3, 64 heads x 400 x 64 causal 28.7 / 25.9; but 32 x 150 x 128 18.1 / 19.3, 64 x 250 x 64 15.2 / 19.9), at 64 for more than a
+//     block of queries (8 x 64 x 4000 28.8 / 34.1, 32 x 100 x 1000 21.1 / 22.6).
 //   * A mask tensor: with its visible-tile map, as there is no test of a tile by each wave.  The pass that makes the map and a range's start cost
 //     20 - 30 us: head dimension 256 from 150 K mask values on (causal 8 heads x 250 x 600 58.8 / 57.2, 400 58.4 / 54.8, 2000 231 / 139); 128 from 6 M values
 //     over all heads (8 x 100 x 8000 87.5 / 69.1, 8 x 1000 60.8 / 44.9; but 8 x 797 39.0 / 42.6, 32 x 250 x 600 39.5 / 43.7); 64 from 11 M in masks of
@@ -1329,7 +1353,7 @@ bool attention_split_wanted(const AttnArgsF32& args, int64_t batch_heads)
 		if (D == 64) return values >= 600 * 1000 && batch_heads * values >= 11 * 1000 * 1000;
 		return values >= 150 * 1000 && (D == 256 || batch_heads * values >= 6 * 1000 * 1000);
 	}
-	else return D == 256 || (args.n_k >= 350 && (D == 128 || args.n_q > 128));
+	else return D == 256 || (args.n_k >= 350 && (D == 128 || args.n_q > 128) && attention_split_fills<D>(args, batch_heads));
 }
 
 template <int D, bool SOFTCAP, bool MASK>

@@ -217,6 +217,18 @@ __global__ __launch_bounds__(256) void sdp_attention_merge_halves_kernel(const f
 	store_merged(y + (bh * n_q + q_row) * D + 4 * quad, acc * inv);
 }
 
+// Key tiles that a query block sees under the index rules.
+inline int64_t attention_block_tiles(int64_t block, int n_q, int n_k, int causal, int diag, int window, int queries_per_block, int keys_per_tile)
+{
+	const int64_t q0 = block * queries_per_block;
+	const int64_t q_last = std::min<int64_t>(q0 + queries_per_block - 1, n_q - 1);
+	int64_t key_hi = n_k - 1;
+	if (causal && q_last + diag < key_hi) key_hi = q_last + diag;
+	int64_t key_lo = 0;
+	if (window > 0 && q0 + diag - window + 1 > 0) key_lo = q0 + diag - window + 1;
+	return key_hi >= 0 && key_hi >= key_lo ? key_hi / keys_per_tile - key_lo / keys_per_tile + 1 : (int64_t)0;
+}
+
 // How many of a head's latest query blocks to dispatch in two key halves (and how many unsplit ones go out before the
 // halves).  Worth it when whole blocks cannot be packed evenly: at least a block per CU, and the longest block a large
 // share of what a CU gets of the whole launch.  Bounded by the workspace of the stream (the K-split workspace of the
@@ -230,15 +242,7 @@ inline AttnSplitPlan plan_attention_split(int n_q, int n_k, int causal, int diag
 	const int64_t q_blocks = (n_q + queries_per_block - 1) / queries_per_block;
 	const int cus = device_cu_count();
 	if (q_blocks * batch_heads < cus || q_blocks > 65536 || capacity == 0) return plan;
-	const auto tiles_of = [&](int64_t b) {
-		const int64_t q0 = b * queries_per_block;
-		const int64_t q_last = std::min<int64_t>(q0 + queries_per_block - 1, n_q - 1);
-		int64_t key_hi = n_k - 1;
-		if (causal && q_last + diag < key_hi) key_hi = q_last + diag;
-		int64_t key_lo = 0;
-		if (window > 0 && q0 + diag - window + 1 > 0) key_lo = q0 + diag - window + 1;
-		return key_hi >= 0 && key_hi >= key_lo ? key_hi / keys_per_tile - key_lo / keys_per_tile + 1 : (int64_t)0;
-	};
+	const auto tiles_of = [&](int64_t b) { return attention_block_tiles(b, n_q, n_k, causal, diag, window, queries_per_block, keys_per_tile); };
 	int64_t total = 0, longest = 0;
 	for (int64_t b = 0; b < q_blocks; ++b)
 	{

@@ -46,7 +46,8 @@ def hidden_keys(n_q, n_k, causal, window):
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("heads,kv,n_q,n_k,softcap,causal,window", [
     (2, 2, 65, 350, 0.0, True, 0), (2, 2, 130, 349, 0.0, False, 0), (4, 2, 129, 352, 0.0, False, 0), (2, 1, 129, 383, 30.0, True, 100), (3, 3, 300, 1025, 0.0, True, 0),
-    (2, 2, 400, 400, 0.0, True, 33), (2, 2, 500, 353, 0.0, True, 0), (1, 1, 1000, 1000, 50.0, True, 256), (40, 8, 1100, 1100, 0.0, True, 0)])
+    (2, 2, 400, 400, 0.0, True, 33), (2, 2, 500, 353, 0.0, True, 0), (1, 1, 1000, 1000, 50.0, True, 256), (40, 8, 1100, 1100, 0.0, True, 0),
+    (40, 8, 900, 900, 0.0, True, 40), (2, 2, 700, 700, 30.0, True, 600)])
 def test_attention_f32_in_bf16_parts(ops, d, heads, kv, n_q, n_k, softcap, causal, window):
     q, k, v = (synth.normal(s + n_q, (1, h, n, d)) for s, h, n in ((1, heads, n_q), (2, kv, n_k), (3, kv, n_k)))
     alpha = d ** -0.5
@@ -114,7 +115,7 @@ def test_attention_f32_in_bf16_parts_of_values_without_parts(ops, d, masked):
     # an infinity or a NaN reaches the queries that see its key, in the column it stands in, and no other block of queries; the largest floats
     # and floats near the smallest one have parts like all others
     import torch
-    heads, n = (26, 800) if masked else (2, 800)
+    heads, n = (26, 800) if masked else (30, 800)
     q, k, v = (synth.normal(s, (1, heads, n, d)) for s in (1, 2, 3))
     alpha = d ** -0.5
 
@@ -146,7 +147,7 @@ def test_attention_f32_in_bf16_parts_of_values_without_parts(ops, d, masked):
 
 
 @pytest.mark.parametrize("d,block", [(64, 64), (128, 64), (256, 128)])
-@pytest.mark.parametrize("heads,window", [(2, 0), (2, 200), (50, 0)])
+@pytest.mark.parametrize("heads,window", [(2, 0), (2, 200), (50, 0), (50, 200)])
 def test_attention_f32_value_that_is_not_finite_reaches_its_query_block(ops, d, block, heads, window):
     # the queries that see its key, and of those that the rules hide it from at most the rest of a block of 64 (head dimension 256: 128): the blocks of the fp32 instruction
     n, key = 800, 485
