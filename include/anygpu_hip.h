@@ -293,9 +293,9 @@ int anygpu_sdp_attention_fwd_f16(const void* q, const void* k, const void* v, vo
 /*
  * anygpu_sdp_attention_fwd_f16 in float32: operands, scores, sums and output are fp32.  A product of floats is six products
  * of their bf16 parts, summed in fp32 (what is left out lies below 2^-24 of it, of either sign; weights below 2^-110 of a query's
- * largest may lose bits below 2^-133); small launches, short windows at head dimensions 64 and 128, and blocks of queries whose results are not finite or whose operands have
- * bits below 2^-133 (floats below 2^-110 do), run on the fp32 matrix instruction; results agree with the unfused float32 path to
- * fp32 rounding.  Same arguments and rules.  Replaces cu_flash_sdpa_fwd_d256_v1 (srcs/kernels/cuda/flash_sdpa_fwd.cuh:6-15: one head, head_dim 256,
+ * largest may lose bits below 2^-133); small launches, short windows at head dimensions 64 and 128, and blocks of queries whose
+ * results are not finite or whose operands have bits below 2^-133 (floats below 2^-110 do), run on the fp32 matrix instruction;
+ * results agree with the unfused float32 path to fp32 rounding.  Same arguments and rules.  Replaces cu_flash_sdpa_fwd_d256_v1 (srcs/kernels/cuda/flash_sdpa_fwd.cuh:6-15: one head, head_dim 256,
  * no mask; here any number of heads, head_dim 64 / 128 / 256, the index-rule masks) and, for masks that are
  * index rules, the per-head loop of sdp_attention_masked_scaled_fwd (srcs/transformers/sdp.hpp:258-271).
  */
