@@ -1,20 +1,22 @@
 // Fused attention, fp16, head dimensions 64 and 128: 32 queries per wave.
 //
-// What bounds it.  Per tile of 64 keys a wave of 32 queries has 1024 (head dimension 64: 512) cycles of MFMAs, about 900 (770) of
-// vector instructions and 32 (16) KB of fragments to read out of LDS.  With v_mfma_f32_32x32x16_f16 every fragment feeds 32 x 32
-// scores, so the LDS stays below half of its rate; the 16-queries-per-wave kernel this one replaces read twice the bytes
-// per score, and its 8-wave blocks of 128 or 256 queries ran one to a CU in lockstep.  Here a block is FOUR waves with 128
-// queries, and two blocks (head dimension 64: three) share a CU without a barrier between them, so that one block's
-// softmax, loads and ends run beside the other's products, and causal launches of ordinary prompts have twice as many
-// pieces to pack onto the CUs.  Scores sit 32 to a lane (S^T = K Q^T: a lane holds one query), so row maxima are in-lane
-// but for one exchange of lane halves.  Sums are those of the fp32 p, and the maximum is exact in every tile, so that the largest p is
+// What bounds it.  Per tile of 64 keys a wave of 32 queries has 1024 (head dimension 64: 512) cycles of MFMAs, some 700 of vector
+// instructions (22 clocks a score with two waves on a SIMD) and 32 (16) KB of fragments to read out of LDS.  With v_mfma_f32_32x32x16_f16 every
+// fragment feeds 32 x 32 scores, so the LDS stays below half of its rate.  A block is FOUR waves with 128 queries, and two blocks (head dimension 64:
+// three) share a CU without a barrier between them.  Scores sit 32 to a lane (S^T = K Q^T: a lane holds one query), so row maxima are in-lane
+// but for one exchange of lane halves.  The two halves of a tile's work come from DIFFERENT tiles, so that a wave has vector instructions to issue
+// behind every MFMA (a wave of such a mix and another like it on its SIMD keep the matrix cores busy, 33.7 clocks per MFMA of 32, where products and
+// softmax in turn took 66): S(t + 1) = K(t + 1) Q^T beside p(t) = 2^(z(t) - m), then O^T += V(t)^T P(t)^T beside the rest of p(t) and the maximum of
+// S(t + 1).  What is left is the power the part may draw: 16 heads x 8192 x 128 without the causal rule 548 us on operands of N(0, 1) and 345 (1.6
+// PFLOP/s) on zeros, where the form with products and softmax in turn took 571 and 407; eight waves and 256 queries to a block, half of the tile
+// loads, measured 540 there and up to a quarter slower where blocks are few.
+// Sums are those of the fp32 p, and the maximum is exact in every tile, so that the largest p is
 // a power of two, which rounds to a half without an error (a maximum that lags until it is outgrown by 2^8 and sums of the
 // rounded p by v_dot2 measured 5 % faster, but up to a tenth further from 64-bit results: 16 heads x 4096 x 128, q of
 // N(0, 4): 2.36e-4 against 2.17e-4 (2-norm), of which the result's own rounding is 2.1e-4).
-// Measured, causal (us; 16-queries-per-wave kernels -> here): 32 / 8 heads x 3000 x 128 126.6 -> 94.9 (0.78 PFLOP/s), 16 x 4096 x 128 115.9 ->
-// 101.4, 64 / 8 x 1000 x 128 45.1 -> 31.8, 16 x 8192 x 128 367 -> 313 (0.88 PFLOP/s; a kernel that overlaps the products and the softmax
-// inside a wave ran at the same rate there, as the clock drops under the matrix units' power), 32 x 2038 x 64 41.9 -> 36.6; without the causal
-// rule 32 / 8 x 3000 x 128 183 -> 172, but 16 x 8192 x 128 542 -> 570 (the former kernel's rounds are full there).
+// Measured, causal (us; products and softmax in turn -> here, the same bits): 16 x 4096 x 128 102.3 -> 91.7, 64 / 8 x 1000 x 128 32.0 -> 29.9, 16 x 8192 x
+// 128 315 -> 299, 2 x 16 x 2280 x 128 63.3 -> 58.7, 32 x 2038 x 64 36.5 -> 32.8, 32 x 4000 x 64 window 500 36.9 -> 34.5, 32 / 8 x 3000 x 128 93.7 -> 95.0 (query
+// blocks of 1 to 47 tiles that do not pack evenly, 20 % of the CU time idle); without the causal rule 32 / 8 x 3000 x 128 173 -> 161.
 #pragma once
 
 #include "attention_walk.hpp"
@@ -49,7 +51,7 @@ __device__ __forceinline__ float max_over_lane_halves(float x)
 }
 
 template <int D, bool SOFTCAP>
-__global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_kernel(const AttnArgs a, const AttnWalk walk)
+__global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention_fwd_f16_q32_kernel(const AttnArgs a, const AttnWalk walk)
 {
 	constexpr int kRow = 2 * D;                              // bytes of a tile row
 	constexpr int KT = kAttnKeysPerTile, KB = KT / 32;
@@ -59,8 +61,8 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 	constexpr int DC = D / 32;                               // 32-wide column blocks of the output
 	constexpr int kSlots = kTile / 1024 / kQ32Waves;         // direct loads of a tile per wave
 	constexpr int kChunks = kRow / 16, kRowsPerLoad = 1024 / kRow;
-	constexpr int kAhead = 4;                                // steps that the K fragments are read ahead
-	constexpr int kVRing = 8;                                // V fragments in registers, read ahead of the softmax
+	constexpr int kAhead = 4;                                // steps that a fragment is read ahead
+	constexpr int kLoadSpacing = D == 128 ? 4 : 2;           // steps from one load of the next tiles to the next
 	extern __shared__ __align__(16) char lds[];
 
 	const int tid = threadIdx.x;
@@ -134,19 +136,19 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 		load_v[j] = row * kRow + ((lane % kChunks) ^ q32_v_swizzle<D>(row)) * 16;
 	}
 	typedef int int4_t __attribute__((ext_vector_type(4)));
-	auto issue_tile = [&](int t, int stage) {
+	// load j of this wave's share (K: j < kSlots, V behind it) of the tile at `at` into a stage
+	auto rsrc_of = [&](const half_t* src, int t) {
 		const int bytes = min(KT, a.n_k - t * KT) * kRow;
-		const uint64_t at_k = reinterpret_cast<uint64_t>(kp) + (int64_t)t * kTile, at_v = reinterpret_cast<uint64_t>(vp) + (int64_t)t * kTile;
-		const int4_t rsrc_k = {(int)(uint32_t)at_k, (int)(uint32_t)(at_k >> 32), bytes, 0x00020000};
-		const int4_t rsrc_v = {(int)(uint32_t)at_v, (int)(uint32_t)(at_v >> 32), bytes, 0x00020000};
-#pragma unroll
-		for (int j = 0; j < kSlots; ++j)
-		{
-			const unsigned m0k = lds_base + stage * kStage + (wave + kQ32Waves * j) * 1024;
-			const unsigned m0v = m0k + kTile;
-			asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(load_k[j]), "s"(rsrc_k), "s"(m0k) : "memory", "m0");
-			asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(load_v[j]), "s"(rsrc_v), "s"(m0v) : "memory", "m0");
-		}
+		const uint64_t at = reinterpret_cast<uint64_t>(src) + (int64_t)t * kTile;
+		return int4_t{(int)(uint32_t)at, (int)(uint32_t)(at >> 32), bytes, 0x00020000};
+	};
+	auto issue_k = [&](int4_t rsrc, int stage, int j) {
+		const unsigned m0 = lds_base + stage * kStage + (wave + kQ32Waves * j) * 1024;
+		asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(load_k[j]), "s"(rsrc), "s"(m0) : "m0");
+	};
+	auto issue_v = [&](int4_t rsrc, int stage, int j) {
+		const unsigned m0 = lds_base + stage * kStage + kTile + (wave + kQ32Waves * j) * 1024;
+		asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(load_v[j]), "s"(rsrc), "s"(m0) : "m0");
 	};
 	typedef __attribute__((address_space(3))) const half8_t* LdsHalf8;
 	const unsigned k_addr = lds_base + n * kRow + ((h ^ q32_k_swizzle<D>(n)) * 16);          // ^ 32 st, + 32 kb rows
@@ -154,89 +156,76 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 	const int vr = (lane & 15) >> 2;
 	const unsigned v_addr = lds_base + kTile + (4 * h + vr) * kRow +
 	                        (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ q32_v_swizzle<D>(vr)) * 16) + (lane & 1) * 8;   // ^ 64 c
-	if (t_first <= t_last) issue_tile(t_first, 0);
-	for (int t = t_first; t <= t_last; ++t)
-	{
-		__builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0)
-		__syncthreads();
-		const int stage = (t - t_first) & 1;
-		const int key0 = t * KT;
-		const bool any_visible = key0 <= any_hi && key0 + KT - 1 >= any_lo;        // wave-uniform
-		const unsigned ka = k_addr + stage * kStage, va = v_addr + stage * kStage;
-		// the first K fragments, on their way while the next tile's loads are issued
-		half8_t kf[KS][KB];
-		auto read_k = [&](int st) {
-#pragma unroll
-			for (int kb = 0; kb < KB; ++kb) kf[st][kb] = *(LdsHalf8)(uintptr_t)((ka ^ (32 * st)) + kb * 32 * kRow);
-		};
-		if (any_visible)
-		{
-#pragma unroll
-			for (int st = 0; st < kAhead; ++st) read_k(st);
-		}
-		__builtin_amdgcn_sched_barrier(0);
-		if (t < t_last) issue_tile(t + 1, stage ^ 1);
-		if (!any_visible) continue;
 
-		// ---- S^T = K Q^T ----
-		float16_t s[KB];
+	// the tiles in which some query of this wave sees a key
+	const int wt_first = any_lo > 0 && any_lo / KT > t_first ? any_lo / KT : t_first;
+	const int wt_last = any_hi < 0 ? -1 : (any_hi / KT < t_last ? any_hi / KT : t_last);
+
+	float mt = -INFINITY;                                    // maximum of the scores of the tile ahead (raw; with softcap logits)
+	constexpr int kStepsA = KS * KB, kStepsB = 2 * KB * DC, kSteps = kStepsA + kStepsB;
+	typedef float16_t Scores[KB];
+
+	auto is_interior = [&](int t) { return t * KT >= all_lo && t * KT + KT - 1 <= all_hi; };      // wave-uniform
+	auto max_pair = [&](const Scores& s, int y) {
+		const float x0 = s[y / 8][2 * (y % 8)], x1 = s[y / 8][2 * (y % 8) + 1];
+		mt = y == 0 ? fmaxf(x0, x1) : fmaxf(fmaxf(mt, x0), x1);
+	};
+	auto logits_of_pair = [&](Scores& s, int y) {
+		if constexpr (SOFTCAP)
+		{
+			s[y / 8][2 * (y % 8)] = logit2<true>(s[y / 8][2 * (y % 8)], k_in, a.k_cap);
+			s[y / 8][2 * (y % 8) + 1] = logit2<true>(s[y / 8][2 * (y % 8) + 1], k_in, a.k_cap);
+		}
+	};
+	auto max_scores = [&](const Scores& s) {
+#pragma unroll
+		for (int y = 0; y < 8 * KB; ++y) max_pair(s, y);
+	};
+	auto mask_scores = [&](Scores& s, int t) {
+		// (through an empty statement: the compiler would do without the branch around this and test every tile's scores)
+		int lo = vis_lo - t * KT - 4 * h, hi = vis_hi - t * KT - 4 * h;
+		asm volatile("" : "+v"(lo), "+v"(hi));
 #pragma unroll
 		for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-			for (int i = 0; i < 16; ++i) s[kb][i] = 0.0f;
-		__builtin_amdgcn_s_setprio(1);
-#pragma unroll
-		for (int st = 0; st < KS; ++st)
+			for (int i = 0; i < 16; ++i)
+			{
+				const int key = 32 * kb + 8 * (i / 4) + i % 4;           // + 4 h
+				s[kb][i] = (key >= lo && key <= hi) ? s[kb][i] : -INFINITY;
+			}
+		max_scores(s);
+	};
+	// own loads have landed; behind the barrier everybody's have, and everybody is done with what the loads issued behind it overwrite:
+	// at the turn of tile t K(t + 1) and V(t) are there, K(t) and V(t - 1) free
+	auto tile_barrier = [&]() {
+		__builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0)
+		__syncthreads();
+	};
+	auto issue_all = [&](int t) {
+		const int stage = (t + 1 - t_first) & 1;
+		if (t + 1 <= t_last && t >= t_first)
 		{
+			const int4_t rsrc = rsrc_of(vp, t + 1);
 #pragma unroll
-			for (int kb = 0; kb < KB; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[st][kb], qf[st], s[kb], 0, 0, 0);
-			if (st + kAhead < KS) read_k(st + kAhead);
-			__builtin_amdgcn_sched_barrier(0);
+			for (int j = 0; j < kSlots; ++j) issue_v(rsrc, stage, j);
 		}
-		__builtin_amdgcn_s_setprio(0);
-		// V^T fragments, the first of them on their way during the softmax.  K slot (h, j) of 16-key step u is key
-		// 16 u + 8 (j / 4) + 4 h + j % 4
-		half8_t vf[kVRing];
-		auto read_v = [&](int i) {
-			const int u = i / DC, c = i % DC;
-			const unsigned src = (va ^ (64 * c)) + 16 * u * kRow;
-			const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)src);
-			const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)(src + 8 * kRow));
-			vf[i % kVRing] = __builtin_shufflevector(__builtin_bit_cast(half4_t, lo), __builtin_bit_cast(half4_t, hi), 0, 1, 2, 3, 4, 5, 6, 7);
-		};
-#pragma unroll
-		for (int i = 0; i < kVRing; ++i) read_v(i);
-		__builtin_amdgcn_sched_barrier(0);
-
-		// ---- online softmax ----
-		if constexpr (SOFTCAP)
+		if (t + 2 <= t_last && t >= t_first)
 		{
+			const int4_t rsrc = rsrc_of(kp, t + 2);
 #pragma unroll
-			for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-				for (int i = 0; i < 16; ++i) s[kb][i] = logit2<true>(s[kb][i], k_in, a.k_cap);
+			for (int j = 0; j < kSlots; ++j) issue_k(rsrc, stage ^ 1, j);
 		}
-		if (!(key0 >= all_lo && key0 + KT - 1 <= all_hi))
-		{
-#pragma unroll
-			for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-				for (int i = 0; i < 16; ++i)
-				{
-					const int key = key0 + 32 * kb + 8 * (i / 4) + 4 * h + i % 4;
-					s[kb][i] = (key >= vis_lo && key <= vis_hi) ? s[kb][i] : -INFINITY;
-				}
-		}
-		float mt = fmaxf(s[0][0], s[1][0]);
-#pragma unroll
-		for (int i = 1; i < 16; ++i) mt = fmaxf(fmaxf(mt, s[0][i]), s[1][i]);
-		mt = max_over_lane_halves(mt);
-		if constexpr (!SOFTCAP) mt *= k_in;
+	};
+	// the maximum of tile t joins the running one
+	float z_in = 1.0f, z_add = 0.0f;
+	auto take_maximum = [&](Scores& cur) {
+		float m_tile = max_over_lane_halves(mt);
+		if constexpr (!SOFTCAP) m_tile *= k_in;
 		// the running maximum settles after some tiles; while no query of the wave raises it, the pass over the accumulators is
 		// left out
-		if (__builtin_amdgcn_ballot_w64(mt > m_run) != 0)
+		if (__builtin_amdgcn_ballot_w64(m_tile > m_run) != 0)
 		{
-			const float m_new = fmaxf(m_run, mt);
+			const float m_new = fmaxf(m_run, m_tile);
 			const float corr = fast_exp2(m_run - (m_new == -INFINITY ? 0.0f : m_new));
 			m_run = m_new;
 			l_run *= corr;
@@ -248,7 +237,8 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 		const float m_safe = m_run == -INFINITY ? 0.0f : m_run;
 		// p = 2^(z_in s + z_add).  The maximum is a rounded product, which the fma does not see as such: from 2^20 on, before
 		// the rounding can take p out of the halves' range, the difference is taken between rounded products
-		float z_in = SOFTCAP ? 1.0f : k_in, z_add = kQ32HeadRoom - m_safe;
+		z_in = SOFTCAP ? 1.0f : k_in;
+		z_add = kQ32HeadRoom - m_safe;
 		if (__builtin_amdgcn_ballot_w64(fabsf(m_safe) > 0x1p20f) != 0)
 		{
 #pragma clang fp contract(off)
@@ -257,40 +247,167 @@ __global__ __launch_bounds__(64 * kQ32Waves, 2) void sdp_attention_fwd_f16_q32_k
 #pragma unroll
 				for (int i = 0; i < 16; ++i)
 				{
-					const float z = SOFTCAP ? s[kb][i] : s[kb][i] * k_in;
-					s[kb][i] = z - m_safe;
+					const float z = SOFTCAP ? cur[kb][i] : cur[kb][i] * k_in;
+					cur[kb][i] = z - m_safe;
 				}
 			z_in = 1.0f;
 			z_add = kQ32HeadRoom;
 		}
+	};
+	auto p_of_score = [&](const Scores& s, int e) { return fast_exp2(fmaf(s[e / 16][e % 16], z_in, z_add)); };
+
+	// One tile: S(t + 1) = K(t + 1) Q^T (SCORES) beside p(t) = 2^(z(t) - m), then O^T += V(t)^T P(t)^T (OUTPUT) beside the
+	// maximum of S(t + 1), as steps of one MFMA.
+	auto tile = [&](auto scores_tag, auto output_tag, Scores& cur, Scores& next, int t) {
+		constexpr bool SCORES = decltype(scores_tag)::value, OUTPUT = decltype(output_tag)::value, BOTH = SCORES && OUTPUT;
+		constexpr int kFirst = SCORES ? 0 : kStepsA, kEnd = OUTPUT ? kSteps : kStepsA;
+		const int stage = (t + 1 - t_first) & 1;
+		const unsigned ka = k_addr + stage * kStage, va = v_addr + (stage ^ 1) * kStage;
+		half8_t frag[kAhead];
+		auto read_operand = [&](int i) {
+			if (i < kStepsA)
+			{
+				const int st = i / KB, kb = i % KB;
+				frag[i % kAhead] = *(LdsHalf8)(uintptr_t)((ka ^ (32 * st)) + kb * 32 * kRow);
+				return;
+			}
+			// K slot (h, j) of 16-key step u is key 16 u + 8 (j / 4) + 4 h + j % 4
+			const int u = (i - kStepsA) / DC, c = (i - kStepsA) % DC;
+			const unsigned src = (va ^ (64 * c)) + 16 * u * kRow;
+			const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)src);
+			const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)(src + 8 * kRow));
+			frag[i % kAhead] = __builtin_shufflevector(__builtin_bit_cast(half4_t, lo), __builtin_bit_cast(half4_t, hi), 0, 1, 2, 3, 4, 5, 6, 7);
+		};
+		const int4_t rsrc_v = rsrc_of(vp, t + 1), rsrc_k = rsrc_of(kp, t + 2 <= t_last ? t + 2 : t_last);
 		half8_t pf[2 * KB];
 		float psum[2] = {0.0f, 0.0f};
+		float x[32];
+		auto pair_into_p = [&](int y) {
+			psum[0] += x[2 * y];
+			psum[1] += x[2 * y + 1];
+			pf[y / 4][2 * (y % 4)] = (half_t)x[2 * y];
+			pf[y / 4][2 * (y % 4) + 1] = (half_t)x[2 * y + 1];
+		};
+		auto vector_work = [&](int i) {
 #pragma unroll
-		for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-			for (int i = 0; i < 16; i += 2)
+			for (int y = 0; y < 8 * KB; ++y)
 			{
-				const float z0 = SOFTCAP ? s[kb][i] + z_add : fmaf(s[kb][i], z_in, z_add);
-				const float z1 = SOFTCAP ? s[kb][i + 1] + z_add : fmaf(s[kb][i + 1], z_in, z_add);
-				const float p0 = fast_exp2(z0), p1 = fast_exp2(z1);
-				psum[0] += p0;
-				psum[1] += p1;
-				pf[2 * kb + i / 8][i % 8] = (half_t)p0;
-				pf[2 * kb + i / 8][i % 8 + 1] = (half_t)p1;
+				const int at = y * 3 * kSteps / 64;
+				if (i == at)
+				{
+					x[2 * y] = p_of_score(cur, 2 * y);
+					x[2 * y + 1] = p_of_score(cur, 2 * y + 1);
+				}
+				if (i == at + 1) pair_into_p(y);
+				if (i == kStepsA + 2 + y * (kStepsB - 2) / (8 * KB))
+				{
+					logits_of_pair(next, y);
+					max_pair(next, y);
+				}
 			}
-		l_run += psum[0] + psum[1];
-
-		// ---- O^T += V^T P^T ----
-		__builtin_amdgcn_sched_barrier(0);
-		__builtin_amdgcn_s_setprio(1);
+		};
+		float16_t zero;
 #pragma unroll
-		for (int i = 0; i < 2 * KB * DC; ++i)
-		{
-			o[i % DC] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i % kVRing], pf[i / DC], o[i % DC], 0, 0, 0);
-			if (i + kVRing < 2 * KB * DC) read_v(i + kVRing);
+		for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
+		auto step = [&](auto step_tag) {
+			constexpr int i = decltype(step_tag)::value;
 			__builtin_amdgcn_sched_barrier(0);
+			if constexpr (i < kStepsA)
+				next[i % KB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[i % kAhead], qf[i / KB], i < KB ? zero : next[i % KB], 0, 0, 0);
+			else
+				o[(i - kStepsA) % DC] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[i % kAhead], pf[(i - kStepsA) / DC], o[(i - kStepsA) % DC], 0, 0, 0);
+			if constexpr (i + kAhead < kEnd) read_operand(i + kAhead);
+			// the next tiles' loads, spread over the steps (past the end: the last tile's K once more, into the free stage)
+			if constexpr (BOTH && i % kLoadSpacing == 1 && i / kLoadSpacing < 2 * kSlots)
+			{
+				constexpr int m = i / kLoadSpacing;
+				if constexpr (m < kSlots) issue_v(rsrc_v, stage, m);
+				else issue_k(rsrc_k, stage ^ 1, m - kSlots);
+			}
+			if constexpr (BOTH) vector_work(i);
+		};
+#pragma unroll
+		for (int i = kFirst; i < kFirst + kAhead; ++i) read_operand(i);
+		if constexpr (!BOTH) issue_all(t);
+		if constexpr (OUTPUT && !SCORES)
+		{
+#pragma unroll
+			for (int y = 0; y < 8 * KB; ++y)
+			{
+				x[2 * y] = p_of_score(cur, 2 * y);
+				x[2 * y + 1] = p_of_score(cur, 2 * y + 1);
+				pair_into_p(y);
+			}
 		}
-		__builtin_amdgcn_s_setprio(0);
+		[&]<int... I>(std::integer_sequence<int, I...>) { (step(std::integral_constant<int, kFirst + I>{}), ...); }(std::make_integer_sequence<int, kEnd - kFirst>{});
+		__builtin_amdgcn_sched_barrier(0);
+		if constexpr (OUTPUT) l_run += psum[0] + psum[1];
+		// (uses here, or the compiler moves the sums and the maximum behind the branch that follows)
+		if constexpr (BOTH) asm volatile("" : "+v"(l_run), "+v"(mt));
+		if constexpr (SCORES)
+		{
+			if constexpr (!OUTPUT)
+			{
+#pragma unroll
+				for (int y = 0; y < 8 * KB; ++y) logits_of_pair(next, y);
+				max_scores(next);
+			}
+			if (!is_interior(t + 1)) mask_scores(next, t + 1);
+		}
+	};
+	if (t_first > t_last) {}
+	else
+	{
+		// K of the first tile, then (the turn of the tile before the first has nothing else to load) its V and K of the second
+		const int4_t rsrc_k = rsrc_of(kp, t_first), rsrc_v = rsrc_of(vp, t_first), rsrc_k2 = rsrc_of(kp, t_first < t_last ? t_first + 1 : t_first);
+#pragma unroll
+		for (int j = 0; j < kSlots; ++j) issue_k(rsrc_k, 0, j);
+#pragma unroll
+		for (int j = 0; j < kSlots; ++j) issue_v(rsrc_v, 0, j);
+#pragma unroll
+		for (int j = 0; j < kSlots; ++j) issue_k(rsrc_k2, 1, j);
+		constexpr std::true_type yes{};
+		constexpr std::false_type no{};
+		const bool any = wt_first <= wt_last;
+		int t = t_first - 1;
+		__builtin_amdgcn_s_waitcnt(0x0F70 | (2 * kSlots));   // vmcnt: the first tile's K
+		__syncthreads();
+		for (const int until = any ? wt_first - 1 : t_last + 1; t < until;)
+		{
+			issue_all(t);
+			++t;
+			if (t <= t_last) tile_barrier();
+		}
+		if (any)
+		{
+			Scores s0, s1;
+			tile(yes, no, s1, s0, t++);
+			for (; t + 1 < wt_last; t += 2)
+			{
+				take_maximum(s0);
+				tile_barrier();
+				tile(yes, yes, s0, s1, t);
+				take_maximum(s1);
+				tile_barrier();
+				tile(yes, yes, s1, s0, t + 1);
+			}
+			if (t < wt_last)
+			{
+				take_maximum(s0);
+				tile_barrier();
+				tile(yes, yes, s0, s1, t++);
+#pragma unroll
+				for (int kb = 0; kb < KB; ++kb) s0[kb] = s1[kb];
+			}
+			take_maximum(s0);
+			tile_barrier();
+			tile(no, yes, s0, s1, t++);
+			for (; t <= t_last; ++t)
+			{
+				tile_barrier();
+				issue_all(t);
+			}
+		}
 	}
 
 	// ---- normalise and store: lane (n, h) holds y[row][32 c + 8 (i / 4) + 4 h + i % 4] ----

@@ -159,6 +159,25 @@ def test_sdp_attention_fused_kernel_32_queries_per_wave(ops, oracle, n_q, n_k, c
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# the same kernel's walk over two tiles at a time: waves that see one to seven tiles, odd and even in number, whose first and last ones lie
+# before, on and behind those of the block's other waves, the last tile whole, of one key and one short
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("n_q,n_k,causal,window", [(128, 192, True, 0), (128, 193, True, 65), (100, 319, True, 130), (130, 385, True, 200), (60, 447, False, 0),
+                                                    (256, 256, True, 33), (129, 448, True, 64), (97, 384, False, 90)])
+def test_sdp_attention_32_queries_per_wave_tiles_in_pairs(ops, oracle, n_q, n_k, causal, window, d):
+    copies, heads = 132, 4
+    q, k, v = (synth.normal(80 + i, (1, heads, n, d)).astype(np.float16) for i, n in enumerate((n_q, n_k, n_k)))
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), d ** -0.5, causal=causal, window=window,
+                                     decode=False)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=d ** -0.5, softcap=0.0,
+                                      causal=causal, window=window, q_per_kv=1, threads=8)
+    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
+    assert not got[0][blind].any() and np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    # p rounded to fp16 (2^-11 each, weights that sum to 1) and the result's own rounding, values of up to about 4
+    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
+
+
 # The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
 # many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
 
