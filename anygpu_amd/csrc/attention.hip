@@ -946,37 +946,39 @@ namespace {
 // Head dimensions 64 and 128, index rules: whether the longest query blocks go out in two halves of their key range (`blocks` of 128
 // queries in all; us, whole / cut).
 //   * Under a window, where most blocks are equally long, while they are one to one and a half for each CU: 9 heads x 4086 x 128, window 1024
-//     55.0 / 43.0, 12 heads 57.1 / 56.6; but 14 heads 46.0 / 62.0, 16 / 8 heads x 4096 52.5 / 61.8.
-//   * One block for each CU: where the blocks run from near nothing to the whole range from 31 tiles on (8 heads x 4086 x 128 78.5 / 61.8, 16 x
-//     2038 45.8 / 46.0; but 32 x 1014 26.7 / 30.0), else from 61 on, where two shorter blocks on a CU overlap enough to pay for the partial
-//     results' way through memory (no causal rule: 4 heads x 8182 x 64 114 / 104, 8 x 4086 x 64 61.6 / 61.0; but 16 x 2038 x 128 51.1 / 58.9).
-//   * More blocks: such a triangle of blocks only, up to one and a quarter for each CU (10 heads x 4086 x 128 81.2 / 69.7; 11 heads 77.7 /
-//     79.2), at head dimension 64 with very long ranges up to two (7 heads x 8182 x 64 122 / 105).
+//     52.9 / 41.1, 12 heads 54.6 / 54.3; but 14 heads 46.0 / 62.0, 16 / 8 heads x 4096 52.5 / 61.8.
+//   * One block for each CU: where the blocks run from near nothing to the whole range from 41 tiles on (8 heads x 4086 x 128 68.5 / 56.7, 8 x 4000
+//     x 64 49.5 / 37.8; but 16 x 2038 x 128 37.9 / 41.2, x 64 28.2 / 29.1), else from 101 on, where two shorter blocks on a CU overlap enough to pay
+//     for the partial results' way through memory (no causal rule: 4 heads x 8182 x 64 98.7 / 95.9; but 8 x 4086 x 64 52.9 / 56.6).
+//   * More blocks: such a triangle of blocks only, up to one and a quarter for each CU (10 heads x 4086 x 128 77.6 / 66.5, 18 x 2038 45.1 / 43.9; 11
+//     x 4086 77.7 / 79.2), at head dimension 64 with very long ranges up to two (7 heads x 8182 x 64 104 / 102).
 template <int D>
 bool attention_cut_longest(const AttnArgs& args, int64_t blocks)
 {
 	const int64_t cus = device_cu_count(), tiles = (args.n_k + kAttnKeysPerTile - 1) / kAttnKeysPerTile;
 	if (args.window > 0) return blocks > cus && 2 * blocks <= 3 * cus;
 	const bool triangle = args.causal && 2 * args.diag <= args.n_q;
-	if (blocks <= cus) return tiles > (triangle ? 30 : 60);
+	if (blocks <= cus) return tiles > (triangle ? 40 : 100);
 	return triangle && ((tiles > 30 && 4 * blocks <= 5 * cus) || (D == 64 && tiles >= 96 && blocks <= 2 * cus));
 }
 
 // Head dimensions 64 and 128, index rules: whether the kernel with 32 queries per wave takes the launch (`blocks` of 128 queries in all).
-// It does twice the work per wave and tile in half of the waves, which needs two blocks on a CU to pay: with up to one block per CU
-// the 16-queries-per-wave kernel is 7 - 13 % ahead (us, 32 / 16 queries: 8 heads x 64 x 128 5.7 / 5.0, 16 heads x 300 x 64 8.0 / 7.2, 32 heads x
-// 600 x 128 17.5 / 16.5, 16 heads x 1700 x 128 39.6 / 35.5), with more it falls behind (36 heads x 1014 x 128 28.9 / 31.3, 32 x 1200 x 128
-// 30.5 / 33.5, 32 x 3000 x 128 93 / 107, 16 x 8192 x 64 178 / 197); under a window at head dimension 128 from one and a half blocks on (12 /
-// 4 heads x 4096, window 512 45.8 / 42.9; 13 x 4000, window 1024 43.9 / 57.4).
+// It does twice the work per wave in half of the waves, so that a block without another on its CU has longer to start and end: with up to one block
+// per CU the 16-queries-per-wave kernel is ahead on short key ranges (us, 32 / 16 queries: 64 heads x 100 x 128 7.8 / 7.0, 16 heads x 300 x 64 7.6 / 7.1, 64 x
+// 330 x 128 11.7 / 11.6, 64 x 500 x 64 11.2 / 11.0), from 10 key tiles on behind (32 x 640 x 64 12.2 / 12.5, 32 x 640 x 128 16.6 / 17.5, 36 x 760 x 128 20.3 / 21.8,
+// 16 x 1700 x 128 31.9 / 35.8, 32 / 8 x 777 x 5000 x 128 87.2 / 96.9), with more blocks it always is (36 heads x 1014 x 128 28.9 / 31.3, 32 x 3000 x 128 93 / 107);
+// under a window at head dimension 64 from one block per CU on (5 heads x 4000 x 64, window 1024 20.6 / 19.9), at 128 from one and a half (12 /
+// 4 heads x 4096, window 512 45.8 / 42.9; 10 x 4000, window 300 41.5 / 38.7; 13 x 4000, window 1024 43.9 / 57.4).
 // Launches of up to half a block per CU go out in several parts of their key range per block, which makes the blocks: there 32
 // queries pay from 32 key tiles per CU on, where the workspace holds the parts' results (32 / 8 heads x 128 queries x 4000 keys x 128
-// 33.1 / 31.6, 20000 68.0 / 68.4; 64 / 8 x 64 x 20000 80.7 / 98.4, 16 x 1000 x 20000 x 64 116 / 126).
+// 31.4 / 30.3, 20000 68.0 / 68.4; 64 / 8 x 64 x 20000 80.7 / 98.4, 16 x 1000 x 20000 x 64 116 / 126).
 template <int D>
 bool attention_q32_wanted(const AttnArgs& args, int64_t blocks, bool in_parts)
 {
 	const int64_t cus = device_cu_count(), tiles = (args.n_k + kAttnKeysPerTile - 1) / kAttnKeysPerTile;
 	if (args.window > 0) return D == 64 ? blocks > cus : 2 * blocks > 3 * cus;
-	return blocks > cus || (2 * blocks <= cus && blocks * tiles > 32 * cus && in_parts);
+	if (2 * blocks > cus) return blocks > cus || tiles >= 10;
+	return blocks * tiles > 32 * cus && in_parts;
 }
 
 template <int D, bool SOFTCAP>
