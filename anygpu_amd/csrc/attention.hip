@@ -938,6 +938,7 @@ __global__ __launch_bounds__(64 * WAVES) void sdp_attention_fwd_f16_skew_kernel(
 }  // namespace anygpu
 
 #include "attention_f16_q32.hpp"
+#include "attention_f16_kwave.hpp"
 
 namespace anygpu {
 
@@ -1029,21 +1030,9 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 	constexpr int kLdsBytes = 2 * AttnLds<D>::kBytes;           // two stages
 	constexpr int kQueriesPerBlock = 16 * QB * WAVES;
 	(void)hipGetLastError();
-	if (kLdsBytes > 64 * 1024)
-	{
-		// more than 64 KB of dynamic LDS has to be granted per function and per device, once
-		static std::atomic<uint64_t> configured_devices{0};
-		int device = 0;
-		hipError_t e = hipGetDevice(&device);
-		if (e != hipSuccess) return e;
-		const uint64_t bit = 1ull << (device & 63);
-		if ((configured_devices.load(std::memory_order_relaxed) & bit) == 0)
-		{
-			e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-			if (e != hipSuccess) return e;
-			configured_devices.fetch_or(bit, std::memory_order_relaxed);
-		}
-	}
+	static std::atomic<uint64_t> configured_devices{0};
+	const hipError_t lds_err = grant_lds(kernel, kLdsBytes, configured_devices);
+	if (lds_err != hipSuccess) return lds_err;
 	AttnArgs args = args_in;
 	const int64_t q_blocks = (args.n_q + kQueriesPerBlock - 1) / kQueriesPerBlock;
 	AttnSplitPlan plan{0, 0};
@@ -1070,6 +1059,33 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 	return hipGetLastError();
 }
 
+// `heads` of `rows` rows each, `per_kv` of them on one key / value head
+template <int D, bool SOFTCAP, int WAVES>
+hipError_t launch_kwave_variant(const AttnArgs& args, int64_t heads, int64_t rows, int64_t per_kv, hipStream_t stream)
+{
+	constexpr int kLdsBytes = kKeyWaveLdsBytes<D, WAVES>;
+	const auto kernel = sdp_attention_fwd_f16_kwave_kernel<D, SOFTCAP, WAVES>;
+	(void)hipGetLastError();
+	static std::atomic<uint64_t> configured_devices{0};
+	const hipError_t lds_err = grant_lds(kernel, kLdsBytes, configured_devices);
+	if (lds_err != hipSuccess) return lds_err;
+	const AttnWalk walk = make_attn_walk((rows + kKeyWaveRows - 1) / kKeyWaveRows, heads, per_kv);
+	if (attn_walk_blocks(walk) > 0x7FFFFFFFLL) return hipErrorInvalidValue;
+	kernel<<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * WAVES), kLdsBytes, stream>>>(args, walk, (int)rows);
+	return hipGetLastError();
+}
+
+template <int D, bool SOFTCAP>
+hipError_t launch_kwave(const AttnArgs& args, int64_t heads, int64_t rows, int64_t per_kv, hipStream_t stream)
+{
+	// (head dimension 256: a block's LDS is a CU's either way, and eight waves are always ahead)
+	if constexpr (D != 256)
+	{
+		if (heads * ((rows + kKeyWaveRows - 1) / kKeyWaveRows) > device_cu_count()) return launch_kwave_variant<D, SOFTCAP, 4>(args, heads, rows, per_kv, stream);
+	}
+	return launch_kwave_variant<D, SOFTCAP, 8>(args, heads, rows, per_kv, stream);
+}
+
 // Head dimensions 64 and 128 take 32 queries per wave and two to three blocks per CU (attention_f16_q32.hpp) where there are blocks enough,
 // else 16 queries per wave.  At 256 the accumulators and queries of 32 rows leave that kernel no registers (8 / 4 heads x 8192 x 256, softcap 50, window 4096: 357 us against 300); the
 // skewed kernel serves it (16 queries per wave; the kernel above in one process: softcap 50 321 -> 276 us, without softcap
@@ -1077,6 +1093,8 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 template <int D>
 hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, hipStream_t stream)
 {
+	if (attention_kwave_wanted(D, batch_heads, args.n_q, args.n_k, args.causal, args.diag, args.window, device_cu_count()))
+		return softcap ? launch_kwave<D, true>(args, batch_heads, args.n_q, args.q_per_kv, stream) : launch_kwave<D, false>(args, batch_heads, args.n_q, args.q_per_kv, stream);
 	if constexpr (D == 256)
 		return softcap ? launch_variant<D, true, 1, true>(args, batch_heads, stream) : launch_variant<D, false, 1, true>(args, batch_heads, stream);
 	else
@@ -1388,7 +1406,8 @@ hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const v
 {
 	if (batch_heads == 0 || n_q == 0) return hipSuccess;
 	const int64_t kv_heads = batch_heads / q_per_kv;
-	const DecodePlan p = plans_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window).within(workspace_bytes);
+	const DecodePlansF16 plans = plans_decode_f16(batch_heads, q_per_kv, n_q, n_k, head_dim, causal, window);
+	const DecodePlan p = plans.within(workspace_bytes);
 	DecodeArgs da;
 	da.a.q = static_cast<const half_t*>(q);
 	da.a.k = static_cast<const half_t*>(k);
@@ -1411,6 +1430,19 @@ hipError_t launch_sdp_attention_decode_f16(const void* q, const void* k, const v
 	da.tiles_per_split = p.tiles_per_split;
 	da.t_first = p.t_first;
 	da.t_last = p.t_last;
+	// (by the finer tiles: the same for every size of workspace)
+	if (decode_kwave_wanted(head_dim, kv_heads * da.groups, plans.fine.t_last - plans.fine.t_first + 1, device_cu_count()))
+	{
+#define ANYGPU_DECODE_DIM(DIM) \
+		return capped ? launch_kwave<DIM, true>(da.a, kv_heads, da.rows, 1, stream) : launch_kwave<DIM, false>(da.a, kv_heads, da.rows, 1, stream)
+		switch (head_dim)
+		{
+		case 64: ANYGPU_DECODE_DIM(64);
+		case 128: ANYGPU_DECODE_DIM(128);
+		default: ANYGPU_DECODE_DIM(256);
+		}
+#undef ANYGPU_DECODE_DIM
+	}
 #define ANYGPU_DECODE_DIM(DIM) \
 	return capped ? launch_decode_variant<DIM, true>(da, kv_heads, stream) : launch_decode_variant<DIM, false>(da, kv_heads, stream)
 	switch (head_dim)

@@ -1226,24 +1226,6 @@ __global__ __launch_bounds__(split_threads(D, MASK), 2) void sdp_attention_fwd_f
 	}
 }
 
-// More than 64 KB of dynamic LDS has to be granted per function and per device, once.
-template <typename Kernel>
-hipError_t grant_lds(Kernel kernel, int bytes, std::atomic<uint64_t>& configured_devices)
-{
-	if (bytes <= 64 * 1024) return hipSuccess;
-	int device = 0;
-	hipError_t e = hipGetDevice(&device);
-	if (e != hipSuccess) return e;
-	const uint64_t bit = 1ull << (device & 63);
-	if ((configured_devices.load(std::memory_order_relaxed) & bit) == 0)
-	{
-		e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-		if (e != hipSuccess) return e;
-		configured_devices.fetch_or(bit, std::memory_order_relaxed);
-	}
-	return hipSuccess;
-}
-
 template <int D, bool MASK>
 constexpr int split_lds_bytes()
 {

@@ -232,4 +232,22 @@ hipError_t launch_gemm_band_ncontig(const float* A, const float* B, const float*
                                     int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                                     int epilogue, float ep_param, hipStream_t stream);
 
+// More than 64 KB of dynamic LDS has to be granted per function and per device, once.
+template <typename Kernel>
+inline hipError_t grant_lds(Kernel kernel, int bytes, std::atomic<uint64_t>& configured_devices)
+{
+	if (bytes <= 64 * 1024) return hipSuccess;
+	int device = 0;
+	hipError_t e = hipGetDevice(&device);
+	if (e != hipSuccess) return e;
+	const uint64_t bit = 1ull << (device & 63);
+	if ((configured_devices.load(std::memory_order_relaxed) & bit) == 0)
+	{
+		e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+		if (e != hipSuccess) return e;
+		configured_devices.fetch_or(bit, std::memory_order_relaxed);
+	}
+	return hipSuccess;
+}
+
 }  // namespace anygpu

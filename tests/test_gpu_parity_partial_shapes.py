@@ -178,6 +178,52 @@ def test_sdp_attention_32_queries_per_wave_tiles_in_pairs(ops, oracle, n_q, n_k,
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# launches of few query blocks: 16 rows per block, the tiles of 32 keys shared out among eight waves (up to a block per CU) or four (more: the copies).
+# Rows and keys on both sides of 16 and 32, as many tiles as waves and one more, blocks whose window starts behind the first tile,
+# queries that see nothing, and generation steps whose rows of several heads and queries share a block
+@pytest.mark.parametrize("copies", [1, 40])
+@pytest.mark.parametrize("heads,kv_heads,n_q,n_k,causal,window", [(4, 2, 17, 17, True, 0), (4, 1, 16, 31, False, 0), (2, 2, 33, 32, True, 0), (4, 4, 40, 257, True, 0),
+                                                                   (4, 2, 31, 288, False, 0), (4, 2, 100, 129, True, 33), (2, 1, 70, 600, False, 64), (4, 2, 60, 40, True, 0),
+                                                                   (4, 2, 80, 150, True, 1), (6, 2, 5, 300, True, 0), (8, 4, 1, 256, True, 0), (4, 4, 4, 319, True, 100),
+                                                                   (12, 4, 3, 290, False, 0), (40, 2, 1, 260, True, 0)])
+@pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 30.0, -0.0884), (256, 0.0, 0.0625), (256, 50.0, 0.0625)])
+def test_sdp_attention_few_rows_keys_over_waves(ops, oracle, heads, kv_heads, n_q, n_k, causal, window, d, cap, alpha, copies):
+    q = synth.normal(1 + n_q, (1, heads, n_q, d)).astype(np.float16)
+    k = synth.normal(2 + n_k, (1, kv_heads, n_k, d)).astype(np.float16) * np.float16(4.0)        # (scores of tens: the running maximum moves)
+    v = synth.normal(3 + d, (1, kv_heads, n_k, d)).astype(np.float16)
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, softcap=cap, causal=causal, window=window)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=alpha, softcap=cap,
+                                      causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
+    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
+    assert not got[0][blind].any() and np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    # p rounded to fp16 (2^-11 each, weights that sum to 1) and the result's own rounding, values of up to about 4
+    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
+
+
+@pytest.mark.parametrize("n_q", [1, 40])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_sdp_attention_few_rows_nan_infinities_and_large_scores(ops, n_q, d):
+    # a NaN in a query reaches its row, a NaN in the last key every row that sees it; among scores of 10^9 the largest one's row of v,
+    # bit for bit, whichever wave has it; strangers around the keys are never read
+    import torch
+    heads, n = 4, 288
+    q, k, v = (synth.normal(70 + i, (heads, m, d)).astype(np.float16) for i, m in enumerate((n_q, n, n)))
+    q[1, n_q // 2, 3] = np.nan
+    k[2, n - 1, 0] = np.nan
+    got = host(ops.sdp_attention_fwd(*(dev(t) for t in (q, k, v)), d ** -0.5, causal=True))
+    seen = np.zeros((heads, n_q), dtype=bool)
+    seen[1, n_q // 2] = seen[2, n_q - 1] = True
+    assert np.array_equal(np.isnan(got).all(-1), seen) and np.array_equal(np.isnan(got).any(-1), seen)
+    order = np.random.default_rng(6).permutation(n)
+    q = torch.full((1, heads, n_q, d), 10000.0, dtype=torch.half, device="cuda")
+    pool = torch.full((n + 64, d), math.nan, dtype=torch.half, device="cuda")
+    pool[32:32 + n] = dev((10000.0 - 16.0 * order)[:, None].repeat(d, axis=1).astype(np.float16))
+    v = synth.normal(9, (1, 1, n, d)).astype(np.float16)
+    got = host(ops.sdp_attention_fwd(q, pool[32:32 + n].view(1, 1, n, d), dev(v), 1.0))
+    assert np.array_equal(got, np.broadcast_to(v[0, 0, int(np.argmin(order))], got.shape))
+
+
 # The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
 # many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
 
