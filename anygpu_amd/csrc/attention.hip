@@ -1060,11 +1060,11 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 }
 
 // `heads` of `rows` rows each, `per_kv` of them on one key / value head
-template <int D, bool SOFTCAP, int WAVES>
+template <int D, bool SOFTCAP, bool MASK, int WAVES>
 hipError_t launch_kwave_variant(const AttnArgs& args, int64_t heads, int64_t rows, int64_t per_kv, hipStream_t stream)
 {
 	constexpr int kLdsBytes = kKeyWaveLdsBytes<D, WAVES>;
-	const auto kernel = sdp_attention_fwd_f16_kwave_kernel<D, SOFTCAP, WAVES>;
+	const auto kernel = sdp_attention_fwd_f16_kwave_kernel<D, SOFTCAP, MASK, WAVES>;
 	(void)hipGetLastError();
 	static std::atomic<uint64_t> configured_devices{0};
 	const hipError_t lds_err = grant_lds(kernel, kLdsBytes, configured_devices);
@@ -1075,15 +1075,15 @@ hipError_t launch_kwave_variant(const AttnArgs& args, int64_t heads, int64_t row
 	return hipGetLastError();
 }
 
-template <int D, bool SOFTCAP>
+template <int D, bool SOFTCAP, bool MASK = false>
 hipError_t launch_kwave(const AttnArgs& args, int64_t heads, int64_t rows, int64_t per_kv, hipStream_t stream)
 {
 	// (head dimension 256: a block's LDS is a CU's either way, and eight waves are always ahead)
 	if constexpr (D != 256)
 	{
-		if (heads * ((rows + kKeyWaveRows - 1) / kKeyWaveRows) > device_cu_count()) return launch_kwave_variant<D, SOFTCAP, 4>(args, heads, rows, per_kv, stream);
+		if (heads * ((rows + kKeyWaveRows - 1) / kKeyWaveRows) > device_cu_count()) return launch_kwave_variant<D, SOFTCAP, MASK, 4>(args, heads, rows, per_kv, stream);
 	}
-	return launch_kwave_variant<D, SOFTCAP, 8>(args, heads, rows, per_kv, stream);
+	return launch_kwave_variant<D, SOFTCAP, MASK, 8>(args, heads, rows, per_kv, stream);
 }
 
 // Head dimensions 64 and 128 take 32 queries per wave and two to three blocks per CU (attention_f16_q32.hpp) where there are blocks enough,
@@ -1093,7 +1093,7 @@ hipError_t launch_kwave(const AttnArgs& args, int64_t heads, int64_t rows, int64
 template <int D>
 hipError_t launch_dim(const AttnArgs& args, bool softcap, int64_t batch_heads, hipStream_t stream)
 {
-	if (attention_kwave_wanted(D, batch_heads, args.n_q, args.n_k, args.causal, args.diag, args.window, device_cu_count()))
+	if (attention_kwave_wanted(D, false, batch_heads, args.n_q, args.n_k, args.causal, args.diag, args.window, device_cu_count()))
 		return softcap ? launch_kwave<D, true>(args, batch_heads, args.n_q, args.q_per_kv, stream) : launch_kwave<D, false>(args, batch_heads, args.n_q, args.q_per_kv, stream);
 	if constexpr (D == 256)
 		return softcap ? launch_variant<D, true, 1, true>(args, batch_heads, stream) : launch_variant<D, false, 1, true>(args, batch_heads, stream);
@@ -1347,6 +1347,18 @@ hipError_t launch_sdp_attention_fwd_f16(const void* q, const void* k, const void
 	{
 		args.causal = 0;
 		args.window = 0;
+		if (attention_mask_map_from() == nullptr && attention_kwave_wanted((int)head_dim, true, batch_heads, args.n_q, args.n_k, 0, args.diag, 0, device_cu_count()))
+		{
+#define ANYGPU_ATTN_F16_MASK_DIM(DIM) \
+			return capped ? launch_kwave<DIM, true, true>(args, batch_heads, n_q, q_per_kv, stream) : launch_kwave<DIM, false, true>(args, batch_heads, n_q, q_per_kv, stream)
+			switch (head_dim)
+			{
+			case 64: ANYGPU_ATTN_F16_MASK_DIM(64);
+			case 128: ANYGPU_ATTN_F16_MASK_DIM(128);
+			default: ANYGPU_ATTN_F16_MASK_DIM(256);
+			}
+#undef ANYGPU_ATTN_F16_MASK_DIM
+		}
 		// The visible-tile map of the mask, at the front of the stream's workspace (the partial results of a split key
 		// range go behind it): worth its pass over the mask for large masks and long key ranges
 		// (attention_mask_map_wanted), and left out where the stream has no workspace to offer (a capture without a

@@ -27,7 +27,7 @@ constexpr int kKeyWaveTile = 32;                // keys of a tile: one MFMA step
 constexpr float kKeyWaveHeadRoom = 15.0f;
 
 // `walk`: blocks of 16 rows of a "head" of `rows` rows; row r is query r % n_q (rows = n_q, or where a key / value head's rows are
-// taken together, q_per_kv * n_q with fewer than 16 queries).
+// taken together, q_per_kv * n_q with fewer than 16 queries).  MASK: an additive mask tensor instead of the index rules.
 // Whether that kernel takes a launch of `heads` x n_q queries, by its blocks of 16 queries, the tiles of the longest (t_last) and what all of them cost: a
 // block's start and end are some five tiles.  us, 128 queries per block / here:
 //   * Up to a block for each CU the longest one decides: head dimension 256 up to 48 tiles (8 heads x 100 x 1400 23.3 / 20.8; but 100 x 2000 24.3 / 27.7), 128 up to 100 (16 x
@@ -36,7 +36,9 @@ constexpr float kKeyWaveHeadRoom = 15.0f;
 //     300 17.5 / 19.5, 8 x 949 without the causal rule 29.7 / 33.3.  128, up to three: 32 x 300 10.0 / 8.5, 32 x 250 x 1000 20.5 / 16.6, 64 x 160 7.7 / 7.2; but 64 x 200
 //     9.0 / 9.5, 32 x 400 x 1000 23.8 / 26.0; up to four where the kernels of 128 queries would have half a block for each CU, which they cut into parts: 16 x 800 21.8 / 14.5, 16 x
 //     1000 24.5 / 21.9.  64, up to four: 32 x 500 14.1 / 7.5, 64 x 250 7.3 / 5.9, 16 x 1000 without the causal rule 21.9 / 16.9; but 64 x 300 7.4 / 8.7.
-inline bool attention_kwave_wanted(int head_dim, int64_t heads, int n_q, int n_k, int causal, int diag, int window, int64_t cus)
+//   * A mask tensor, whose hidden tiles are not known ahead: 8 x 400 x 256 24.8 / 12.6, 200 x 1500 25.9 / 24.1 (but 600 26.8 / 26.3, 100 x 3000 28.2 / 40.1), 16 x 600 x 128 21.2 / 16.9,
+//     64 x 167 11.4 / 9.6 (but 32 x 422 17.1 / 18.4, 64 x 300 14.3 / 18.0, 64 x 200 x 1500 39.8 / 41.8), 16 x 1000 x 64 22.4 / 18.7, 32 x 100 x 3000 25.1 / 15.7 (but 32 x 1000 28.8 / 32.8).
+inline bool attention_kwave_wanted(int head_dim, bool mask, int64_t heads, int n_q, int n_k, int causal, int diag, int window, int64_t cus)
 {
 	const int64_t groups = (n_q + kKeyWaveRows - 1) / kKeyWaveRows, blocks = heads * groups;
 	if (blocks > 4 * cus) return false;
@@ -45,6 +47,7 @@ inline bool attention_kwave_wanted(int head_dim, int64_t heads, int n_q, int n_k
 	const int64_t longest = std::max(t_first, t_last);
 	if (blocks <= cus) return longest <= (head_dim == 256 ? 48 : head_dim == 128 ? 100 : 200);
 	const int64_t cost = blocks * (t_first + t_last + 10) / 2;          // (tiles grow evenly from the first group to the last, but for a window)
+	if (mask) return blocks <= (head_dim == 64 ? 4 : 3) * cus && cost <= (head_dim == 256 ? 26 : head_dim == 128 ? 110 : 200) * cus;
 	if (head_dim == 256) return 4 * blocks <= 9 * cus && longest <= 48 && cost <= 56 * cus;
 	if (head_dim == 128) return (blocks <= 3 * cus && cost <= 75 * cus) || (2 * heads * ((n_q + 127) / 128) <= cus && cost <= 90 * cus);
 	return cost <= 160 * cus;
@@ -61,7 +64,7 @@ inline bool decode_kwave_wanted(int64_t head_dim, int64_t blocks, int64_t tiles,
 template <int D, int WAVES>
 constexpr int kKeyWaveLdsBytes = (WAVES * kKeyWaveTile + kKeyWaveRows) * AttnLds<D>::kPitchV;
 
-template <int D, bool SOFTCAP, int WAVES>
+template <int D, bool SOFTCAP, bool MASK, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void sdp_attention_fwd_f16_kwave_kernel(const AttnArgs a, const AttnWalk walk, int rows)
 {
 	constexpr int ROWS = kKeyWaveRows, THREADS = 64 * WAVES;
@@ -111,6 +114,25 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 			*reinterpret_cast<float4_t*>(lds + (idx / VPR) * kPitchV + (idx % VPR) * 16) = src[i];
 		}
 	};
+	const int q_idx = one_head ? row0 + n : (row0 + n) % a.n_q;
+	// MASK: the values of this lane's scores of a tile, four consecutive halves of each half tile at any alignment; in the last tile keys
+	// past the end read nothing (their scores are masked)
+	half4_t mk[2] = {};
+	const half_t* const mask_row = MASK ? a.mask + (int64_t)(q_idx < a.n_q ? q_idx : a.n_q - 1) * a.mask_stride : nullptr;
+	auto fetch_mask = [&](int u) {
+		typedef half4_t LooseHalf4 __attribute__((aligned(2)));
+		const int key = kKeyWaveTile * u + 4 * g;
+#pragma unroll
+		for (int kb = 0; kb < 2; ++kb)
+		{
+			if ((u + 1) * kKeyWaveTile <= a.n_k) mk[kb] = *reinterpret_cast<const LooseHalf4*>(mask_row + key + 16 * kb);
+			else
+			{
+#pragma unroll
+				for (int r = 0; r < 4; ++r) mk[kb][r] = key + 16 * kb + r < a.n_k ? mask_row[key + 16 * kb + r] : (half_t)-INFINITY;
+			}
+		}
+	};
 	// the tile is this wave's alone: what it wrote is there, or what it reads has been read, once its counter says so
 	auto wait_lds = [&]() {
 		__builtin_amdgcn_s_waitcnt(0xC07F);               // lgkmcnt(0)
@@ -131,6 +153,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	if (u <= u_last)
 	{
 		fetch(kr, kp, u);
+		if constexpr (MASK) fetch_mask(u);
 		fetch(vr, vp, u);
 	}
 #pragma unroll
@@ -139,7 +162,6 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 		const int idx = tid + THREADS * i;
 		if (idx < ROWS * VPR) *reinterpret_cast<float4_t*>(q_lds + (idx / VPR) * kPitchV + (idx % VPR) * 16) = q_vec[i];
 	}
-	const int q_idx = one_head ? row0 + n : (row0 + n) % a.n_q;
 	const int vis_hi = a.causal && q_idx + a.diag < a.n_k - 1 ? q_idx + a.diag : a.n_k - 1;
 	const int vis_lo = a.window > 0 ? q_idx + a.diag - a.window + 1 : 0;
 
@@ -152,7 +174,12 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	{
 		const bool more = u + WAVES <= u_last;
 		put(kr);
-		if (more) fetch(kr, kp, u + WAVES);
+		const half4_t mask_now[2] = {mk[0], mk[1]};
+		if (more)
+		{
+			fetch(kr, kp, u + WAVES);
+			if constexpr (MASK) fetch_mask(u + WAVES);
+		}
 		wait_lds();
 		// ---- S^T = K Q^T ----
 		float4_t s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
@@ -180,7 +207,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 			for (int r = 0; r < 4; ++r)
 			{
 				const int key = kKeyWaveTile * u + 16 * kb + 4 * g + r;
-				const float zz = logit2<SOFTCAP>(s[kb][r], a.k_in, a.k_cap);
+				const float zz = logit2<SOFTCAP>(s[kb][r], a.k_in, a.k_cap) + (MASK ? (float)mask_now[kb][r] * kLog2e : 0.0f);
 				z[kb][r] = (key >= vis_lo && key <= vis_hi) ? zz : -INFINITY;
 				mt = fmaxf(mt, z[kb][r]);
 			}

@@ -67,6 +67,14 @@ __global__ __launch_bounds__(1024) void attention_mask_tile_map_kernel(const T* 
 	if (threadIdx.x == 0) map[(int64_t)q_block * groups + group] = (unsigned short)bits;
 }
 
+// The number in the environment that says from how many mask values on there is a map, or nullptr.  With one the launch goes to the kernels that have a form
+// with and without the map, whatever its size.
+inline const char* attention_mask_map_from()
+{
+	const char* text = std::getenv("ANYGPU_ATTN_MASK_MAP_FROM");
+	return text != nullptr && *text != 0 ? text : nullptr;
+}
+
 // Whether the map is made for a mask of n_q x n_k values.  Its pass costs a launch and a few memory latencies (8 - 12 us for
 // small masks, 5.6 TB/s for large ones), which short key ranges do not earn back: from 4 M mask values on, or from 16384 keys
 // on whatever the queries (a sliding window over a long cache hides most of them from a few queries as well).  The
@@ -75,8 +83,7 @@ __global__ __launch_bounds__(1024) void attention_mask_tile_map_kernel(const T* 
 // `needed`: the launch's kernel works on the map.
 inline bool attention_mask_map_wanted(int64_t n_q, int64_t n_k, bool needed = false)
 {
-	const char* text = std::getenv("ANYGPU_ATTN_MASK_MAP_FROM");
-	if (text != nullptr && *text != 0) return n_q * n_k >= std::atoll(text);
+	if (const char* text = attention_mask_map_from()) return n_q * n_k >= std::atoll(text);
 	return needed || n_q * n_k >= (4ll << 20) || n_k >= 16384;
 }
 

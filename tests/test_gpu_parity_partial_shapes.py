@@ -224,6 +224,47 @@ def test_sdp_attention_few_rows_nan_infinities_and_large_scores(ops, n_q, d):
     assert np.array_equal(got, np.broadcast_to(v[0, 0, int(np.argmin(order))], got.shape))
 
 
+# the same in float32 (tiles of 16 keys): fp32 sums of up to 300 products and weights
+@pytest.mark.parametrize("copies", [1, 40])
+@pytest.mark.parametrize("heads,kv_heads,n_q,n_k,causal,window", [(4, 2, 17, 17, True, 0), (4, 1, 16, 15, False, 0), (2, 2, 33, 16, True, 0), (4, 4, 40, 129, True, 0),
+                                                                   (4, 2, 31, 128, False, 0), (4, 2, 100, 145, True, 33), (2, 1, 70, 300, False, 64), (4, 2, 60, 40, True, 0),
+                                                                   (4, 2, 80, 150, True, 1), (4, 4, 1, 31, True, 0)])
+@pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 30.0, -0.0884), (256, 0.0, 0.0625), (256, 50.0, 0.0625)])
+def test_sdp_attention_f32_few_rows_keys_over_waves(ops, oracle, heads, kv_heads, n_q, n_k, causal, window, d, cap, alpha, copies):
+    q, k, v = (synth.normal(s + n, (1, h, n, d)) for s, h, n in ((1, heads, n_q), (2, kv_heads, n_k), (3, kv_heads, n_k)))
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, softcap=cap, causal=causal, window=window, decode=False))
+    want = oracle.sdp_attention_rules(q[0], k[0], v[0], alpha=alpha, softcap=cap, causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
+    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
+    assert not got[0][blind].any() and np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F32
+
+
+# and with a mask tensor: rows and tiles that it hides altogether, values of either sign, the type's lowest, keys that end inside a tile
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("heads,n_q,n_k", [(3, 1, 1), (2, 17, 15), (4, 33, 32), (2, 40, 257), (150, 30, 100), (3, 100, 131), (2, 16, 300)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_sdp_attention_mask_tensor_few_rows_keys_over_waves(ops, oracle, heads, n_q, n_k, d, dtype):
+    ndt = np.float16 if dtype == "f16" else np.float32
+    q, k, v = (synth.normal(s + n, (1, heads, n, d)).astype(ndt) for s, n in ((1, n_q), (2, n_k), (3, n_k)))
+    mask = synth.normal(7, (n_q, n_k)).astype(ndt)
+    if n_q > 2:
+        mask[:, n_k // 2:] = np.where(synth.normal(8, (n_q, n_k - n_k // 2)) > 0, -np.inf, mask[:, n_k // 2:])
+        mask[n_q // 3, :] = -np.inf                              # sees nothing: zeros
+        mask[n_q - 1, :] = np.finfo(ndt).min if dtype == "f16" else -1e30
+        mask[1, :n_k - 1] = -np.inf
+        mask[1, n_k - 1] = 0.0
+    if n_k > 64:
+        mask[:, 32:64] = -np.inf
+    got = host(ops.sdp_attention_masked_scaled_fwd(*(dev(t) for t in (q, k, v)), dev(mask).reshape(1, 1, n_q, n_k), d ** -0.5)).astype(np.float32)
+    wide = [oracle.cvt_f16_to_f32(t) if dtype == "f16" else t for t in (q, k, v, mask)]
+    want = oracle.sdp_attention_masked_scaled_fwd(*(t[:, :3] for t in wide[:3]), wide[3].reshape(1, 1, n_q, n_k), d ** -0.5, threads=8)
+    seen = np.isfinite(wide[3]).any(axis=-1)
+    assert not got[:, :, ~seen].any() and np.isfinite(got).all()
+    tol = TOL_F16_ROWOPS * 2 if dtype == "f16" else TOL_F32
+    assert scaled_rel_err(got[:, :3][:, :, seen], want[:, :, seen], 1.0) <= tol
+
+
 # The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
 # many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
 
