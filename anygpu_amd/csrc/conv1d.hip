@@ -7,8 +7,8 @@
 // neighbouring lane's vector, so every lane publishes the tail of its vector in LDS and reads
 // its left neighbour's after one barrier.  The halo in front of the whole tile comes from
 // global memory (zeros at the start of a row).
-// Element kernel: one thread per output sample, for sequence lengths or pointers that do not
-// allow 16-byte row access.
+// Rows whose tiles would be mostly empty or off the vectors' boundaries go as one run of vectors, short ones as (row, vector) pairs.
+// Element kernel: one thread per output sample, for rows shorter than a vector.
 #include "device_utils.hpp"
 #include "launch.hpp"
 
@@ -142,6 +142,140 @@ __global__ __launch_bounds__(256) void causal_conv1d_silu_tile_kernel(
 	}
 }
 
+// n / d for n < 2^32, inverse = floor(2^32 / d)
+__device__ __forceinline__ unsigned divide(unsigned n, unsigned d, unsigned inverse)
+{
+	const unsigned q = __umulhi(n, inverse);              // at most one too small
+	return n - q * d >= d ? q + 1 : q;
+}
+
+// The rows as one run of aligned vectors, wherever a row begins and ends: x and y are dense, so the vectors of the whole tensor are numbered and a block takes
+// 256 * U of them.  A thread's vector lies in one row or, at most eight samples from its end, in two; those that hold a row's first samples or
+// two rows go the long way, sample by sample with the taps of either channel.  Bound: HBM.  Rows of any length then move in whole tiles of aligned vectors, where the
+// kernel above takes a row of 4259 halves in two tiles of 512 vectors, the second with 21, at addresses off any boundary: 4 x 8320 x 4259 159 -> 99 us
+// (5.7 TB/s), 4224 x 8191 36.2 -> 25.8, aligned rows of 4264 (4 x 4224) 68.3 -> 51.7; float32 8320 x 2314 31.8 -> 25.7.
+template <typename T, int WIDTH, int U>
+__global__ __launch_bounds__(256) void causal_conv1d_silu_flat_kernel(
+	const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias, T* __restrict__ y,
+	unsigned chan, unsigned seqlen, unsigned chan_inverse, unsigned seq_inverse, int64_t total)
+{
+	constexpr int EPV = 16 / (int)sizeof(T);
+	constexpr int TPV = (int)(sizeof(typename ConvVec<T>::tail_type) / sizeof(T));
+	using Vec = typename ConvVec<T>::type;
+	using Tail = typename ConvVec<T>::tail_type;
+	// the taps of a channel at any alignment
+	struct Taps { T v[WIDTH]; __device__ T operator[](int k) const { return v[k]; } };
+	__shared__ Tail tails[U][256];
+
+	const int tid = threadIdx.x;
+	const int64_t start = (int64_t)blockIdx.x * (256 * U * EPV);       // sample of the tensor
+	Vec xv[U];
+#pragma unroll
+	for (int u = 0; u < U; ++u)
+	{
+		const int64_t at = start + (u * 256 + tid) * EPV;
+		Vec val = {};
+		if (at + EPV <= total) val = __builtin_nontemporal_load(reinterpret_cast<const Vec*>(x + at));
+		else
+		{
+#pragma unroll
+			for (int e = 0; e < EPV; ++e)
+				if (at + e < total) val[e] = x[at + e];
+		}
+		xv[u] = val;
+	}
+	Tail front = {};
+	if (tid == 0 && start > 0) front = *reinterpret_cast<const Tail*>(x + start - TPV);
+
+	// while the loads are on their way: the block's first row and its place in it, and of each vector
+	const unsigned row0 = total < (1ll << 32) ? divide((unsigned)start, seqlen, seq_inverse) : (unsigned)(start / seqlen);
+	const unsigned first = (unsigned)(start - (int64_t)row0 * seqlen), ch0 = row0 - divide(row0, chan, chan_inverse) * chan;
+	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	unsigned pos[U], ch[U];                                // pos: of the vector's first sample in its row
+	bool inside[U];                                        // the wave's 64 vectors are, in one row
+	Taps taps[U];
+	T bv[U];
+#pragma unroll
+	for (int u = 0; u < U; ++u)
+	{
+		const unsigned from = first + (unsigned)((u * 256 + wave * 64) * EPV);
+		const unsigned down = divide(from, seqlen, seq_inverse), pos0 = from - down * seqlen;
+		inside[u] = pos0 >= (unsigned)kHalo && pos0 + 64 * EPV <= seqlen;
+		pos[u] = pos0 + (tid & 63) * EPV;
+		ch[u] = ch0 + down;
+		if (!inside[u])
+		{
+			const unsigned more = divide(pos[u], seqlen, seq_inverse);
+			pos[u] -= more * seqlen;
+			ch[u] += more;
+		}
+		ch[u] -= divide(ch[u], chan, chan_inverse) * chan;
+		taps[u] = *reinterpret_cast<const Taps*>(w + (int64_t)ch[u] * WIDTH);
+		bv[u] = bias[ch[u]];
+	}
+#pragma unroll
+	for (int u = 0; u < U; ++u)
+	{
+		Tail t;
+#pragma unroll
+		for (int e = 0; e < TPV; ++e) t[e] = xv[u][EPV - TPV + e];
+		tails[u][tid] = t;
+	}
+	__syncthreads();
+
+#pragma unroll
+	for (int u = 0; u < U; ++u)
+	{
+		const int64_t at = start + (u * 256 + tid) * EPV;
+		if (at >= total) continue;
+		Tail prev;
+		if (tid > 0) prev = tails[u][tid - 1];
+		else if (u > 0) prev = tails[u - 1][255];
+		else prev = front;
+		float wv[kMaxWidth] = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+		for (int k = 0; k < WIDTH; ++k) wv[kMaxWidth - WIDTH + k] = (float)taps[u][k];
+		float s[kHalo + EPV];
+#pragma unroll
+		for (int e = 0; e < kHalo; ++e) s[e] = (float)prev[TPV - kHalo + e];
+#pragma unroll
+		for (int e = 0; e < EPV; ++e) s[kHalo + e] = (float)xv[u][e];
+		Vec out;
+		if (inside[u] || (pos[u] >= (unsigned)kHalo && pos[u] + EPV <= seqlen))
+		{
+#pragma unroll
+			for (int e = 0; e < EPV; ++e) out[e] = (T)conv_point<WIDTH>(wv, (float)bv[u], s[e], s[e + 1], s[e + 2], s[e + 3]);
+		}
+		else
+		{
+			const unsigned ch2 = ch[u] + 1 == chan ? 0 : ch[u] + 1;
+			const Taps taps2 = *reinterpret_cast<const Taps*>(w + (int64_t)ch2 * WIDTH);
+			float wv2[kMaxWidth] = { 0.f, 0.f, 0.f, 0.f };
+#pragma unroll
+			for (int k = 0; k < WIDTH; ++k) wv2[kMaxWidth - WIDTH + k] = (float)taps2[k];
+			const float bv2 = (float)bias[ch2];
+#pragma unroll
+			for (int e = 0; e < EPV; ++e)
+			{
+				const bool next = pos[u] + e >= seqlen;
+				const unsigned p = next ? pos[u] + e - seqlen : pos[u] + e;
+				float wp[kMaxWidth];
+#pragma unroll
+				for (int k = 0; k < kMaxWidth; ++k) wp[k] = next ? wv2[k] : wv[k];
+				// (samples in front of the row's first are zeros, whatever the row before holds)
+				out[e] = (T)conv_point<WIDTH>(wp, next ? bv2 : (float)bv[u], p >= 3 ? s[e] : 0.0f, p >= 2 ? s[e + 1] : 0.0f, p >= 1 ? s[e + 2] : 0.0f, s[e + 3]);
+			}
+		}
+		if (at + EPV <= total) __builtin_nontemporal_store(out, reinterpret_cast<Vec*>(y + at));
+		else
+		{
+#pragma unroll
+			for (int e = 0; e < EPV; ++e)
+				if (at + e < total) y[at + e] = out[e];
+		}
+	}
+}
+
 // Short rows: a row has fewer vectors than a tile of the kernel above has slots, so the tile would be mostly idle.
 // Here the (row, vector) pairs of the whole tensor are numbered consecutively and a block takes 256 of them,
 // whichever rows they belong to; a thread finds its halo in its left neighbour's tail unless its vector is
@@ -266,6 +400,19 @@ static hipError_t launch_width(const void* x, const void* w, const void* bias, v
 		// vectors per row, a partial last one included; rows shorter than the halo take the element kernel
 		const int64_t nvec = (seqlen + EPV - 1) / EPV;
 		const int64_t tiles_per_row = (nvec + 256 * U - 1) / (256 * U);
+		// Rows of four waves' vectors and more that start off the vectors' boundaries, or whose last tile would be mostly empty (one in sixteen vectors
+		// of the tiles and more), as one run of vectors, where the tensors themselves are aligned.  Below, every other wave holds a row's end and goes
+		// the long way: 2 x 4224 rows of 1170 halves 5 % slower, of 1000 17 % (with the norm beside it).
+		const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+		const bool wasteful = nvec >= 256 * U && 16 * nvec < 15 * tiles_per_row * 256 * U;
+		const int64_t total = rows * seqlen, flat_blocks = (total + 256 * U * EPV - 1) / (256 * U * EPV);
+		if (aligned && nvec >= 256 && (!vec_ok || wasteful) && flat_blocks <= 0x7FFFFFFFLL && rows < (1ll << 31) && seqlen < (1ll << 31))
+		{
+			discard_stale_error();
+			causal_conv1d_silu_flat_kernel<T, WIDTH, U><<<dim3((unsigned)flat_blocks), dim3(256), 0, stream>>>(xp, wp, bp, yp, (unsigned)chan, (unsigned)seqlen,
+				(unsigned)((1ull << 32) / (uint64_t)chan), (unsigned)((1ull << 32) / (uint64_t)seqlen), total);
+			return hipGetLastError();
+		}
 		const int64_t blocks = rows * tiles_per_row;
 		if (nvec < 256 * U && seqlen >= EPV && (rows * nvec + 255) / 256 <= 0x7FFFFFFFLL)
 		{

@@ -555,3 +555,23 @@ def test_mm_f16_small_products_as_they_lie(ops, m, n, k, layout, shift):
     got = host(ops.tensor_mm(av, wv, b_layout=lay)).astype(np.float64)
     assert np.all(np.isnan(got[0])) and not np.isfinite(got[1:, n - 1]).any()
     assert np.array_equal(got[1:, :n - 1], want[1:, :n - 1])
+
+
+# convolution over rows of any length as one run of vectors (256 vectors and more, off their boundaries or in tiles mostly empty): every remainder of
+# a row's end in a vector, rows that end with a block and one sample on, a single row, a last vector that is not whole; what
+# the row before holds (here NaN and infinities at its end) never reaches a row
+@pytest.mark.parametrize("dtype,b,d,s,width", [("f16", 1, 1, 2049, 4), ("f16", 3, 5, 2055, 4), ("f16", 2, 3, 4093, 3), ("f16", 1, 3, 4095, 4), ("f16", 2, 2, 4097, 2), ("f16", 3, 3, 4099, 1),
+                                               ("f16", 2, 7, 2042, 4), ("f16", 1, 5, 4168, 4), ("f16", 2, 3, 8190, 4), ("f32", 1, 1, 1021, 4), ("f32", 3, 5, 1026, 4),
+                                               ("f32", 2, 3, 2047, 3), ("f32", 2, 7, 2049, 2), ("f32", 1, 3, 2108, 4), ("f32", 2, 2, 1023, 1)])
+def test_conv1d_rows_as_one_run_of_vectors(ops, oracle, dtype, b, d, s, width):
+    ndt = np.float16 if dtype == "f16" else np.float32
+    x = synth.normal(s, (b, d, s)).astype(ndt)
+    w, bias = synth.normal(1, (d, width), std=0.5).astype(ndt), synth.normal(2, (d,), std=0.1).astype(ndt)
+    wide = [oracle.cvt_f16_to_f32(t) if dtype == "f16" else t for t in (x, w, bias)]
+    want = oracle.tensor_causal_conv1d(*wide, threads=4)
+    got = host(ops.tensor_causal_conv1d(dev(x), dev(w), dev(bias))).astype(np.float32)
+    assert scaled_rel_err(got, want, 1.0) <= (TOL_F16_ROWOPS if dtype == "f16" else TOL_F32)
+    x[0, 0, -3:] = np.array([np.nan, np.inf, np.nan])
+    again = host(ops.tensor_causal_conv1d(dev(x), dev(w), dev(bias))).astype(np.float32)
+    rows = again.reshape(b * d, s)
+    assert np.array_equal(rows[1:], got.reshape(b * d, s)[1:]) and np.array_equal(rows[0, :-3], got[0, 0, :-3]) and np.isnan(rows[0, -3:]).any()
