@@ -1038,7 +1038,7 @@ hipError_t launch_variant(const AttnArgs& args_in, int64_t batch_heads, hipStrea
 	AttnSplitPlan plan{0, 0};
 	if (D == 256 || MASK || attention_cut_longest<D>(args, q_blocks * batch_heads))
 		plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads,
-		                            kQueriesPerBlock, kAttnKeysPerTile, D, band::workspace_capacity(stream));
+		                            kQueriesPerBlock, kAttnKeysPerTile, D, band::workspace_capacity(stream), SKEW ? 1 : 0, SKEW);
 	// (or, with too few query blocks for the chip, every block in several parts of its key range)
 	const int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kQueriesPerBlock,
 	                                                                    kAttnKeysPerTile, D, band::workspace_capacity(stream));

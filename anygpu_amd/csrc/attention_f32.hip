@@ -1244,13 +1244,14 @@ namespace anygpu {
 
 namespace {
 
-// One launch over query blocks of QUERIES and tiles of KEYS, with the merge of whatever goes out in parts of its key range.
+// One launch over query blocks of QUERIES and tiles of KEYS, with the merge of whatever goes out in parts of its key range.  resident: as plan_attention_split
+// takes it.
 template <int D, int QUERIES, int KEYS, typename Launch>
-hipError_t launch_blocks_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t stream, Launch launch)
+hipError_t launch_blocks_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t stream, int resident, Launch launch)
 {
 	const int64_t q_blocks = (args.n_q + QUERIES - 1) / QUERIES;
 	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, QUERIES, KEYS, D,
-	                                                band::workspace_capacity(stream));
+	                                                band::workspace_capacity(stream), resident);
 	// (or, with too few query blocks for the chip, every block in several parts of its key range)
 	const int64_t parts_all = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, QUERIES, KEYS, D,
 	                                                                        band::workspace_capacity(stream));
@@ -1270,10 +1271,14 @@ hipError_t launch_blocks_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t
 	return hipGetLastError();
 }
 
+// blocks of the bf16 form that a CU holds (a mask tensor's have no lengths that are known ahead: 0)
+template <int D, bool MASK>
+constexpr int kSplitResident = MASK ? 0 : split_narrow(D, MASK) ? 1 : 2;
+
 template <int D, bool SOFTCAP, bool MASK>
 hipError_t launch_split_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t stream)
 {
-	return launch_blocks_f32<D, kSplitQueries, kSplitKeys>(args, batch_heads, stream, [&](const AttnWalk& walk) {
+	return launch_blocks_f32<D, kSplitQueries, kSplitKeys>(args, batch_heads, stream, kSplitResident<D, MASK>, [&](const AttnWalk& walk) {
 		auto kernel = sdp_attention_fwd_f32_split_kernel<D, SOFTCAP, MASK, false>;
 		static std::atomic<uint64_t> configured_devices{0};
 		const hipError_t err = grant_lds(kernel, split_lds_bytes<D, MASK>(), configured_devices);
@@ -1293,7 +1298,7 @@ hipError_t launch_plain_f32(AttnArgsF32& args, int64_t batch_heads, hipStream_t 
 	constexpr int WAVES = DIRECT ? 8 : 4;
 	constexpr int KT = DIRECT ? 32 : 64;
 	constexpr int kLdsBytes = AttnLdsF32<D, KT>::kStageFloats * 4 * (DIRECT ? 2 : 1);
-	return launch_blocks_f32<D, 16 * WAVES, KT>(args, batch_heads, stream, [&](const AttnWalk& walk) {
+	return launch_blocks_f32<D, 16 * WAVES, KT>(args, batch_heads, stream, 0, [&](const AttnWalk& walk) {
 		auto kernel = sdp_attention_fwd_f32_kernel<D, SOFTCAP, WAVES, KT, DIRECT, MASK>;
 		static std::atomic<uint64_t> configured_devices{0};
 		const hipError_t err = grant_lds(kernel, kLdsBytes, configured_devices);
@@ -1318,7 +1323,7 @@ bool attention_split_fills(const AttnArgsF32& args, int64_t batch_heads)
 	int64_t longest = 0;
 	for (int64_t b = q_blocks - 1, step = q_blocks / 64 + 1; b >= 0; b = args.window > 0 ? b - step : -1)
 		longest = std::max(longest, attention_block_tiles(b, args.n_q, args.n_k, args.causal, args.diag, args.window, kSplitQueries, kSplitKeys));
-	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, kSplitQueries, kSplitKeys, D, kRoom);
+	const AttnSplitPlan plan = plan_attention_split(args.n_q, args.n_k, args.causal, args.diag, args.window, batch_heads, kSplitQueries, kSplitKeys, D, kRoom, 2);
 	const int64_t parts = plan.n_split > 0 ? 1 : plan_attention_parts(args.n_q, args.n_k, args.causal, args.diag, batch_heads, kSplitQueries, kSplitKeys, D, kRoom);
 	if (parts == 1) return args.window == 0 || longest >= 21 || (longest >= 5 && q_blocks * batch_heads >= device_cu_count());
 	if (longest < 11) return false;

@@ -233,10 +233,18 @@ inline int64_t attention_block_tiles(int64_t block, int n_q, int n_k, int causal
 // halves).  Worth it when whole blocks cannot be packed evenly: at least a block per CU, and the longest block a large
 // share of what a CU gets of the whole launch.  Bounded by the workspace of the stream (the K-split workspace of the
 // GEMMs: a caller's, or the library's own for eager launches; none under capture without a caller's: then no split).
+//
+// `resident` > 0, the blocks that a CU holds at once: whole blocks also where they pack well enough.  A CU without a block is not lost altogether: the others run at a
+// higher clock, and the partial results cost their way through memory.  Not split: the longest block at most 1.31 of what a place for a block gets, and the second
+// round's longest on top of the first round's shortest at most 1.3 (one block per CU, us, split / whole, causal: half 8 heads x 8192 x 256 353 / 304, 16 x 3639 187 / 155, 16 x 3000
+// 136 / 112, 32 / 8 x 1339 67 / 54, 8 / 4 x 6000 window 4096 209 / 170; float32 32 / 8 x 1339 x 256 214 / 192, two per CU 32 / 8 x 3000 x 128 429 / 402).
+// `few`: of the blocks that would be split only as many as pay (half, head dimension 256): those beyond 1.35 of a place's share where the longest is beyond 1.45 (all /
+// whole / here: 8 x 4096 114 / 129 / 111, 8 x 4500 143 / 153 / 140, 16 x 2100 82 / 77 / 75; none at 8 / 4 x 5000 window 4096 162 / 151, 16 x 2600 106 / 96, whose longest are 1.39 and 1.42, nor
+// below 32 tiles: 32 / 16 x 1100 56 / 45), half of the longest ones where it is the second round that does not fit (8 / 4 x 8192 window 4096 278 / 299 / 271).
 struct AttnSplitPlan { int64_t n_split, n_big; };
 
 inline AttnSplitPlan plan_attention_split(int n_q, int n_k, int causal, int diag, int window, int64_t batch_heads,
-                                          int queries_per_block, int keys_per_tile, int head_dim, size_t capacity)
+                                          int queries_per_block, int keys_per_tile, int head_dim, size_t capacity, int resident = 0, bool few = false)
 {
 	AttnSplitPlan plan{0, 0};
 	const int64_t q_blocks = (n_q + queries_per_block - 1) / queries_per_block;
@@ -251,11 +259,33 @@ inline AttnSplitPlan plan_attention_split(int n_q, int n_k, int causal, int diag
 	}
 	const double per_cu = (double)total * (double)batch_heads / (double)cus;
 	if (longest < 16 || (double)longest <= 0.6 * per_cu) return plan;
-	const int64_t split_min = std::max<int64_t>(16, (int64_t)(0.6 * per_cu));
+	int64_t split_min = std::max<int64_t>(16, (int64_t)(0.6 * per_cu));
+	int64_t at_most = q_blocks;
+	if (resident > 0)
+	{
+		const double place = per_cu / resident;
+		// (the latest blocks are the longest)
+		const int64_t places = (int64_t)cus * resident, blocks = q_blocks * batch_heads;
+		const int64_t second = blocks > places ? tiles_of(q_blocks - 1 - (places - 1) / batch_heads) + tiles_of(q_blocks - 1 - places / batch_heads) : 0;
+		const bool unpacked = (double)second > 1.3 * place;
+		if ((double)longest <= 1.31 * place && !unpacked) return plan;
+		if (few && (double)longest > 1.45 * place)
+		{
+			if (longest < 32) return plan;
+			split_min = std::max(split_min, (int64_t)(1.35 * place) + 1);
+		}
+		else if (few)
+		{
+			if (!unpacked) return plan;
+			int64_t long_ones = 0;
+			while (long_ones < q_blocks && 10 * tiles_of(q_blocks - 1 - long_ones) >= 9 * longest) ++long_ones;
+			at_most = long_ones / 2;
+		}
+	}
 	// the latest blocks that are long enough, as far as the workspace holds their partial results
 	const int64_t room = (int64_t)(capacity / ((size_t)batch_heads * 2 * queries_per_block * (head_dim + 2) * sizeof(float)));
 	int64_t n_split = 0;
-	while (n_split < q_blocks && n_split < room && tiles_of(q_blocks - 1 - n_split) >= split_min) ++n_split;
+	while (n_split < at_most && n_split < room && tiles_of(q_blocks - 1 - n_split) >= split_min) ++n_split;
 	if (n_split == 0) return plan;
 	int64_t n_big = 0;
 	while (n_split + n_big < q_blocks && 2 * tiles_of(q_blocks - 1 - n_split - n_big) > longest) ++n_big;
