@@ -1006,7 +1006,8 @@ hipError_t launch_q32(const AttnArgs& args_in, int64_t batch_heads, hipStream_t 
 		const hipError_t ws_err = band::workspace_acquire(stream, &args.partials);
 		if (ws_err != hipSuccess) return ws_err;
 	}
-	const AttnWalk walk = make_attn_walk(q_blocks, batch_heads, args.q_per_kv, plan.n_split, plan.n_big, parts_all);
+	const AttnWalk walk = make_attn_walk(q_blocks, batch_heads, args.q_per_kv, plan.n_split, plan.n_big, parts_all,
+	                                     plan.n_split > 0 || parts_all > 1 ? 0 : device_cu_count() / kAttnXcds);
 	if (attn_walk_blocks(walk) > 0x7FFFFFFFLL) return hipErrorInvalidValue;
 	sdp_attention_fwd_f16_q32_kernel<D, SOFTCAP><<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * kQ32Waves), kLdsBytes, stream>>>(args, walk);
 	hipError_t err = hipGetLastError();

@@ -15,8 +15,9 @@
 // rounded p by v_dot2 measured 5 % faster, but up to a tenth further from 64-bit results: 16 heads x 4096 x 128, q of
 // N(0, 4): 2.36e-4 against 2.17e-4 (2-norm), of which the result's own rounding is 2.1e-4).
 // Measured, causal (us; products and softmax in turn -> here, the same bits): 16 x 4096 x 128 102.3 -> 91.7, 64 / 8 x 1000 x 128 32.0 -> 29.9, 16 x 8192 x
-// 128 315 -> 299, 2 x 16 x 2280 x 128 63.3 -> 58.7, 32 x 2038 x 64 36.5 -> 32.8, 32 x 4000 x 64 window 500 36.9 -> 34.5, 32 / 8 x 3000 x 128 93.7 -> 95.0 (query
-// blocks of 1 to 47 tiles that do not pack evenly, 20 % of the CU time idle); without the causal rule 32 / 8 x 3000 x 128 173 -> 161.
+// 128 315 -> 299, 2 x 16 x 2280 x 128 63.3 -> 58.7, 32 / 8 x 3000 x 128 93.3 -> 91.4, 4096 166 -> 153, 32 x 2038 x 64 36.5 -> 32.8, 32 x 4000 x 64 window 500
+// 36.9 -> 34.5; without the causal rule 32 / 8 x 3000 x 128 177 -> 159.  Slower where many blocks walk some five tiles (128 / 8 x 300 x 128 12.4 -> 13.1), and where the
+// last of them do not fill the places (16 / 8 x 2600 x 128 52.2 -> 53.7).
 #pragma once
 
 #include "attention_walk.hpp"
@@ -91,6 +92,10 @@ __global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention
 		t_first += part * per;
 		if (t_first + per - 1 < t_last) t_last = t_first + per - 1;
 	}
+
+	// A SIMD issues from the older of its two waves while that one can: blocks behind the first two rounds go first instead, whose partner is nearer to its end (us, causal: 32 /
+	// 8 heads x 3000 x 128 91.2 -> 90.1, 3200 100.3 -> 98.4, window 1024 60.6 -> 58.7, 128 / 8 x 579 27.8 -> 26.9; three blocks on a CU, head dimension 64, are slower with it: 32 / 8 x 3000 55.0 / 57.9).
+	if (D == 128 && walk.turn > 0 && (int)blockIdx.x >= 2 * kAttnXcds * walk.turn) __builtin_amdgcn_s_setprio(1);
 
 	// this wave's queries as second operands: lane (n, h) holds q[row][16 s + 8 h .. + 7]
 	const int wq0 = q0 + 32 * wave;

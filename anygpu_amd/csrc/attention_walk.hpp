@@ -42,12 +42,18 @@ struct AttnWalk
 	int n_split;         // the latest n_split query blocks of a head are dispatched in two halves of their key range
 	int n_big;           // unsplit blocks dispatched before the halves
 	int parts_all;       // > 1: every query block is dispatched as that many blocks, one per part of its key range
+	int turn;            // > 0: the blocks turn .. 2 turn - 1 of an XCD are dispatched lightest first
 };
 
 // parts_all > 1 (launches with too few query blocks for the chip, long key ranges): n_split and n_big do not apply, the
 // partial results are laid out as if every query block were a split one (slot = blocks from the last).
+//
+// turn (kernels of two or three blocks per CU, whole blocks): the CUs of an XCD.  The first round of blocks puts one on each of them, heaviest first, and the
+// second, in the same order, would put its heaviest with the heaviest of the first: backwards, the sums are nearly equal (half, causal: 32 / 8 heads x 3000 x 128 91.2 ->
+// 88.0 us, 32 / 8 x 4096 x 128 150 -> 146, 32 / 8 x 3000 x 64 55.0 -> 50.5, 64 / 8 x 1404 x 128 48.7 -> 46.5; third rounds backwards 93 and 158 us of the first two).
+// Only where the second round is nearly full, as its lightest blocks go where a place is first: 16 / 8 x 3600 (58 blocks per XCD) 75.0 -> 72.7, but 2600 (42) 51.9 / 52.9, 3000 (48) 62.5 / 64.7.
 inline AttnWalk make_attn_walk(int64_t q_blocks, int64_t batch_heads, int64_t q_per_kv, int64_t n_split = 0, int64_t n_big = 0,
-                               int64_t parts_all = 1)
+                               int64_t parts_all = 1, int64_t turn = 0)
 {
 	AttnWalk w;
 	w.real_q_blocks = (int)q_blocks;
@@ -67,6 +73,7 @@ inline AttnWalk make_attn_walk(int64_t q_blocks, int64_t batch_heads, int64_t q_
 	w.chunks = (w.q_blocks + w.chunk - 1) / w.chunk;
 	w.units = w.chunks * w.groups;
 	w.units_per_xcd = (w.units + kAttnXcds - 1) / kAttnXcds;
+	w.turn = 4 * (int64_t)w.units_per_xcd * w.chunk * w.q_per_kv >= 7 * turn ? (int)turn : 0;
 	return w;
 }
 
@@ -90,8 +97,13 @@ __device__ __forceinline__ bool attn_walk_locate_part(const AttnWalk& w, unsigne
                                                       int& part, int& parts, int& split_slot)
 {
 	const int xcd = (int)(block % kAttnXcds);
-	const int slot = (int)(block / kAttnXcds);
+	int slot = (int)(block / kAttnXcds);
 	const int per_unit = w.chunk * w.q_per_kv;
+	if (slot >= w.turn && slot < 2 * w.turn)
+	{
+		const int all = w.units_per_xcd * per_unit;
+		slot = w.turn - 1 + (all < 2 * w.turn ? all : 2 * w.turn) - slot;
+	}
 	const int unit = (slot / per_unit) * kAttnXcds + xcd;
 	const int member = slot % per_unit;
 	if (unit >= w.units) return false;

@@ -178,6 +178,17 @@ def test_sdp_attention_32_queries_per_wave_tiles_in_pairs(ops, oracle, n_q, n_k,
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# the same kernel where the second round of blocks is dispatched backwards: 55 to 76 blocks per XCD, with padding at the end of a head and of the launch
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("copies,heads,kv_heads,n,causal", [(7, 4, 2, 1930, True), (40, 4, 2, 300, True), (37, 4, 2, 300, True), (31, 5, 1, 260, True), (64, 4, 4, 200, False), (33, 4, 2, 510, True)])
+def test_sdp_attention_32_queries_per_wave_second_round_backwards(ops, oracle, copies, heads, kv_heads, n, causal, d):
+    q, k, v = (synth.normal(s + n, (1, h, n, d)).astype(np.float16) for s, h in ((1, heads), (2, kv_heads), (3, kv_heads)))
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), d ** -0.5, causal=causal)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=d ** -0.5, softcap=0.0, causal=causal, window=0, q_per_kv=heads // kv_heads, threads=8)
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2
+
+
 # launches of few query blocks: 16 rows per block, the tiles of 32 keys shared out among eight waves (up to a block per CU) or four (more: the copies).
 # Rows and keys on both sides of 16 and 32, as many tiles as waves and one more, blocks whose window starts behind the first tile,
 # queries that see nothing, and generation steps whose rows of several heads and queries share a block
