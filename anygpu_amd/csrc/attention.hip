@@ -951,8 +951,9 @@ namespace {
 //   * One block for each CU: where the blocks run from near nothing to the whole range from 41 tiles on (8 heads x 4086 x 128 68.5 / 56.7, 8 x 4000
 //     x 64 49.5 / 37.8; but 16 x 2038 x 128 37.9 / 41.2, x 64 28.2 / 29.1), else from 101 on, where two shorter blocks on a CU overlap enough to pay
 //     for the partial results' way through memory (no causal rule: 4 heads x 8182 x 64 98.7 / 95.9; but 8 x 4086 x 64 52.9 / 56.6).
-//   * More blocks: such a triangle of blocks only, up to one and a quarter for each CU (10 heads x 4086 x 128 77.6 / 66.5, 18 x 2038 45.1 / 43.9; 11
-//     x 4086 77.7 / 79.2), at head dimension 64 with very long ranges up to two (7 heads x 8182 x 64 104 / 102).
+//   * More blocks: such a triangle of blocks only, up to one and a quarter for each CU (10 heads x 4086 x 128 77.6 / 66.5, 18 x 2038 45.1 / 43.9), up to 1.4
+//     where it starts at the first key (16 / 8 x 2600 x 128 52.7 / 48.2, 12 / 4 x 3500 66.9 / 59.2, 8 x 5300 x 64 52.7 / 52.0, 11 x 4086 x 128 76.8 / 74.7; but 16 / 8 x 2600 x
+//     3200 keys 69.5 / 71.2, 8 x 5200 x 6000 99.9 / 101.9, 10 x 4700 x 128 86.6 / 89.1), at head dimension 64 with very long ranges up to two (7 heads x 8182 x 64 104 / 102).
 template <int D>
 bool attention_cut_longest(const AttnArgs& args, int64_t blocks)
 {
@@ -960,7 +961,7 @@ bool attention_cut_longest(const AttnArgs& args, int64_t blocks)
 	if (args.window > 0) return blocks > cus && 2 * blocks <= 3 * cus;
 	const bool triangle = args.causal && 2 * args.diag <= args.n_q;
 	if (blocks <= cus) return tiles > (triangle ? 40 : 100);
-	return triangle && ((tiles > 30 && 4 * blocks <= 5 * cus) || (D == 64 && tiles >= 96 && blocks <= 2 * cus));
+	return triangle && ((tiles > 30 && (4 * blocks <= 5 * cus || (5 * blocks <= 7 * cus && 8 * args.diag <= args.n_q))) || (D == 64 && tiles >= 96 && blocks <= 2 * cus));
 }
 
 // Head dimensions 64 and 128, index rules: whether the kernel with 32 queries per wave takes the launch (`blocks` of 128 queries in all).

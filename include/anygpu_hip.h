@@ -348,7 +348,8 @@ int anygpu_sdp_attention_fwd_masked_f16(const void* q, const void* k, const void
  * arguments the decode form rejects); workspace must be 16-byte aligned device memory of at least that size and
  * may be reused by the next call on the same stream.  (The range is cut in tiles of 32 keys; a workspace below that size
  * which still holds the partial results of a cut in tiles of 64 is accepted and gets that cut, whose sums round
- * differently.  From that size on the bytes handed in make no difference.)  The reference has no decode kernel: its generation step
+ * differently.  From that size on the bytes handed in make no difference.)  Short ranges run in one launch without partial results in memory; their
+ * workspace is checked as any other's and left alone.  The reference has no decode kernel: its generation step
  * runs the per-head loop of srcs/transformers/sdp.hpp:258-271 against the cached keys.
  */
 int64_t anygpu_sdp_attention_decode_workspace_bytes(int64_t batch_heads, int64_t q_per_kv, int64_t n_q, int64_t n_k,

@@ -251,15 +251,16 @@ def test_sdp_attention_f32_few_rows_keys_over_waves(ops, oracle, heads, kv_heads
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F32
 
 
-# head dimension 256, the long query blocks of a causal launch: some in two halves of their keys and some that as long stay whole (2100 keys; two rounds of blocks
-# under a window), all of them (float32), none (1100 and 1339); sequence ends inside and on a block and a tile
-@pytest.mark.parametrize("dtype,copies,heads,kv_heads,n,window", [("f16", 4, 4, 2, 2100, 0), ("f16", 8, 4, 2, 2048, 1024), ("f16", 8, 4, 2, 1100, 0), ("f16", 5, 3, 1, 2111, 1500),
-                                                                  ("f32", 2, 4, 4, 2100, 0), ("f32", 8, 4, 1, 1339, 0), ("f32", 4, 4, 2, 1536, 1000)])
-def test_sdp_attention_causal_blocks_partly_in_halves(ops, oracle, dtype, copies, heads, kv_heads, n, window):
-    half = dtype == "f16"
-    q, k, v = (synth.normal(s + n, (1, h, n, 256)).astype(np.float16 if half else np.float32) for s, h in ((1, heads), (2, kv_heads), (3, kv_heads)))
-    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), 0.0625, softcap=50.0, causal=True, window=window)).astype(np.float32)
-    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] if half else t[0] for t in (q, k, v)), alpha=0.0625, softcap=50.0, causal=True, window=window,
+# the long query blocks of a causal launch: at head dimension 256 some in two halves of their keys and some that as long stay whole (2100 keys; two rounds of blocks
+# under a window), all of them (float32), none (1100 and 1339); at 64 and 128 up to one and a third block per CU; sequence ends inside and on a block and a tile
+@pytest.mark.parametrize("dtype,copies,heads,kv_heads,n,window,d", [("f16", 4, 4, 2, 2100, 0, 256), ("f16", 8, 4, 2, 2048, 1024, 256), ("f16", 8, 4, 2, 1100, 0, 256), ("f16", 5, 3, 1, 2111, 1500, 256),
+                                                                    ("f32", 2, 4, 4, 2100, 0, 256), ("f32", 8, 4, 1, 1339, 0, 256), ("f32", 4, 4, 2, 1536, 1000, 256),
+                                                                    ("f16", 4, 4, 2, 2600, 0, 128), ("f16", 4, 4, 2, 2600, 0, 64), ("f16", 4, 4, 2, 2688, 0, 128)])
+def test_sdp_attention_causal_blocks_partly_in_halves(ops, oracle, dtype, copies, heads, kv_heads, n, window, d):
+    half, alpha = dtype == "f16", d ** -0.5
+    q, k, v = (synth.normal(s + n, (1, h, n, d)).astype(np.float16 if half else np.float32) for s, h in ((1, heads), (2, kv_heads), (3, kv_heads)))
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, softcap=50.0, causal=True, window=window)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] if half else t[0] for t in (q, k, v)), alpha=alpha, softcap=50.0, causal=True, window=window,
                                       q_per_kv=heads // kv_heads, threads=8)
     assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
     assert scaled_rel_err(got[0], want, 1.0) <= (TOL_F16_ROWOPS * 2 if half else TOL_F32)
