@@ -142,7 +142,8 @@ __global__ __launch_bounds__(256) void causal_conv1d_silu_tile_kernel(
 	}
 }
 
-// n / d for n < 2^32, inverse = floor(2^32 / d)
+// n / d for n < 2^32 with inverse = inverse_of(d): floor(2^32 / d), for d = 1 the 2^32 - 1 that an unsigned holds
+__host__ __device__ __forceinline__ unsigned inverse_of(unsigned d) { return d == 1 ? 0xFFFFFFFFu : (unsigned)((1ull << 32) / d); }
 __device__ __forceinline__ unsigned divide(unsigned n, unsigned d, unsigned inverse)
 {
 	const unsigned q = __umulhi(n, inverse);              // at most one too small
@@ -410,7 +411,7 @@ static hipError_t launch_width(const void* x, const void* w, const void* bias, v
 		{
 			discard_stale_error();
 			causal_conv1d_silu_flat_kernel<T, WIDTH, U><<<dim3((unsigned)flat_blocks), dim3(256), 0, stream>>>(xp, wp, bp, yp, (unsigned)chan, (unsigned)seqlen,
-				(unsigned)((1ull << 32) / (uint64_t)chan), (unsigned)((1ull << 32) / (uint64_t)seqlen), total);
+				inverse_of((unsigned)chan), inverse_of((unsigned)seqlen), total);
 			return hipGetLastError();
 		}
 		const int64_t blocks = rows * tiles_per_row;

@@ -601,3 +601,20 @@ def test_conv1d_rows_as_one_run_of_vectors(ops, oracle, dtype, b, d, s, width):
     again = host(ops.tensor_causal_conv1d(dev(x), dev(w), dev(bias))).astype(np.float32)
     rows = again.reshape(b * d, s)
     assert np.array_equal(rows[1:], got.reshape(b * d, s)[1:]) and np.array_equal(rows[0, :-3], got[0, 0, :-3]) and np.isnan(rows[0, -3:]).any()
+
+
+# one channel, where every row has the same taps: batches of two to sixteen rows, whose row number is no channel's, off the vectors' boundaries and with a nearly empty
+# last tile, taps and bias as slices of buffers that hold NaN everywhere else
+@pytest.mark.parametrize("dtype,b,s,width", [("f16", 2, 2049, 4), ("f16", 3, 4095, 2), ("f16", 4, 2049, 4), ("f16", 9, 4259, 3), ("f16", 16, 4168, 4), ("f16", 4, 4168, 1),
+                                             ("f32", 2, 1025, 4), ("f32", 4, 1025, 4), ("f32", 9, 2049, 2), ("f32", 16, 2108, 4)])
+def test_conv1d_rows_as_one_run_of_vectors_one_channel(ops, oracle, dtype, b, s, width):
+    import torch
+    ndt = np.float16 if dtype == "f16" else np.float32
+    x = synth.normal(s, (b, 1, s)).astype(ndt)
+    w, bias = synth.normal(1, (1, width), std=0.5).astype(ndt), synth.normal(2, (1,), std=0.1).astype(ndt)
+    wide = [oracle.cvt_f16_to_f32(t) if dtype == "f16" else t for t in (x, w, bias)]
+    want = oracle.tensor_causal_conv1d(*wide, threads=4)
+    pool = torch.full((256,), math.nan, dtype=torch.float16 if dtype == "f16" else torch.float32, device="cuda")
+    pool[64:64 + width], pool[160] = dev(w[0]), float(bias[0])
+    got = host(ops.tensor_causal_conv1d(dev(x), pool[64:64 + width].view(1, width), pool[160:161])).astype(np.float32)
+    assert scaled_rel_err(got, want, 1.0) <= (TOL_F16_ROWOPS if dtype == "f16" else TOL_F32)
