@@ -175,6 +175,17 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 		const bool more = u + WAVES <= u_last;
 		put(kr);
 		const half4_t mask_now[2] = {mk[0], mk[1]};
+		// a tile that the mask hides from every query of the block takes no part, whatever its keys and values hold
+		bool visible = true;
+		if constexpr (MASK)
+		{
+			bool any = false;
+#pragma unroll
+			for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+				for (int r = 0; r < 4; ++r) any |= mask_now[kb][r] > (half_t)(-INFINITY);
+			visible = __builtin_amdgcn_ballot_w64(any) != 0;
+		}
 		if (more)
 		{
 			fetch(kr, kp, u + WAVES);
@@ -183,20 +194,24 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 		wait_lds();
 		// ---- S^T = K Q^T ----
 		float4_t s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-#pragma unroll
-		for (int st = 0; st < KS; ++st)
+		if (visible)
 		{
-			const half8_t qf = *reinterpret_cast<const half8_t*>(q_lds + n * kPitchV + (32 * st + 8 * g) * 2);
 #pragma unroll
-			for (int kb = 0; kb < 2; ++kb)
+			for (int st = 0; st < KS; ++st)
 			{
-				const half8_t kf = *reinterpret_cast<const half8_t*>(lds + (16 * kb + n) * kPitchV + (32 * st + 8 * g) * 2);
-				s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf, s[kb], 0, 0, 0);
+				const half8_t qf = *reinterpret_cast<const half8_t*>(q_lds + n * kPitchV + (32 * st + 8 * g) * 2);
+#pragma unroll
+				for (int kb = 0; kb < 2; ++kb)
+				{
+					const half8_t kf = *reinterpret_cast<const half8_t*>(lds + (16 * kb + n) * kPitchV + (32 * st + 8 * g) * 2);
+					s[kb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf, s[kb], 0, 0, 0);
+				}
 			}
 		}
 		wait_lds();
 		put(vr);
 		if (more) fetch(vr, vp, u + WAVES);
+		if (!visible) continue;
 
 		// ---- online softmax ----
 		float z[2][4];

@@ -133,6 +133,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	if (u <= u_last)
 	{
 		fetch_k(u);
+		if constexpr (MASK) fetch_mask(u);
 		fetch_v(u);
 	}
 #pragma unroll
@@ -160,60 +161,77 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 			const int idx = lane + 64 * i;
 			*reinterpret_cast<float4_t*>(lds + (idx / VPR) * kPitch + (idx % VPR) * 4) = kr[i];
 		}
-		if constexpr (MASK) fetch_mask(u);
-		if (more) fetch_k(u + WAVES);
+		const float4_t mask_now = mk;
+		// a tile that the mask hides from every query of the block (-inf, or the lowest float, which is -inf as a logit) takes no part, whatever its
+		// keys and values hold
+		bool visible = true;
+		if constexpr (MASK)
+		{
+			bool any = false;
+#pragma unroll
+			for (int r = 0; r < 4; ++r) any |= mask_now[r] * kLog2e > -INFINITY;
+			visible = __builtin_amdgcn_ballot_w64(any) != 0;
+		}
+		if (more)
+		{
+			fetch_k(u + WAVES);
+			if constexpr (MASK) fetch_mask(u + WAVES);
+		}
 		wait_lds();
 		// ---- S^T = K Q^T: even and odd elements in sums of their own ----
 		float4_t s[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-#pragma unroll
-		for (int st = 0; st < KS; ++st)
+		if (visible)
 		{
-			const float4_t kf = *reinterpret_cast<const float4_t*>(lds + n * kPitch + 16 * st + 4 * g);
-			const float4_t qf = *reinterpret_cast<const float4_t*>(q_lds + n * kPitch + 16 * st + 4 * g);
 #pragma unroll
-			for (int e = 0; e < 4; ++e) s[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], s[e & 1], 0, 0, 0);
-		}
-		wait_lds();
+			for (int st = 0; st < KS; ++st)
+			{
+				const float4_t kf = *reinterpret_cast<const float4_t*>(lds + n * kPitch + 16 * st + 4 * g);
+				const float4_t qf = *reinterpret_cast<const float4_t*>(q_lds + n * kPitch + 16 * st + 4 * g);
+#pragma unroll
+				for (int e = 0; e < 4; ++e) s[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], s[e & 1], 0, 0, 0);
+			}
+			wait_lds();
 
-		// ---- online softmax ----
-		float z[4];
-		float mt = -INFINITY;
+			// ---- online softmax ----
+			float z[4];
+			float mt = -INFINITY;
 #pragma unroll
-		for (int r = 0; r < 4; ++r)
-		{
-			const int key = KT * u + 4 * g + r;
-			const float zz = logit2<SOFTCAP>(s[0][r] + s[1][r], a.k_in, a.k_cap) + (MASK ? mk[r] * kLog2e : 0.0f);
-			z[r] = (key >= vis_lo && key <= vis_hi) ? zz : -INFINITY;
-			mt = fmaxf(mt, z[r]);
-		}
-		mt = max_over_lane_rows(mt);
-		const float m_new = fmaxf(m_run, mt);
-		const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
-		if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0)
-		{
-			const float corr = fast_exp2(m_run - m_safe);
-			l_run *= corr;
+			for (int r = 0; r < 4; ++r)
+			{
+				const int key = KT * u + 4 * g + r;
+				const float zz = logit2<SOFTCAP>(s[0][r] + s[1][r], a.k_in, a.k_cap) + (MASK ? mask_now[r] * kLog2e : 0.0f);
+				z[r] = (key >= vis_lo && key <= vis_hi) ? zz : -INFINITY;
+				mt = fmaxf(mt, z[r]);
+			}
+			mt = max_over_lane_rows(mt);
+			const float m_new = fmaxf(m_run, mt);
+			const float m_safe = (m_new == -INFINITY) ? 0.0f : m_new;
+			if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0)
+			{
+				const float corr = fast_exp2(m_run - m_safe);
+				l_run *= corr;
 #pragma unroll
-			for (int c = 0; c < DC; ++c)
+				for (int c = 0; c < DC; ++c)
 #pragma unroll
-				for (int e = 0; e < 4; ++e) o[c][e] *= corr;
-		}
-		m_run = m_new;
-		float p[4];
+					for (int e = 0; e < 4; ++e) o[c][e] *= corr;
+			}
+			m_run = m_new;
+			float p[4];
 #pragma unroll
-		for (int r = 0; r < 4; ++r)
-		{
-			p[r] = fast_exp2(z[r] - m_safe);
-			l_run += p[r];
-		}
+			for (int r = 0; r < 4; ++r)
+			{
+				p[r] = fast_exp2(z[r] - m_safe);
+				l_run += p[r];
+			}
 
-		// ---- O^T += V^T P^T ----
+			// ---- O^T += V^T P^T ----
 #pragma unroll
-		for (int r = 0; r < 4; ++r)
+			for (int r = 0; r < 4; ++r)
 #pragma unroll
-			for (int c = 0; c < DC; ++c)
+				for (int c = 0; c < DC; ++c)
 #pragma unroll
-				for (int e = 0; e < 4; ++e) o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[r][c][e], p[r], o[c][e], 0, 0, 0);
+					for (int e = 0; e < 4; ++e) o[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[r][c][e], p[r], o[c][e], 0, 0, 0);
+		}
 		if (more) fetch_v(u + WAVES);
 	}
 

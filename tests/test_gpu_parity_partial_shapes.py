@@ -291,6 +291,33 @@ def test_sdp_attention_mask_tensor_few_rows_keys_over_waves(ops, oracle, heads, 
     assert scaled_rel_err(got[:, :3][:, :, seen], want[:, :, seen], 1.0) <= tol
 
 
+# what a mask tensor hides from all queries of a wave (whole tiles of 64 keys) takes no part in their results, whatever it holds: the tail of a padded cache,
+# a stretch within, and one that the first sixteen queries see and the others do not; 16 rows per block with eight waves (3 heads) and four (100),
+# 128 queries per block (700)
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("heads", [3, 100, 700])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_sdp_attention_mask_tensor_hidden_tiles_hold_anything(ops, heads, d, dtype):
+    ndt = np.float16 if dtype == "f16" else np.float32
+    n_q, n_k = 40, 300
+    q, k, v = (synth.normal(s + n, (1, heads, n, d)).astype(ndt) for s, n in ((1, n_q), (2, n_k), (3, n_k)))
+    mask = synth.normal(7, (n_q, n_k)).astype(ndt)
+    mask[:, 128:192] = -np.inf
+    mask[:, 256:] = -np.inf
+    mask[16:, 64:128] = np.finfo(ndt).min if dtype == "f32" else -np.inf
+    run = lambda kk, vv: host(ops.sdp_attention_masked_scaled_fwd(dev(q), dev(kk), dev(vv), dev(mask).reshape(1, 1, n_q, n_k), d ** -0.5))
+    clean = run(k, v)
+    assert np.isfinite(clean).all()
+    for value in (np.nan, np.inf):
+        kk, vv = k.copy(), v.copy()
+        kk[:, :, 128:192] = vv[:, :, 128:192] = value
+        kk[:, :, 257::3] = vv[:, :, 256:] = value
+        assert np.array_equal(run(kk, vv), clean)
+        kk[:, :, 70] = vv[:, :, 64:128] = value
+        got = run(kk, vv)
+        assert np.array_equal(got[:, :, 16:], clean[:, :, 16:]) and not np.isfinite(got[:, :, :16]).any()
+
+
 # The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
 # many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
 
