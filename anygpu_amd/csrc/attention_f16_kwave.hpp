@@ -99,7 +99,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 
 	float4_t kr[VPS], vr[VPS];
 	// a tile of K or V as it lies, 1 KB of consecutive memory per load (in operand layout, 16 rows x 64 bytes, a CU fetches a quarter of that
-	// rate: 16 bytes per clock); rows past the last key come out as zeros (their scores are masked, their p is 0)
+	// rate: 16 bytes per clock); rows past the last key come out as zeros (their scores are masked, their p is 0): for a buffer without a
+	// stride the range check counts the scalar offset as well (a lane's offset against the buffer's bytes less the scalar one)
 	auto fetch = [&](float4_t (&dst)[VPS], const half_t* src, int u) {
 		const int keys = a.n_k - kKeyWaveTile * u;
 		const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(src) + (int64_t)u * (kKeyWaveTile * D), 0, (keys < kKeyWaveTile ? keys : kKeyWaveTile) * (2 * D), 0x00020000);

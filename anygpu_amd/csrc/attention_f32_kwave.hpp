@@ -79,7 +79,8 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	const int u_first = key_lo / KT, u_last = key_hi >= 0 ? key_hi / KT : -1;
 
 	// K passes through LDS (1 KB of consecutive memory per load), V is fetched as it is needed: four columns of four rows per lane, 256
-	// consecutive bytes for sixteen lanes.  Rows past the last key come out as zeros (their scores are masked, their p is 0).
+	// consecutive bytes for sixteen lanes.  Rows past the last key come out as zeros (their scores are masked, their p is 0): for a buffer without
+	// a stride the range check counts the scalar offset as well.  (All of it in the lane's offset takes 15 registers more at head dimension 256, 8 heads x 650 30.4 -> 31.5 us.)
 	float4_t kr[VPS], vr[4][DC];
 	const auto rsrc_of = [&](const float* src, int u) {
 		const int keys = a.n_k - KT * u;

@@ -318,6 +318,30 @@ def test_sdp_attention_mask_tensor_hidden_tiles_hold_anything(ops, heads, d, dty
         assert np.array_equal(got[:, :, 16:], clean[:, :, 16:]) and not np.isfinite(got[:, :, :16]).any()
 
 
+# keys and values that end inside a tile (one key over whole tiles of 32 and 16, one short, in between), with NaN in memory in front of the first and behind the last
+# of them, and in place of the head in the middle: no result takes any of it
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("n_k", [33, 129, 143, 257, 273, 287])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_sdp_attention_few_rows_nothing_behind_the_last_key(ops, n_k, d, dtype):
+    import torch
+    ndt, tdt = (np.float16, torch.float16) if dtype == "f16" else (np.float32, torch.float32)
+    for n_q in (40, 1):
+        q, k, v = (dev(synth.normal(s + n, (1, 3, n, d)).astype(ndt)) for s, n in ((1, n_q), (2, n_k), (3, n_k)))
+        mask = dev(synth.normal(7, (1, 1, n_q, n_k)).astype(ndt))
+
+        def among_nan(t):
+            pool = torch.full((3 * n_k + 128, d), math.nan, dtype=tdt, device="cuda")
+            view = pool[64:64 + 3 * n_k].view(1, 3, n_k, d)
+            view.copy_(t)
+            view[:, 1] = math.nan
+            return view
+        for run in (lambda kk, vv: ops.sdp_attention_fwd(q, kk, vv, d ** -0.5), lambda kk, vv: ops.sdp_attention_fwd(q, kk, vv, d ** -0.5, causal=True, window=50),
+                    lambda kk, vv: ops.sdp_attention_fwd(q, kk, vv, d ** -0.5, decode=False), lambda kk, vv: ops.sdp_attention_masked_scaled_fwd(q, kk, vv, mask, d ** -0.5)):
+            clean, got = host(run(k, v)), host(run(among_nan(k), among_nan(v)))
+            assert np.isfinite(clean).all() and np.array_equal(got[:, ::2], clean[:, ::2])
+
+
 # The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
 # many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
 
