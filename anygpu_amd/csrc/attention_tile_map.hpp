@@ -11,6 +11,7 @@
 #include "device_utils.hpp"
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <cstdlib>
 
@@ -67,25 +68,28 @@ __global__ __launch_bounds__(1024) void attention_mask_tile_map_kernel(const T* 
 	if (threadIdx.x == 0) map[(int64_t)q_block * groups + group] = (unsigned short)bits;
 }
 
-// The number in the environment that says from how many mask values on there is a map, or nullptr.  With one the launch goes to the kernels that have a form
-// with and without the map, whatever its size.
-inline const char* attention_mask_map_from()
+// The environment variable ANYGPU_ATTN_MASK_MAP_FROM, read at every launch: from how many mask values on there is a map (0: always, a huge
+// value: never), -1 without it.
+inline int64_t attention_mask_map_from()
 {
 	const char* text = std::getenv("ANYGPU_ATTN_MASK_MAP_FROM");
-	return text != nullptr && *text != 0 ? text : nullptr;
+	return text != nullptr && *text != 0 ? std::max(std::atoll(text), 0ll) : -1;
 }
 
 // Whether the map is made for a mask of n_q x n_k values.  Its pass costs a launch and a few memory latencies (8 - 12 us for
 // small masks, 5.6 TB/s for large ones), which short key ranges do not earn back: from 4 M mask values on, or from 16384 keys
 // on whatever the queries (a sliding window over a long cache hides most of them from a few queries as well).  The
-// environment variable ANYGPU_ATTN_MASK_MAP_FROM, read at every launch, replaces the rule by "from that many mask values
-// on" (0: always, a huge value: never).
+// environment variable replaces the rule.
 // `needed`: the launch's kernel works on the map.
 inline bool attention_mask_map_wanted(int64_t n_q, int64_t n_k, bool needed = false)
 {
-	if (const char* text = attention_mask_map_from()) return n_q * n_k >= std::atoll(text);
+	const int64_t from = attention_mask_map_from();
+	if (from >= 0) return n_q * n_k >= from;
 	return needed || n_q * n_k >= (4ll << 20) || n_k >= 16384;
 }
+
+// Whether the environment variable asks for a map, which the kernels of 16 rows per block do not read: the launch then goes to those that do.
+inline bool attention_mask_map_asked(int64_t n_q, int64_t n_k) { return attention_mask_map_from() >= 0 && attention_mask_map_wanted(n_q, n_k); }
 
 // 64-bit words of the map per query block
 inline int64_t attention_tile_map_words(int64_t n_k, int keys_per_tile)

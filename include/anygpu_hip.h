@@ -313,7 +313,9 @@ int anygpu_sdp_attention_fwd_f32(const float* q, const float* k, const float* v,
  * ANYGPU_ATTN_MASK_MAP_FROM, read at every call, replaces both by a number of mask values) a pass over the mask ahead of the kernel (once, not per head) notes which key tiles it hides from which
  * blocks of queries; those are neither loaded nor multiplied.  The note lives at the front of the stream's workspace;
  * under a capture without a caller's workspace there is none, every tile is loaded and the hidden ones cost no products.
- * The results are the same bit for bit either way, except where few query blocks go out in parts of their key range:
+ * Launches of few queries and heads, which blocks of 16 queries serve better, take neither note nor workspace and leave the hidden tiles' products out as well;
+ * where the environment variable asks for a note they go to the kernels that read one, whose sums are taken in another order.
+ * The results of those kernels are the same bit for bit with the note and without, except where few query blocks go out in parts of their key range:
  * with the note the parts divide the visible tiles among them (a sliding window over a long cache leaves most equal
  * parts of the range empty), without it the range, and the sums are taken in another order.  The float32 form's products of bf16
  * parts need the note: masks for which they pay (150 K values and more at head dimension 256) get one whatever their size, unless

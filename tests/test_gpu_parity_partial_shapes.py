@@ -342,6 +342,59 @@ def test_sdp_attention_few_rows_nothing_behind_the_last_key(ops, n_k, d, dtype):
             assert np.isfinite(clean).all() and np.array_equal(got[:, ::2], clean[:, ::2])
 
 
+# the note of a mask's hidden tiles (always / never) in launches of so many heads that blocks of 128 queries (float32 at 64 and 128: 64) take them: masks below the
+# sizes that get one by default, ragged last tiles and blocks, queries that see nothing, mask rows at an odd pitch; and the launches of few query blocks, which have none by
+# default, with the same bits where the variable says never, and on the kernels that read one, in another order of sums, where it says always
+@pytest.mark.parametrize("dtype,d,heads,n_q,n_k,kind", [("f16", 64, 70, 300, 333, "slide"), ("f16", 64, 140, 130, 1500, "stripes"), ("f16", 128, 48, 300, 300, "blind rows"), ("f16", 128, 96, 130, 700, "odd stride"),
+                                                        ("f16", 256, 26, 300, 301, "slide"), ("f16", 256, 26, 130, 1030, "stripes"), ("f32", 64, 120, 300, 333, "slide"), ("f32", 64, 64, 200, 2100, "stripes"),
+                                                        ("f32", 128, 80, 300, 300, "blind rows"), ("f32", 128, 40, 200, 1500, "odd stride"), ("f32", 256, 24, 300, 301, "slide"), ("f32", 256, 4, 150, 1100, "stripes")])
+def test_sdp_attention_mask_tensor_with_and_without_note(ops, oracle, monkeypatch, dtype, d, heads, n_q, n_k, kind):
+    import torch
+    from anygpu_amd import capi
+    half, alpha = dtype == "f16", d ** -0.5
+    q, k, v = (synth.normal(s + n, (heads, n, d)).astype(np.float16 if half else np.float32) for s, n in ((1, n_q), (2, n_k), (3, n_k)))
+    if kind == "slide":
+        mask = oracle.slide_mask(oracle.causal_mask(n_q, n_k, diag=n_k - n_q), n_k // 3)
+    else:
+        rng = np.random.default_rng(n_q * 1000 + n_k)
+        mask = rng.normal(0.0, 2.0, (n_q, n_k)).astype(np.float32)
+        hide_key_stripes(mask, rng)
+        if kind == "blind rows":
+            mask[[5, n_q // 2]] = -np.inf
+    with np.errstate(over="ignore"):
+        mask = np.ascontiguousarray(mask).astype(q.dtype)
+    pitch = n_k + (3 if kind == "odd stride" else 0)
+    rows = torch.full((n_q * pitch + 1,), float("nan"), dtype=torch.float16 if half else torch.float32, device="cuda")[1:].view(n_q, pitch)
+    rows[:, :n_k] = dev(mask)
+    fn = getattr(capi.load(), f"anygpu_sdp_attention_fwd_masked_{dtype}")
+
+    def run(count, env):
+        if env is None:
+            monkeypatch.delenv("ANYGPU_ATTN_MASK_MAP_FROM", raising=False)
+        else:
+            monkeypatch.setenv("ANYGPU_ATTN_MASK_MAP_FROM", env)
+        args = [dev(t[:count]) for t in (q, k, v)]
+        y = torch.empty_like(args[0])
+        assert fn(*(t.data_ptr() for t in args), rows.data_ptr(), y.data_ptr(), count, 1, n_q, n_k, d, pitch, alpha, 0.0, None) == capi.ANYGPU_OK
+        return host(y).astype(np.float32)
+    tol = TOL_F16_ROWOPS * 2 if half else TOL_F32
+    always, never = run(heads, "0"), run(heads, str(1 << 60))
+    assert scaled_rel_err(always, never, 1.0) <= (TOL_F16_ROWOPS if half else 1e-5)
+    some = [0, heads // 2, heads - 1]
+    wide = [(oracle.cvt_f16_to_f32(t) if half else t) for t in (q[some], k[some], v[some], mask)]
+    seen = np.isfinite(wide[3]).any(axis=-1)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = oracle.sdp_attention_masked_scaled_fwd(*(t[None] for t in wide[:3]), wide[3].reshape(1, 1, n_q, n_k), alpha, threads=8)[0]
+    for got in (always[some], never[some]):
+        assert not got[:, ~seen].any() and np.isfinite(got).all()
+        assert scaled_rel_err(got[:, seen], want[:, seen], 1.0) <= tol
+    if n_k < 500:
+        few = [run(2, env) for env in (None, "0", str(1 << 60))]
+        assert np.array_equal(few[0], few[2]) and not np.array_equal(few[0], few[1])
+        for got in few[:2]:
+            assert not got[:, ~seen].any() and scaled_rel_err(got[0][seen], want[0][seen], 1.0) <= tol
+
+
 # The next tests reach the kernel with 32 queries per wave by more than one query block per CU (512 heads), or by few blocks with so
 # many key tiles that each goes out in parts.  Scores are set by the first component of q and k alone.
 
