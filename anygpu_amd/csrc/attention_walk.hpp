@@ -51,7 +51,8 @@ struct AttnWalk
 // turn (kernels of two or three blocks per CU, whole blocks): the CUs of an XCD.  The first round of blocks puts one on each of them, heaviest first, and the
 // second, in the same order, would put its heaviest with the heaviest of the first: backwards, the sums are nearly equal (half, causal: 32 / 8 heads x 3000 x 128 91.2 ->
 // 88.0 us, 32 / 8 x 4096 x 128 150 -> 146, 32 / 8 x 3000 x 64 55.0 -> 50.5, 64 / 8 x 1404 x 128 48.7 -> 46.5; third rounds backwards 93 and 158 us of the first two).
-// Only where the second round is nearly full, as its lightest blocks go where a place is first: 16 / 8 x 3600 (58 blocks per XCD) 75.0 -> 72.7, but 2600 (42) 51.9 / 52.9, 3000 (48) 62.5 / 64.7.
+// Only where the second round is nearly full, as its lightest blocks go where a place is first: 16 / 8 x 3600 (58 blocks per XCD) 75.0 -> 72.7, but 2600 (42) 51.9 / 52.9, 3000 (48) 62.5 / 64.7;
+// blocks that there are, without the padding of units and rounds (7 x 8 heads x 543 x 128, 35 blocks and 21 of padding per XCD, softcap 19.8 / 26.3, 7 x 16 / 8 x 294 x 128 11.8 / 13.5).
 inline AttnWalk make_attn_walk(int64_t q_blocks, int64_t batch_heads, int64_t q_per_kv, int64_t n_split = 0, int64_t n_big = 0,
                                int64_t parts_all = 1, int64_t turn = 0)
 {
@@ -73,7 +74,7 @@ inline AttnWalk make_attn_walk(int64_t q_blocks, int64_t batch_heads, int64_t q_
 	w.chunks = (w.q_blocks + w.chunk - 1) / w.chunk;
 	w.units = w.chunks * w.groups;
 	w.units_per_xcd = (w.units + kAttnXcds - 1) / kAttnXcds;
-	w.turn = 4 * (int64_t)w.units_per_xcd * w.chunk * w.q_per_kv >= 7 * turn ? (int)turn : 0;
+	w.turn = 4 * q_blocks * batch_heads >= 7 * turn * kAttnXcds ? (int)turn : 0;
 	return w;
 }
 
