@@ -983,6 +983,21 @@ bool attention_q32_wanted(const AttnArgs& args, int64_t blocks, bool in_parts)
 	return blocks * tiles > 32 * cus && in_parts;
 }
 
+// The kernel with 32 queries per wave: whether its blocks take a tile's products and softmax one after the other, a third of the code to fetch and neither a tile of
+// scores ahead of the loop nor one of output behind it.  By the tiles of an average block (us, overlapped / in turn, causal): head dimension 128 up to 3.75 (4 x 64 / 8 heads
+// x 200 13.7 / 12.1, 6 x 32 / 8 x 300 20.0 / 18.5, window 25 8 x 64 / 8 x 1377 166 / 148; but 16 x 16 x 300 23.0 / 24.8, at 5 tiles 4 % behind), with softcap up to 5 (3 x 128 / 16 x 216 window 8 26.7 / 21.5, 18 x
+// 16 / 4 x 296 30.6 / 27.8; at 6 equal), 64 up to 5 (8 x 32 / 8 x 250 10.0 / 9.0, 14 x 8 / 4 x 266 9.7 / 8.4; at 6 3 % behind), with softcap up to 7 (9 x 16 x 422 window 16 15.5 / 13.5; at 8 equal).
+template <int D, bool SOFTCAP>
+bool attention_q32_in_turn(const AttnArgs& args)
+{
+	const int64_t q_blocks = (args.n_q + kQ32QueriesPerBlock - 1) / kQ32QueriesPerBlock;
+	const auto tiles_of = [&](int64_t b) {
+		return attention_block_tiles(b, args.n_q, args.n_k, args.causal, args.diag, args.window, kQ32QueriesPerBlock, kAttnKeysPerTile);
+	};
+	const int64_t four_blocks = tiles_of(0) + 2 * tiles_of(q_blocks / 2) + tiles_of(q_blocks - 1);        // four times an average block
+	return four_blocks <= (D == 64 ? (SOFTCAP ? 28 : 20) : (SOFTCAP ? 20 : 15));
+}
+
 template <int D, bool SOFTCAP>
 hipError_t launch_q32(const AttnArgs& args_in, int64_t batch_heads, hipStream_t stream)
 {
@@ -1010,7 +1025,9 @@ hipError_t launch_q32(const AttnArgs& args_in, int64_t batch_heads, hipStream_t 
 	const AttnWalk walk = make_attn_walk(q_blocks, batch_heads, args.q_per_kv, plan.n_split, plan.n_big, parts_all,
 	                                     plan.n_split > 0 || parts_all > 1 ? 0 : device_cu_count() / kAttnXcds);
 	if (attn_walk_blocks(walk) > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-	sdp_attention_fwd_f16_q32_kernel<D, SOFTCAP><<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * kQ32Waves), kLdsBytes, stream>>>(args, walk);
+	const dim3 grid((unsigned)attn_walk_blocks(walk));
+	if (attention_q32_in_turn<D, SOFTCAP>(args)) sdp_attention_fwd_f16_q32_kernel<D, SOFTCAP, true><<<grid, dim3(64 * kQ32Waves), kLdsBytes, stream>>>(args, walk);
+	else sdp_attention_fwd_f16_q32_kernel<D, SOFTCAP, false><<<grid, dim3(64 * kQ32Waves), kLdsBytes, stream>>>(args, walk);
 	hipError_t err = hipGetLastError();
 	if (err != hipSuccess || walk.n_split == 0) return err;
 	const int64_t items = batch_heads * walk.n_split * kQueriesPerBlock * (D / 4);

@@ -16,8 +16,8 @@
 // N(0, 4): 2.36e-4 against 2.17e-4 (2-norm), of which the result's own rounding is 2.1e-4).
 // Measured, causal (us; products and softmax in turn -> here, the same bits): 16 x 4096 x 128 102.3 -> 91.7, 64 / 8 x 1000 x 128 32.0 -> 29.9, 16 x 8192 x
 // 128 315 -> 299, 2 x 16 x 2280 x 128 63.3 -> 58.7, 32 / 8 x 3000 x 128 93.3 -> 91.4, 4096 166 -> 153, 32 x 2038 x 64 36.5 -> 32.8, 32 x 4000 x 64 window 500
-// 36.9 -> 34.5; without the causal rule 32 / 8 x 3000 x 128 177 -> 159.  Slower where many blocks walk some five tiles (128 / 8 x 300 x 128 12.4 -> 13.1), and where the
-// last of them do not fill the places (16 / 8 x 2600 x 128 52.2 -> 53.7).
+// 36.9 -> 34.5; without the causal rule 32 / 8 x 3000 x 128 177 -> 159.  Blocks of some three tiles and fewer paid for its longer
+// code (4 x 64 / 8 x 200 x 128 12.2 -> 13.7): they take products and softmax in turn (attention_q32_in_turn), with the same bits.
 #pragma once
 
 #include "attention_walk.hpp"
@@ -51,8 +51,9 @@ __device__ __forceinline__ float max_over_lane_halves(float x)
 	return fmaxf(a, b);
 }
 
-template <int D, bool SOFTCAP>
-__global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention_fwd_f16_q32_kernel(const AttnArgs a, const AttnWalk walk)
+// IN_TURN: the products and the softmax of a tile one after the other, for blocks of few tiles
+template <int D, bool SOFTCAP, bool IN_TURN>
+__global__ __launch_bounds__(64 * kQ32Waves, D == 64 && !IN_TURN ? 3 : 2) void sdp_attention_fwd_f16_q32_kernel(const AttnArgs a, const AttnWalk walk)
 {
 	constexpr int kRow = 2 * D;                              // bytes of a tile row
 	constexpr int KT = kAttnKeysPerTile, KB = KT / 32;
@@ -198,7 +199,6 @@ __global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention
 				const int key = 32 * kb + 8 * (i / 4) + i % 4;           // + 4 h
 				s[kb][i] = (key >= lo && key <= hi) ? s[kb][i] : -INFINITY;
 			}
-		max_scores(s);
 	};
 	// own loads have landed; behind the barrier everybody's have, and everybody is done with what the loads issued behind it overwrite:
 	// at the turn of tile t K(t + 1) and V(t) are there, K(t) and V(t - 1) free
@@ -261,6 +261,15 @@ __global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention
 	};
 	auto p_of_score = [&](const Scores& s, int e) { return fast_exp2(fmaf(s[e / 16][e % 16], z_in, z_add)); };
 
+	// fragment i (16-key step u = i / DC, columns 32 c ..) of the V tile at `va`: K slot (h, j) is key 16 u + 8 (j / 4) + 4 h + j % 4
+	auto v_fragment = [&](unsigned va, int i) {
+		const int u = i / DC, c = i % DC;
+		const unsigned src = (va ^ (64 * c)) + 16 * u * kRow;
+		const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)src);
+		const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)(src + 8 * kRow));
+		return __builtin_shufflevector(__builtin_bit_cast(half4_t, lo), __builtin_bit_cast(half4_t, hi), 0, 1, 2, 3, 4, 5, 6, 7);
+	};
+
 	// One tile: S(t + 1) = K(t + 1) Q^T (SCORES) beside p(t) = 2^(z(t) - m), then O^T += V(t)^T P(t)^T (OUTPUT) beside the
 	// maximum of S(t + 1), as steps of one MFMA.
 	auto tile = [&](auto scores_tag, auto output_tag, Scores& cur, Scores& next, int t) {
@@ -276,12 +285,7 @@ __global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention
 				frag[i % kAhead] = *(LdsHalf8)(uintptr_t)((ka ^ (32 * st)) + kb * 32 * kRow);
 				return;
 			}
-			// K slot (h, j) of 16-key step u is key 16 u + 8 (j / 4) + 4 h + j % 4
-			const int u = (i - kStepsA) / DC, c = (i - kStepsA) % DC;
-			const unsigned src = (va ^ (64 * c)) + 16 * u * kRow;
-			const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)src);
-			const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4_t*)(uintptr_t)(src + 8 * kRow));
-			frag[i % kAhead] = __builtin_shufflevector(__builtin_bit_cast(half4_t, lo), __builtin_bit_cast(half4_t, hi), 0, 1, 2, 3, 4, 5, 6, 7);
+			frag[i % kAhead] = v_fragment(va, i - kStepsA);
 		};
 		const int4_t rsrc_v = rsrc_of(vp, t + 1), rsrc_k = rsrc_of(kp, t + 2 <= t_last ? t + 2 : t_last);
 		half8_t pf[2 * KB];
@@ -357,10 +361,98 @@ __global__ __launch_bounds__(64 * kQ32Waves, D == 64 ? 3 : 2) void sdp_attention
 				for (int y = 0; y < 8 * KB; ++y) logits_of_pair(next, y);
 				max_scores(next);
 			}
-			if (!is_interior(t + 1)) mask_scores(next, t + 1);
+			if (!is_interior(t + 1))
+			{
+				mask_scores(next, t + 1);
+				max_scores(next);
+			}
 		}
 	};
 	if (t_first > t_last) {}
+	else if constexpr (IN_TURN)
+	{
+		auto issue_tile = [&](int t, int stage) {
+			const int4_t rsrc_k = rsrc_of(kp, t), rsrc_v = rsrc_of(vp, t);
+#pragma unroll
+			for (int j = 0; j < kSlots; ++j)
+			{
+				issue_k(rsrc_k, stage, j);
+				issue_v(rsrc_v, stage, j);
+			}
+		};
+		constexpr int kVRing = 8;                            // V fragments in registers, read ahead of the softmax
+		issue_tile(t_first, 0);
+		for (int t = t_first; t <= t_last; ++t)
+		{
+			tile_barrier();
+			const int stage = (t - t_first) & 1;
+			const bool any_visible = t >= wt_first && t <= wt_last;        // wave-uniform
+			const unsigned ka = k_addr + stage * kStage, va = v_addr + stage * kStage;
+			// the first K fragments, on their way while the next tile's loads are issued
+			half8_t kf[KS][KB];
+			auto read_k = [&](int st) {
+#pragma unroll
+				for (int kb = 0; kb < KB; ++kb) kf[st][kb] = *(LdsHalf8)(uintptr_t)((ka ^ (32 * st)) + kb * 32 * kRow);
+			};
+			if (any_visible)
+			{
+#pragma unroll
+				for (int st = 0; st < kAhead; ++st) read_k(st);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+			if (t < t_last) issue_tile(t + 1, stage ^ 1);
+			if (!any_visible) continue;
+
+			Scores s;
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+				for (int i = 0; i < 16; ++i) s[kb][i] = 0.0f;
+			__builtin_amdgcn_s_setprio(1);
+#pragma unroll
+			for (int st = 0; st < KS; ++st)
+			{
+#pragma unroll
+				for (int kb = 0; kb < KB; ++kb) s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[st][kb], qf[st], s[kb], 0, 0, 0);
+				if (st + kAhead < KS) read_k(st + kAhead);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			__builtin_amdgcn_s_setprio(0);
+			half8_t vf[kVRing];
+			auto read_v = [&](int i) { vf[i % kVRing] = v_fragment(va, i); };
+#pragma unroll
+			for (int i = 0; i < kVRing; ++i) read_v(i);
+			__builtin_amdgcn_sched_barrier(0);
+
+#pragma unroll
+			for (int y = 0; y < 8 * KB; ++y) logits_of_pair(s, y);
+			if (!is_interior(t)) mask_scores(s, t);
+			max_scores(s);
+			take_maximum(s);
+			half8_t pf[2 * KB];
+			float psum[2] = {0.0f, 0.0f};
+#pragma unroll
+			for (int y = 0; y < 8 * KB; ++y)
+			{
+				const float p0 = p_of_score(s, 2 * y), p1 = p_of_score(s, 2 * y + 1);
+				psum[0] += p0;
+				psum[1] += p1;
+				pf[y / 4][2 * (y % 4)] = (half_t)p0;
+				pf[y / 4][2 * (y % 4) + 1] = (half_t)p1;
+			}
+			l_run += psum[0] + psum[1];
+			__builtin_amdgcn_sched_barrier(0);
+			__builtin_amdgcn_s_setprio(1);
+#pragma unroll
+			for (int i = 0; i < kStepsB; ++i)
+			{
+				o[i % DC] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i % kVRing], pf[i / DC], o[i % DC], 0, 0, 0);
+				if (i + kVRing < kStepsB) read_v(i + kVRing);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			__builtin_amdgcn_s_setprio(0);
+		}
+	}
 	else
 	{
 		// K of the first tile, then (the turn of the tile before the first has nothing else to load) its V and K of the second

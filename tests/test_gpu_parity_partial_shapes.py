@@ -178,6 +178,24 @@ def test_sdp_attention_32_queries_per_wave_tiles_in_pairs(ops, oracle, n_q, n_k,
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# blocks of enough tiles that the scores of one run beside the softmax of the one before (those above take them in turn): the first query block of a causal launch with
+# waves of one and two tiles, ranges that begin and end within and between blocks, odd and even numbers of tiles
+@pytest.mark.parametrize("d,cap", [(64, 0.0), (128, 0.0), (64, 30.0), (128, 30.0)])
+@pytest.mark.parametrize("n_q,n_k,causal,window", [(1000, 1000, True, 0), (897, 960, True, 0), (1100, 1161, True, 600), (130, 641, False, 0), (97, 577, True, 0), (385, 1025, False, 520)])
+def test_sdp_attention_32_queries_per_wave_tiles_overlapped(ops, oracle, n_q, n_k, causal, window, d, cap):
+    copies, heads = 66, 4
+    q, k, v = (synth.normal(80 + i, (1, heads, n, d)).astype(np.float16) for i, n in enumerate((n_q, n_k, n_k)))
+    k *= np.float16(2.0)
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), d ** -0.5, softcap=cap, causal=causal, window=window,
+                                     decode=False)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=d ** -0.5, softcap=cap,
+                                      causal=causal, window=window, q_per_kv=1, threads=8)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    # p rounded to fp16 (2^-11 each, weights that sum to 1) and the result's own rounding, values of up to about 4
+    assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2
+
+
 # the same kernel where the second round of blocks is dispatched backwards: 55 to 76 blocks per XCD, with padding at the end of a head and of the launch
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("copies,heads,kv_heads,n,causal", [(7, 4, 2, 1930, True), (40, 4, 2, 300, True), (37, 4, 2, 300, True), (31, 5, 1, 260, True), (64, 4, 4, 200, False), (33, 4, 2, 510, True)])
@@ -473,11 +491,12 @@ def test_sdp_attention_scores_beyond_the_mantissa(ops, d, alpha, heads):
     assert np.array_equal(got, np.broadcast_to(v[0, 0, int(np.argmin(order))], got.shape))
 
 
+@pytest.mark.parametrize("n", [200, 900])                        # a tile's products and softmax in turn, and overlapped
 @pytest.mark.parametrize("d", [64, 128])
-def test_sdp_attention_32_queries_per_wave_nan_and_infinities(ops, d):
+def test_sdp_attention_32_queries_per_wave_nan_and_infinities(ops, d, n):
     # a NaN in a query reaches its row; a NaN in a key, or a score of +inf, the rows that see the key; a score of -inf hides it
     import torch
-    copies, heads, n = 64, 8, 200
+    copies, heads = 64, 8
     q, k, v = (synth.normal(70 + i, (heads, n, d)).astype(np.float16) for i in range(3))
     q[1, 37, 3] = np.nan
     k[2, 150, 0] = np.nan
