@@ -1366,7 +1366,7 @@ hipError_t launch_sdp_attention_fwd_f16(const void* q, const void* k, const void
 	{
 		args.causal = 0;
 		args.window = 0;
-		if (!attention_mask_map_asked(n_q, n_k) && attention_kwave_wanted((int)head_dim, true, batch_heads, args.n_q, args.n_k, 0, args.diag, 0, device_cu_count()))
+		if (!attention_mask_map_set() && attention_kwave_wanted((int)head_dim, true, batch_heads, args.n_q, args.n_k, 0, args.diag, 0, device_cu_count()))
 		{
 #define ANYGPU_ATTN_F16_MASK_DIM(DIM) \
 			return capped ? launch_kwave<DIM, true, true>(args, batch_heads, n_q, q_per_kv, stream) : launch_kwave<DIM, false, true>(args, batch_heads, n_q, q_per_kv, stream)

@@ -1386,7 +1386,7 @@ hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, h
 	AttnArgsF32 args = args_in;
 	args.tile_map = nullptr;
 	args.map_words = 0;
-	if (!(MASK && attention_mask_map_asked(args.n_q, args.n_k)) &&
+	if (!(MASK && attention_mask_map_set()) &&
 	    attention_kwave_wanted_f32(D, MASK, batch_heads, args.n_q, args.n_k, args.causal, args.diag, args.window, device_cu_count()))
 		return launch_kwave_f32<D, SOFTCAP, MASK>(args, batch_heads, args.n_q, args.q_per_kv, stream);
 	const bool split = attention_split_wanted<D, MASK>(args, batch_heads);

@@ -88,8 +88,8 @@ inline bool attention_mask_map_wanted(int64_t n_q, int64_t n_k, bool needed = fa
 	return needed || n_q * n_k >= (4ll << 20) || n_k >= 16384;
 }
 
-// Whether the environment variable asks for a map, which the kernels of 16 rows per block do not read: the launch then goes to those that do.
-inline bool attention_mask_map_asked(int64_t n_q, int64_t n_k) { return attention_mask_map_from() >= 0 && attention_mask_map_wanted(n_q, n_k); }
+// With the variable set, a launch of few query blocks stays on the kernels that have a form with the map and one without it, alike to the last bit (blocks of 16 rows have neither).
+inline bool attention_mask_map_set() { return attention_mask_map_from() >= 0; }
 
 // 64-bit words of the map per query block
 inline int64_t attention_tile_map_words(int64_t n_k, int keys_per_tile)

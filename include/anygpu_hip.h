@@ -314,7 +314,7 @@ int anygpu_sdp_attention_fwd_f32(const float* q, const float* k, const float* v,
  * blocks of queries; those are neither loaded nor multiplied.  The note lives at the front of the stream's workspace;
  * under a capture without a caller's workspace there is none, every tile is loaded and the hidden ones cost no products.
  * Launches of few queries and heads, which blocks of 16 queries serve better, take neither note nor workspace and leave the hidden tiles' products out as well;
- * where the environment variable asks for a note they go to the kernels that read one, whose sums are taken in another order.
+ * with the environment variable set, to whatever number, they go to the kernels that know the note, whose sums are taken in another order.
  * The results of those kernels are the same bit for bit with the note and without, except where few query blocks go out in parts of their key range:
  * with the note the parts divide the visible tiles among them (a sliding window over a long cache leaves most equal
  * parts of the range empty), without it the range, and the sums are taken in another order.  The float32 form's products of bf16

@@ -361,8 +361,8 @@ def test_sdp_attention_few_rows_nothing_behind_the_last_key(ops, n_k, d, dtype):
 
 
 # the note of a mask's hidden tiles (always / never) in launches of so many heads that blocks of 128 queries (float32 at 64 and 128: 64) take them: masks below the
-# sizes that get one by default, ragged last tiles and blocks, queries that see nothing, mask rows at an odd pitch; and the launches of few query blocks, which have none by
-# default, with the same bits where the variable says never, and on the kernels that read one, in another order of sums, where it says always
+# sizes that get one by default, ragged last tiles and blocks, queries that see nothing, mask rows at an odd pitch; and the launches of few query blocks, which have none while
+# the variable is not set
 @pytest.mark.parametrize("dtype,d,heads,n_q,n_k,kind", [("f16", 64, 70, 300, 333, "slide"), ("f16", 64, 140, 130, 1500, "stripes"), ("f16", 128, 48, 300, 300, "blind rows"), ("f16", 128, 96, 130, 700, "odd stride"),
                                                         ("f16", 256, 26, 300, 301, "slide"), ("f16", 256, 26, 130, 1030, "stripes"), ("f32", 64, 120, 300, 333, "slide"), ("f32", 64, 64, 200, 2100, "stripes"),
                                                         ("f32", 128, 80, 300, 300, "blind rows"), ("f32", 128, 40, 200, 1500, "odd stride"), ("f32", 256, 24, 300, 301, "slide"), ("f32", 256, 4, 150, 1100, "stripes")])
@@ -408,8 +408,8 @@ def test_sdp_attention_mask_tensor_with_and_without_note(ops, oracle, monkeypatc
         assert scaled_rel_err(got[:, seen], want[:, seen], 1.0) <= tol
     if n_k < 500:
         few = [run(2, env) for env in (None, "0", str(1 << 60))]
-        assert np.array_equal(few[0], few[2]) and not np.array_equal(few[0], few[1])
-        for got in few[:2]:
+        assert scaled_rel_err(few[1], few[2], 1.0) <= (TOL_F16_ROWOPS if half else 1e-5) and not np.array_equal(few[0], few[1])
+        for got in few:
             assert not got[:, ~seen].any() and scaled_rel_err(got[0][seen], want[0][seen], 1.0) <= tol
 
 
