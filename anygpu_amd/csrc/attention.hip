@@ -994,8 +994,7 @@ bool attention_q32_in_turn(const AttnArgs& args)
 	const auto tiles_of = [&](int64_t b) {
 		return attention_block_tiles(b, args.n_q, args.n_k, args.causal, args.diag, args.window, kQ32QueriesPerBlock, kAttnKeysPerTile);
 	};
-	const int64_t four_blocks = tiles_of(0) + 2 * tiles_of(q_blocks / 2) + tiles_of(q_blocks - 1);        // four times an average block
-	return four_blocks <= (D == 64 ? (SOFTCAP ? 28 : 20) : (SOFTCAP ? 20 : 15));
+	return four_average_blocks(q_blocks, tiles_of) <= (D == 64 ? (SOFTCAP ? 28 : 20) : (SOFTCAP ? 20 : 15));
 }
 
 template <int D, bool SOFTCAP>

@@ -26,8 +26,6 @@ constexpr int kKeyWaveTile = 32;                // keys of a tile: one MFMA step
 // p is 2^15 for a score at the running maximum (attention_f16_q32.hpp)
 constexpr float kKeyWaveHeadRoom = 15.0f;
 
-// `walk`: blocks of 16 rows of a "head" of `rows` rows; row r is query r % n_q (rows = n_q, or where a key / value head's rows are
-// taken together, q_per_kv * n_q with fewer than 16 queries).  MASK: an additive mask tensor instead of the index rules.
 // Whether that kernel takes a launch of `heads` x n_q queries, by its blocks of 16 queries, the tiles of the longest (t_last) and what all of them cost: a
 // block's start and end are some five tiles.  us, 128 queries per block / here:
 //   * Up to a block for each CU the longest one decides: head dimension 256 up to 48 tiles (8 heads x 100 x 1400 23.3 / 20.8; but 100 x 2000 24.3 / 27.7), 128 up to 100 (16 x
@@ -38,18 +36,27 @@ constexpr float kKeyWaveHeadRoom = 15.0f;
 //     1000 24.5 / 21.9.  64, up to four: 32 x 500 14.1 / 7.5, 64 x 250 7.3 / 5.9, 16 x 1000 without the causal rule 21.9 / 16.9; but 64 x 300 7.4 / 8.7.
 //   * A mask tensor, whose hidden tiles are not known ahead: 8 x 400 x 256 24.8 / 12.6, 200 x 1500 25.9 / 24.1 (but 600 26.8 / 26.3, 100 x 3000 28.2 / 40.1), 16 x 600 x 128 21.2 / 16.9,
 //     64 x 167 11.4 / 9.6 (but 32 x 422 17.1 / 18.4, 64 x 300 14.3 / 18.0, 64 x 200 x 1500 39.8 / 41.8), 16 x 1000 x 64 22.4 / 18.7, 32 x 100 x 3000 25.1 / 15.7 (but 32 x 1000 28.8 / 32.8).
+//   * Not where blocks of 128 queries are many or have few tiles themselves: at 64 and 128 with a single tile of 64 keys (84 heads x 29 x 64 4.0 / 4.5, 7 x 4 x 34 x 128 4.7 / 5.2), at 256, and at 128
+//     by a little, where estimated times say so (176 heads x 34 x 256 6.7 / 12.5, 10 x 8 x 81 x 242 x 256 14.7 / 25.9, 20 x 4 x 75 x 256 10.8 / 14.0, mask tensor 64 x 153 x 256 15.6 / 20.5, 31 x 8 x 68 x 128
+//     6.5 / 8.1).  The constants are fitted to 2800 launches of 16 to 1600 queries; of the 1860 that the lines above give to this kernel 350 were slower by more than 4 %, 27 of the 1390 that are left.
 inline bool attention_kwave_wanted(int head_dim, bool mask, int64_t heads, int n_q, int n_k, int causal, int diag, int window, int64_t cus)
 {
 	const int64_t groups = (n_q + kKeyWaveRows - 1) / kKeyWaveRows, blocks = heads * groups;
 	if (blocks > 4 * cus) return false;
 	const int64_t t_first = attention_block_tiles(0, n_q, n_k, causal, diag, window, kKeyWaveRows, kKeyWaveTile);
 	const int64_t t_last = attention_block_tiles(groups - 1, n_q, n_k, causal, diag, window, kKeyWaveRows, kKeyWaveTile);
-	const int64_t longest = std::max(t_first, t_last);
+	const int64_t longest = std::max(t_first, t_last), q_blocks = (n_q + 127) / 128;
+	if (!mask && head_dim != 256 && attention_block_tiles(0, n_q, n_k, causal, diag, window, 128, 64) <= 1 && attention_block_tiles(q_blocks - 1, n_q, n_k, causal, diag, window, 128, 64) <= 1) return false;
+	if (head_dim == 256 || (head_dim == 128 && !mask))
+	{
+		const KeyWaveCost cost = head_dim == 128 ? KeyWaveCost{0.53, 0.21, 0.0, 1.38, 0.0, 1.65} : mask ? KeyWaveCost{3.13, 0.58, 2.2, 2.35, 0.85, 4.5} : KeyWaveCost{2.39, 0.59, 1.0, 2.46, 0.1, 4.2};
+		if (!attention_kwave_ahead(cost, head_dim == 256, heads, n_q, n_k, causal, diag, window, kKeyWaveRows, kKeyWaveTile, cus)) return false;
+	}
 	if (blocks <= cus) return longest <= (head_dim == 256 ? 48 : head_dim == 128 ? 100 : 200);
 	const int64_t cost = blocks * (t_first + t_last + 10) / 2;          // (tiles grow evenly from the first group to the last, but for a window)
 	if (mask) return blocks <= (head_dim == 64 ? 4 : 3) * cus && cost <= (head_dim == 256 ? 26 : head_dim == 128 ? 110 : 200) * cus;
 	if (head_dim == 256) return 4 * blocks <= 9 * cus && longest <= 48 && cost <= 56 * cus;
-	if (head_dim == 128) return (blocks <= 3 * cus && cost <= 75 * cus) || (2 * heads * ((n_q + 127) / 128) <= cus && cost <= 90 * cus);
+	if (head_dim == 128) return (blocks <= 3 * cus && cost <= 75 * cus) || (2 * heads * q_blocks <= cus && cost <= 90 * cus);
 	return cost <= 160 * cus;
 }
 
@@ -64,6 +71,8 @@ inline bool decode_kwave_wanted(int64_t head_dim, int64_t blocks, int64_t tiles,
 template <int D, int WAVES>
 constexpr int kKeyWaveLdsBytes = (WAVES * kKeyWaveTile + kKeyWaveRows) * AttnLds<D>::kPitchV;
 
+// `walk`: blocks of 16 rows of a "head" of `rows` rows; row r is query r % n_q (rows = n_q, or where the query heads of a key / value head are
+// taken together, q_per_kv * n_q, at most kDecodeMaxRows).  MASK: an additive mask tensor instead of the index rules.
 template <int D, bool SOFTCAP, bool MASK, int WAVES>
 __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void sdp_attention_fwd_f16_kwave_kernel(const AttnArgs a, const AttnWalk walk, int rows)
 {

@@ -27,6 +27,8 @@ constexpr int kKeyWaveTile = 16;
 //   * With more, all of them.  256: 8 x 800 47.8 / 36.2, 4 x 8 x 400 56.9 / 45.9, 8 x 1200 70.0 / 72.9.  128: 16 x 800 38.1 / 33.1, 64 x 350 36.4 / 31.1; but 32 x 200 x 1500 47.9 / 55.8; mask
 //     tensor 16 x 600 57.4 / 39.2, 64 x 300 60.1 / 41.9; but 64 x 400 56.7 / 67.1.  64: 16 x 800 27.6 / 19.5, 64 x 350 22.4 / 16.9; but 32 x 200 x 1500 30.9 / 31.6; mask tensor
 //     32 x 200 x 1500 41.7 / 38.1, 32 x 400 27.1 / 20.8; but 16 x 1000 44.3 / 44.4.
+//   * Not at 256 where blocks of 128 queries are many or have few tiles themselves, by estimated times (240 heads x 105 31.5 / 52.6, 80 x 232 x 280 49.5 / 70.2, 32 x 783 window 51 39.8 / 57.0, mask tensor
+//     99 x 93 25.5 / 33.7).  The constants are fitted to 1000 launches; of the 780 that the lines above give to this kernel 122 were slower by more than 4 %, 28 of the 630 that are left.
 inline bool attention_kwave_wanted_f32(int head_dim, bool mask, int64_t heads, int n_q, int n_k, int causal, int diag, int window, int64_t cus)
 {
 	const int64_t groups = (n_q + kKeyWaveRows - 1) / kKeyWaveRows, blocks = heads * groups;
@@ -34,6 +36,8 @@ inline bool attention_kwave_wanted_f32(int head_dim, bool mask, int64_t heads, i
 	const int64_t t_first = attention_block_tiles(0, n_q, n_k, causal, diag, window, kKeyWaveRows, kKeyWaveTile);
 	const int64_t t_last = attention_block_tiles(groups - 1, n_q, n_k, causal, diag, window, kKeyWaveRows, kKeyWaveTile);
 	const int64_t longest = std::max(t_first, t_last);
+	if (head_dim == 256 && !attention_kwave_ahead(mask ? KeyWaveCost{3.95, 0.81, 2.4, 11.4, 1.2, 4.0} : KeyWaveCost{3.91, 0.71, 7.7, 5.5, 0.0, 13.3}, true, heads, n_q, n_k, causal, diag, window,
+	                                              kKeyWaveRows, kKeyWaveTile, cus)) return false;
 	if (blocks <= cus) return longest <= (head_dim == 256 ? (mask ? 34 : 48) : head_dim == 128 && !mask ? 80 : 190);
 	const int64_t cost = blocks * (t_first + t_last + 12) / 2;          // (tiles grow evenly from the first group to the last, but for a window)
 	if (head_dim == 256) return longest <= (mask ? 34 : 60) && cost <= (mask ? 40 : 80) * cus;

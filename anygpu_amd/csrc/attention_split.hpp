@@ -229,6 +229,31 @@ inline int64_t attention_block_tiles(int64_t block, int n_q, int n_k, int causal
 	return key_hi >= 0 && key_hi >= key_lo ? key_hi / keys_per_tile - key_lo / keys_per_tile + 1 : (int64_t)0;
 }
 
+// Key tiles of an average one of `blocks` query blocks, four times: they grow or fall evenly, under a window to or from a plateau.
+template <typename TilesOf>
+inline int64_t four_average_blocks(int64_t blocks, TilesOf tiles_of) { return tiles_of(0) + 2 * tiles_of(blocks / 2) + tiles_of(blocks - 1); }
+
+// What a launch takes beyond its 4 us, us, on blocks of 16 rows whose keys are shared out among their waves: per block and tile of an average block, for one block on each CU; and on
+// blocks of 128 queries: the longest one's start and tiles (of 64 keys), or what the CUs get, per block and tile of an average one.
+struct KeyWaveCost { double block, tile, first, step, block_128, tile_128; };
+
+// Whether blocks of 16 rows with tiles of keys_per_tile keys are ahead of blocks of 128 queries, where there is more than one of them for each CU and the key range is too short for parts of it
+// to go out by themselves.  single: the blocks are one to a CU, so that rounds count.
+inline bool attention_kwave_ahead(const KeyWaveCost& cost, bool single, int64_t heads, int n_q, int n_k, int causal, int diag, int window, int rows, int keys_per_tile, int64_t cus)
+{
+	const int64_t groups = (n_q + rows - 1) / rows, blocks = heads * groups, q_blocks = (n_q + 127) / 128;
+	if (blocks <= cus) return true;
+	const auto tiles_128 = [&](int64_t b) { return attention_block_tiles(b, n_q, n_k, causal, diag, window, 128, 64); };
+	const int64_t longest = std::max(tiles_128(0), tiles_128(q_blocks - 1));
+	// (few blocks of 128 queries go out in parts of the range, most of which a window empties: 8 heads x 1824 x 256 float32, window 53 54.9 / 37.9)
+	if (longest > 16 || (window > 0 && n_k >= 512 && 2 * heads * q_blocks <= cus)) return true;
+	const double average = 0.25 * four_average_blocks(groups, [&](int64_t b) { return attention_block_tiles(b, n_q, n_k, causal, diag, window, rows, keys_per_tile); });
+	const double average_128 = 0.25 * four_average_blocks(q_blocks, tiles_128), shares = (double)blocks / cus;
+	const double rounds = single ? 0.5 * (shares + (blocks + cus - 1) / cus) : shares;
+	return rounds * (cost.block + cost.tile * average) <
+	       std::max(cost.first + cost.step * longest, (double)(heads * q_blocks) / cus * (cost.block_128 + cost.tile_128 * average_128));
+}
+
 // How many of a head's latest query blocks to dispatch in two key halves (and how many unsplit ones go out before the
 // halves).  Worth it when whole blocks cannot be packed evenly: at least a block per CU, and the longest block a large
 // share of what a CU gets of the whole launch.  Bounded by the workspace of the stream (the K-split workspace of the
