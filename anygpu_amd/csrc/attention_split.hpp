@@ -265,7 +265,10 @@ inline bool attention_kwave_ahead(const KeyWaveCost& cost, bool single, int64_t 
 // 136 / 112, 32 / 8 x 1339 67 / 54, 8 / 4 x 6000 window 4096 209 / 170; float32 32 / 8 x 1339 x 256 214 / 192, two per CU 32 / 8 x 3000 x 128 429 / 402).
 // `few`: of the blocks that would be split only as many as pay (half, head dimension 256): those beyond 1.35 of a place's share where the longest is beyond 1.45 (all /
 // whole / here: 8 x 4096 114 / 129 / 111, 8 x 4500 143 / 153 / 140, 16 x 2100 82 / 77 / 75; none at 8 / 4 x 5000 window 4096 162 / 151, 16 x 2600 106 / 96, whose longest are 1.39 and 1.42, nor
-// below 32 tiles: 32 / 16 x 1100 56 / 45), half of the longest ones where it is the second round that does not fit (8 / 4 x 8192 window 4096 278 / 299 / 271).
+// below 32 tiles: 32 / 16 x 1100 56 / 45), half of the longest ones where it is the second round that does not fit: under a window (all / none / here, 8 / 4 heads: 8192 window 4096 281 / 298 / 273, 7940
+// 270 / 289 / 266, 6988 window 3000 205 / 218 / 192, 6180 window 2048 149 / 158 / 138, 5600 window 1536 123 / 123 / 110; none is ahead only at the ends of its range: 4740 window 1024 97 / 78 / 83, 7000
+// window 1536 145 / 129 / 144), and of a chunk of queries against its cache (all / here: 40 / 20 heads x 840 x 2106 125 / 107, 24 / 8 x 1556 x 3725 195 / 183, 16 / 4 x 2005 x 8741 446 / 430, 33 launches that have it 3 % in the
+// mean; but 40 / 10 x 1100 x 5179 293 / 309).
 struct AttnSplitPlan { int64_t n_split, n_big; };
 
 inline AttnSplitPlan plan_attention_split(int n_q, int n_k, int causal, int diag, int window, int64_t batch_heads,

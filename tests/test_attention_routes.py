@@ -101,3 +101,39 @@ def forms(tmp_path_factory):
 
 def test_timed_launches_take_the_faster_kernel(forms):
     assert [(case, got) for (case, _), got in zip(TIMED, forms([case for case, _ in TIMED]))] == TIMED
+
+
+def _launches(test_cases, dtype="f16", mask=RULE, dims=(64, 128), capped=0):
+    """(heads, queries, keys, causal, window) of GPU tests as launches; a window without the causal rule as one with it, which sees fewer keys"""
+    return [(dtype, mask, d, h, n_q, n_k, w if w else CAUSAL if causal else NONE, capped, 0) for h, n_q, n_k, causal, w in test_cases for d in dims]
+
+
+def test_gpu_tests_reach_the_kernels_they_name(forms):
+    def of(*launches, **more):
+        return set(forms(_launches(launches, **more)))
+    # 32 queries per wave, overlapped and in turn
+    assert of((264, 1000, 1000, True, 0), (264, 897, 960, True, 0), (264, 1100, 1161, True, 600), (264, 130, 641, False, 0), (264, 97, 577, True, 0), (512, 900, 900, True, 0)) == {"q32"}
+    assert of((528, 128, 192, True, 0), (528, 256, 256, True, 33), (512, 200, 200, True, 0)) == {"q32 in turn"}
+    # 16 queries per wave
+    sixteen = [(140, 31, 64, True, 0), (140, 127, 129, True, 0), (140, 128, 128, True, 0), (140, 113, 63, False, 0), (120, 129, 257, True, 70), (120, 160, 100, True, 0), (56, 300, 321, False, 0),
+               (64, 257, 600, True, 1), (120, 130, 513, True, 0), (120, 130, 300, False, 0)]
+    assert of(*sixteen) == {"q16"}
+    # 16 rows per block with eight waves and four
+    assert of((4, 40, 257, True, 0), (4, 31, 288, False, 0), (4, 100, 129, True, 33), (4, 130, 97, True, 0), (4, 33, 65, True, 0), (3, 16, 95, False, 0)) == {"rows8"}
+    assert of((160, 40, 257, True, 0), (160, 31, 288, False, 0), (80, 70, 600, False, 0)) == {"rows4"}
+    assert of((4, 17, 17, True, 0), (2, 33, 32, True, 0), (4, 60, 40, True, 0), dims=(256,)) == {"rows8"}
+    assert of((160, 17, 17, True, 0), (160, 40, 257, True, 0), (160, 80, 150, True, 1), dtype="f32") == {"rows4"}
+    # head dimension 256: blocks of 128 queries with many heads
+    from test_gpu_parity import ATTN_D256_CASES
+    many = [(h * (1030 // (h * ((n_q + 15) // 16)) + 1), n_q, n_k, causal, w) for h, _, n_q, n_k, _, _, _, causal, w in ATTN_D256_CASES if n_k < 1500]
+    assert of(*many, (2, 129, 3000, True, 1800), dims=(256,)) == {"skew"}
+    # mask tensors: what they hide, softcap and grouped heads
+    for dtype in ("f16", "f32"):
+        assert of((3, 40, 300, False, 0), (4, 40, 257, False, 0), (6, 17, 130, False, 0), (8, 100, 90, False, 0), dtype=dtype, mask=MASK, dims=(64, 128, 256)) == {"rows8"}
+        assert of((100, 40, 300, False, 0), (160, 40, 300, False, 0), dtype=dtype, mask=MASK) == {"rows4"}
+        assert of((700, 40, 300, False, 0), dtype=dtype, mask=MASK, dims=(64, 128, 256)) == {"blocks"}
+    note = {"f16": [(64, 70, 300, 333), (64, 140, 130, 1500), (128, 48, 300, 300), (128, 96, 130, 700), (256, 26, 300, 301), (256, 30, 130, 1030)],
+            "f32": [(64, 120, 300, 333), (64, 64, 200, 2100), (128, 80, 300, 300), (128, 40, 200, 1500), (256, 24, 300, 301), (256, 4, 150, 1100)]}
+    for dtype, shapes in note.items():
+        for d, *shape in shapes:
+            assert of((*shape, False, 0), dtype=dtype, mask=MASK, dims=(d,)) == {"blocks"}, (dtype, d, shape)

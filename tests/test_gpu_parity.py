@@ -2022,8 +2022,8 @@ def test_sdp_attention_fused_kernel_random_shapes(ops, oracle, dtype):
         assert scaled_rel_err(got[0], want, 1.0) <= tol, case
 
 
-# head_dim 256 runs the kernel that takes S of tile t + 1 beside the softmax of tile t: tile counts of
-# one and two (the pipelined loop body not entered / entered once), a last tile that is not whole, a key range longer
+# head_dim 256: tile counts of one and two of the kernel that takes S of tile t + 1 beside the softmax of tile t (the pipelined loop body not entered / entered once; the few heads
+# of this test run on 16 rows per block up to 48 tiles of 32 keys, many heads of the same shapes in test_gpu_parity_partial_shapes.py on that kernel), a last tile that is not whole, a key range longer
 # than the queries, windows below a tile and without the causal rule, queries without a visible key, grouped heads
 ATTN_D256_CASES = [
     (2, 2, 17, 63, 256, 0.0625, 50.0, True, 0),

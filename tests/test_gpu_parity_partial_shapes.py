@@ -7,7 +7,7 @@ import pytest
 
 from anygpu_amd import synth
 from helpers import exact_int_product, scaled_rel_err
-from test_gpu_parity import TOL_F16_GEMM, TOL_F16_ROWOPS, TOL_F32, dev, hide_key_stripes, host
+from test_gpu_parity import ATTN_D256_CASES, TOL_F16_GEMM, TOL_F16_ROWOPS, TOL_F32, dev, hide_key_stripes, host
 
 pytestmark = pytest.mark.gpu
 
@@ -133,7 +133,7 @@ def test_sdp_attention_f32_mask_tensor_blocks_in_parts_that_fill_the_rounds(ops,
 
 
 # head dimensions 64 and 128 run 32 queries per wave, four waves and 128 queries per block, tiles of 64 keys, where there are more query
-# blocks than CUs (here: 66 copies of four heads), 16 queries per wave in eight waves where there are fewer: one query and
+# blocks than CUs (here: 66 copies of four heads), 16 rows per block or, with a single tile of keys, 16 queries per wave in eight waves where there are few: one query and
 # the edges of a wave's and a block's queries, tiles of one key, one short of whole and whole, queries of a wave that see
 # nothing, and the first and last tile of a window that only some waves of a block see
 @pytest.mark.parametrize("copies", [1, 66])
@@ -196,7 +196,7 @@ def test_sdp_attention_32_queries_per_wave_tiles_overlapped(ops, oracle, n_q, n_
     assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2
 
 
-# the same kernel where the second round of blocks is dispatched backwards: 55 to 76 blocks per XCD, with padding at the end of a head and of the launch
+# the same kernel where the second round of blocks is dispatched backwards: 56 to 66 blocks per XCD (55.5 are just too few), with padding at the end of a head and of the launch
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("copies,heads,kv_heads,n,causal", [(7, 4, 2, 1930, True), (40, 4, 2, 300, True), (37, 4, 2, 300, True), (31, 5, 1, 260, True), (64, 4, 4, 200, False), (33, 4, 2, 510, True)])
 def test_sdp_attention_32_queries_per_wave_second_round_backwards(ops, oracle, copies, heads, kv_heads, n, causal, d):
@@ -207,14 +207,16 @@ def test_sdp_attention_32_queries_per_wave_second_round_backwards(ops, oracle, c
     assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2
 
 
-# launches of few query blocks: 16 rows per block, the tiles of 32 keys shared out among eight waves (up to a block per CU) or four (more: the copies).
+# launches of few query blocks: 16 rows per block, the tiles of 32 keys shared out among eight waves (up to a block per CU) or four (more, at 64 and 128: most of the copies; copies of few keys, and at 64
+# and 128 a single tile of 64 keys, run on the kernels of 128 queries per block).
 # Rows and keys on both sides of 16 and 32, as many tiles as waves and one more, blocks whose window starts behind the first tile,
 # queries that see nothing, and generation steps whose rows of several heads and queries share a block
 @pytest.mark.parametrize("copies", [1, 40])
 @pytest.mark.parametrize("heads,kv_heads,n_q,n_k,causal,window", [(4, 2, 17, 17, True, 0), (4, 1, 16, 31, False, 0), (2, 2, 33, 32, True, 0), (4, 4, 40, 257, True, 0),
                                                                    (4, 2, 31, 288, False, 0), (4, 2, 100, 129, True, 33), (2, 1, 70, 600, False, 64), (4, 2, 60, 40, True, 0),
                                                                    (4, 2, 80, 150, True, 1), (6, 2, 5, 300, True, 0), (8, 4, 1, 256, True, 0), (4, 4, 4, 319, True, 100),
-                                                                   (12, 4, 3, 290, False, 0), (40, 2, 1, 260, True, 0)])
+                                                                   (12, 4, 3, 290, False, 0), (40, 2, 1, 260, True, 0),
+                                                                   (4, 2, 130, 97, True, 0), (4, 4, 33, 65, True, 0), (3, 1, 16, 95, False, 0)])
 @pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 30.0, -0.0884), (256, 0.0, 0.0625), (256, 50.0, 0.0625)])
 def test_sdp_attention_few_rows_keys_over_waves(ops, oracle, heads, kv_heads, n_q, n_k, causal, window, d, cap, alpha, copies):
     q = synth.normal(1 + n_q, (1, heads, n_q, d)).astype(np.float16)
@@ -269,9 +271,10 @@ def test_sdp_attention_f32_few_rows_keys_over_waves(ops, oracle, heads, kv_heads
     assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F32
 
 
-# the long query blocks of a causal launch: at head dimension 256 some in two halves of their keys and some that as long stay whole (2100 keys; two rounds of blocks
-# under a window), all of them (float32), none (1100 and 1339); at 64 and 128 up to one and a third block per CU; sequence ends inside and on a block and a tile
-@pytest.mark.parametrize("dtype,copies,heads,kv_heads,n,window,d", [("f16", 4, 4, 2, 2100, 0, 256), ("f16", 8, 4, 2, 2048, 1024, 256), ("f16", 8, 4, 2, 1100, 0, 256), ("f16", 5, 3, 1, 2111, 1500, 256),
+# the long query blocks of a causal launch: at head dimension 256 those beyond their share in two halves of their keys (2100 keys), half of the longest ones where the second round of blocks does
+# not fit (3108 and 3332 under a window), none (2048 under a window, 1100, 1339; 2111 has fewer blocks than CUs), at 64 and 128 up to one and a third block per CU; in float32 some; sequence
+# ends inside and on a block and a tile
+@pytest.mark.parametrize("dtype,copies,heads,kv_heads,n,window,d", [("f16", 4, 4, 2, 2100, 0, 256), ("f16", 8, 4, 2, 2048, 1024, 256), ("f16", 8, 4, 2, 1100, 0, 256), ("f16", 5, 3, 1, 2111, 1500, 256), ("f16", 4, 4, 2, 3108, 1024, 256), ("f16", 4, 4, 1, 3332, 1536, 256),
                                                                     ("f32", 2, 4, 4, 2100, 0, 256), ("f32", 8, 4, 1, 1339, 0, 256), ("f32", 4, 4, 2, 1536, 1000, 256),
                                                                     ("f16", 4, 4, 2, 2600, 0, 128), ("f16", 4, 4, 2, 2600, 0, 64), ("f16", 4, 4, 2, 2688, 0, 128)])
 def test_sdp_attention_causal_blocks_partly_in_halves(ops, oracle, dtype, copies, heads, kv_heads, n, window, d):
@@ -307,6 +310,80 @@ def test_sdp_attention_mask_tensor_few_rows_keys_over_waves(ops, oracle, heads, 
     assert not got[:, :, ~seen].any() and np.isfinite(got).all()
     tol = TOL_F16_ROWOPS * 2 if dtype == "f16" else TOL_F32
     assert scaled_rel_err(got[:, :3][:, :, seen], want[:, :, seen], 1.0) <= tol
+
+
+# head dimensions 64 and 128, half a block of 128 queries to one for each CU and fewer than ten tiles: 16 queries per wave in eight waves
+@pytest.mark.parametrize("copies,n_q,n_k,causal,window", [(35, 31, 64, True, 0), (35, 127, 129, True, 0), (35, 128, 128, True, 0), (35, 113, 63, False, 0), (30, 129, 257, True, 70), (30, 160, 100, True, 0),
+                                                           (14, 300, 321, False, 64), (16, 257, 600, True, 1), (30, 130, 513, True, 0)])
+@pytest.mark.parametrize("d,cap,alpha", [(64, 0.0, 0.125), (128, 0.0, -0.0884), (64, 30.0, 0.125), (128, 50.0, 0.0884)])
+def test_sdp_attention_16_queries_per_wave(ops, oracle, copies, n_q, n_k, causal, window, d, cap, alpha):
+    heads, kv_heads = 4, 2
+    q = synth.normal(1 + n_q, (1, heads, n_q, d)).astype(np.float16)
+    k = synth.normal(2 + n_k, (1, kv_heads, n_k, d)).astype(np.float16) * np.float16(4.0)        # (scores of tens: the running maximum moves)
+    v = synth.normal(3 + d, (1, kv_heads, n_k, d)).astype(np.float16)
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, softcap=cap, causal=causal, window=window, decode=False)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=alpha, softcap=cap, causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
+    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
+    assert not got[0][blind].any() and np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
+
+
+# head dimension 256 with so many heads that blocks of 128 queries take the launch, whose scores of a tile run beside the softmax of the one before: the shapes of one and two tiles, short last
+# tiles, windows and queries that see nothing that few heads run on 16 rows per block
+@pytest.mark.parametrize("case", [case for case in ATTN_D256_CASES if case[3] < 1500] + [(2, 2, 129, 3000, 256, 0.0625, 0.0, True, 1800)])
+def test_sdp_attention_head_dim_256_many_heads(ops, oracle, case):
+    heads, kv_heads, n_q, n_k, d, alpha, cap, causal, window = case
+    copies = 1030 // (heads * ((n_q + 15) // 16)) + 1 if n_k < 1500 else 1
+    q, k, v = (synth.normal(s + n, (1, h, n, d)).astype(np.float16) for s, h, n in ((1, heads, n_q), (2, kv_heads, n_k), (3, kv_heads, n_k)))
+    got = host(ops.sdp_attention_fwd(*(dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)), alpha, softcap=cap, causal=causal, window=window, decode=False)).astype(np.float32)
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=alpha, softcap=cap, causal=causal, window=window, q_per_kv=heads // kv_heads, threads=8)
+    blind = ~np.isfinite(want).all(axis=-1)                      # queries without a visible key: zeros
+    assert not got[0][blind].any() and np.isfinite(got).all()
+    assert np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+    assert scaled_rel_err(got[0][~blind], want[~blind], 1.0) <= TOL_F16_ROWOPS * 2
+
+
+# alpha 0 without a softcap: the mean of the visible values, on every kernel (16 rows per block, 16 and 32 queries per wave, head dimension 256, float32 in either form), and nothing of the hidden ones
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("heads,n", [(4, 100), (60, 300), (160, 130), (512, 200), (300, 700)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_sdp_attention_alpha_zero(ops, heads, n, d, dtype):
+    import torch
+    q, k, v = (dev(synth.normal(s, (1, 4, n, d)).astype(np.float16 if dtype == "f16" else np.float32)).repeat(1, heads // 4, 1, 1) for s in (1, 2, 3))
+    got = host(ops.sdp_attention_fwd(q, k, v, 0.0, causal=True, window=90)).astype(np.float64)
+    sums = np.cumsum(np.concatenate([np.zeros((4, 1, d)), host(v[0, :4]).astype(np.float64)], axis=1), axis=1)
+    at = np.arange(1, n + 1)
+    lo = np.maximum(at - 90, 0)
+    want = (sums[:, at] - sums[:, lo]) / (at - lo)[None, :, None]
+    assert scaled_rel_err(got[0, :4], want, 1.0) <= (2.0 ** -10 if dtype == "f16" else TOL_F32)
+    assert np.array_equal(got[0].reshape(-1, 4, n, d), np.broadcast_to(got[:, :4], (heads // 4, 4, n, d)))
+
+
+# a mask tensor with softcap (logits capped before the mask is added) and grouped heads, which only the C entry points take: 16 rows per block with eight waves and with four, 128 queries per block
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("heads,q_per_kv,n_q,n_k", [(4, 2, 40, 257), (6, 3, 17, 130), (160, 4, 40, 300), (8, 8, 100, 90), (200, 2, 100, 200)])
+@pytest.mark.parametrize("d,cap,alpha", [(64, 30.0, 0.3), (128, 0.0, 0.0884), (128, 50.0, 0.2), (256, 30.0, 0.2), (256, 0.0, 0.0625)])
+def test_sdp_attention_mask_tensor_softcap_and_grouped_heads(ops, heads, q_per_kv, n_q, n_k, d, cap, alpha, dtype):
+    import torch
+    from anygpu_amd import capi
+    from test_gpu_attention_f32_parts import attend64
+    ndt = np.float16 if dtype == "f16" else np.float32
+    q, k, v = (synth.normal(s + n, (h, n, d)).astype(ndt) for s, h, n in ((1, heads, n_q), (2, heads // q_per_kv, n_k), (3, heads // q_per_kv, n_k)))
+    mask = synth.normal(7, (n_q, n_k), std=2.0).astype(ndt)
+    mask[synth.normal(8, (n_q, n_k)) > 0.5] = -np.inf
+    mask[:, 64:96] = -np.inf
+    mask[n_q // 2] = -np.inf                                     # sees nothing: zeros
+    dq, dk, dv, dm = (dev(t) for t in (q, k, v, mask))
+    y = torch.full_like(dq, 9.0)
+    fn = getattr(capi.load(), f"anygpu_sdp_attention_fwd_masked_{dtype}")
+    assert fn(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dm.data_ptr(), y.data_ptr(), heads, q_per_kv, n_q, n_k, d, n_k, alpha, cap, None) == capi.ANYGPU_OK
+    got, bias = host(y).astype(np.float64), mask.astype(np.float64)
+    some = sorted({0, 1, heads // 2, heads - 1})
+    want = np.stack([attend64(q[h:h + 1], k[h // q_per_kv:h // q_per_kv + 1], v[h // q_per_kv:h // q_per_kv + 1], alpha, cap, bias=bias)[0] for h in some])
+    assert not got[:, n_q // 2].any() and np.isfinite(got).all()
+    # (float32: logits of up to about 20 carry the hardware exponential's 2^-22 of themselves into the weights)
+    assert scaled_rel_err(got[some], want, 1.0) <= (TOL_F16_ROWOPS * 2 if dtype == "f16" else TOL_F32)
 
 
 # what a mask tensor hides from all queries of a wave (whole tiles of 64 keys) takes no part in their results, whatever it holds: the tail of a padded cache,
@@ -364,7 +441,7 @@ def test_sdp_attention_few_rows_nothing_behind_the_last_key(ops, n_k, d, dtype):
 # sizes that get one by default, ragged last tiles and blocks, queries that see nothing, mask rows at an odd pitch; and the launches of few query blocks, which have none while
 # the variable is not set
 @pytest.mark.parametrize("dtype,d,heads,n_q,n_k,kind", [("f16", 64, 70, 300, 333, "slide"), ("f16", 64, 140, 130, 1500, "stripes"), ("f16", 128, 48, 300, 300, "blind rows"), ("f16", 128, 96, 130, 700, "odd stride"),
-                                                        ("f16", 256, 26, 300, 301, "slide"), ("f16", 256, 26, 130, 1030, "stripes"), ("f32", 64, 120, 300, 333, "slide"), ("f32", 64, 64, 200, 2100, "stripes"),
+                                                        ("f16", 256, 26, 300, 301, "slide"), ("f16", 256, 30, 130, 1030, "stripes"), ("f32", 64, 120, 300, 333, "slide"), ("f32", 64, 64, 200, 2100, "stripes"),
                                                         ("f32", 128, 80, 300, 300, "blind rows"), ("f32", 128, 40, 200, 1500, "odd stride"), ("f32", 256, 24, 300, 301, "slide"), ("f32", 256, 4, 150, 1100, "stripes")])
 def test_sdp_attention_mask_tensor_with_and_without_note(ops, oracle, monkeypatch, dtype, d, heads, n_q, n_k, kind):
     import torch
@@ -477,10 +554,10 @@ def test_sdp_attention_32_queries_per_wave_moving_maximum(ops, d, step):
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("alpha", [1.0, -1.0])
-@pytest.mark.parametrize("heads", [4, 512])
+@pytest.mark.parametrize("heads", [4, 120, 512])
 def test_sdp_attention_scores_beyond_the_mantissa(ops, d, alpha, heads):
     # scores of 10^9 and more, whose rounding as a float is larger than the halves' range of exponents: still the row of the key
-    # with the largest score, bit for bit (16 queries per wave with few heads, 32 with many)
+    # with the largest score, bit for bit (16 rows per block with few heads, 16 queries per wave with 120, 32 with 512)
     import torch
     n = 300
     order = np.random.default_rng(6).permutation(n)
