@@ -1353,9 +1353,8 @@ bool attention_split_wanted(const AttnArgsF32& args, int64_t batch_heads)
 	else return D == 256 || (args.n_k >= 350 && (D == 128 || args.n_q > 128) && attention_split_fills<D>(args, batch_heads));
 }
 
-// `heads` of `rows` rows each, `per_kv` of them on one key / value head
 template <int D, bool SOFTCAP, bool MASK, int WAVES>
-hipError_t launch_kwave_variant_f32(const AttnArgsF32& args, int64_t heads, int64_t rows, int64_t per_kv, hipStream_t stream)
+hipError_t launch_kwave_variant_f32(const AttnArgsF32& args, int64_t batch_heads, hipStream_t stream)
 {
 	constexpr int kLdsBytes = kKeyWaveLdsBytes<D, WAVES>;
 	const auto kernel = sdp_attention_fwd_f32_kwave_kernel<D, SOFTCAP, MASK, WAVES>;
@@ -1363,20 +1362,20 @@ hipError_t launch_kwave_variant_f32(const AttnArgsF32& args, int64_t heads, int6
 	static std::atomic<uint64_t> configured_devices{0};
 	const hipError_t lds_err = grant_lds(kernel, kLdsBytes, configured_devices);
 	if (lds_err != hipSuccess) return lds_err;
-	const AttnWalk walk = make_attn_walk((rows + kKeyWaveRows - 1) / kKeyWaveRows, heads, per_kv);
+	const AttnWalk walk = make_attn_walk((args.n_q + kKeyWaveRows - 1) / kKeyWaveRows, batch_heads, args.q_per_kv);
 	if (attn_walk_blocks(walk) > 0x7FFFFFFFLL) return hipErrorInvalidValue;
-	kernel<<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * WAVES), kLdsBytes, stream>>>(args, walk, (int)rows);
+	kernel<<<dim3((unsigned)attn_walk_blocks(walk)), dim3(64 * WAVES), kLdsBytes, stream>>>(args, walk);
 	return hipGetLastError();
 }
 
 template <int D, bool SOFTCAP, bool MASK>
-hipError_t launch_kwave_f32(const AttnArgsF32& args, int64_t heads, int64_t rows, int64_t per_kv, hipStream_t stream)
+hipError_t launch_kwave_f32(const AttnArgsF32& args, int64_t batch_heads, hipStream_t stream)
 {
 	if constexpr (D != 256)
 	{
-		if (heads * ((rows + kKeyWaveRows - 1) / kKeyWaveRows) > device_cu_count()) return launch_kwave_variant_f32<D, SOFTCAP, MASK, 4>(args, heads, rows, per_kv, stream);
+		if (batch_heads * ((args.n_q + kKeyWaveRows - 1) / kKeyWaveRows) > device_cu_count()) return launch_kwave_variant_f32<D, SOFTCAP, MASK, 4>(args, batch_heads, stream);
 	}
-	return launch_kwave_variant_f32<D, SOFTCAP, MASK, 8>(args, heads, rows, per_kv, stream);
+	return launch_kwave_variant_f32<D, SOFTCAP, MASK, 8>(args, batch_heads, stream);
 }
 
 template <int D, bool SOFTCAP, bool MASK>
@@ -1388,7 +1387,7 @@ hipError_t launch_variant_f32(const AttnArgsF32& args_in, int64_t batch_heads, h
 	args.map_words = 0;
 	if (!(MASK && attention_mask_map_set()) &&
 	    attention_kwave_wanted_f32(D, MASK, batch_heads, args.n_q, args.n_k, args.causal, args.diag, args.window, device_cu_count()))
-		return launch_kwave_f32<D, SOFTCAP, MASK>(args, batch_heads, args.n_q, args.q_per_kv, stream);
+		return launch_kwave_f32<D, SOFTCAP, MASK>(args, batch_heads, stream);
 	const bool split = attention_split_wanted<D, MASK>(args, batch_heads);
 	if constexpr (!MASK) return split ? launch_split_f32<D, SOFTCAP, false>(args, batch_heads, stream) : launch_plain_f32<D, SOFTCAP, false>(args, batch_heads, stream);
 	else

@@ -48,10 +48,9 @@ inline bool attention_kwave_wanted_f32(int head_dim, bool mask, int64_t heads, i
 template <int D, int WAVES>
 constexpr int kKeyWaveLdsBytes = (WAVES * kKeyWaveTile + kKeyWaveRows) * (D + 8) * 4;
 
-// `walk`: blocks of 16 rows of a "head" of `rows` rows; row r is query r % n_q (rows = n_q, or where a key / value head's rows are
-// taken together, q_per_kv * n_q with fewer than 16 queries).  MASK: an additive mask tensor instead of the index rules.
+// `walk`: blocks of 16 queries of a head.  MASK: an additive mask tensor instead of the index rules.
 template <int D, bool SOFTCAP, bool MASK, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void sdp_attention_fwd_f32_kwave_kernel(const AttnArgsF32 a, const AttnWalk walk, int rows)
+__global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void sdp_attention_fwd_f32_kwave_kernel(const AttnArgsF32 a, const AttnWalk walk)
 {
 	constexpr int ROWS = kKeyWaveRows, THREADS = 64 * WAVES, KT = kKeyWaveTile;
 	constexpr int kPitch = D + 8, kPitchO = D + 4;       // floats
@@ -67,19 +66,17 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	float* const lds = lds_all + wave * (KT * kPitch);
 	int head, group;
 	if (!attn_walk_locate(walk, blockIdx.x, head, group)) return;      // the whole block
-	const float* qp = a.q + (int64_t)head * rows * D;
-	const float* kp = a.k + (int64_t)(head / walk.q_per_kv) * a.n_k * D;
-	const float* vp = a.v + (int64_t)(head / walk.q_per_kv) * a.n_k * D;
-	float* yp = a.y + (int64_t)head * rows * D;
+	const float* qp = a.q + (int64_t)head * a.n_q * D;
+	const float* kp = a.k + (int64_t)(head / a.q_per_kv) * a.n_k * D;
+	const float* vp = a.v + (int64_t)(head / a.q_per_kv) * a.n_k * D;
+	float* yp = a.y + (int64_t)head * a.n_q * D;
 
-	// the visible keys of the block: of its first and last query, or of all queries where rows of several heads are together
-	const int row0 = ROWS * group;
-	const bool one_head = rows == a.n_q;
-	const int q_first = one_head ? row0 : 0, q_last = one_head && row0 + ROWS < a.n_q ? row0 + ROWS - 1 : a.n_q - 1;
+	// the visible keys of the block: of its first and last query
+	const int row0 = ROWS * group, q_last = row0 + ROWS < a.n_q ? row0 + ROWS - 1 : a.n_q - 1;
 	int key_hi = a.n_k - 1;
 	if (a.causal && q_last + a.diag < key_hi) key_hi = q_last + a.diag;
 	int key_lo = 0;
-	if (a.window > 0 && q_first + a.diag - a.window + 1 > 0) key_lo = q_first + a.diag - a.window + 1;
+	if (a.window > 0 && row0 + a.diag - a.window + 1 > 0) key_lo = row0 + a.diag - a.window + 1;
 	const int u_first = key_lo / KT, u_last = key_hi >= 0 ? key_hi / KT : -1;
 
 	// K passes through LDS (1 KB of consecutive memory per load), V is fetched as it is needed: four columns of four rows per lane, 256
@@ -103,7 +100,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 			for (int c = 0; c < DC; ++c)
 				vr[r][c] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, g * (16 * D) + n * 16, r * (4 * D) + c * 256, 0));
 	};
-	const int q_idx = one_head ? row0 + n : (row0 + n) % a.n_q;
+	const int q_idx = row0 + n;
 	// MASK: the values of this lane's scores of a tile, four consecutive floats at any alignment; in the last tile keys past the end read
 	// nothing (their scores are masked)
 	float4_t mk = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -131,7 +128,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	for (int i = 0; i < kQVecs; ++i)
 	{
 		const int idx = tid + THREADS * i;
-		if (idx < ROWS * VPR) q_vec[i] = *reinterpret_cast<const float4_t*>(qp + (int64_t)min(row0 + idx / VPR, rows - 1) * D + (idx % VPR) * 4);
+		if (idx < ROWS * VPR) q_vec[i] = *reinterpret_cast<const float4_t*>(qp + (int64_t)min(row0 + idx / VPR, a.n_q - 1) * D + (idx % VPR) * 4);
 	}
 	__builtin_amdgcn_sched_barrier(0);
 	int u = u_first + wave;
@@ -263,7 +260,7 @@ __global__ __launch_bounds__(64 * WAVES, D == 256 ? 2 : D == 128 ? 3 : 4) void s
 	for (int i = tid; i < ROWS * VPR; i += THREADS)
 	{
 		const int r = i / VPR, quad = i % VPR;
-		if (row0 + r >= rows) continue;
+		if (row0 + r >= a.n_q) continue;
 		float big = row_max[0][r];
 		for (int w = 1; w < waves; ++w) big = fmaxf(big, row_max[w][r]);
 		const float safe = big == -INFINITY ? 0.0f : big;
