@@ -3,7 +3,8 @@
 // The kernels with 128 queries per block leave most CUs idle on a prompt of a few hundred tokens, and the block that has the most keys walks them alone
 // (8 heads x 394 x 256: 32 blocks, seven tiles of 64 keys at 2.7 us each).  Here every 16 rows are a block, and its four or eight waves take tiles of 32 keys in turn,
 // each with its own running maximum, without a barrier; their results meet in LDS.  One launch, no workspace.
-// What bounds it: the rate at which a CU fetches, since every 16 rows read their keys again.  Rows of K and of the queries fetched straight in operand
+// What bounds it: a block's chain of queries, first tile, some tiles per wave and the meeting of the waves (matrix cores busy 3 - 6 %, 9 - 14 bytes fetched per clock and CU over the launch), and in
+// it the rate at which a CU fetches, since every 16 rows read their keys again.  Rows of K and of the queries fetched straight in operand
 // layout (16 rows x 64 bytes an instruction) come at 16 bytes per clock and CU, 1 KB of consecutive memory at 55 - 60 (all CUs at once, out of the L2s), so
 // K passes through LDS like V, through the same wave-private tile, and the queries are fetched once per block (8 heads x 394 x 256 14.9 us with both
 // in operand layout, 11.5 now).  A tile of K and V is requested while the one before is used.  Eight waves hide the latency where blocks are at most one to a CU; with more of
