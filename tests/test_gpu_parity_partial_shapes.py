@@ -196,6 +196,31 @@ def test_sdp_attention_32_queries_per_wave_tiles_overlapped(ops, oracle, n_q, n_
     assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2
 
 
+# a window over a long cache: blocks of two or three tiles, products and softmax in turn, in parts of the range that the window leaves mostly empty, and whole without a workspace for them
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("cap", [0.0, 30.0])
+def test_sdp_attention_32_queries_per_wave_short_window_in_parts(ops, oracle, d, cap):
+    import torch
+    copies, heads, n_q, n_k, window = (40 if d == 64 else 65), 4, 200, 6000, 100        # one and a quarter and two rounds of blocks, cut into three and two parts
+    q, k, v = (synth.normal(80 + i, (1, heads, n, d)).astype(np.float16) for i, n in enumerate((n_q, n_k, n_k)))
+    args = [dev(t).repeat(copies, 1, 1, 1) for t in (q, k, v)]
+
+    def run(workspace_bytes):
+        workspace = torch.empty((workspace_bytes,), dtype=torch.uint8, device="cuda")
+        ops.set_workspace(workspace)
+        try:
+            return host(ops.sdp_attention_fwd(*args, d ** -0.5, softcap=cap, causal=True, window=window, decode=False)).astype(np.float32)
+        finally:
+            torch.cuda.synchronize()
+            ops.set_workspace(None)
+    parts, whole = run(160 << 20), run(256)
+    assert not np.array_equal(parts, whole), "the launch was expected to take parts of the key range"
+    want = oracle.sdp_attention_rules(*(oracle.cvt_f16_to_f32(t)[0] for t in (q, k, v)), alpha=d ** -0.5, softcap=cap, causal=True, window=window, q_per_kv=1, threads=8)
+    for got in (parts, whole):
+        assert np.isfinite(got).all() and np.array_equal(got, np.broadcast_to(got[:1], got.shape))
+        assert scaled_rel_err(got[0], want, 1.0) <= TOL_F16_ROWOPS * 2
+
+
 # the same kernel where the second round of blocks is dispatched backwards: 56 to 66 blocks per XCD (55.5 are just too few), with padding at the end of a head and of the launch
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("copies,heads,kv_heads,n,causal", [(7, 4, 2, 1930, True), (40, 4, 2, 300, True), (37, 4, 2, 300, True), (31, 5, 1, 260, True), (64, 4, 4, 200, False), (33, 4, 2, 510, True)])
